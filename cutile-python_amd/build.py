@@ -19,7 +19,10 @@ CSRC = ROOT / "csrc"
 INCLUDE = ROOT.parent / "include"
 OUT = ROOT / "cutile_amd" / "libmxgemm.so"
 OBJ = ROOT / "build"
-SOURCES = ["mx_api.hip", "mx_gemm_mfma.hip", "mx_gemm_pp.hip", "mx_gemm_pp32.hip", "mx_gemm_w4.hip", "mx_gemm_generic.hip", "mx_gemm_decode.hip", "mx_aux.hip", "mx_probe.hip"]
+SOURCES = ["mx_api.hip", "mx_gemm_mfma.hip", "mx_gemm_pp32.hip", "mx_gemm_w4.hip", "mx_gemm_generic.hip", "mx_gemm_decode.hip", "mx_aux.hip", "mx_probe.hip"]
+# sources compiled once per value of a macro, so that their instances build in parallel: (file, macro, count)
+SPLIT = [("mx_gemm_pp.hip", "MX_PP_PAIR", 4)]
+UNITS = [(s, None) for s in SOURCES] + [(f, f"-D{m}={i}") for f, m, n in SPLIT for i in range(n)]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          f"-I{INCLUDE}", f"-I{CSRC}", "-Wno-unused-command-line-argument"]
@@ -45,11 +48,12 @@ def _flags_changed() -> bool:
     return True
 
 
-def _compile(src: str, force: bool) -> pathlib.Path:
+def _compile(unit, force: bool) -> pathlib.Path:
+    src, define = unit
     s = CSRC / src
-    o = OBJ / (s.stem + ".o")
+    o = OBJ / (s.stem + (define.replace("=", "_").replace("-D", "_") if define else "") + ".o")
     if force or _newer(s, o):
-        cmd = ["hipcc", *FLAGS, "-c", str(s), "-o", str(o)]
+        cmd = ["hipcc", *FLAGS, *([define] if define else []), "-c", str(s), "-o", str(o)]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")
@@ -59,9 +63,9 @@ def _compile(src: str, force: bool) -> pathlib.Path:
 def build(force: bool = False, jobs: int | None = None) -> pathlib.Path:
     OBJ.mkdir(exist_ok=True)
     force = _flags_changed() or force
-    jobs = jobs or min(len(SOURCES), os.cpu_count() or 4, 8)
+    jobs = jobs or min(len(UNITS), os.cpu_count() or 4, 8)
     with ThreadPoolExecutor(jobs) as ex:
-        objs = list(ex.map(lambda s: _compile(s, force), SOURCES))
+        objs = list(ex.map(lambda u: _compile(u, force), sorted(UNITS, key=lambda u: u[1] is None)))
     (OBJ / "flags.txt").write_text(" ".join(FLAGS))
     cmd = ["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(OUT), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)

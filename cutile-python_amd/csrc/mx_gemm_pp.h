@@ -74,4 +74,8 @@ inline int64_t pp_grid(int M, int N, int K, int ksub) {
   return (can_walk && tiles > num_cus()) ? num_cus() : tiles;
 }
 
+// the ping-pong kernels of one element-format pair (mx_gemm_pp.hip, compiled once per pair)
+template <int AF, int BF>
+int launch_pp_pair(const GemmArgs& g, hipStream_t stream);
+
 }  // namespace mx

@@ -167,4 +167,60 @@ __device__ inline void store8_full<uint16_t>(uint16_t* p, const v4f& v0, const v
   *(u4*)p = w;
 }
 
+// Eight consecutive outputs (two accumulator quads) of which the first `nvalid` (>= 1) exist, at any element alignment.
+// A whole group is one 16-byte store for bf16 (two for fp32): global memory takes dwordx4 stores at any byte address.
+// A partial one is taken apart into a 4-, a 2- and a 1-element store, so a lane never issues more than three.
+typedef uint32_t u4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u2_any __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u1_any __attribute__((aligned(2)));
+
+template <typename OutT>
+__device__ inline void store8_edge(OutT* p, const v4f& v0, const v4f& v1, int nvalid);
+
+template <>
+__device__ inline void store8_edge<uint16_t>(uint16_t* p, const v4f& v0, const v4f& v1, int nvalid) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  const uint32_t x = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){v0.x, v0.y}, b2));
+  const uint32_t y = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){v0.z, v0.w}, b2));
+  const uint32_t z = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){v1.x, v1.y}, b2));
+  const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){v1.z, v1.w}, b2));
+  if (nvalid >= 8) {
+    *(u4_any*)p = (u4_any){x, y, z, w};
+  } else if (nvalid > 0) {
+    if (nvalid & 4) *(u2_any*)p = (u2_any){x, y};
+    if (nvalid & 2) *(u1_any*)(p + (nvalid & 4)) = nvalid & 4 ? z : x;
+    if (nvalid & 1) p[nvalid & 6] = (uint16_t)(nvalid & 4 ? (nvalid & 2 ? w : z) : (nvalid & 2 ? y : x));
+  }
+}
+
+template <>
+__device__ inline void store8_edge<float>(float* p, const v4f& v0, const v4f& v1, int nvalid) {
+  typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+  typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
+  if (nvalid >= 8) {
+    *(f4*)p = v0;
+    *(f4*)(p + 4) = v1;
+  } else if (nvalid > 0) {
+    if (nvalid & 4) *(f4*)p = v0;
+    if (nvalid & 2) *(f2*)(p + (nvalid & 4)) = nvalid & 4 ? (f2){v1.x, v1.y} : (f2){v0.x, v0.y};
+    if (nvalid & 1) p[nvalid & 6] = nvalid & 4 ? (nvalid & 2 ? v1.z : v1.x) : (nvalid & 2 ? v0.z : v0.x);
+  }
+}
+
+// what C holds already, added to the group that store8_edge is about to write
+template <typename OutT>
+__device__ inline void add8_edge(const OutT* p, v4f& v0, v4f& v1, int nvalid) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float old = 0.f;
+    if (e < nvalid) {
+      if constexpr (sizeof(OutT) == 4) old = p[e];
+      else old = bf16_to_f32(p[e]);
+    }
+    if (e < 4) v0[e] += old;
+    else v1[e - 4] += old;
+  }
+}
+
 }  // namespace mx
