@@ -8,6 +8,7 @@ cutile-python_amd/cutile_amd/libmxgemm.so.  hipcc cross-compiles: no GPU is need
 from __future__ import annotations
 
 import argparse
+import importlib.util
 import os
 import pathlib
 import subprocess
@@ -18,6 +19,7 @@ ROOT = pathlib.Path(__file__).resolve().parent
 CSRC = ROOT / "csrc"
 INCLUDE = ROOT.parent / "include"
 OUT = ROOT / "cutile_amd" / "libmxgemm.so"
+HOST_OUT = ROOT / "cutile_amd" / "_mxhost.so"   # csrc/mx_host.cpp: the operators' native host path
 OBJ = ROOT / "build"
 SOURCES = ["mx_api.hip", "mx_gemm_mfma.hip", "mx_gemm_pp32.hip", "mx_gemm_w4.hip", "mx_gemm_generic.hip", "mx_gemm_decode.hip", "mx_aux.hip", "mx_probe.hip"]
 # sources compiled once per value of a macro, so that their instances build in parallel: (file, macro, count)
@@ -60,12 +62,31 @@ def _compile(unit, force: bool) -> pathlib.Path:
     return o
 
 
+def _build_host(force: bool) -> None:
+    """The native host path of the Python operators: host code only, against the torch that will load it."""
+    import sysconfig
+    spec = importlib.util.find_spec("torch")   # torch's place, without importing it
+    torch_dir = pathlib.Path(spec.submodule_search_locations[0])
+    src, rocm = CSRC / "mx_host.cpp", pathlib.Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    if not force and not _newer(src, HOST_OUT):
+        return
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-I{INCLUDE}", f"-I{rocm / 'include'}", f"-I{torch_dir / 'include'}",
+           f"-I{torch_dir / 'include/torch/csrc/api/include'}", f"-I{sysconfig.get_paths()['include']}", "-o", str(HOST_OUT),
+           str(src), f"-L{torch_dir / 'lib'}", "-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for {src.name}:\n{r.stdout}\n{r.stderr}")
+
+
 def build(force: bool = False, jobs: int | None = None) -> pathlib.Path:
     OBJ.mkdir(exist_ok=True)
     force = _flags_changed() or force
     jobs = jobs or min(len(UNITS), os.cpu_count() or 4, 8)
     with ThreadPoolExecutor(jobs) as ex:
+        host = ex.submit(_build_host, force)
         objs = list(ex.map(lambda u: _compile(u, force), sorted(UNITS, key=lambda u: u[1] is None)))
+        host.result()
     (OBJ / "flags.txt").write_text(" ".join(FLAGS))
     cmd = ["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(OUT), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)

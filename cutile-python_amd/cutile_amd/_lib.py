@@ -114,6 +114,28 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The native host path (module ``_mxhost``, csrc/mx_host.cpp) bound to the library that :func:`lib` loaded.
+    Like the library itself it has no fallback: without it nothing runs."""
+    global _host
+    if _host is None:
+        h = lib()
+        with _lock:
+            if _host is None:
+                try:
+                    from . import _mxhost
+                except ImportError as e:
+                    raise MXLibraryError(f"{_HERE / '_mxhost.so'} cannot be loaded ({e}): build it with "
+                                         "`python cutile-python_amd/build.py`.") from e
+                from .ops import PackedScales
+                _mxhost.bind(h._handle, PackedScales)
+                _host = _mxhost
+    return _host
+
+
 def last_error() -> str:
     return lib().mx_last_error().decode("utf-8", "replace")
 
@@ -145,4 +167,4 @@ def desc(t: torch.Tensor, mx_dtype: int, packed_dim: int = -1) -> MxTensor:
 
 
 def stream_ptr(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)

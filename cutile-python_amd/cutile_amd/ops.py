@@ -1,7 +1,9 @@
 """Host-side mirror of the reference's block-scaled matmul interface, on PyTorch-ROCm tensors.
 
 Every function validates like its reference counterpart (same argument order, same error
-classes and messages) and then calls libmxgemm.so through ctypes on the current HIP stream.
+classes and messages) and then calls libmxgemm.so on the current HIP stream.  Ordinary calls of the hot
+operators go through the native module ``_mxhost`` (csrc/mx_host.cpp), which declines whatever it does not
+know before anything is enqueued; such calls are validated here and go through ctypes.
 PyTorch is used for device memory and streams only; there is no PyTorch or CPU compute
 fallback: if the library is missing, calls raise.
 
@@ -58,6 +60,13 @@ def _check(rc: int):
         # cext/tile_kernel.cpp:3910-3916
         raise RuntimeError(f"Failed to launch mxgemm kernel: {msg}")
     raise RuntimeError(msg)
+
+
+def _raise_code(rc: int):
+    """Raises for the error code a native operator returned."""
+    if rc == L.MX_ERR_WORKSPACE:
+        raise ValueError(L.last_error())
+    _check(rc)
 
 
 def _dtype_name(dt) -> str:
@@ -167,9 +176,31 @@ class _ScaleCache:
         self._lock = threading.Lock()
         self._entries = collections.OrderedDict()   # key -> (weakref to base, version, PackedScales, event, stream)
 
+        # the same copies by scale tensor object: (id(tensor), transposed) -> (weakref to it, version, stream,
+        # PackedScales, key into _entries).  A repeated call with the same object costs a dictionary look-up this way
+        # instead of building a key from its base, shape and strides.
+        self._by_object = {}
+
     def clear(self):
         with self._lock:
             self._entries.clear()
+            self._by_object.clear()
+
+    def lookup_object(self, s: torch.Tensor, transposed: bool, stream: int) -> Optional[PackedScales]:
+        e = self._by_object.get((id(s), transposed))
+        if e is None or e[0]() is not s or e[1] != s._version or e[2] != stream:
+            return None
+        with self._lock:
+            if e[4] in self._entries:
+                self._entries.move_to_end(e[4])
+        return e[3]
+
+    def _remember_object(self, s, transposed, version, stream, packed, key):   # under the lock
+        if len(self._by_object) >= 2 * self.max_entries:   # views that are gone, entries that were dropped
+            self._by_object = {k: v for k, v in self._by_object.items() if v[0]() is not None and v[4] in self._entries}
+            if len(self._by_object) >= 2 * self.max_entries:
+                self._by_object.clear()
+        self._by_object[(id(s), transposed)] = (weakref.ref(s), version, stream, packed, key)
 
     def lookup(self, s: torch.Tensor, transposed: bool) -> PackedScales:
         base = s._base if s._base is not None else s
@@ -184,6 +215,8 @@ class _ScaleCache:
                     # the copy belongs to the allocator pool of that stream: tell it that this one reads it too,
                     # so that dropping the entry while this stream's GEMM is in flight does not recycle the block
                     e[2].data.record_stream(stream)
+                else:
+                    self._remember_object(s, transposed, base._version, stream.cuda_stream, e[2], key)
                 return e[2]
         packed = pack_scales(s, transposed=transposed, operand="b" if transposed else "a")
         if torch.cuda.is_current_stream_capturing():
@@ -197,6 +230,7 @@ class _ScaleCache:
                 del self._entries[k]
             while len(self._entries) > self.max_entries:
                 self._entries.popitem(last=False)
+            self._by_object = {k: v for k, v in self._by_object.items() if v[4] in self._entries}
         return packed
 
 
@@ -358,6 +392,19 @@ def block_scaled_matmul(A: torch.Tensor, A_scale, B: torch.Tensor, B_scale, *,
     it while that tensor object lives and torch has not written to it (``_version``), so that repeated calls with
     the same weights launch the GEMM kernel only; :func:`clear_scale_cache` drops the copies.
     """
+    code = L.KERNELS.get(kernel)
+    if code is not None and not static_scratch:
+        As_n, Bs_n = A_scale, B_scale
+        if cache_scales and A.is_cuda and isinstance(A_scale, torch.Tensor) and isinstance(B_scale, torch.Tensor):
+            stream = L.stream_ptr(A.device)
+            As_n = _SCALE_CACHE.lookup_object(A_scale, False, stream)
+            Bs_n = _SCALE_CACHE.lookup_object(B_scale, True, stream)
+        if not cache_scales or (As_n is not None and Bs_n is not None and kernel != "generic"):
+            r = L.host().gemm(A, As_n, B, Bs_n, C, out_dtype, a_format, b_format, accumulate, code, split_k)
+            if isinstance(r, torch.Tensor):
+                return r
+            if r is not None and not cache_scales:   # (a problem of the general kernel refuses the cached layout: below)
+                _raise_code(r)
     a_fmt, b_fmt = _elem_format(A, a_format), _elem_format(B, b_format)
     if a_fmt is None or b_fmt is None:
         bad = A if a_fmt is None else B
@@ -404,6 +451,13 @@ def grouped_block_scaled_matmul(As, A_scales, Bs, B_scales, *, out_dtype: torch.
     ``grouped_matmul_kernel(As, Bs, Cs, ...)`` (test/kernels/group_gemm.py:10-38, driven as in
     test/test_group_gemm.py).  Every problem follows the rules of :func:`block_scaled_matmul`; all are
     enqueued by one library call on the current stream.  Returns the list of outputs."""
+    code = L.KERNELS.get(kernel)
+    if code is not None:
+        r = L.host().gemm_list(As, A_scales, Bs, B_scales, Cs, out_dtype, code)
+        if isinstance(r, list):
+            return r
+        if r is not None:
+            _raise_code(r)
     n = len(As)
     if not (len(A_scales) == len(Bs) == len(B_scales) == n) or (Cs is not None and len(Cs) != n):
         raise ValueError("As, A_scales, Bs, B_scales (and Cs) must be lists of the same length")
@@ -564,6 +618,12 @@ def block_quantize(x: torch.Tensor, block_size: int = 32, dtype=torch.float8_e4m
     scale_mode "ceil": the reference's rule 2^ceil(log2(max(amax/448, 1e-12))) with a non-saturating
     cast; "floor": the OCP MX rule 2^(floor(log2 amax) - emax_elem) with a saturating cast.
     """
+    if block_size == 32 and scale_mode in ("floor", "ceil"):
+        r = L.host().quantize(x, dtype, 1 if scale_mode == "floor" else 0, False)
+        if type(r) is tuple:
+            return r
+        if r is not None:
+            _check(r)
     if block_size != 32:
         raise TileValueError(f"only the MX block size 32 is supported by the quantiser, got {block_size}")
     if x.shape[-1] < block_size:
@@ -762,6 +822,11 @@ def silu_and_mul_quantize(gate_up: torch.Tensor, dtype=torch.float8_e4m3fn, *, s
     :func:`block_quantize`."""
     if scale_mode not in ("ceil", "floor"):
         raise TileValueError(f"scale_mode must be 'ceil' or 'floor', got {scale_mode!r}")
+    r = L.host().quantize(gate_up, dtype, 1 if scale_mode == "floor" else 0, True)
+    if type(r) is tuple:
+        return r
+    if r is not None:
+        _check(r)
     fmt = dtype if isinstance(dtype, str) else _DTYPE_FMT.get(dtype)
     if fmt not in _FMT_CODE:
         raise TileTypeError(f"Unsupported quantisation dtype {dtype}")
