@@ -21,7 +21,7 @@ INCLUDE = ROOT.parent / "include"
 OUT = ROOT / "cutile_amd" / "libmxgemm.so"
 HOST_OUT = ROOT / "cutile_amd" / "_mxhost.so"   # csrc/mx_host.cpp: the operators' native host path
 OBJ = ROOT / "build"
-SOURCES = ["mx_api.hip", "mx_gemm_mfma.hip", "mx_gemm_pp32.hip", "mx_gemm_w4.hip", "mx_gemm_generic.hip", "mx_gemm_decode.hip", "mx_aux.hip", "mx_probe.hip"]
+SOURCES = ["mx_api.hip", "mx_gemm_mfma.hip", "mx_gemm_pp32.hip", "mx_gemm_w4.hip", "mx_gemm_generic.hip", "mx_gemm_decode.hip", "mx_gemm_stream.hip", "mx_aux.hip", "mx_probe.hip"]
 # sources compiled once per value of a macro, so that their instances build in parallel: (file, macro, count)
 SPLIT = [("mx_gemm_pp.hip", "MX_PP_PAIR", 4)]
 UNITS = [(s, None) for s in SOURCES] + [(f, f"-D{m}={i}") for f, m, n in SPLIT for i in range(n)]
@@ -37,6 +37,12 @@ def _newer(src: pathlib.Path, obj: pathlib.Path) -> bool:
     if not obj.exists():
         return True
     deps = [src, *CSRC.glob("*.h"), INCLUDE / "mxgemm.h"]
+    listed = obj.with_suffix(".d")   # what the compiler read of this tree the last time
+    if listed.exists():
+        names = [pathlib.Path(w) for w in listed.read_text().replace("\\\n", " ").split()[1:]]
+        deps = [d for d in names if ROOT.parent in d.resolve().parents]
+        if not all(d.exists() for d in deps):
+            return True
     return any(d.stat().st_mtime > obj.stat().st_mtime for d in deps)
 
 
@@ -55,7 +61,7 @@ def _compile(unit, force: bool) -> pathlib.Path:
     s = CSRC / src
     o = OBJ / (s.stem + (define.replace("=", "_").replace("-D", "_") if define else "") + ".o")
     if force or _newer(s, o):
-        cmd = ["hipcc", *FLAGS, *([define] if define else []), "-c", str(s), "-o", str(o)]
+        cmd = ["hipcc", *FLAGS, *([define] if define else []), "-MD", "-MF", str(o.with_suffix(".d")), "-c", str(s), "-o", str(o)]
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "mx_common.h"
+#include "mx_stream.h"
 
 // Scratch of mx_gemm_static: lives in the library's device image, one copy per GPU the library runs on, held
 // until the process ends.  Host code never uses this name as an address: static_scratch() below resolves the
@@ -48,25 +49,19 @@ inline int native_layout_of(int kernel) {
 }
 inline bool is_native(int layout) { return layout == MX_SCALE_NATIVE || layout == MX_SCALE_NATIVE32; }
 
-// The decode kernel takes K up to kDecodeChunk per launch; a longer K runs as one launch per chunk, the chunks adding
-// up in an fp32 buffer of the workspace that a last pass converts into C.
-constexpr int64_t kDecodeChunk = 8192;
-// One launch of it multiplies up to 32 rows of X; more rows run slab by slab, each slab streaming the weights again
-// (the second pass finds most of a weight matrix of up to 256 MiB in the Infinity Cache).  MX_KERNEL_AUTO does that
-// up to kDecodeAutoM rows (measured on 28672 x 8192 FP4 weights: M = 64 takes 2 x 26 us this way against 62 us on the
-// tiled kernel, whose time hardly grows up to M = 128); an explicit MX_KERNEL_DECODE up to kDecodeMaxM.
-constexpr int64_t kDecodeAutoM = 64, kDecodeMaxM = 128;
-inline bool decode_shape(int64_t M, int64_t N, int64_t K) {
-  return M >= 1 && M <= kDecodeMaxM && K % 512 == 0 && N % 16 == 0;
+// The decode kernel keeps X in registers: K up to kDecodeMaxK, 32 rows per launch (MX_KERNEL_AUTO gives it no more; an
+// explicit MX_KERNEL_DECODE runs up to kDecodeMaxM rows slab by slab, each slab streaming the weights again).
+constexpr int64_t kDecodeMaxK = 8192, kDecodeMaxM = 128;
+// Rows up to which MX_KERNEL_AUTO streams the weights through registers (MX_KERNEL_STREAM).
+constexpr int64_t kStreamAutoM = 64;
+// FP4 weights with plain scales at up to 32 rows: the decode kernel keeps X in registers for the whole launch, which
+// pays once a workgroup walks several weight tiles (28672 x 8192: 26 - 29 us against 28 - 36 us at 4 - 32 rows, 14336 x
+// 4096 at 16 rows 11.4 against 10.9); beyond 16 rows, where X is as much as the weights, from the start, unless K is
+// so short that its tiles are all start-up.
+inline bool decode_beats_stream(int64_t M, int64_t N, int64_t K) {
+  if (K > kDecodeMaxK || K % 512 != 0 || N % 16 != 0) return false;
+  return M <= 16 ? (N >= 16384 && K >= 4096) : (K >= 2048 || N <= 8192);
 }
-// workspace of that buffer; depends on (M, N, K, opts) only, so it is also counted for problems whose operand types
-// then send them to another kernel
-inline int64_t decode_partial_bytes(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
-  if ((o.kernel != MX_KERNEL_AUTO && o.kernel != MX_KERNEL_DECODE) || !decode_shape(M, N, K) || K <= kDecodeChunk)
-    return 0;
-  return round256(M * N * 4);
-}
-
 const mx_gemm_opts kDefaultOpts = {sizeof(mx_gemm_opts), 0, MX_SCALE_2D, MX_SCALE_2D, MX_KERNEL_AUTO, 32, 0, 0};
 
 // Number of K-slices for a problem that ends up on a one-tile MFMA kernel (1 = no split).  Depends only on
@@ -171,9 +166,8 @@ int64_t mx_packed_scale_bytes(int64_t rows, int64_t K) {
 
 int64_t mx_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, const mx_gemm_opts* opts) {
   const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
-  if (o.kernel == MX_KERNEL_GENERIC) return 0;
-  if (o.kernel == MX_KERNEL_DECODE) return decode_partial_bytes(M, N, K, o);
-  int64_t b = decode_partial_bytes(M, N, K, o);
+  if (o.kernel == MX_KERNEL_GENERIC || o.kernel == MX_KERNEL_STREAM || o.kernel == MX_KERNEL_DECODE) return 0;
+  int64_t b = 0;
   const int S = plan_k_splits(M, N, K, o);
   if (S > 1) {   // per-slice packed scales and the fp32 partial products
     b += S * (mx_packed_scale_bytes(M, K / S) + mx_packed_scale_bytes(N, K / S));
@@ -376,10 +370,35 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
   else if (C->stride[1] != 1) why = "C is not row-major";
   else if (M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 30)) why = "extent too large";
 
+  // what keeps the weight-streaming kernel from taking the problem (it also takes E5M2 x E2M1, which the tiled
+  // kernels do not)
+  const char* why_stream = nullptr;
+  if (batched) why_stream = "batched operands";
+  else if (o.block_size != 32 || As->dtype != MX_E8M0) why_stream = "it reads E8M0 scales with block 32";
+  else if (!stream_supports(A->dtype, B->dtype)) why_stream = "it takes 8-bit A with FP4 B or B of A's format";
+  else if (K < 128 || K % 128 != 0) why_stream = "K is not a multiple of 128";
+  else if ((why_stream = mfma_operand_issue(A->ptr, M, a_ld, A->stride[1], A->dtype, 1))) {}
+  else if ((why_stream = mfma_operand_issue(B->ptr, N, b_ld, B->stride[0], B->dtype, B->packed_dim == 0))) {}
+  else if (C->stride[1] != 1) why_stream = "C is not row-major";
+  else if (o.a_scale_layout != MX_SCALE_2D || As->stride[1] != 1 || As->stride[0] % 4 != 0 ||
+           ((uintptr_t)As->ptr) % 4 != 0)
+    why_stream = "A_scale must be the plain 2-D layout with 4-byte aligned rows";
+  else if (o.b_scale_layout != MX_SCALE_NATIVE &&
+           (o.b_scale_layout != MX_SCALE_2D || Bs->stride[0] != 1 || Bs->stride[1] % 4 != 0 || ((uintptr_t)Bs->ptr) % 4 != 0))
+    why_stream = "B_scale must be MX_SCALE_NATIVE or K-contiguous with 4-byte aligned rows";
+
   int kernel = o.kernel;
-  if (kernel == MX_KERNEL_AUTO) {
-    if (why) kernel = MX_KERNEL_GENERIC;
-    else if (M <= kDecodeAutoM && o.split_k <= 1 && A->dtype != MX_E2M1 && B->dtype == MX_E2M1 &&
+  if (kernel == MX_KERNEL_DECODE && K > kDecodeMaxK && M <= kDecodeMaxM && N % 16 == 0 && K % 512 == 0 && !why_stream &&
+      o.b_scale_layout == MX_SCALE_2D && B->dtype == MX_E2M1)
+    kernel = MX_KERNEL_STREAM;   // beyond what the decode kernel keeps of X in registers
+  if (kernel == MX_KERNEL_STREAM) {
+    if (why_stream) return set_error(MX_ERR_LAYOUT, "the streaming kernel cannot run this problem: %s", why_stream);
+  } else if (kernel == MX_KERNEL_AUTO) {
+    if (!plan && !why_stream && o.split_k <= 1 && (why || M <= kStreamAutoM) &&
+        !(M <= 32 && decode_beats_stream(M, N, K) && B->dtype == MX_E2M1 && o.b_scale_layout == MX_SCALE_2D))
+      kernel = MX_KERNEL_STREAM;
+    else if (why) kernel = MX_KERNEL_GENERIC;
+    else if (M <= 32 && o.split_k <= 1 && A->dtype != MX_E2M1 && B->dtype == MX_E2M1 &&
              o.a_scale_layout == MX_SCALE_2D &&
              o.b_scale_layout == MX_SCALE_2D && Bs->stride[0] == 1 && As->stride[1] == 1 && K % 512 == 0 &&
              N % 16 == 0 && Bs->stride[1] % 16 == 0 && ((uintptr_t)Bs->ptr) % 16 == 0 &&
@@ -437,6 +456,17 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     return launch_gemm_generic(g, (hipStream_t)stream);
   }
 
+  if (kernel == MX_KERNEL_STREAM) {
+    StreamArgs d = {};
+    d.X = (const uint8_t*)A->ptr; d.Xs = (const uint8_t*)As->ptr;
+    d.W = (const uint8_t*)B->ptr; d.Ws = (const uint8_t*)Bs->ptr; d.C = C->ptr;
+    d.M = (int32_t)M; d.N = (int32_t)N; d.K = (int32_t)K;
+    d.ldx = a_ld; d.ldxs = As->stride[0]; d.ldw = b_ld; d.ldws = Bs->stride[1]; d.ldc = C->stride[0];
+    d.x_fmt = A->dtype; d.w_fmt = B->dtype; d.c_dtype = C->dtype; d.accumulate = o.accumulate;
+    d.ws_packed = o.b_scale_layout == MX_SCALE_NATIVE;
+    return launch_gemm_stream(d, (hipStream_t)stream);
+  }
+
   if (kernel == MX_KERNEL_DECODE) {
     if (M > kDecodeMaxM)
       return set_error(MX_ERR_SHAPE, "the decode kernel handles M <= %lld (got %lld)", (long long)kDecodeMaxM, (long long)M);
@@ -454,7 +484,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     d.ldx = a_ld; d.ldxs = As->stride[0]; d.ldw = b_ld; d.ldws = Bs->stride[1]; d.ldc = C->stride[0];
     d.x_fmt = A->dtype; d.w_fmt = B->dtype; d.c_dtype = C->dtype; d.accumulate = o.accumulate;
     const int c_bytes = C->dtype == MX_BF16 ? 2 : 4;
-    // slabs of 32 rows of X (and of C, or of the chunk buffer)
+    // slabs of 32 rows of X and C
     auto launch_slabs = [&](const DecodeArgs& full, int out_bytes) {
       for (int64_t m0 = 0; m0 < M; m0 += 32) {
         DecodeArgs s = full;
@@ -465,24 +495,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       }
       return (int)MX_OK;
     };
-    if (K <= kDecodeChunk) return launch_slabs(d, c_bytes);
-    // a longer K (the down-projection of an MoE layer, K = 14336 / 28672): chunks of kDecodeChunk elements, each
-    // streaming its part of the weights once, summed in fp32 in the workspace in chunk order
-    const int64_t need = decode_partial_bytes(M, N, K, o);
-    if (!workspace || workspace_bytes < need)
-      return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
-                       (long long)workspace_bytes);
-    if (((uintptr_t)workspace) % 256 != 0) return set_error(MX_ERR_WORKSPACE, "workspace must be 256-byte aligned");
-    for (int64_t k0 = 0; k0 < K; k0 += kDecodeChunk) {
-      DecodeArgs c = d;
-      c.X = d.X + k0; c.Xs = d.Xs + k0 / 32;          // 8-bit activations: one byte per element
-      c.W = d.W + k0 / 2; c.Ws = d.Ws + k0 / 32;      // FP4 weights: two elements per byte
-      c.K = (int32_t)(K - k0 < kDecodeChunk ? K - k0 : kDecodeChunk);
-      c.C = workspace; c.ldc = N; c.c_dtype = MX_F32; c.accumulate = k0 > 0;
-      if (int rc = launch_slabs(c, 4)) return rc;
-    }
-    return launch_splitk_reduce((const float*)workspace, 1, M, N, C->ptr, C->stride[0], C->dtype, o.accumulate,
-                                (hipStream_t)stream);
+    return launch_slabs(d, c_bytes);
   }
 
   // ---- MFMA path: bring the scales into the native layout if they are not ----------------------------
