@@ -457,6 +457,11 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
   }
 
   if (kernel == MX_KERNEL_STREAM) {
+    // it uses no workspace, but a caller of MX_KERNEL_AUTO is held to what mx_gemm_workspace_bytes says, whatever is picked
+    const int64_t need = mx_gemm_workspace_bytes(M, N, K, &o);
+    if (B->dtype != MX_E2M1 && need > 0 && (!workspace || workspace_bytes < need))
+      return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
+                       (long long)workspace_bytes);
     StreamArgs d = {};
     d.X = (const uint8_t*)A->ptr; d.Xs = (const uint8_t*)As->ptr;
     d.W = (const uint8_t*)B->ptr; d.Ws = (const uint8_t*)Bs->ptr; d.C = C->ptr;
