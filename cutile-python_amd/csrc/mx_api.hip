@@ -896,8 +896,158 @@ int mx_moe_align(const int32_t* topk_ids, int64_t num_ids, int32_t num_experts, 
     return set_error(MX_ERR_WORKSPACE, "moe_align: workspace of %lld bytes required, %lld given", (long long)need,
                      (long long)workspace_bytes);
   if (need > 0 && ((uintptr_t)workspace) % 4 != 0) return set_error(MX_ERR_WORKSPACE, "moe_align: workspace must be 4-byte aligned");
-  return launch_moe_align(topk_ids, num_ids, num_experts, tile_m, sorted_token_ids, sorted_expert_ids,
+  return launch_moe_align(topk_ids, 0, num_ids, num_experts, tile_m, sorted_token_ids, sorted_expert_ids,
                           num_slots_out, max_slots, (int32_t*)workspace, (hipStream_t)stream);
+}
+
+namespace {
+// Sizes of a mixture-of-experts layer and where its pieces lie in the workspace.
+struct MoePlan {
+  int64_t T, n, E, H, F, H_out;
+  bool stream;          // experts' weights streamed for a few rows each; otherwise grouped GEMMs on aligned slots
+  int32_t tile_m;
+  int64_t q, qs, c3, c1, slots, max_slots, blocks, align, grouped, grouped_bytes, total;   // offsets (bytes)
+};
+// Rows per expert up to which the weights are streamed.
+constexpr int64_t kMoeStreamRows = 48;
+
+MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& W2, const mx_gemm_opts& o) {
+  MoePlan p = {};
+  p.T = T; p.n = T * topk; p.E = W1.shape[0]; p.H = W1.shape[2]; p.F = W1.shape[1] / 2; p.H_out = W2.shape[1];
+  p.stream = p.n <= kMoeMaxIds && p.n <= p.E * kMoeStreamRows && p.H % 128 == 0 && p.F % 128 == 0;
+  int64_t off = 0;
+  auto take = [&](int64_t bytes) { const int64_t at = off; off += round256(bytes); return at; };
+  p.q = take(p.n * p.F);
+  p.qs = take(p.n * (p.F / 32));
+  p.c3 = take(p.n * p.H_out * 4);
+  if (!p.stream) {
+    p.tile_m = 256;
+    p.max_slots = mx_moe_align_max_slots(p.n, (int32_t)p.E, p.tile_m);
+    p.c1 = take(p.n * p.F * 4);
+    p.slots = take(p.max_slots * 4);
+    p.blocks = take(p.max_slots / p.tile_m * 4);
+    p.align = take(mx_moe_align_workspace_bytes(p.n, (int32_t)p.E));
+    mx_gemm_opts g1 = kDefaultOpts, g2 = kDefaultOpts;
+    g1.b_scale_layout = o.a_scale_layout;
+    g2.b_scale_layout = o.b_scale_layout;
+    const int64_t b1 = mx_gemm_grouped_workspace_bytes(p.max_slots, 2 * p.F, p.H, p.E, &g1);
+    const int64_t b2 = mx_gemm_grouped_workspace_bytes(p.max_slots, p.H_out, p.F, p.E, &g2);
+    p.grouped_bytes = b1 > b2 ? b1 : b2;
+    p.grouped = take(p.grouped_bytes);
+  }
+  p.total = off;
+  return p;
+}
+
+inline mx_tensor tensor2d(void* ptr, int dtype, int64_t rows, int64_t cols, int64_t ld) {
+  return mx_tensor{ptr, dtype, 2, {rows, cols, 0, 0}, {ld, 1, 0, 0}, -1, 0};
+}
+}  // namespace
+
+int64_t mx_moe_forward_workspace_bytes(int64_t T, int32_t topk, const mx_tensor* W1, const mx_tensor* W2,
+                                       const mx_gemm_opts* opts) {
+  if (T <= 0 || topk <= 0 || !W1 || !W2 || W1->ndim != 3 || W2->ndim != 3) return 0;
+  return moe_plan(T, topk, *W1, *W2, opts ? *opts : kDefaultOpts).total;
+}
+
+int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1, const mx_tensor* W1s,
+                   const mx_tensor* W2, const mx_tensor* W2s, const float* topk_weights, const void* topk_ids,
+                   int32_t ids64, int32_t topk, mx_tensor* out, int32_t scale_mode, const mx_gemm_opts* opts,
+                   void* workspace, int64_t workspace_bytes, void* stream) {
+  const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
+  if (int rc = check_tensor(X, "X", 2, 2)) return rc;
+  if (int rc = check_tensor(Xs, "X_scale", 2, 2)) return rc;
+  if (int rc = check_tensor(W1, "W1", 3, 3)) return rc;
+  if (int rc = check_tensor(W1s, "W1_scale", 3, 3)) return rc;
+  if (int rc = check_tensor(W2, "W2", 3, 3)) return rc;
+  if (int rc = check_tensor(W2s, "W2_scale", 3, 3)) return rc;
+  if (int rc = check_tensor(out, "out", 2, 2)) return rc;
+  if (!topk_weights || !topk_ids) return set_error(MX_ERR_INVALID, "null routing arrays");
+  const int64_t T = X->shape[0], H = X->shape[1], E = W1->shape[0], F = W1->shape[1] / 2, H_out = W2->shape[1];
+  if (topk <= 0) return set_error(MX_ERR_INVALID, "topk must be positive");
+  if (W1->shape[1] % 2 != 0 || W1->shape[2] != H || W2->shape[0] != E || W2->shape[2] != F)
+    return set_error(MX_ERR_SHAPE, "W1 must be [E, 2F, H] and W2 [E, H_out, F]");
+  if (out->shape[0] != T || out->shape[1] != H_out) return set_error(MX_ERR_SHAPE, "out must be [T, H_out]");
+  if (X->dtype != MX_E4M3 || W1->dtype != W2->dtype || (W1->dtype != MX_E4M3 && W1->dtype != MX_E2M1) ||
+      Xs->dtype != MX_E8M0 || W1s->dtype != MX_E8M0 || W2s->dtype != MX_E8M0)
+    return set_error(MX_ERR_DTYPE, "mx_moe_forward takes E4M3 activations and E4M3 or E2M1 weights with E8M0 scales");
+  if (out->dtype != MX_F32 && out->dtype != MX_BF16) return set_error(MX_ERR_DTYPE, "out must be MX_F32 or MX_BF16");
+  if (scale_mode != 0 && scale_mode != 1) return set_error(MX_ERR_INVALID, "scale_mode must be 0 (ceil) or 1 (floor)");
+  if (H % 32 != 0 || F % 32 != 0 || E <= 0 || T * topk >= 0x7FFFFFFF)
+    return set_error(MX_ERR_SHAPE, "H and F must be multiples of 32");
+  if (Xs->shape[0] != T || Xs->shape[1] != H / 32) return set_error(MX_ERR_SHAPE, "X_scale must be [T, H/32]");
+  if (T == 0 || H_out == 0) return MX_OK;
+  // every condition under which one of the steps below could refuse its operands, before anything is enqueued
+  auto weights_issue = [&](const mx_tensor* W, const mx_tensor* Ws, int32_t layout) -> const char* {
+    if (W->dtype == MX_E2M1 && W->packed_dim != 2) return "FP4 weights are not packed along K";
+    if (const char* why = mfma_operand_issue(W->ptr, W->shape[1], W->stride[1], W->stride[2], W->dtype, 1)) return why;
+    if (W->stride[0] % 16 != 0) return "expert pitch of W is not a multiple of 16 bytes";
+    if (E * mx_packed_scale_bytes(W->shape[1], W->shape[2]) >= ((int64_t)1 << 31)) return "the packed scales span 2 GiB or more";
+    if (layout == MX_SCALE_NATIVE) return ((uintptr_t)Ws->ptr) % 16 != 0 ? "packed scales are not 16-byte aligned" : nullptr;
+    if (layout != MX_SCALE_2D) return "scale layout";
+    if (Ws->shape[0] != E || Ws->shape[1] != W->shape[1] || Ws->shape[2] != W->shape[2] / 32) return "W_scale must be [E, rows, K/32]";
+    if (Ws->stride[2] != 1 || Ws->stride[1] % 4 != 0 || Ws->stride[0] % 4 != 0 || ((uintptr_t)Ws->ptr) % 4 != 0 ||
+        W->shape[1] * Ws->stride[1] >= ((int64_t)1 << 31))
+      return "W_scale rows are not contiguous and 4-byte aligned";
+    return nullptr;
+  };
+  const char* why = mfma_operand_issue(X->ptr, T, X->stride[0], X->stride[1], X->dtype, 1);
+  if (!why) why = weights_issue(W1, W1s, o.a_scale_layout);
+  if (!why) why = weights_issue(W2, W2s, o.b_scale_layout);
+  if (!why && (Xs->stride[1] != 1 || Xs->stride[0] % 4 != 0 || ((uintptr_t)Xs->ptr) % 4 != 0)) why = "X_scale rows are not contiguous and 4-byte aligned";
+  if (!why && (out->stride[1] != 1 || out->stride[0] != H_out)) why = "out is not contiguous";
+  if (!why && 2 * F <= 128) why = "F is too small";
+  if (!why && H_out <= 128) why = "H_out is too small";
+  if (why) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: %s", why);
+  const MoePlan p = moe_plan(T, topk, *W1, *W2, o);
+  if (p.n * p.F >= ((int64_t)1 << 31)) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: the activation spans 2 GiB or more");
+  if (!workspace || workspace_bytes < p.total)
+    return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)p.total, (long long)workspace_bytes);
+  if (((uintptr_t)workspace) % 256 != 0) return set_error(MX_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+  uint8_t* const ws = (uint8_t*)workspace;
+  hipStream_t st = (hipStream_t)stream;
+
+  if (p.stream) {
+    MoeStreamArgs a = {};
+    a.ids = topk_ids; a.ids64 = ids64; a.n_ids = (int32_t)p.n; a.E = (int32_t)E;
+    a.w_fmt = W1->dtype; a.scale_mode = scale_mode;
+    a.X = (const uint8_t*)X->ptr; a.Xs = (const uint8_t*)Xs->ptr; a.ldx = X->stride[0]; a.ldxs = Xs->stride[0];
+    a.x_rows = (int32_t)T; a.replicas = topk;
+    a.W = (const uint8_t*)W1->ptr; a.ldw = W1->stride[1]; a.w_es = W1->stride[0];
+    a.Ws = (const uint8_t*)W1s->ptr; a.ws_packed = o.a_scale_layout == MX_SCALE_NATIVE;
+    a.ldws = W1s->stride[1]; a.ws_es = a.ws_packed ? mx_packed_scale_bytes(2 * F, H) : W1s->stride[0];
+    a.N = (int32_t)(2 * F); a.K = (int32_t)H; a.F = (int32_t)F;
+    a.q = ws + p.q; a.qs = ws + p.qs;
+    if (int rc = launch_moe_stream(a, true, st)) return rc;
+    a.X = ws + p.q; a.Xs = ws + p.qs; a.ldx = F; a.ldxs = F / 32;
+    a.x_rows = (int32_t)p.n; a.replicas = 1;
+    a.W = (const uint8_t*)W2->ptr; a.ldw = W2->stride[1]; a.w_es = W2->stride[0];
+    a.Ws = (const uint8_t*)W2s->ptr; a.ws_packed = o.b_scale_layout == MX_SCALE_NATIVE;
+    a.ldws = W2s->stride[1]; a.ws_es = a.ws_packed ? mx_packed_scale_bytes(H_out, F) : W2s->stride[0];
+    a.N = (int32_t)H_out; a.K = (int32_t)F;
+    a.weights = topk_weights; a.C = (float*)(ws + p.c3);
+    if (int rc = launch_moe_stream(a, false, st)) return rc;
+  } else {
+    int32_t* const slots = (int32_t*)(ws + p.slots);
+    int32_t* const blocks = (int32_t*)(ws + p.blocks);
+    if (int rc = launch_moe_align(topk_ids, ids64, p.n, (int32_t)E, p.tile_m, slots, blocks, nullptr, p.max_slots,
+                                  (int32_t*)(ws + p.align), st))
+      return rc;
+    mx_gemm_opts g = kDefaultOpts;
+    g.b_scale_layout = o.a_scale_layout;
+    mx_tensor c1 = tensor2d(ws + p.c1, MX_BF16, p.n, 2 * F, 2 * F);
+    if (int rc = mx_gemm_grouped(X, Xs, W1, W1s, &c1, nullptr, slots, p.max_slots, blocks, p.tile_m, topk, p.n, &g, ws + p.grouped,
+                                 p.grouped_bytes, stream))
+      return rc;
+    mx_tensor q = tensor2d(ws + p.q, MX_E4M3, p.n, F, F), qs = tensor2d(ws + p.qs, MX_E8M0, p.n, F / 32, F / 32);
+    if (int rc = mx_silu_mul_quantize(&c1, &q, &qs, scale_mode, stream)) return rc;
+    g.b_scale_layout = o.b_scale_layout;
+    mx_tensor c3 = tensor2d(ws + p.c3, MX_F32, p.n, H_out, H_out);
+    if (int rc = mx_gemm_grouped(&q, &qs, W2, W2s, &c3, topk_weights, slots, p.max_slots, blocks, p.tile_m, 1, p.n, &g,
+                                 ws + p.grouped, p.grouped_bytes, stream))
+      return rc;
+  }
+  return launch_moe_combine((const float*)(ws + p.c3), topk_ids, ids64, (int)E, T, topk, H_out, out->ptr, out->dtype, st);
 }
 
 namespace {

@@ -1,6 +1,7 @@
 // Memory-bound helpers around the block-scaled GEMM: MX quantisation, native scale re-layout and the
 // MoE slot alignment.  All integer / byte work; results must be bit-exact.
 #include "mx_common.h"
+#include "mx_quant.h"
 
 namespace mx {
 namespace {
@@ -8,112 +9,12 @@ namespace {
 // ================================================================================================
 // MX quantiser (replaces the torch-op chain of block_quantize, test/kernels/kernel_utils.py:38-80)
 // ================================================================================================
-// The shared exponent is computed on bit patterns.  Element conversion has two routes with identical
-// results: the gfx950 scaled-conversion instructions for ordinary blocks, and an integer route (value =
-// sig * 2^(ex-150) divided by 2^se by subtracting exponents, then rounded to nearest even onto the target
-// grid in one step) for blocks with a zero / subnormal amax, inf / NaN or an extreme scale, where denormal
-// modes or the instruction's special cases could otherwise change a bit.
-
-struct Unpacked {
-  uint32_t sig;   // 24-bit significand with the leading one at bit 23 (0 for zero)
-  int ex;         // biased exponent such that value = sig * 2^(ex - 150)
-  uint32_t sign;  // 0 or 1
-  int cls;        // 0 finite, 1 inf, 2 nan
-};
-
-__device__ inline Unpacked unpack_f32(uint32_t bits) {
-  Unpacked u;
-  u.sign = bits >> 31;
-  const uint32_t a = bits & 0x7FFFFFFFu;
-  u.cls = a > 0x7F800000u ? 2 : (a == 0x7F800000u ? 1 : 0);
-  int ex = (int)(a >> 23);
-  uint32_t sig = a & 0x7FFFFFu;
-  if (ex == 0) {
-    if (sig != 0) {  // subnormal: normalise
-      const int lz = __builtin_clz(sig) - 8;
-      sig <<= lz;
-      ex = 1 - lz;
-    }
-  } else {
-    sig |= 0x800000u;
-  }
-  u.sig = sig;
-  u.ex = ex;
-  return u;
-}
-
-// round-to-nearest-even of sig / 2^sh, sh in [1, 31]
-__device__ inline uint32_t rne_shift(uint32_t sig, int sh) {
-  return (sig + ((1u << (sh - 1)) - 1u) + ((sig >> sh) & 1u)) >> sh;
-}
-
-// Generic minifloat encoder: MBITS mantissa bits, minimum normal exponent EMIN, exponent bias BIAS.
-// Returns the magnitude code without clamping (may exceed the format's largest finite code).
-template <int MBITS, int EMIN, int BIAS>
-__device__ inline uint32_t encode_mag(const Unpacked& u, int se) {
-  if (u.sig == 0) return 0;
-  const int E = u.ex - 127 - se;            // exponent of x / 2^se
-  const int Eq = E > EMIN ? E : EMIN;
-  int sh = (23 - MBITS) + (Eq - E);
-  if (sh > 31) sh = 31;                     // anything this small rounds to zero
-  const uint32_t n = rne_shift(u.sig, sh);  // in units of 2^(Eq - MBITS); normal range: [2^MBITS, 2^(MBITS+1)]
-  if (E > 300) return 0xFFFFu;              // cannot happen for finite fp32 / E8M0 scales; keeps shifts sane
-  return (uint32_t)((Eq + BIAS - 1) << MBITS) + n;
-}
-
-__device__ inline uint32_t encode_e4m3(const Unpacked& u, int se, bool saturate) {
-  const uint32_t s = u.sign << 7;
-  if (u.cls == 2) return s | 0x7F;
-  if (u.cls == 1) return s | (saturate ? 0x7Eu : 0x7Fu);
-  uint32_t c = encode_mag<3, -6, 7>(u, se);
-  if (c > 0x7E) c = saturate ? 0x7E : 0x7F;   // torch's cast: above 448 after rounding -> NaN
-  return s | c;
-}
-
-__device__ inline uint32_t encode_e5m2(const Unpacked& u, int se, bool saturate) {
-  const uint32_t s = u.sign << 7;
-  if (u.cls == 2) return s | 0x7F;
-  if (u.cls == 1) return s | (saturate ? 0x7Bu : 0x7Cu);
-  uint32_t c = encode_mag<2, -14, 15>(u, se);
-  if (c > 0x7B) c = saturate ? 0x7B : 0x7C;   // IEEE-like: overflow -> inf
-  return s | c;
-}
-
-__device__ inline uint32_t encode_e2m1(const Unpacked& u, int se) {
-  const uint32_t s = u.sign << 3;
-  if (u.cls != 0) return s | 7;
-  uint32_t c = encode_mag<1, 0, 1>(u, se);
-  if (c > 7) c = 7;                           // finite-only format: clamp to +-6
-  return s | c;
-}
+// The shared exponent and the element codes come from encode_block (mx_quant.h), on bit patterns.
 
 __device__ inline float load_as_f32(const void* p, int64_t i, int dtype) {
   if (dtype == MX_F32) return ((const float*)p)[i];
   if (dtype == MX_BF16) return bf16_to_f32(((const uint16_t*)p)[i]);
   return (float)((const _Float16*)p)[i];
-}
-
-// silu(a) * b = a / (1 + exp(-a)) * b as a fixed sequence of correctly rounded fp32 operations (no fused
-// multiply-add, no approximate instruction), so that a host restatement with the same sequence gets the
-// same bits: exp(-a) = 2^z, z = -a * log2(e) clamped to +-125, z = n + f with n = rint(z), 2^f by the
-// degree-7 Taylor polynomial in f * ln 2 (|f| <= 0.5: truncation error below 1e-8), scaled by 2^n exactly.
-__device__ inline float silu_mul_f32(float a, float b) {
-  float z = __fmul_rn(-a, 1.44269504f);
-  z = fminf(fmaxf(z, -125.0f), 125.0f);
-  const float n = __builtin_rintf(z);
-  const float f = __fsub_rn(z, n);
-  float p = 1.52527338e-5f;
-  p = __fadd_rn(__fmul_rn(p, f), 1.54035304e-4f);
-  p = __fadd_rn(__fmul_rn(p, f), 1.33335581e-3f);
-  p = __fadd_rn(__fmul_rn(p, f), 9.61812911e-3f);
-  p = __fadd_rn(__fmul_rn(p, f), 5.55041087e-2f);
-  p = __fadd_rn(__fmul_rn(p, f), 2.40226507e-1f);
-  p = __fadd_rn(__fmul_rn(p, f), 6.93147181e-1f);
-  p = __fadd_rn(__fmul_rn(p, f), 1.0f);
-  const float e = __fmul_rn(p, __builtin_bit_cast(float, (uint32_t)((int)n + 127) << 23));
-  const float s = __fdiv_rn(1.0f, __fadd_rn(1.0f, e));
-  const float t = a < -87.5f ? 0.0f : __fmul_rn(a, s);   // exp(-a) is past the clamp: the true value is below 2^-120
-  return __fmul_rn(t, b);
 }
 
 // EPL consecutive elements starting at element index i (all of them inside K checked by the caller for `vec`)
@@ -204,11 +105,10 @@ __device__ inline void quant_store(const QuantArgs& q, const QuantUnit& u, float
     for (int e = 0; e < EPL; ++e) v[e] = (live && e < nvalid) ? silu_mul_f32(v[e], w[e]) : 0.f;
   }
   // amax over the block on |bits| (monotone in |x| for finite values; NaN patterns compare largest)
-  uint32_t bits[EPL], am = 0;
+  uint32_t am = 0;
 #pragma unroll
   for (int e = 0; e < EPL; ++e) {
-    bits[e] = __builtin_bit_cast(uint32_t, v[e]);
-    const uint32_t a = bits[e] & 0x7FFFFFFFu;
+    const uint32_t a = __builtin_bit_cast(uint32_t, v[e]) & 0x7FFFFFFFu;
     am = a > am ? a : am;
   }
 #pragma unroll
@@ -217,94 +117,9 @@ __device__ inline void quant_store(const QuantArgs& q, const QuantUnit& u, float
     am = o > am ? o : am;
   }
 
-  // shared exponent
-  int se;
-  if (q.scale_mode == 0) {
-    // reference rule: 2^ceil(log2(max(amax/448, 1e-12))), ceiling taken exactly on the fp32 quotient
-    // (a block with an inf or NaN amax never uses this exponent: see nonfinite_ceil below)
-    float t = __fdiv_rn(__builtin_bit_cast(float, am), 448.0f);
-    t = t > 1e-12f ? t : 1e-12f;
-    const uint32_t tb = __builtin_bit_cast(uint32_t, t);
-    se = (int)(tb >> 23) - 127 + ((tb & 0x7FFFFFu) ? 1 : 0);
-  } else {
-    // OCP MX v1.0: floor(log2 amax) - emax_elem; all-zero block -> smallest scale
-    const int emax = q.fmt == MX_E4M3 ? 8 : (q.fmt == MX_E5M2 ? 15 : 2);
-    if (am == 0) {
-      se = -127;
-    } else {
-      const int ex = (int)(am >> 23);
-      const int fl = ex ? ex - 127 : (31 - __builtin_clz(am)) - 149;
-      se = fl - emax;
-    }
-  }
-  se = se < -127 ? -127 : (se > 127 ? 127 : se);
-  const bool saturate = q.scale_mode != 0;
-
-  // Reference rule with a non-finite amax: torch.clamp(min=) keeps NaN and inf / 448 stays inf, so the scale is
-  // NaN or inf, both of which the cast to float8_e8m0fnu writes as 0xFF; x / scale is then NaN for every
-  // element of a NaN block (the element's own sign if it is a NaN itself), and for an inf block NaN where
-  // |x| is inf (inf / inf is the default NaN, whose sign bit is set on the hosts the reference runs on) and a
-  // signed zero elsewhere.  E2M1 has no NaN: non-finite elements saturate to +-6 as in the finite case.
-  const bool nonfinite_ceil = q.scale_mode == 0 && am >= 0x7F800000u;
   uint32_t code[EPL];
-  if (nonfinite_ceil) {
-    const bool blk_nan = am > 0x7F800000u;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      const uint32_t a = bits[e] & 0x7FFFFFFFu, sgn = bits[e] >> 31;
-      if (q.fmt == MX_E2M1) code[e] = (sgn << 3) | ((blk_nan || a == 0x7F800000u) ? 7u : 0u);
-      else if (a > 0x7F800000u) code[e] = (sgn << 7) | 0x7Fu;
-      else if (blk_nan) code[e] = 0x7Fu;
-      else if (a == 0x7F800000u) code[e] = 0xFFu;
-      else code[e] = sgn << 7;
-    }
-  } else
-  // Blocks whose amax is a normal finite number and whose scale 2^se is a normal float take the hardware
-  // scaled conversions (v_cvt_scalef32_pk_*: x / 2^se rounded to nearest even; FP8 overflows to NaN / inf,
-  // FP4 saturates -- measured on MI355X against the integer encoders below for 270 k inputs per format).
-  // The saturating FP8 rule clamps the magnitude to max_normal * 2^se first, which is exact.  Everything
-  // else (zero or subnormal amax, inf / NaN, extreme scales) goes through the integer encoders.
-  if (am >= 0x00800000u && am < 0x7F800000u && se > -127 && se < 120) {
-    typedef short s2 __attribute__((ext_vector_type(2)));
-    const float sc = __builtin_bit_cast(float, (uint32_t)(se + 127) << 23);
-    float x[EPL];
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) x[e] = v[e];
-    if (saturate && q.fmt != MX_E2M1) {
-      const float lim = __fmul_rn(q.fmt == MX_E4M3 ? 448.0f : 57344.0f, sc);
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) x[e] = __builtin_copysignf(fminf(__builtin_fabsf(x[e]), lim), x[e]);
-    }
-#pragma unroll
-    for (int h = 0; h < EPL / 4; ++h) {   // four elements at a time
-      uint32_t packed;
-      if (q.fmt == MX_E4M3) {
-        s2 r = {0, 0};
-        r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(r, x[4 * h + 0], x[4 * h + 1], sc, false);
-        r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(r, x[4 * h + 2], x[4 * h + 3], sc, true);
-        packed = __builtin_bit_cast(uint32_t, r);
-      } else if (q.fmt == MX_E5M2) {
-        s2 r = {0, 0};
-        r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(r, x[4 * h + 0], x[4 * h + 1], sc, false);
-        r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(r, x[4 * h + 2], x[4 * h + 3], sc, true);
-        packed = __builtin_bit_cast(uint32_t, r);
-      } else {
-        uint32_t r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, x[4 * h + 0], x[4 * h + 1], sc, 0);
-        r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, x[4 * h + 2], x[4 * h + 3], sc, 1);
-        packed = (r & 0xFu) | ((r & 0xF0u) << 4) | ((r & 0xF00u) << 8) | ((r & 0xF000u) << 12);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) code[4 * h + e] = (packed >> (8 * e)) & 0xFFu;
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      const Unpacked un = unpack_f32(bits[e]);
-      code[e] = q.fmt == MX_E4M3 ? encode_e4m3(un, se, saturate)
-                : q.fmt == MX_E5M2 ? encode_e5m2(un, se, saturate)
-                                   : encode_e2m1(un, se);
-    }
-  }
+  uint8_t scale_byte;
+  encode_block<EPL>(v, am, q.fmt, q.scale_mode, code, scale_byte);
   if (!live) return;
   if (q.fmt == MX_E2M1) {
     // low nibble = even element (test/test_mma_scaled.py:155-160)
@@ -335,7 +150,7 @@ __device__ inline void quant_store(const QuantArgs& q, const QuantUnit& u, float
       for (int e = 0; e < EPL; ++e) out[e] = (uint8_t)code[e];
     }
   }
-  if (sub == 0) q.scale[row * q.sc_ld + kb] = nonfinite_ceil ? (uint8_t)0xFF : (uint8_t)(se + 127);
+  if (sub == 0) q.scale[row * q.sc_ld + kb] = scale_byte;
 }
 
 // 32 / EPL lanes per 32-element block, EPL consecutive elements per lane (8: half as many threads, and the
@@ -486,6 +301,7 @@ __global__ __launch_bounds__(256) void pack_scales_list_kernel(const PackList pl
 // ================================================================================================
 // A stable counting sort of the flattened expert ids over several workgroups, without atomics on global
 // memory and without any slot written twice.  The ids are cut into B contiguous chunks, one per workgroup.
+// (The ids may be int64: id_shift = 1 reads their low halves.)
 //   moe_hist_kernel (only when B > 1): workgroup b counts the ids of every expert in chunk b -> counts[b][e].
 //   moe_place_kernel: workgroup b
 //     1. sums column e of `counts` (thread e): ids of expert e in all chunks (total) and in the chunks before
@@ -502,7 +318,7 @@ constexpr int kAlignThreads = 256;
 constexpr int kAlignSegExperts = 256;      // up to this many experts the segment placement is used
 constexpr int64_t kAlignMaxChunk = 65535;  // ids per workgroup (u16 prefixes inside a chunk)
 
-__global__ __launch_bounds__(kAlignThreads) void moe_hist_kernel(const int32_t* __restrict__ topk_ids, int64_t n,
+__global__ __launch_bounds__(kAlignThreads) void moe_hist_kernel(const int32_t* __restrict__ topk_ids, int id_shift, int64_t n,
                                                                  int32_t E, int64_t chunk,
                                                                  int32_t* __restrict__ counts) {
   extern __shared__ int32_t sh[];   // [E]
@@ -511,14 +327,14 @@ __global__ __launch_bounds__(kAlignThreads) void moe_hist_kernel(const int32_t* 
   __syncthreads();
   const int64_t lo = (int64_t)blockIdx.x * chunk, hi = lo + chunk < n ? lo + chunk : n;
   for (int64_t i = lo + tid; i < hi; i += kAlignThreads) {
-    const int e = topk_ids[i];
+    const int e = topk_ids[i << id_shift];
     if (e >= 0 && e < E) atomicAdd(&sh[e], 1);
   }
   __syncthreads();
   for (int e = tid; e < E; e += kAlignThreads) counts[(int64_t)blockIdx.x * E + e] = sh[e];
 }
 
-__global__ __launch_bounds__(kAlignThreads) void moe_place_kernel(const int32_t* __restrict__ topk_ids, int64_t n,
+__global__ __launch_bounds__(kAlignThreads) void moe_place_kernel(const int32_t* __restrict__ topk_ids, int id_shift, int64_t n,
                                                                   int32_t E, int32_t tile_m, int64_t chunk,
                                                                   const int32_t* __restrict__ counts,
                                                                   int32_t* __restrict__ sorted_ids,
@@ -543,7 +359,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_place_kernel(const int32_t*
     for (int i = tid; i < E * LD / 2; i += T) ((uint32_t*)cnt)[i] = 0;
     __syncthreads();
     for (int64_t i = slo; i < shi; ++i) {
-      const int e = topk_ids[i];
+      const int e = topk_ids[i << id_shift];
       if (e >= 0 && e < E) cnt[e * LD + tid] += 1;
     }
     __syncthreads();
@@ -561,7 +377,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_place_kernel(const int32_t*
     for (int e = tid; e < E; e += T) total[e] = 0;
     __syncthreads();
     for (int64_t i = lo + tid; i < hi; i += T) {
-      const int e = topk_ids[i];
+      const int e = topk_ids[i << id_shift];
       if (e >= 0 && e < E) atomicAdd(&total[e], 1);
     }
   }
@@ -610,7 +426,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_place_kernel(const int32_t*
   // ---- 3. placement -------------------------------------------------------------------------------------
   if (seg_mode) {
     for (int64_t i = slo; i < shi; ++i) {
-      const int e = topk_ids[i];
+      const int e = topk_ids[i << id_shift];
       if (e >= 0 && e < E) {
         const int32_t pos = start[e] + base[e] + cnt[e * LD + tid];
         cnt[e * LD + tid] += 1;
@@ -623,7 +439,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_place_kernel(const int32_t*
     if (tid < 64) {
       for (int64_t i0 = lo; i0 < hi; i0 += 64) {
         const int64_t i = i0 + tid;
-        int e = i < hi ? topk_ids[i] : -1;
+        int e = i < hi ? topk_ids[i << id_shift] : -1;
         if (e >= E) e = -1;
         bool todo = e >= 0;
         while (__any(todo)) {
@@ -775,11 +591,13 @@ int64_t moe_align_workspace_bytes(int64_t num_ids, int32_t num_experts) {
   return blocks > 1 ? blocks * num_experts * (int64_t)sizeof(int32_t) : 0;
 }
 
-int launch_moe_align(const int32_t* topk_ids, int64_t num_ids, int32_t num_experts, int32_t tile_m,
+int launch_moe_align(const void* ids, int ids64, int64_t num_ids, int32_t num_experts, int32_t tile_m,
                      int32_t* sorted_token_ids, int32_t* sorted_expert_ids, int32_t* num_slots_out,
                      int64_t max_slots, int32_t* counts, hipStream_t stream) {
   int64_t chunk, blocks;
   moe_align_plan(num_ids, chunk, blocks);
+  const int32_t* topk_ids = (const int32_t*)ids;
+  const int id_shift = ids64 ? 1 : 0;
   const bool seg = num_experts <= kAlignSegExperts;
   const size_t lds = (size_t)(3 * num_experts + 1 + kAlignThreads) * sizeof(int32_t) +
                      (seg ? (size_t)num_experts * (kAlignThreads + 2) * sizeof(uint16_t) : 0);
@@ -794,11 +612,11 @@ int launch_moe_align(const int32_t* topk_ids, int64_t num_ids, int32_t num_exper
   }
   if (blocks > 1) {
     hipLaunchKernelGGL(moe_hist_kernel, dim3((unsigned)blocks), dim3(kAlignThreads), (size_t)num_experts * sizeof(int32_t),
-                       stream, topk_ids, num_ids, num_experts, chunk, counts);
+                       stream, topk_ids, id_shift, num_ids, num_experts, chunk, counts);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_hist_kernel launch: %s", hipGetErrorString(e));
   }
-  hipLaunchKernelGGL(moe_place_kernel, dim3((unsigned)blocks), dim3(kAlignThreads), lds, stream, topk_ids, num_ids,
+  hipLaunchKernelGGL(moe_place_kernel, dim3((unsigned)blocks), dim3(kAlignThreads), lds, stream, topk_ids, id_shift, num_ids,
                      num_experts, tile_m, chunk, counts, sorted_token_ids, sorted_expert_ids, num_slots_out, max_slots);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_place_kernel launch: %s", hipGetErrorString(e));

@@ -112,12 +112,19 @@ struct GemmArgs {
   int64_t b_expert_stride;   // bytes between experts in B
   int64_t bs_expert_stride;  // dwords between experts in Bs
   int64_t a_rows;            // rows of the A tensor (for the buffer descriptor)
-  int32_t stagger;           // 1: workgroups start their K walk at different quads
   // split-K (one-tile kernels only): K is the slice length, slice i reads the scales / writes the partial
   // output i strides further on
   int32_t k_splits;
   int64_t as_split_stride, bs_split_stride;   // dwords
   int64_t c_split_stride;                     // elements of C
+  // batch of equal products (one-tile kernels only, blockIdx.z): bytes / dwords / elements of C from one to the next
+  int32_t batch;
+  int64_t a_batch, b_batch, as_batch, bs_batch, c_batch;
+  const float* acc;          // what is added to the product (fp32, laid out like C); null: C itself if `accumulate`
+  // grouped gate + up projection with the activation quantised in the epilogue (ping-pong kernel): W holds up_half gate
+  // rows, then up_half up rows; silu(gate) * up goes to q [slot id][up_half] (E4M3) and qs [slot id][up_half / 32]
+  uint8_t* q; uint8_t* qs;
+  int32_t up_half, scale_mode;
 };
 
 int launch_gemm_mfma(const GemmArgs& g, int kernel_id, hipStream_t stream);
@@ -182,7 +189,7 @@ int launch_quantize(const QuantArgs& q, hipStream_t stream);
 
 // `counts`: moe_align_workspace_bytes(num_ids, num_experts) bytes of scratch (per-chunk histograms)
 int64_t moe_align_workspace_bytes(int64_t num_ids, int32_t num_experts);
-int launch_moe_align(const int32_t* topk_ids, int64_t num_ids, int32_t num_experts, int32_t tile_m,
+int launch_moe_align(const void* topk_ids, int ids64, int64_t num_ids, int32_t num_experts, int32_t tile_m,
                      int32_t* sorted_token_ids, int32_t* sorted_expert_ids, int32_t* num_slots_out,
                      int64_t max_slots, int32_t* counts, hipStream_t stream);
 

@@ -43,7 +43,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, lds_u8* const smem,
 
   // ---- tile of C owned by this workgroup: XCD-aware, then grouped along M --------------------------
   const int tiles_m = (g.M + C::BM - 1) / C::BM, tiles_n = (g.N + C::BN - 1) / C::BN;
-  int tile_m, tile_n, tile_lid;
+  int tile_m, tile_n;
   {
     const int total = tiles_m * tiles_n;
     // workgroup ids are dealt round-robin to the 8 XCDs (each has its own L2): give every XCD one
@@ -57,7 +57,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, lds_u8* const smem,
     const int in = lid % in_group;
     tile_m = first_m + in % gsz;
     tile_n = in / gsz;
-    tile_lid = lid;
   }
   const int m0 = tile_m * C::BM, n0 = tile_n * C::BN;
 
@@ -170,28 +169,21 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, lds_u8* const smem,
   constexpr int LOAD_ITERS = C::MT >= 2 ? C::MT / 2 : 1;
   constexpr int LPI = (TOTAL_LOADS + LOAD_ITERS - 1) / LOAD_ITERS;
 
-  // K is walked in quads of four 128-element steps.  Workgroups that run side by side start at different
-  // quads (and wrap around): with power-of-two row pitches all rows of a stage live in the same memory
-  // channel, and without the stagger every workgroup would ask that one channel at the same time.
+  // K is walked in quads of four 128-element steps.
   constexpr int SPQ = 4 / C::KSUB;   // stages per quad
-  const int q_start = (g.stagger && ksteps % 4 == 0) ? tile_lid % KQ : 0;
-  load_scales(q_start, sa, sb);
+  load_scales(0, sa, sb);
 #pragma unroll
-  for (int idx = 0; idx < TOTAL_LOADS; ++idx) issue_one(idx, q_start * SPQ, 0, true);
+  for (int idx = 0; idx < TOTAL_LOADS; ++idx) issue_one(idx, 0, 0, true);
   int buf = 0;
-  for (int Qi = 0; Qi < KQ; ++Qi) {
-    const int Q = Qi + q_start < KQ ? Qi + q_start : Qi + q_start - KQ;
-    const int Qn = Q + 1 < KQ ? Q + 1 : 0;
-    load_scales(Qn, sa_n, sb_n);
+  for (int Q = 0; Q < KQ; ++Q) {
+    load_scales(Q + 1, sa_n, sb_n);
 #pragma unroll
     for (int t0 = 0; t0 < 4; t0 += C::KSUB) {
       const int s = Q * SPQ + t0 / C::KSUB;
-      const int it = Qi * SPQ + t0 / C::KSUB;        // position in the (rotated) walk
-      if (it < nstages) {
+      if (s < nstages) {
         __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this thread's LDS-DMA of stage s landed
         __syncthreads();                      // everyone's landed; everyone left stage s-1's buffer
-        const bool more = it + 1 < nstages;
-        const int sn = (t0 / C::KSUB + 1 < SPQ) ? s + 1 : Qn * SPQ;   // stage that follows in the walk
+        const bool more = s + 1 < nstages;
         lds_u8* const atile = smem + buf * C::STAGE + (wm0 + r) * C::A_RB;
         // B rows go to the instruction in the order bperm_row (mx_common.h): tile j of a 64-row group is rows
         // bperm_tile_off(j) + bperm_lane_off(lane % 16), which is also the order of the packed B scales
@@ -214,7 +206,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, lds_u8* const smem,
             if (kk == 0 && i < LOAD_ITERS) {
 #pragma unroll
               for (int l = 0; l < LPI; ++l)
-                if (i * LPI + l < TOTAL_LOADS) issue_one(i * LPI + l, sn, buf ^ 1, more);
+                if (i * LPI + l < TOTAL_LOADS) issue_one(i * LPI + l, s + 1, buf ^ 1, more);
             }
             // keep the DMA loads in the tile iteration they were written in; everything else may move
             __builtin_amdgcn_sched_barrier(0x78F);

@@ -502,6 +502,9 @@ int launch_pp_pair(const GemmArgs& g, hipStream_t stream) {
 }
 #if MX_PP_PAIR == 0
 template int launch_pp_pair<MX_E4M3, MX_E4M3>(const GemmArgs&, hipStream_t);
+extern template int launch_pp_pair<MX_E5M2, MX_E5M2>(const GemmArgs&, hipStream_t);
+extern template int launch_pp_pair<MX_E2M1, MX_E2M1>(const GemmArgs&, hipStream_t);
+extern template int launch_pp_pair<MX_E4M3, MX_E2M1>(const GemmArgs&, hipStream_t);
 
 int launch_gemm_pingpong(const GemmArgs& g, hipStream_t stream) {
   if (g.c_dtype != MX_F32 && g.c_dtype != MX_BF16)

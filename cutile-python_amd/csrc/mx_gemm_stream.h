@@ -28,22 +28,24 @@
 
 namespace mx {
 
-constexpr int kStreamWaves = 8;
-
-template <int XF_, int WF_, int NT_, int MT_, bool PACKED_>
+// UP: the four tiles of a wave are 32 rows of the gate half of W and the 32 rows of the up half that belong to them.
+template <int XF_, int WF_, int NT_, int MT_, bool PACKED_, int WAVES_ = 8, bool UP_ = false>
 struct StreamCfg {
-  static constexpr int XF = XF_, WF = WF_, NT = NT_, MT = MT_;
-  static constexpr bool PACKED = PACKED_;
+  static constexpr int XF = XF_, WF = WF_, NT = NT_, MT = MT_, WAVES = WAVES_;
+  static constexpr bool PACKED = PACKED_, UP = UP_;
+  static constexpr int NSW = PACKED ? (UP ? 2 : 1) : NT;  // scale registers (x 4) of W per K-quad
   static constexpr int SK = WF == MX_E2M1 ? 2 : 1;        // K-steps per stage
   static constexpr int SPQ = 4 / SK;                      // stages per K-quad
   static constexpr int WEB = WF == MX_E2M1 ? 4 : 8;
   static constexpr int L = 2 * MT * SK + 2 * NT;          // load instructions per stage
-  static constexpr int NSC = MT + (PACKED ? 1 : NT);      // scale load instructions per K-quad
+  static constexpr int NSC = MT + NSW;      // scale load instructions per K-quad
   static constexpr int XSLOT = MT * SK * 2048;            // LDS bytes of one stage of X
-  static constexpr int TP = NT >= 2 ? 2 : 1;              // tiles of W re-sorted at a time
+  // tiles of W re-sorted at a time (one where that lets two workgroups of four waves share a CU's LDS)
+  static constexpr int TP = NT >= 2 && !(WAVES == 4 && XSLOT == 8192) ? 2 : 1;
   static constexpr int WAVE_BYTES = 2 * XSLOT + TP * 2048;
-  static constexpr int RED = kStreamWaves * NT * MT * 1024;   // partial sums: [wave][tile][lane] float4
-  static constexpr int LDS_BYTES = kStreamWaves * WAVE_BYTES > RED ? kStreamWaves * WAVE_BYTES : RED;
+  static constexpr int RED = WAVES * NT * MT * 1024;   // partial sums: [wave][tile][lane] float4
+  static constexpr int LDS_BYTES = WAVES * WAVE_BYTES > RED ? WAVES * WAVE_BYTES : RED;
+  static_assert(!UP || NT == 4, "two tiles of gate, two of up");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
   static_assert(L + NSC < 63, "vmcnt range");
 };
@@ -57,15 +59,16 @@ struct StreamWave {
 // LDS as it comes, so its chunks are swizzled on the way in; W is swizzled when it is written to the scratch area.
 __device__ inline uint32_t stream_x_col(int q, int lane) { return (uint32_t)(((lane & 7) ^ swz<8>(8 * q + (lane >> 3))) << 4); }
 
-// acc[i][j] of the wave: rows 16 i + lane % 16 of X, tile j0 + j of its group of W, K-quads [Q0, Q1) (the last one may be
+// acc[i][j] of the wave: rows 16 i + lane % 16 of X, tile j0[0] + j of its group of W, K-quads [Q0, Q1) (the last one may be
 // partial: ksteps in all).  xvo: lane offsets of the 2 MT DMA instructions of a K-step of X (kOobOffset: no such row);
 // xso: lane offset of the 16 scale bytes of row 16 i + lane % 16; wvo: lane offsets of the 2 NT load instructions of a
 // stage of W (rows 8 h + lane / 8 of tile j in instruction 2 j + h); wso: lane offset of the scales of tile j's row
-// lane % 16 (packed: one, of the group).
+// lane % 16 (packed: one, of the group; UP: two, of the groups that the gate and the up rows lie in, whose first tiles
+// are j0[0] and j0[1]).
 template <class C>
 __device__ __forceinline__ void stream_products(const StreamWave& w, lds_u8* const lds, const uint32_t (&xvo)[2 * C::MT],
                                                 const uint32_t (&xso)[C::MT], const uint32_t (&wvo)[2 * C::NT],
-                                                const uint32_t (&wso)[C::PACKED ? 1 : C::NT], const int j0, const int Q0,
+                                                const uint32_t (&wso)[C::NSW], const int (&j0)[C::UP ? 2 : 1], const int Q0,
                                                 const int Q1, const int ksteps, v4f (&acc)[C::MT][C::NT]) {
   constexpr int NT = C::NT, MT = C::MT, SK = C::SK, TP = C::TP;
   typedef __attribute__((address_space(3))) v4i lds_w4i;
@@ -73,19 +76,21 @@ __device__ __forceinline__ void stream_products(const StreamWave& w, lds_u8* con
   const int s1 = Q1 * 4 < ksteps ? Q1 * 4 : ksteps;
   lds_u8* const scr = lds + 2 * C::XSLOT;
   v4i wr[2][NT][2];
-  v4i sx[MT], sxn[MT], sw[C::PACKED ? 1 : NT], swn[C::PACKED ? 1 : NT];
+  v4i sx[MT], sxn[MT], sw[C::NSW], swn[C::NSW];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-  auto load_scales = [&](int Q, v4i (&x)[MT], v4i (&ws)[C::PACKED ? 1 : NT]) {
+  auto load_scales = [&](int Q, v4i (&x)[MT], v4i (&ws)[C::NSW]) {
     const bool live = Q < Q1;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
       x[i] = __builtin_amdgcn_raw_buffer_load_b128(w.rsXs, live ? xso[i] : kOobOffset, Q * 16, 0);
     if constexpr (C::PACKED) {
-      ws[0] = __builtin_amdgcn_raw_buffer_load_b128(w.rsWs, live ? wso[0] : kOobOffset, Q * 1024, 0);
+#pragma unroll
+      for (int j = 0; j < C::NSW; ++j)
+        ws[j] = __builtin_amdgcn_raw_buffer_load_b128(w.rsWs, live ? wso[j] : kOobOffset, Q * 1024, 0);
     } else {
 #pragma unroll
       for (int j = 0; j < NT; ++j)
@@ -156,9 +161,11 @@ __device__ __forceinline__ void stream_products(const StreamWave& w, lds_u8* con
 #pragma unroll
             for (int j = jb; j < jb + TP; ++j) {
               if constexpr (C::PACKED) {
-                // a full group's tiles are the four bytes; fewer tiles per wave start at byte j0, shifted down
-                const int ws = NT == 4 ? sw[0][u] : (int)((uint32_t)sw[0][u] >> (8 * j0));
-                acc[i][j] = mfma_scaled<C::WF, C::XF>(wf[kk][j - jb], xf[kk][i], acc[i][j], j, ws, 0, xs);
+                // a full group's tiles are the four bytes; fewer tiles of a group start at byte j0, shifted down
+                constexpr bool whole = NT == 4 && !C::UP;
+                const int g = C::UP ? j / 2 : 0;
+                const int ws = whole ? sw[0][u] : (int)((uint32_t)sw[g][u] >> (8 * j0[g]));
+                acc[i][j] = mfma_scaled<C::WF, C::XF>(wf[kk][j - jb], xf[kk][i], acc[i][j], C::UP ? j % 2 : j, ws, 0, xs);
               } else {
                 acc[i][j] = mfma_scaled<C::WF, C::XF>(wf[kk][j - jb], xf[kk][i], acc[i][j], 0,
                                                       (int)((uint32_t)sw[j][u] >> (8 * gq)), 0, xs);
@@ -184,7 +191,7 @@ __device__ __forceinline__ void stream_products(const StreamWave& w, lds_u8* con
 #pragma unroll
     for (int i = 0; i < MT; ++i) sx[i] = sxn[i];
 #pragma unroll
-    for (int j = 0; j < (C::PACKED ? 1 : NT); ++j) sw[j] = swn[j];
+    for (int j = 0; j < C::NSW; ++j) sw[j] = swn[j];
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // the trailing zero-fill DMA has left the queue: LDS may be reused
 }

@@ -7,13 +7,13 @@ namespace {
 // Workgroup of 8 waves: kw K ranges x 8 / kw units of NT tiles.  m_tiles row tiles of 16 MT rows are neighbours in
 // dispatch order on the same XCD (workgroup ids go round-robin over 8 XCDs), so W is read from memory once.
 template <class C>
-__global__ __launch_bounds__(kStreamWaves * 64) void stream_kernel(const StreamArgs a) {
+__global__ __launch_bounds__(C::WAVES * 64) void stream_kernel(const StreamArgs a) {
   constexpr int NT = C::NT, MT = C::MT;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_generic[];
   lds_u8* const smem = (lds_u8*)smem_generic;
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, gq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kq = wave % a.kw, nw = wave / a.kw, nwv = kStreamWaves / a.kw;
+  const int kq = wave % a.kw, nw = wave / a.kw, nwv = C::WAVES / a.kw;
   int unit0 = blockIdx.x, mt = 0;
   if (a.m_tiles > 1) {
     const int per = 8 * a.m_tiles, hi = unit0 / per, in = unit0 % per;
@@ -23,7 +23,7 @@ __global__ __launch_bounds__(kStreamWaves * 64) void stream_kernel(const StreamA
   }
   const int m0 = mt * 16 * MT;
   const int u = unit0 * nwv + nw;                    // unit of NT tiles
-  const int G = u * NT / 4, j0 = u * NT % 4;
+  const int G = u * NT / 4, j0[1] = {u * NT % 4};
   const int KQ = (a.K + 511) / 512;
   const int Q0 = kq * KQ / a.kw, Q1 = (kq + 1) * KQ / a.kw;
 
@@ -33,7 +33,7 @@ __global__ __launch_bounds__(kStreamWaves * 64) void stream_kernel(const StreamA
   w.rsW = make_rsrc(a.W, (uint32_t)((int64_t)(a.N - 1) * a.ldw + (int64_t)a.K * (C::WF == MX_E2M1 ? 1 : 2) / 2));
   w.rsWs = C::PACKED ? make_rsrc(a.Ws, (uint32_t)(packed_scale_dwords(a.N, a.K) * 4))
                      : make_rsrc(a.Ws, (uint32_t)((int64_t)(a.N - 1) * a.ldws + a.K / 32));
-  uint32_t xvo[2 * MT], xso[MT], wvo[2 * NT], wso[C::PACKED ? 1 : NT];
+  uint32_t xvo[2 * MT], xso[MT], wvo[2 * NT], wso[C::NSW];
 #pragma unroll
   for (int q = 0; q < 2 * MT; ++q) {
     const int m = m0 + 8 * q + (lane >> 3);
@@ -46,11 +46,11 @@ __global__ __launch_bounds__(kStreamWaves * 64) void stream_kernel(const StreamA
   }
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
-    const int n = 64 * G + bperm_row(j0 + j, r);
+    const int n = 64 * G + bperm_row(j0[0] + j, r);
     if constexpr (!C::PACKED) wso[j] = n < a.N ? (uint32_t)(n * a.ldws) : kOobOffset;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int nl = 64 * G + bperm_row(j0 + j, 8 * h + (lane >> 3));
+      const int nl = 64 * G + bperm_row(j0[0] + j, 8 * h + (lane >> 3));
       wvo[2 * j + h] = nl < a.N ? (uint32_t)(nl * a.ldw + (lane & 7) * 16) : kOobOffset;
     }
   }
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(kStreamWaves * 64) void stream_kernel(const StreamA
   // item = (unit, row tile, tile pair) of the workgroup; lane (c, g) of tile j holds row c, columns
   // bperm_tile_off(j) + 8 g .. + 3 of the group, so a pair of tiles is 8 consecutive outputs of a lane
   constexpr int JP = NT >= 2 ? 2 : 1;
-  for (int it = wave; it < nwv * MT * (NT / JP); it += kStreamWaves) {   // uniform per wave
+  for (int it = wave; it < nwv * MT * (NT / JP); it += C::WAVES) {   // uniform per wave
     const int jp = it % (NT / JP), i = it / (NT / JP) % MT, wv = it / (NT / JP) / MT;
     v4f v[2] = {};
     for (int k = 0; k < a.kw; ++k)
@@ -105,7 +105,7 @@ int launch(const StreamArgs& a, int blocks, hipStream_t stream) {
       return set_error(MX_ERR_LAUNCH, "hipFuncSetAttribute(%d bytes LDS): %s", C::LDS_BYTES, hipGetErrorString(e));
     attr_done = 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kStreamWaves * 64), C::LDS_BYTES, stream, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::WAVES * 64), C::LDS_BYTES, stream, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "stream_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
@@ -160,7 +160,7 @@ int launch_gemm_stream(const StreamArgs& a0, hipStream_t stream) {
   for (int n = 4; n >= 1; n >>= 1)
     for (int kw = 8; kw >= 1; kw >>= 1) {
       if (kw > 1 && kw > KQ) continue;
-      const int units = (tiles + n * (kStreamWaves / kw) - 1) / (n * (kStreamWaves / kw));
+      const int units = (tiles + n * (8 / kw) - 1) / (n * (8 / kw));
       const int64_t rounds = ((int64_t)units * a.m_tiles + 255) / 256;
       const float t = rounds * ((KQ + kw - 1) / kw * (n * wb + xb) + 3.f);
       if (t < best) { best = t; nt = n; a.kw = kw; a.units = units; }

@@ -32,6 +32,8 @@ struct Lib {
   MX_FN(mx_gemm_list_workspace_bytes);
   MX_FN(mx_quantize);
   MX_FN(mx_silu_mul_quantize);
+  MX_FN(mx_moe_forward);
+  MX_FN(mx_moe_forward_workspace_bytes);
 } lib;
 #undef MX_FN
 PyObject* packed_type = nullptr;   // ops.PackedScales
@@ -283,6 +285,69 @@ PyObject* py_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return res;
 }
 
+// scales of a stack of expert weights: a [E, rows, K/32] E8M0 tensor or a PackedScales of it
+bool expert_scale_desc(PyObject* o, int64_t E, int64_t rows, int64_t K, const at::Device& dev, mx_tensor* d, int32_t* layout) {
+  if (THPVariable_Check(o)) {
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (!is_e8m0(t) || t.device() != dev || t.dim() != 3) return false;
+    *d = desc(t, MX_E8M0);
+    *layout = MX_SCALE_2D;
+    return true;
+  }
+  if ((PyObject*)Py_TYPE(o) != packed_type) return false;
+  PyObject* pb = PyObject_GetAttr(o, s_batch);
+  const bool ok = pb && PyLong_AsLongLong(pb) == E;
+  Py_XDECREF(pb);
+  if (PyErr_Occurred()) { PyErr_Clear(); return false; }
+  if (!ok || !scale_desc(o, rows, K, true, dev, d, layout) || *layout != MX_SCALE_NATIVE) return false;
+  d->ndim = 3;
+  d->shape[0] = E; d->shape[1] = rows; d->shape[2] = K / 32;
+  d->stride[0] = rows * (K / 32); d->stride[1] = K / 32; d->stride[2] = 1;
+  return true;
+}
+
+// moe(hidden, hidden_scale, w1, w1_scale, w2, w2_scale, topk_weights, topk_ids, out_dtype, mode, w_format)
+//   -> result, error code, or None
+PyObject* py_moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 11) { PyErr_SetString(PyExc_TypeError, "moe takes 11 arguments"); return nullptr; }
+  for (int i : {0, 1, 2, 4, 6, 7})
+    if (!THPVariable_Check(a[i])) Py_RETURN_NONE;
+  const at::Tensor &X = THPVariable_Unpack(a[0]), &Xs = THPVariable_Unpack(a[1]), &W1 = THPVariable_Unpack(a[2]),
+                   &W2 = THPVariable_Unpack(a[4]), &wt = THPVariable_Unpack(a[6]), &ids = THPVariable_Unpack(a[7]);
+  if (X.dim() != 2 || Xs.dim() != 2 || W1.dim() != 3 || W2.dim() != 3 || ids.dim() != 2 || !on_current_device(X)) Py_RETURN_NONE;
+  const at::Device dev = X.device();
+  if (Xs.device() != dev || W1.device() != dev || W2.device() != dev || wt.device() != dev || ids.device() != dev) Py_RETURN_NONE;
+  const int f1 = elem_format(W1, a[10]), f2 = elem_format(W2, a[10]);
+  if (X.scalar_type() != at::kFloat8_e4m3fn || !is_e8m0(Xs) || f1 != f2 || (f1 != MX_E4M3 && f1 != MX_E2M1)) Py_RETURN_NONE;
+  if (f1 == MX_E2M1 && (W1.stride(2) != 1 || W2.stride(2) != 1)) Py_RETURN_NONE;
+  const int64_t T = X.size(0), topk = ids.size(1), E = W1.size(0);
+  if (ids.size(0) != T || T == 0 || topk == 0 || topk > 1 << 20 || !ids.is_contiguous() ||
+      (ids.scalar_type() != at::kInt && ids.scalar_type() != at::kLong) || wt.scalar_type() != at::kFloat ||
+      !wt.is_contiguous() || wt.numel() != T * topk || !THPDtype_Check(a[8]))
+    Py_RETURN_NONE;
+  const auto out_t = ((THPDtype*)a[8])->scalar_type;
+  if (out_code(out_t) < 0) Py_RETURN_NONE;
+  mx_tensor dX = desc(X, MX_E4M3), dXs = desc(Xs, MX_E8M0), dW1 = desc(W1, f1, f1 == MX_E2M1 ? 2 : -1),
+            dW2 = desc(W2, f2, f2 == MX_E2M1 ? 2 : -1), dW1s, dW2s;
+  mx_gemm_opts o = {sizeof(mx_gemm_opts), 0, 0, 0, MX_KERNEL_AUTO, 32, 0, 0};
+  if (!expert_scale_desc(a[3], E, dW1.shape[1], dW1.shape[2], dev, &dW1s, &o.a_scale_layout) ||
+      !expert_scale_desc(a[5], E, dW2.shape[1], dW2.shape[2], dev, &dW2s, &o.b_scale_layout))
+    Py_RETURN_NONE;
+  at::Tensor out = device_empty({T, dW2.shape[1]}, out_t, dev);
+  mx_tensor dO = desc(out, out_code(out_t));
+  const int mode = (int)PyLong_AsLong(a[9]);
+  const int64_t need = lib.p_mx_moe_forward_workspace_bytes(T, (int32_t)topk, &dW1, &dW2, &o);
+  at::Tensor ws = device_empty({need > 0 ? need : 1}, at::kByte, dev);
+  int rc;
+  {
+    NoGil nogil;
+    rc = lib.p_mx_moe_forward(&dX, &dXs, &dW1, &dW1s, &dW2, &dW2s, (const float*)wt.data_ptr(), ids.data_ptr(),
+                              ids.scalar_type() == at::kLong, (int32_t)topk, &dO, mode, &o, ws.data_ptr(), need, stream_of(dev));
+  }
+  if (rc == MX_ERR_LAYOUT) Py_RETURN_NONE;   // nothing was enqueued: operands for the single operators
+  return rc_or(rc, out);
+}
+
 // bind(handle of the loaded libmxgemm.so, PackedScales class)
 PyObject* py_bind(PyObject*, PyObject* args) {
   unsigned long long h;
@@ -299,6 +364,8 @@ PyObject* py_bind(PyObject*, PyObject* args) {
   MX_FN(mx_gemm_list_workspace_bytes)
   MX_FN(mx_quantize)
   MX_FN(mx_silu_mul_quantize)
+  MX_FN(mx_moe_forward)
+  MX_FN(mx_moe_forward_workspace_bytes)
 #undef MX_FN
   Py_INCREF(cls);
   Py_XDECREF(packed_type);
@@ -319,6 +386,7 @@ PyMethodDef methods[] = {
     {"gemm", (PyCFunction)(void (*)(void))guarded<py_gemm>, METH_FASTCALL, nullptr},
     {"gemm_list", (PyCFunction)(void (*)(void))guarded<py_gemm_list>, METH_FASTCALL, nullptr},
     {"quantize", (PyCFunction)(void (*)(void))guarded<py_quantize>, METH_FASTCALL, nullptr},
+    {"moe", (PyCFunction)(void (*)(void))guarded<py_moe>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_mxhost", nullptr, -1, methods};
 

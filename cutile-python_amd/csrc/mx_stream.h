@@ -17,4 +17,20 @@ struct StreamArgs {
 bool stream_supports(int x_fmt, int w_fmt);
 int launch_gemm_stream(const StreamArgs& a, hipStream_t stream);
 
+// mixture-of-experts layer at decode sizes (mx_moe.hip)
+constexpr int kMoeMaxIds = 2048;   // routed ids that a workgroup sorts out by itself
+struct MoeStreamArgs {
+  const uint8_t* X; const uint8_t* Xs; const uint8_t* W; const uint8_t* Ws;
+  const void* ids; const float* weights;
+  uint8_t* q; uint8_t* qs; float* C;   // up: elements and scales [n_ids][F]; down: [n_ids][N]
+  int64_t ldx, ldxs, ldw, ldws, w_es, ws_es;   // bytes; *_es: between experts
+  int32_t x_rows, N, K, F;             // N: rows of an expert's W (up: 2 F)
+  int32_t n_ids, ids64, E, replicas;   // a routed copy `id` reads row id / replicas of X
+  int32_t w_fmt, ws_packed, scale_mode;
+  int32_t kw, units;                   // chosen by the launcher
+};
+int launch_moe_stream(const MoeStreamArgs& a, bool up, hipStream_t stream);
+int launch_moe_combine(const float* c, const void* ids, int ids64, int E, int64_t T, int topk, int64_t H, void* out,
+                       int out_dtype, hipStream_t stream);
+
 }  // namespace mx

@@ -73,6 +73,11 @@ SYMBOLS = {
     "mx_moe_align": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32,
                                     ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                     ctypes.c_int64, ctypes.c_void_p]),
+    "mx_moe_forward_workspace_bytes": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int32, _P(MxTensor), _P(MxTensor),
+                                                        _P(MxGemmOpts)]),
+    "mx_moe_forward": (ctypes.c_int, [_P(MxTensor)] * 6 + [
+        ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, _P(MxTensor), ctypes.c_int32,
+        _P(MxGemmOpts), ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]),
     "mx_bench_gemm": (ctypes.c_int, [ctypes.c_int32] + [_P(MxTensor)] * 5 + [
         _P(MxGemmOpts), ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32,
         _P(ctypes.c_float), ctypes.c_void_p]),

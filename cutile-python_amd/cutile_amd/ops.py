@@ -880,6 +880,14 @@ def cutile_moe_scaled(hidden_states: torch.Tensor, hidden_scale: torch.Tensor,
     :class:`PackedScales`; topk_weights / topk_ids (tokens, topk).  The intermediate activation is
     re-quantised to E4M3 on the device (one fused pass) so that both GEMMs run block-scaled.  Nothing in the
     call synchronises with the host.  Returns (tokens, H) in ``out_dtype``."""
+    if kernel == "auto" and scale_mode in ("floor", "ceil"):
+        # one library call for the whole layer (tile_m is then the library's choice: results do not depend on it)
+        r = L.host().moe(hidden_states, hidden_scale, w1, w1_scale, w2, w2_scale, topk_weights, topk_ids, out_dtype,
+                         1 if scale_mode == "floor" else 0, w_format)
+        if isinstance(r, torch.Tensor):
+            return r
+        if r is not None:
+            _raise_code(r)
     if hidden_states.dim() != 2 or w1.dim() != 3 or w2.dim() != 3:
         raise TileTypeError("hidden_states must be 2D, w1 and w2 3D")
     T = hidden_states.shape[0]

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define MXGEMM_VERSION 103
+#define MXGEMM_VERSION 104
 
 /* Exported symbols (the library is built with hidden default visibility). */
 #if defined(__GNUC__)
@@ -291,6 +291,25 @@ MX_API int mx_quantize(const mx_tensor* x, mx_tensor* xq, mx_tensor* scale, int3
  */
 MX_API int mx_silu_mul_quantize(const mx_tensor* gate_up, mx_tensor* xq, mx_tensor* scale, int32_t scale_mode,
                          void* stream);
+
+/*
+ * The whole mixture-of-experts layer, cutile_moe (samples/MoE.py:197-288) with block-scaled products:
+ *   out[t,:] = sum_j w[t,j] * ( quantise(silu(g) * u) @ W2[e].T ),  [g | u] = bf16(X[t,:] @ W1[e].T),  e = ids[t,j]
+ *   X [T,H] MX_E4M3, Xs [T,H/32]; W1 [E,2F,H], W2 [E,H_out,F] MX_E4M3 or MX_E2M1 (packed along K), their scales plain
+ *   [E,rows,K/32] or MX_SCALE_NATIVE (operand B; opts->a_scale_layout is W1's, b_scale_layout W2's layout here);
+ *   topk_weights [T,topk] fp32; topk_ids [T,topk] int32 (ids64 = 0) or int64 (1), contiguous; ids outside [0, E) drop
+ *   their copy.  The activation between the projections is E4M3, quantised by scale_mode as in mx_quantize.
+ *   out [T,H_out] MX_F32 or MX_BF16, contiguous.
+ * A few rows per expert stream the experts' weights (three launches in all); more run as alignment, grouped GEMM,
+ * activation, grouped GEMM and sum.  No host synchronisation.  Returns MX_ERR_LAYOUT, with nothing enqueued, for
+ * operands that only the single entry points take (generic-kernel layouts).
+ */
+MX_API int64_t mx_moe_forward_workspace_bytes(int64_t T, int32_t topk, const mx_tensor* W1, const mx_tensor* W2,
+                                       const mx_gemm_opts* opts);
+MX_API int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1, const mx_tensor* W1s,
+                   const mx_tensor* W2, const mx_tensor* W2s, const float* topk_weights, const void* topk_ids,
+                   int32_t ids64, int32_t topk, mx_tensor* out, int32_t scale_mode, const mx_gemm_opts* opts,
+                   void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * Re-lays a scale tensor into an MFMA-ready native layout consumed by the MFMA kernels

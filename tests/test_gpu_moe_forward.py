@@ -1,0 +1,55 @@
+"""GPU parity of the whole mixture-of-experts layer (cutile_moe_scaled -> mx_moe_forward) where its splits can go wrong:
+one row, rows around the row tiles, experts with no row and with more rows than a pass takes, routed ids outside the
+experts, column counts that leave a workgroup partly idle, plain and packed scales, both id widths, and the sizes on
+either side of the switch to grouped GEMMs."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import mx_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _elems(codes, fmt, dev):
+    return torch.from_numpy(O.pack_fp4(codes)).to(dev) if fmt == O.E2M1 else torch.from_numpy(codes).to(dev).view(torch.float8_e4m3fn)
+
+
+def _scale(sc, dev):
+    return torch.from_numpy(sc).to(dev).view(torch.float8_e8m0fnu)
+
+
+# T, H, F, E, topk, skew: share of the copies that go to expert 0
+CASES = [(1, 128, 128, 4, 2, 0.0), (17, 256, 128, 8, 1, 0.0), (48, 512, 256, 4, 2, 0.0), (40, 640, 384, 3, 1, 1.0),
+         (33, 1024, 256, 16, 4, 0.7), (64, 128, 640, 8, 2, 0.5), (150, 256, 128, 2, 2, 0.9), (700, 256, 256, 16, 4, 0.3)]
+
+
+@pytest.mark.parametrize("packed", [False, True], ids=["plain", "packed"])
+@pytest.mark.parametrize("w_fmt", [O.E4M3, O.E2M1], ids=str)
+@pytest.mark.parametrize("T,H,F,E,topk,skew", CASES)
+def test_moe_forward(ct, dev, T, H, F, E, topk, skew, w_fmt, packed):
+    rng = np.random.default_rng(T * 7 + F)
+    H_out = H + 72                       # not a multiple of a tile
+    hq, hs = O.block_quantize(rng.standard_normal((T, H)).astype(np.float32), 32, O.E4M3, "floor")
+    w1q, w1s = O.block_quantize((rng.standard_normal((E, 2 * F, H)) * 0.2).astype(np.float32), 32, w_fmt, "floor")
+    w2q, w2s = O.block_quantize((rng.standard_normal((E, H_out, F)) * 0.2).astype(np.float32), 32, w_fmt, "floor")
+    ids = rng.integers(0, E, (T, topk))
+    ids[rng.random((T, topk)) < skew] = 0
+    lost = rng.random((T, topk)) < 0.1   # copies that no expert claims
+    wts = rng.random((T, topk)).astype(np.float32)
+    want = O.moe_forward(hq, hs, w1q, w1s, w2q, w2s, np.where(lost, 0, wts), ids, w_fmt=w_fmt)
+    ids = np.where(lost, np.where(rng.random((T, topk)) < 0.5, -1, E + 3), ids)
+    s1, s2 = _scale(w1s, dev), _scale(w2s, dev)
+    if packed:
+        s1, s2 = ct.pack_scales(s1, operand="b"), ct.pack_scales(s2, operand="b")
+    for out_dtype, id_dtype in ((torch.float32, torch.int64), (torch.bfloat16, torch.int32)):
+        got = ct.cutile_moe_scaled(_elems(hq, O.E4M3, dev), _scale(hs, dev), _elems(w1q, w_fmt, dev), s1,
+                                   _elems(w2q, w_fmt, dev), s2, torch.from_numpy(wts).to(dev),
+                                   torch.from_numpy(ids).to(dev, id_dtype), out_dtype=out_dtype,
+                                   w_format="e2m1" if w_fmt == O.E2M1 else None)
+        assert got.shape == (T, H_out) and got.dtype == out_dtype
+        # the activation is rounded to bf16 and re-quantised on both sides: a last-bit difference of the first product
+        # can move an element by one E4M3 step, as in test_moe_pipeline_matches_oracle
+        err = O.rel_fro(got.float().cpu(), want)
+        print(f"{T} {H} {F} {E} {topk} {w_fmt} packed={packed} {out_dtype}: {err:.2e}", flush=True)
+        assert err < 2e-2
