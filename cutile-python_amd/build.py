@@ -23,7 +23,7 @@ HOST_OUT = ROOT / "cutile_amd" / "_mxhost.so"   # csrc/mx_host.cpp: the operator
 OBJ = ROOT / "build"
 SOURCES = ["mx_api.hip", "mx_gemm_mfma.hip", "mx_gemm_pp32.hip", "mx_gemm_w4.hip", "mx_gemm_generic.hip", "mx_gemm_decode.hip", "mx_gemm_stream.hip", "mx_moe.hip", "mx_aux.hip", "mx_probe.hip"]
 # sources compiled once per value of a macro, so that their instances build in parallel: (file, macro, count)
-SPLIT = [("mx_gemm_pp.hip", "MX_PP_PAIR", 4)]
+SPLIT = [("mx_gemm_pp.hip", "MX_PP_PAIR", 4), ("mx_gemm_t128.hip", "T128_PAIR", 4)]
 UNITS = [(s, None) for s in SOURCES] + [(f, f"-D{m}={i}") for f, m, n in SPLIT for i in range(n)]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "mx_common.h"
+#include "mx_gemm_t128.h"
 #include "mx_stream.h"
 
 // Scratch of mx_gemm_static: lives in the library's device image, one copy per GPU the library runs on, held
@@ -35,9 +36,7 @@ inline int64_t round256(int64_t b) { return (b + 255) & ~(int64_t)255; }
 // kernel MX_KERNEL_AUTO uses for large problems
 constexpr int big_tile_kernel() { return MX_KERNEL_MFMA_PINGPONG; }
 
-// Problems MX_KERNEL_AUTO gives to the persistent 256x256 kernel: enough 256x256 tiles to occupy most of the
-// 256 CUs (measured crossover against the 128x128 one-tile kernel, which has four times as many workgroups
-// to spread: 128 tiles -> 128x128 is 14 % faster, 144 tiles -> 256x256 is 26 % faster).
+// Problems with enough 256x256 tiles to occupy most of the 256 CUs are never split along K.
 inline bool big_tile_problem(int64_t M, int64_t N) {
   return M > 128 && N > 128 && ((M + 255) / 256) * ((N + 255) / 256) >= 144;
 }
@@ -68,23 +67,40 @@ const mx_gemm_opts kDefaultOpts = {sizeof(mx_gemm_opts), 0, MX_SCALE_2D, MX_SCAL
 // (M, N, K, opts) so that mx_gemm_workspace_bytes and mx_gemm agree.  Automatic rule: split when the tiles
 // of the 128x128 kernel cover less than half of the CUs and every slice keeps at least two K-quads.
 int plan_k_splits(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
-  if (o.split_k == 1 || o.a_scale_layout != MX_SCALE_2D || o.b_scale_layout != MX_SCALE_2D || o.block_size != 32)
-    return 1;
-  if (o.kernel != MX_KERNEL_AUTO && o.kernel != MX_KERNEL_MFMA_128x128 && o.kernel != MX_KERNEL_MFMA_256x256 &&
-      o.kernel != MX_KERNEL_MFMA_256x256_W4)
-    return 1;
-  if (K <= 0 || K % 512 != 0 || M <= 0 || N <= 0) return 1;
+  const bool t256 = o.kernel == MX_KERNEL_MFMA_256x256 || o.kernel == MX_KERNEL_MFMA_256x256_W4;
+  if (o.split_k == 1 || o.block_size != 32 || K <= 0 || M <= 0 || N <= 0) return 1;
+  if (o.kernel != MX_KERNEL_AUTO && o.kernel != MX_KERNEL_MFMA_128x128 && !t256) return 1;
+  if (t256 && (o.a_scale_layout != MX_SCALE_2D || o.b_scale_layout != MX_SCALE_2D || K % 512 != 0)) return 1;
   if (o.split_k > 1) return (K % ((int64_t)512 * o.split_k) == 0) ? o.split_k : -1;   // -1: cannot honour
-  if (o.kernel != MX_KERNEL_AUTO && o.kernel != MX_KERNEL_MFMA_128x128) return 1;
+  if (t256) return 1;
   if (o.kernel == MX_KERNEL_AUTO && big_tile_problem(M, N)) return 1;   // big-tile kernel
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   if (tiles * 2 > 256 || K < 2048) return 1;
-  int64_t s = 256 / tiles;
-  if (s > K / 1024) s = K / 1024;
-  while (s > 1 && K % (512 * s) != 0) --s;
+  const int64_t s = 256 / tiles < K / 1024 ? 256 / tiles : K / 1024;
   return (int)(s < 1 ? 1 : s);
 }
 
+
+// What MX_KERNEL_AUTO weighs beyond kStreamAutoM rows: estimated time (us) of a product on the kernels that can run it.
+// Fitted to measurements of 96 .. 4096 rows x 512 .. 17456 columns x 512 .. 9216 (stages of 128 bytes of a row):
+//   128 x 128 tiles: 0.62 us per stage with one tile on a CU (1024 x 4096 x 4096 24.6 us, 2048 x 2048 x 8192 45 us), 0.97
+//     with two (2048 x 4096 x 4096 36.7 us); FP4 x FP4 0.68 / 1.2.  Split along K: the partial sums are written and read.
+//   256 x 256 tiles: 1.1 us per stage when they leave half of the CUs idle, else 1.45 (1531 x 14336 x 4096: two rounds, 92 us;
+//     4009 x 3171 x 3072: one, 44 us); FP4 1.3 / 1.8; it needs re-laid scales.
+//   streaming: 0.57 us per unit of its own cost estimate (256 x 14336 x 4096 40 us, 1024 x 4096 x 8192 60 us).
+float est_t128(int64_t M, int64_t N, int64_t K, int S, bool fp4) {
+  const int64_t wgs = ((M + 127) / 128) * ((N + 127) / 128) * S;
+  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)) / S;
+  float t = 5.f + st * (wgs <= 256 ? (fp4 ? 0.68f : 0.62f) : (fp4 ? 1.2f : 0.97f) * ((wgs + 511) / 512));
+  if (S > 1) t += 4.f + (float)S * M * N * 8 / 4e6f;
+  return t;
+}
+float est_pp(int64_t M, int64_t N, int64_t K, bool fp4, bool pack) {
+  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128));
+  return 8.f + st * (tiles <= 128 ? (fp4 ? 1.3f : 1.1f) : (fp4 ? 1.8f : 1.45f) * ((tiles + 255) / 256)) + (pack ? 5.f : 0.f);
+}
+float est_stream(int64_t M, int64_t N, int64_t K, int w_fmt) { return 5.f + 0.57f * stream_plan(M, N, K, w_fmt).cost; }
 
 int check_tensor(const mx_tensor* t, const char* name, int min_nd, int max_nd) {
   if (!t) return set_error(MX_ERR_INVALID, "%s: null descriptor", name);
@@ -169,11 +185,7 @@ int64_t mx_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, const mx_gemm_o
   if (o.kernel == MX_KERNEL_GENERIC || o.kernel == MX_KERNEL_STREAM || o.kernel == MX_KERNEL_DECODE) return 0;
   int64_t b = 0;
   const int S = plan_k_splits(M, N, K, o);
-  if (S > 1) {   // per-slice packed scales and the fp32 partial products
-    b += S * (mx_packed_scale_bytes(M, K / S) + mx_packed_scale_bytes(N, K / S));
-    b += round256(S * M * N * 4);
-    return b;
-  }
+  if (S > 1) b += round256(S * M * N * 4);   // the fp32 partial products
   if (!is_native(o.a_scale_layout)) b += mx_packed_scale_bytes(M, K);
   if (!is_native(o.b_scale_layout)) b += mx_packed_scale_bytes(N, K);
   return b;
@@ -257,7 +269,7 @@ namespace {
 // What mx_gemm would launch for a problem that ends on the 128 x 128 one-tile kernel without split-K: the list
 // entry point collects these and runs them as one batched scale re-layout and one persistent GEMM launch.
 struct GemmPlan {
-  GemmArgs g;
+  T128Args g;
   PackArgs pa, pb;
   bool pack_a, pack_b;
 };
@@ -274,7 +286,7 @@ int mx_gemm(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const m
 
 namespace {
 // mx_gemm; with `plan` nothing is launched: a problem of the simple kind is described in *plan (return MX_OK),
-// any other valid problem returns kPlanNotSimple
+// any other valid problem returns kPlanNotSimple.
 int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const mx_tensor* Bs, mx_tensor* C,
               const mx_gemm_opts* opts, void* workspace, int64_t workspace_bytes, void* stream, GemmPlan* plan) {
   const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
@@ -394,7 +406,8 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
   if (kernel == MX_KERNEL_STREAM) {
     if (why_stream) return set_error(MX_ERR_LAYOUT, "the streaming kernel cannot run this problem: %s", why_stream);
   } else if (kernel == MX_KERNEL_AUTO) {
-    if (!plan && !why_stream && o.split_k <= 1 && (why || M <= kStreamAutoM) &&
+    const bool may_stream = !plan && !why_stream && o.split_k <= 1;
+    if (may_stream && (why || M <= kStreamAutoM) &&
         !(M <= 32 && decode_beats_stream(M, N, K) && B->dtype == MX_E2M1 && o.b_scale_layout == MX_SCALE_2D))
       kernel = MX_KERNEL_STREAM;
     else if (why) kernel = MX_KERNEL_GENERIC;
@@ -404,8 +417,13 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
              N % 16 == 0 && Bs->stride[1] % 16 == 0 && ((uintptr_t)Bs->ptr) % 16 == 0 &&
              N * b_ld < ((int64_t)1 << 31) && As->stride[0] % 16 == 0 && ((uintptr_t)As->ptr) % 16 == 0)
       kernel = MX_KERNEL_DECODE;
-    else if (big_tile_problem(M, N)) kernel = big_tile_kernel();
-    else kernel = MX_KERNEL_MFMA_128x128;
+    else {
+      const bool fp4 = A->dtype == MX_E2M1;
+      const float t128 = est_t128(M, N, K, o.split_k > 1 ? 1 : plan_k_splits(M, N, K, o), fp4);
+      const float pp = o.split_k > 1 ? 1e30f : est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout));
+      const float st = may_stream ? est_stream(M, N, K, B->dtype) : 1e30f;
+      kernel = st < t128 && st < pp ? MX_KERNEL_STREAM : t128 <= pp ? MX_KERNEL_MFMA_128x128 : big_tile_kernel();
+    }
   } else if (kernel != MX_KERNEL_GENERIC && why) {
     return set_error(MX_ERR_LAYOUT, "requested kernel %d cannot run this problem: %s", kernel, why);
   }
@@ -522,6 +540,59 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
                        512 * o.split_k);
   }
   if (S > 1 && plan) return kPlanNotSimple;
+  if (kernel == MX_KERNEL_MFMA_128x128) {
+    // scales are read where they are if the kernel can (A alone, or A and B), else re-laid first
+    T128Args g = {};
+    const bool a_can = o.a_scale_layout == MX_SCALE_2D &&
+                       t128_plain_scales(As->ptr, As->stride[0], As->stride[1], M, K, A->dtype, B->dtype);
+    const bool b_can = o.b_scale_layout == MX_SCALE_2D &&
+                       t128_plain_scales(Bs->ptr, Bs->stride[1], Bs->stride[0], N, K, A->dtype, B->dtype);
+    g.a_plain = a_can; g.b_plain = a_can && b_can;
+    const bool pack_a = !a_can && !is_native(o.a_scale_layout), pack_b = !g.b_plain && !is_native(o.b_scale_layout);
+    if ((!a_can && !pack_a && o.a_scale_layout != MX_SCALE_NATIVE) || (!g.b_plain && !pack_b && o.b_scale_layout != MX_SCALE_NATIVE))
+      return set_error(MX_ERR_LAYOUT, "kernel %d reads native-layout scales of kind %d (MX_SCALE_NATIVE for the "
+                       "16x16x128-instruction kernels, MX_SCALE_NATIVE32 for pingpong32 / w4p); pass the matching "
+                       "layout or the plain 2-D scales", kernel, MX_SCALE_NATIVE);
+    g.A = (const uint8_t*)A->ptr; g.B = (const uint8_t*)B->ptr; g.As = (const uint8_t*)As->ptr; g.Bs = (const uint8_t*)Bs->ptr;
+    g.C = C->ptr;
+    g.lda = a_ld; g.ldb = b_ld; g.ldas = As->stride[0]; g.ldbs = Bs->stride[1]; g.ldc = C->stride[0];
+    g.M = (int32_t)M; g.N = (int32_t)N; g.K = (int32_t)K;
+    g.a_fmt = A->dtype; g.b_fmt = B->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate;
+    g.batch = 1; g.k_splits = S; g.a_rows = M;
+    if (pack_a) {
+      if (int rc = make_pack_args(As, o.a_scale_layout, M, K, ws, kPackA, pa)) return rc;
+      g.As = ws;
+      ws += mx_packed_scale_bytes(M, K);
+    }
+    if (pack_b) {
+      mx_tensor t = *Bs;
+      if (o.b_scale_layout == MX_SCALE_2D) {  // [K/32, N] -> view as [N, K/32]
+        t.shape[0] = Bs->shape[1]; t.shape[1] = Bs->shape[0];
+        t.stride[0] = Bs->stride[1]; t.stride[1] = Bs->stride[0];
+      }
+      if (int rc = make_pack_args(&t, o.b_scale_layout, N, K, ws, kPackB, pb)) return rc;
+      g.Bs = ws;
+      ws += mx_packed_scale_bytes(N, K);
+    }
+    if ((!g.a_plain && ((uintptr_t)g.As) % 16 != 0) || (!g.b_plain && ((uintptr_t)g.Bs) % 16 != 0))
+      return set_error(MX_ERR_LAYOUT, "native scale buffers must be 16-byte aligned");
+    if (plan) {
+      if ((pack_a && o.a_scale_layout != MX_SCALE_2D) || (pack_b && o.b_scale_layout != MX_SCALE_2D) ||
+          (g.a_plain && !g.b_plain) || o.accumulate)
+        return kPlanNotSimple;
+      plan->g = g;
+      plan->pack_a = pack_a; plan->pack_b = pack_b;
+      if (pack_a) plan->pa = pa;
+      if (pack_b) plan->pb = pb;
+      return MX_OK;
+    }
+    if (pack_a || pack_b)   // one launch for both operands
+      if (int rc = launch_pack_scales_pair(pack_a ? &pa : nullptr, pack_b ? &pb : nullptr, (hipStream_t)stream)) return rc;
+    if (S == 1) return launch_gemm_t128(g, (hipStream_t)stream);
+    g.partial = (float*)ws;
+    if (int rc = launch_gemm_t128(g, (hipStream_t)stream)) return rc;
+    return launch_splitk_reduce(g.partial, S, M, N, C->ptr, C->stride[0], C->dtype, o.accumulate, (hipStream_t)stream);
+  }
   if (S > 1) {
     // ---- split-K: the slices are a batch for the scale re-layout and a second grid dimension for the GEMM
     const int64_t Ks = K / S, kbs = Ks / 32;
@@ -576,7 +647,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
   }
   if (((uintptr_t)as_native) % 16 != 0 || ((uintptr_t)bs_native) % 16 != 0)
     return set_error(MX_ERR_LAYOUT, "native scale buffers must be 16-byte aligned");
-  if (!plan && (pack_a || pack_b))   // one launch for both operands
+  if (pack_a || pack_b)   // one launch for both operands
     if (int rc = launch_pack_scales_pair(pack_a ? &pa : nullptr, pack_b ? &pb : nullptr, (hipStream_t)stream)) return rc;
 
   GemmArgs g = {};
@@ -586,14 +657,6 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
   g.a_fmt = A->dtype; g.b_fmt = B->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate;
   g.a_rows = M;
   g.replicas = 1;
-  if (plan) {
-    if ((pack_a && o.a_scale_layout != MX_SCALE_2D) || (pack_b && o.b_scale_layout != MX_SCALE_2D)) return kPlanNotSimple;
-    plan->g = g;
-    plan->pack_a = pack_a; plan->pack_b = pack_b;
-    if (pack_a) plan->pa = pa;
-    if (pack_b) plan->pb = pb;
-    return MX_OK;
-  }
   return launch_gemm_mfma(g, kernel, (hipStream_t)stream);
 }
 }  // namespace
@@ -676,7 +739,7 @@ int mx_gemm_list(int32_t count, const mx_tensor* A, const mx_tensor* As, const m
     items.push_back(it);
   }
   // Pass 2: one scale re-layout launch per 64 scale tensors, one persistent GEMM launch per 32 problems of one
-  // element-format pair and output type
+  // element-format pair and scale layout
   std::vector<PackArgs> packs;
   for (const Item& it : items) {
     if (!it.simple) continue;
@@ -688,16 +751,17 @@ int mx_gemm_list(int32_t count, const mx_tensor* A, const mx_tensor* As, const m
   std::vector<char> done(items.size(), 0);
   for (size_t i = 0; i < items.size(); ++i) {
     if (!items[i].simple || done[i]) continue;
-    std::vector<GemmArgs> group;
-    const GemmArgs& g0 = items[i].plan.g;
+    std::vector<T128Args> group;
+    const T128Args& g0 = items[i].plan.g;
     for (size_t j = i; j < items.size(); ++j) {
-      const GemmArgs& g = items[j].plan.g;
-      if (items[j].simple && !done[j] && g.a_fmt == g0.a_fmt && g.b_fmt == g0.b_fmt && g.c_dtype == g0.c_dtype) {
+      const T128Args& g = items[j].plan.g;
+      if (items[j].simple && !done[j] && g.a_fmt == g0.a_fmt && g.b_fmt == g0.b_fmt && g.a_plain == g0.a_plain &&
+          g.b_plain == g0.b_plain) {
         group.push_back(g);
         done[j] = 1;
       }
     }
-    if (int rc = launch_gemm_mfma_list(group.data(), (int)group.size(), (hipStream_t)stream)) return rc;
+    if (int rc = launch_gemm_t128_list(group.data(), (int)group.size(), (hipStream_t)stream)) return rc;
   }
   // Pass 3: the rest (large problems for the persistent 256 x 256 kernel, skinny ones for the decode kernel,
   // split-K, batched operands, layouts only the general kernel reads), one call each
@@ -831,6 +895,44 @@ int mx_gemm_grouped(const mx_tensor* A, const mx_tensor* As, const mx_tensor* W,
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                      (long long)workspace_bytes);
   if (((uintptr_t)ws) % 256 != 0) return set_error(MX_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+  if (kernel == MX_KERNEL_MFMA_128x128) {
+    T128Args g = {};
+    g.a_plain = t128_plain_scales(As->ptr, As->stride[0], As->stride[1], T, K, A->dtype, W->dtype);
+    PackArgs pa = {}, pw;
+    g.As = (const uint8_t*)As->ptr; g.ldas = As->stride[0];
+    if (!g.a_plain) {   // gathered into slot order while re-laying
+      pa.target = kPackA;
+      pa.src = (const uint8_t*)As->ptr; pa.dst = (uint32_t*)ws;
+      pa.rows = num_slots; pa.K = K; pa.s_row = As->stride[0]; pa.s_kb = As->stride[1];
+      pa.layout = MX_SCALE_2D; pa.batch = 1;
+      pa.gather_ids = sorted_token_ids; pa.replicas = num_token_replicas; pa.num_valid_ids = num_valid_ids;
+      g.As = ws;
+      ws += mx_packed_scale_bytes(num_slots, K);
+    }
+    g.Bs = (const uint8_t*)Ws->ptr;
+    const bool pack_w = !is_native(o.b_scale_layout);
+    if (!pack_w && o.b_scale_layout != MX_SCALE_NATIVE)
+      return set_error(MX_ERR_LAYOUT, "kernel %d reads native-layout scales of kind %d, W_scale has kind %d", kernel,
+                       MX_SCALE_NATIVE, o.b_scale_layout);
+    if (E * mx_packed_scale_bytes(N, K) >= ((int64_t)1 << 31))
+      return set_error(MX_ERR_SHAPE, "the packed scales of all experts must stay below 2 GiB");
+    if (pack_w) {
+      if (o.b_scale_layout != MX_SCALE_2D) return set_error(MX_ERR_LAYOUT, "W_scale must be [E, N, K/32] or native");
+      if (int rc = make_pack_args(Ws, MX_SCALE_2D, N, K, ws, kPackB, pw)) return rc;
+      g.Bs = ws;
+    }
+    if (!g.a_plain || pack_w)
+      if (int rc = launch_pack_scales_pair(g.a_plain ? nullptr : &pa, pack_w ? &pw : nullptr, (hipStream_t)stream)) return rc;
+    g.A = (const uint8_t*)A->ptr; g.B = (const uint8_t*)W->ptr; g.C = C->ptr;
+    g.lda = A->stride[0]; g.ldb = W->stride[1]; g.ldc = C->stride[0];
+    g.M = (int32_t)num_slots; g.N = (int32_t)N; g.K = (int32_t)K;
+    g.a_fmt = A->dtype; g.b_fmt = W->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate;
+    g.batch = 1; g.k_splits = 1;
+    g.sorted_token_ids = sorted_token_ids; g.sorted_expert_ids = sorted_expert_ids; g.topk_weights = topk_weights;
+    g.tile_m = tile_m; g.replicas = num_token_replicas; g.num_valid_ids = num_valid_ids; g.num_experts = (int32_t)E;
+    g.a_rows = T; g.b_expert = W->stride[0]; g.bs_expert = mx_packed_scale_bytes(N, K);
+    return launch_gemm_t128(g, (hipStream_t)stream);
+  }
   // A scales: gathered into slot order while re-laying; W scales of all experts ride in the same launch
   const int native = native_layout_of(kernel);
   const bool t32 = native == MX_SCALE_NATIVE32;

@@ -117,10 +117,6 @@ struct GemmArgs {
   int32_t k_splits;
   int64_t as_split_stride, bs_split_stride;   // dwords
   int64_t c_split_stride;                     // elements of C
-  // batch of equal products (one-tile kernels only, blockIdx.z): bytes / dwords / elements of C from one to the next
-  int32_t batch;
-  int64_t a_batch, b_batch, as_batch, bs_batch, c_batch;
-  const float* acc;          // what is added to the product (fp32, laid out like C); null: C itself if `accumulate`
   // grouped gate + up projection with the activation quantised in the epilogue (ping-pong kernel): W holds up_half gate
   // rows, then up_half up rows; silu(gate) * up goes to q [slot id][up_half] (E4M3) and qs [slot id][up_half / 32]
   uint8_t* q; uint8_t* qs;
@@ -128,10 +124,6 @@ struct GemmArgs {
 };
 
 int launch_gemm_mfma(const GemmArgs& g, int kernel_id, hipStream_t stream);
-// A list of independent plain products (no grouping, no split-K, one element format pair and output dtype for the
-// whole list) on the 128 x 128 one-tile kernel body: one persistent launch per 32 problems walks the concatenated
-// tile list (the scheme of grouped_matmul_kernel, test/kernels/group_gemm.py:10-38).
-int launch_gemm_mfma_list(const GemmArgs* problems, int n, hipStream_t stream);
 int launch_gemm_pingpong(const GemmArgs& g, hipStream_t stream);
 // the 32x32x64-instruction variant: 8-bit element formats only
 bool pingpong32_supports(int a_fmt, int b_fmt);

@@ -130,6 +130,30 @@ bool stream_supports(int x_fmt, int w_fmt) {
          (x_fmt == MX_E5M2 && (w_fmt == MX_E5M2 || w_fmt == MX_E2M1));
 }
 
+// How the 8 waves of a workgroup split the problem: kw K ranges x 8 / kw units of nt tiles; M in tiles of 16 mt rows.  The
+// cost that is minimised is a wave's K-quads times what a K-step of it moves (nt tiles of W, the rows of X), plus a
+// start-up per workgroup, for every round of workgroups over the 256 CUs: X is fetched once per unit, so wide units
+// save traffic, but a second, partly filled round costs more (28672 x 8192 FP4 at 4 rows: 224 workgroups 28 us, 448
+// 33.6 us; 14336 x 8192 FP8 at 64 rows: 224 of 4 tiles 34 us, 448 of 2 45 us).
+// (tiles of a 64-row group interleave its rows, so groups are covered whole)
+StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int w_fmt) {
+  StreamPlan p = {};
+  p.mt = M <= 16 ? 1 : M <= 32 || w_fmt == MX_E2M1 ? 2 : 4;
+  p.m_tiles = (int)((M + 16 * p.mt - 1) / (16 * p.mt));
+  const int tiles = (int)((N + 63) / 64 * 4), KQ = (int)((K + 511) / 512);
+  const float wb = w_fmt == MX_E2M1 ? 1.f : 2.f, xb = (M < 16 * p.mt ? M : 16 * p.mt) / 16.f;
+  p.cost = 1e30f;
+  for (int n = 4; n >= 1; n >>= 1)
+    for (int kw = 8; kw >= 1; kw >>= 1) {
+      if (kw > 1 && kw > KQ) continue;
+      const int units = (tiles + n * (8 / kw) - 1) / (n * (8 / kw));
+      const int64_t rounds = ((int64_t)units * p.m_tiles + 255) / 256;
+      const float t = rounds * ((KQ + kw - 1) / kw * (n * wb + xb) + 3.f);
+      if (t < p.cost) { p.cost = t; p.nt = n; p.kw = kw; p.units = units; }
+    }
+  return p;
+}
+
 int launch_gemm_stream(const StreamArgs& a0, hipStream_t stream) {
   StreamArgs a = a0;
   if (!stream_supports(a.x_fmt, a.w_fmt))
@@ -145,26 +169,9 @@ int launch_gemm_stream(const StreamArgs& a0, hipStream_t stream) {
   if ((int64_t)a.M * a.ldx >= lim || (int64_t)a.N * a.ldw >= lim || (int64_t)a.M * a.ldxs >= lim ||
       (a.ws_packed ? packed_scale_dwords(a.N, a.K) * 4 : (int64_t)a.N * a.ldws) >= lim || wrow > a.ldw)
     return set_error(MX_ERR_LAYOUT, "stream kernel: an operand spans 2 GiB or more");
-  const int mt = a.M <= 16 ? 1 : a.M <= 32 || a.w_fmt == MX_E2M1 ? 2 : 4;
-  a.m_tiles = (a.M + 16 * mt - 1) / (16 * mt);
-  // How the 8 waves of a workgroup split the problem: kw K ranges x 8 / kw units of nt tiles.  The estimate that is
-  // minimised is a wave's K-quads times what a K-step of it moves (nt tiles of W, the rows of X), plus a start-up per
-  // workgroup, for every round of workgroups over the 256 CUs: X is fetched once per unit, so wide units save traffic,
-  // but a second, partly filled round costs more (28672 x 8192 FP4 at 4 rows: 224 workgroups 28 us, 448 33.6 us; 14336
-  // x 8192 FP8 at 64 rows: 224 of 4 tiles 34 us, 448 of 2 45 us).
-  // (tiles of a 64-row group interleave its rows, so groups are covered whole)
-  const int tiles = (a.N + 63) / 64 * 4, KQ = (a.K + 511) / 512;
-  const float wb = a.w_fmt == MX_E2M1 ? 1.f : 2.f, xb = (a.M < 16 * mt ? a.M : 16 * mt) / 16.f;
-  int nt = 1;
-  float best = 1e30f;
-  for (int n = 4; n >= 1; n >>= 1)
-    for (int kw = 8; kw >= 1; kw >>= 1) {
-      if (kw > 1 && kw > KQ) continue;
-      const int units = (tiles + n * (8 / kw) - 1) / (n * (8 / kw));
-      const int64_t rounds = ((int64_t)units * a.m_tiles + 255) / 256;
-      const float t = rounds * ((KQ + kw - 1) / kw * (n * wb + xb) + 3.f);
-      if (t < best) { best = t; nt = n; a.kw = kw; a.units = units; }
-    }
+  const StreamPlan p = stream_plan(a.M, a.N, a.K, a.w_fmt);
+  const int mt = p.mt, nt = p.nt;
+  a.m_tiles = p.m_tiles; a.kw = p.kw; a.units = p.units;
   const int blocks = a.m_tiles > 1 ? (a.units + 7) / 8 * 8 * a.m_tiles : a.units;
 #define MX_CASE(XF, WF)                                                                       \
   if (a.x_fmt == XF && a.w_fmt == WF)                                                         \

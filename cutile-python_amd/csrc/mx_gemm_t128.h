@@ -1,0 +1,39 @@
+// Interface of the 128 x 128 one-tile kernel (mx_gemm_t128.hip): small and mid-size products, batches of them, lists of
+// unequal ones, split-K, and the grouped form with 128-slot tiles.
+#pragma once
+#include "mx_common.h"
+
+namespace mx {
+
+struct T128Args {
+  const uint8_t* A;        // [M rows][lda bytes], K contiguous
+  const uint8_t* B;        // [N rows][ldb bytes]
+  const uint8_t* As;       // a_plain: [M rows][ldas bytes]; else the native layout (operand A, slot order when grouped)
+  const uint8_t* Bs;       // b_plain: [N rows][ldbs bytes]; else the native layout (operand B)
+  void* C;
+  const float* acc;        // what is added to the product (fp32, laid out like C); null: C itself if `accumulate`
+  int64_t lda, ldb, ldas, ldbs, ldc;   // bytes; ldc in elements
+  int64_t a_batch, b_batch, as_batch, bs_batch, c_batch;   // from one product of a batch to the next: bytes, elements of C
+  float* partial;          // k_splits > 1: fp32 partial products [split][M][N]
+  int32_t M, N, K;
+  int32_t a_fmt, b_fmt, c_dtype, accumulate;
+  int32_t a_plain, b_plain;
+  int32_t batch, k_splits; // 1 each unless used
+  // grouped (MoE) extension; sorted_token_ids == nullptr otherwise.  M is the number of slots.
+  const int32_t* sorted_token_ids;
+  const int32_t* sorted_expert_ids;
+  const float* topk_weights;
+  int32_t tile_m, replicas, num_experts;
+  int64_t num_valid_ids, a_rows, b_expert, bs_expert;      // rows of A; bytes between experts
+};
+
+// scales that the kernel reads where they are: K-contiguous rows of 4-byte aligned E8M0 bytes, K a whole number of stages
+inline bool t128_plain_scales(const void* ptr, int64_t ld, int64_t k_stride, int64_t rows, int64_t K, int a_fmt, int b_fmt) {
+  const int stage = a_fmt == MX_E2M1 && b_fmt == MX_E2M1 ? 256 : 128;
+  return k_stride == 1 && K % stage == 0 && ld % 4 == 0 && ((uintptr_t)ptr) % 4 == 0 && rows * ld < ((int64_t)1 << 31);
+}
+int launch_gemm_t128(const T128Args& g, hipStream_t stream);
+// any number of independent plain products of one element-format pair: one persistent launch per 32 of them
+int launch_gemm_t128_list(const T128Args* problems, int n, hipStream_t stream);
+
+}  // namespace mx

@@ -15,6 +15,8 @@ struct StreamArgs {
   int32_t kw, m_tiles, units;
 };
 bool stream_supports(int x_fmt, int w_fmt);
+struct StreamPlan { int mt, m_tiles, nt, kw, units; float cost; };
+StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int w_fmt);
 int launch_gemm_stream(const StreamArgs& a, hipStream_t stream);
 
 // mixture-of-experts layer at decode sizes (mx_moe.hip)

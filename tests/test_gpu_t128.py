@@ -1,0 +1,46 @@
+"""GPU parity of the pipelined 128 x 128 kernel at the edges of its dispatch: grids either side of one workgroup per CU
+(its two pipeline depths), K that ends inside a stage or a K-quad, scales read in place or from the native layout, K
+split over the workgroups."""
+import pytest
+import torch
+
+from mxutil import oracle_matmul, raw_operand
+from oracle import mx_oracle as O
+from test_gpu_edges import _check_guarded, _guarded
+
+pytestmark = pytest.mark.gpu
+PAIRS = [(O.E4M3, O.E4M3), (O.E5M2, O.E5M2), (O.E2M1, O.E2M1), (O.E4M3, O.E2M1)]
+# The matrix instruction aligns the 128 products of a K-step to the largest of them and drops what falls below its
+# accumulator, at most 2^-17 of the largest for each E4M3 product of these operands (raw codes, scales over 15 binades):
+# 128 * 2^-17 = 1e-3 of the norm.  A scale, row or K-step taken from the wrong place is an error of the order of 1.
+TOL = 1e-3
+
+
+def _run(ct, a, b, layout, **kw):
+    sa = ct.pack_scales(a.scale_t, operand="a") if layout == "packed" else a.scale_t
+    sb = ct.pack_scales(b.scale_t, operand="b") if layout in ("packed", "b packed") else b.scale_t.T
+    return ct.block_scaled_matmul(a.storage, sa, b.storage.T, sb, a_format=a.fmt_kw, b_format=b.fmt_kw,
+                                  kernel="mfma128", **kw)
+
+
+@pytest.mark.parametrize("layout", ["plain", "b packed", "packed"])
+@pytest.mark.parametrize("fa,fb", PAIRS, ids=str)
+@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (128, 128, 128), (129, 127, 384), (64, 200, 640), (300, 260, 1184),
+                                   (130, 136, 256), (2048, 2176, 256), (2177, 1930, 160)])
+def test_t128_kernel(ct, dev, layout, fa, fb, M, N, K):
+    a, b = raw_operand(M, K, fa, 100 + M, dev), raw_operand(N, K, fb, 200 + N, dev)
+    ref = oracle_matmul(a, b)
+    out = _run(ct, a, b, layout, out_dtype=torch.float32)
+    assert O.rel_fro(out.cpu(), ref) <= TOL
+    c, buf = _guarded(M, N, N + 3, torch.bfloat16, dev)
+    _run(ct, a, b, layout, C=c)
+    _check_guarded(c, buf, ref)
+
+
+@pytest.mark.parametrize("fa,fb", PAIRS, ids=str)
+@pytest.mark.parametrize("layout", ["plain", "packed"])
+@pytest.mark.parametrize("M,N,K", [(70, 130, 2048), (256, 128, 4096 + 128), (33, 65, 6144 + 32)])
+def test_t128_splits_k(ct, dev, layout, fa, fb, M, N, K):
+    a, b = raw_operand(M, K, fa, 300 + M, dev), raw_operand(N, K, fb, 400 + N, dev)
+    out = _run(ct, a, b, layout, out_dtype=torch.float32)
+    assert O.rel_fro(out.cpu(), oracle_matmul(a, b)) <= TOL
