@@ -88,8 +88,8 @@ int plan_k_splits(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
 //   256 x 256 tiles: 1.1 us per stage when they leave half of the CUs idle, else 1.45 (1531 x 14336 x 4096: two rounds, 92 us;
 //     4009 x 3171 x 3072: one, 44 us); FP4 1.3 / 1.8; it needs re-laid scales.
 //   streaming: 0.57 us per unit of its own cost estimate (256 x 14336 x 4096 40 us, 1024 x 4096 x 8192 60 us).
-float est_t128(int64_t M, int64_t N, int64_t K, int S, bool fp4) {
-  const int64_t wgs = ((M + 127) / 128) * ((N + 127) / 128) * S;
+float est_t128(int64_t M, int64_t N, int64_t K, int S, bool fp4, int64_t batch = 1) {
+  const int64_t wgs = ((M + 127) / 128) * ((N + 127) / 128) * S * batch;
   const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)) / S;
   float t = 5.f + st * (wgs <= 256 ? (fp4 ? 0.68f : 0.62f) : (fp4 ? 1.2f : 0.97f) * ((wgs + 511) / 512));
   if (S > 1) t += 4.f + (float)S * M * N * 8 / 4e6f;
@@ -274,9 +274,11 @@ struct GemmPlan {
   bool pack_a, pack_b;
 };
 constexpr int kPlanNotSimple = 1;   // gemm_impl with a plan: the problem needs its own mx_gemm call
+constexpr int kAccNeedsCopy = 2;    // gemm_impl with an addend: the kernel can only accumulate into C (nothing enqueued)
 
 int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const mx_tensor* Bs, mx_tensor* C,
-              const mx_gemm_opts* opts, void* workspace, int64_t workspace_bytes, void* stream, GemmPlan* plan);
+              const mx_gemm_opts* opts, void* workspace, int64_t workspace_bytes, void* stream, GemmPlan* plan,
+              const float* acc = nullptr);
 }  // namespace
 
 int mx_gemm(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const mx_tensor* Bs, mx_tensor* C,
@@ -284,11 +286,38 @@ int mx_gemm(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const m
   return gemm_impl(A, As, B, Bs, C, opts, workspace, workspace_bytes, stream, nullptr);
 }
 
+int mx_gemm_add(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const mx_tensor* Bs, const mx_tensor* D,
+                mx_tensor* C, const mx_gemm_opts* opts, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (int rc = check_tensor(D, "D", 2, 3)) return rc;
+  if (int rc = check_tensor(C, "C", 2, 3)) return rc;
+  if (D->dtype != MX_F32 || C->dtype != MX_F32) return set_error(MX_ERR_DTYPE, "mx_gemm_add: D and C must be MX_F32");
+  if (D->ndim != C->ndim) return set_error(MX_ERR_SHAPE, "mx_gemm_add: D and C must have the same shape");
+  int64_t numel = 1;
+  for (int i = C->ndim - 1; i >= 0; --i) {
+    if (D->shape[i] != C->shape[i]) return set_error(MX_ERR_SHAPE, "mx_gemm_add: D and C must have the same shape");
+    if (C->shape[i] > 1 && (D->stride[i] != numel || C->stride[i] != numel))
+      return set_error(MX_ERR_LAYOUT, "mx_gemm_add: D and C must be contiguous");
+    numel *= C->shape[i];
+  }
+  mx_gemm_opts o = opts ? *opts : kDefaultOpts;
+  o.accumulate = 0;
+  const int rc = gemm_impl(A, As, B, Bs, C, &o, workspace, workspace_bytes, stream, nullptr, (const float*)D->ptr);
+  if (rc != kAccNeedsCopy) return rc;
+  if (numel == 0) return MX_OK;
+  if (C->ptr != D->ptr) {
+    const hipError_t e = hipMemcpyAsync(C->ptr, D->ptr, (size_t)numel * 4, hipMemcpyDeviceToDevice, (hipStream_t)stream);
+    if (e != hipSuccess) return set_error(MX_ERR_DEVICE, "mx_gemm_add: %s", hipGetErrorString(e));
+  }
+  o.accumulate = 1;
+  return gemm_impl(A, As, B, Bs, C, &o, workspace, workspace_bytes, stream, nullptr);
+}
+
 namespace {
 // mx_gemm; with `plan` nothing is launched: a problem of the simple kind is described in *plan (return MX_OK),
-// any other valid problem returns kPlanNotSimple.
+// any other valid problem returns kPlanNotSimple.  acc: fp32 addend laid out like C (contiguous)
 int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const mx_tensor* Bs, mx_tensor* C,
-              const mx_gemm_opts* opts, void* workspace, int64_t workspace_bytes, void* stream, GemmPlan* plan) {
+              const mx_gemm_opts* opts, void* workspace, int64_t workspace_bytes, void* stream, GemmPlan* plan,
+              const float* acc) {
   const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
   if (int rc = check_tensor(A, "A", 2, 3)) return rc;
   if (int rc = check_tensor(B, "B", 2, 3)) return rc;
@@ -361,6 +390,72 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       }
       return v;
     };
+    // small products: the whole batch as one launch of the 128 x 128 kernel (behind one scale re-layout launch), in chunks
+    // of what the workspace holds packed scales for
+    {
+      const mx_tensor a2 = slice(A, 0, 1), b2 = slice(B, 0, 1), as2 = slice(As, 0, 1), bs2 = slice(Bs, 0, 1);
+      auto bstride = [](const mx_tensor* t) { return t->ndim == 3 && t->shape[0] > 1 ? t->stride[0] : (int64_t)0; };
+      const int64_t per = mx_packed_scale_bytes(M, K) + mx_packed_scale_bytes(N, K);
+      const bool fp4 = A->dtype == MX_E2M1;
+      bool ok = (o.kernel == MX_KERNEL_AUTO || o.kernel == MX_KERNEL_MFMA_128x128) && o.split_k <= 1 && K > 0 &&
+                pair_supported_by_mfma(A->dtype, B->dtype) && C->stride[2] == 1 && bstride(A) % 16 == 0 && bstride(B) % 16 == 0 &&
+                !mfma_operand_issue(a2.ptr, M, a2.stride[0], a2.stride[1], A->dtype, a2.packed_dim == 1) &&
+                !mfma_operand_issue(b2.ptr, N, b2.stride[1], b2.stride[0], B->dtype, b2.packed_dim == 0) &&
+                M < (1 << 30) && N < (1 << 30) && K < (1 << 30);
+      const bool plain = ok && t128_plain_scales(as2.ptr, as2.stride[0], as2.stride[1], M, K, A->dtype, B->dtype) &&
+                         t128_plain_scales(bs2.ptr, bs2.stride[1], bs2.stride[0], N, K, A->dtype, B->dtype) &&
+                         bstride(As) % 4 == 0 && bstride(Bs) % 4 == 0;
+      int64_t chunk = plain ? batch : (workspace ? workspace_bytes / per : 0);
+      if (chunk > 32768) chunk = 32768;
+      if (ok && batch > 1) {   // few long products are better off one by one with K split, large ones gain nothing
+        float alone = est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4);
+        if (o.kernel == MX_KERNEL_AUTO) {
+          const float pp = est_pp(M, N, K, fp4, true);
+          if (pp < alone) alone = pp;
+          if (!fp4 && M <= kStreamAutoM && est_stream(M, N, K, B->dtype) < alone) alone = est_stream(M, N, K, B->dtype);
+        }
+        ok = est_t128(M, N, K, 1, fp4, batch) <= batch * alone;
+      }
+      if (!plain && workspace && ((uintptr_t)workspace) % 256 != 0) ok = false;
+      if (ok && chunk >= 1) {
+        for (int64_t b0 = 0; b0 < batch; b0 += chunk) {
+          const int64_t nb = batch - b0 < chunk ? batch - b0 : chunk;
+          T128Args g = {};
+          g.A = (const uint8_t*)A->ptr + b0 * bstride(A); g.a_batch = bstride(A);
+          g.B = (const uint8_t*)B->ptr + b0 * bstride(B); g.b_batch = bstride(B);
+          g.As = (const uint8_t*)As->ptr + b0 * bstride(As); g.as_batch = bstride(As);
+          g.Bs = (const uint8_t*)Bs->ptr + b0 * bstride(Bs); g.bs_batch = bstride(Bs);
+          g.c_batch = C->stride[0];
+          g.C = (uint8_t*)C->ptr + b0 * g.c_batch * (C->dtype == MX_BF16 ? 2 : 4);
+          if (acc) g.acc = acc + b0 * g.c_batch;
+          g.lda = a2.stride[0]; g.ldb = b2.stride[1]; g.ldas = as2.stride[0]; g.ldbs = bs2.stride[1]; g.ldc = C->stride[1];
+          g.M = (int32_t)M; g.N = (int32_t)N; g.K = (int32_t)K;
+          g.a_fmt = A->dtype; g.b_fmt = B->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate;
+          g.a_plain = g.b_plain = plain;
+          g.batch = (int32_t)nb; g.k_splits = 1; g.a_rows = M;
+          if (!plain) {
+            PackArgs pa, pb;
+            mx_tensor t = bs2;
+            t.shape[0] = bs2.shape[1]; t.shape[1] = bs2.shape[0];
+            t.stride[0] = bs2.stride[1]; t.stride[1] = bs2.stride[0];
+            uint8_t* const wa = (uint8_t*)workspace;
+            const int64_t na = g.as_batch ? nb : 1, nbb = g.bs_batch ? nb : 1;   // a broadcast operand is re-laid once
+            uint8_t* const wb = wa + na * mx_packed_scale_bytes(M, K);
+            if (int rc = make_pack_args(&as2, MX_SCALE_2D, M, K, wa, kPackA, pa)) return rc;
+            if (int rc = make_pack_args(&t, MX_SCALE_2D, N, K, wb, kPackB, pb)) return rc;
+            pa.src = g.As; pa.batch = (int32_t)na; pa.s_batch = g.as_batch;
+            pb.src = g.Bs; pb.batch = (int32_t)nbb; pb.s_batch = g.bs_batch;
+            if (int rc = launch_pack_scales_pair(&pa, &pb, (hipStream_t)stream)) return rc;
+            g.As = wa; g.Bs = wb;
+            g.as_batch = g.as_batch ? mx_packed_scale_bytes(M, K) : 0;
+            g.bs_batch = g.bs_batch ? mx_packed_scale_bytes(N, K) : 0;
+          }
+          if (int rc = launch_gemm_t128(g, (hipStream_t)stream)) return rc;
+        }
+        return MX_OK;
+      }
+    }
+    if (acc) return kAccNeedsCopy;
     const int c_bytes = C->dtype == MX_BF16 ? 2 : 4;
     for (int64_t b = 0; b < batch; ++b) {
       const mx_tensor a2 = slice(A, b, 1), as2 = slice(As, b, 1), b2 = slice(B, b, 1), bs2 = slice(Bs, b, 1);
@@ -433,6 +528,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     return set_error(MX_ERR_LAYOUT, "split_k = %d is only available on the one-tile MFMA kernels (kernel %d chosen)",
                      o.split_k, kernel);
   if (plan && kernel != MX_KERNEL_MFMA_128x128) return kPlanNotSimple;
+  if (acc && kernel != MX_KERNEL_MFMA_128x128) return kAccNeedsCopy;
   if (kernel == MX_KERNEL_GENERIC) {
     if (is_native(o.a_scale_layout) || is_native(o.b_scale_layout))
       return set_error(MX_ERR_LAYOUT, "the generic kernel cannot read native-layout scales");
@@ -540,6 +636,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
                        512 * o.split_k);
   }
   if (S > 1 && plan) return kPlanNotSimple;
+  if (S > 1 && acc) return kAccNeedsCopy;
   if (kernel == MX_KERNEL_MFMA_128x128) {
     // scales are read where they are if the kernel can (A alone, or A and B), else re-laid first
     T128Args g = {};
@@ -557,7 +654,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     g.C = C->ptr;
     g.lda = a_ld; g.ldb = b_ld; g.ldas = As->stride[0]; g.ldbs = Bs->stride[1]; g.ldc = C->stride[0];
     g.M = (int32_t)M; g.N = (int32_t)N; g.K = (int32_t)K;
-    g.a_fmt = A->dtype; g.b_fmt = B->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate;
+    g.a_fmt = A->dtype; g.b_fmt = B->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate; g.acc = acc;
     g.batch = 1; g.k_splits = S; g.a_rows = M;
     if (pack_a) {
       if (int rc = make_pack_args(As, o.a_scale_layout, M, K, ws, kPackA, pa)) return rc;

@@ -27,6 +27,7 @@ namespace {
 #define MX_FN(name) decltype(&name) p_##name = nullptr
 struct Lib {
   MX_FN(mx_gemm);
+  MX_FN(mx_gemm_add);
   MX_FN(mx_gemm_workspace_bytes);
   MX_FN(mx_gemm_list);
   MX_FN(mx_gemm_list_workspace_bytes);
@@ -236,6 +237,47 @@ PyObject* py_gemm_list(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return res;
 }
 
+// mma(x, x_scale, y, y_scale, acc, x_format, y_format, allow_mixed) -> acc + x @ y (a new tensor), error code, or None.
+// Every rule of mma_scaled that could fail is a condition here: what is not the plain block-32 case is left to ops.py.
+PyObject* py_mma(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  if (n != 8) { PyErr_SetString(PyExc_TypeError, "mma takes 8 arguments"); return nullptr; }
+  for (int i = 0; i < 5; ++i)
+    if (!THPVariable_Check(a[i])) Py_RETURN_NONE;
+  const at::Tensor &x = THPVariable_Unpack(a[0]), &xs = THPVariable_Unpack(a[1]), &y = THPVariable_Unpack(a[2]),
+                   &ys = THPVariable_Unpack(a[3]), &acc = THPVariable_Unpack(a[4]);
+  const int xd = (int)x.dim(), yd = (int)y.dim();
+  if ((xd != 2 && xd != 3) || (yd != 2 && yd != 3) || xs.dim() != xd || ys.dim() != yd || !on_current_device(x)) Py_RETURN_NONE;
+  const at::Device dev = x.device();
+  if (xs.device() != dev || y.device() != dev || ys.device() != dev || acc.device() != dev) Py_RETURN_NONE;
+  const int fx = elem_format(x, a[5]), fy = elem_format(y, a[6]);
+  if (fx < 0 || fy < 0 || (fx != fy && !PyObject_IsTrue(a[7])) || !is_e8m0(xs) || !is_e8m0(ys)) Py_RETURN_NONE;
+  if ((fx == MX_E2M1 && x.stride(-1) != 1) || (fy == MX_E2M1 && y.stride(-2) != 1)) Py_RETURN_NONE;
+  mx_tensor dx = desc(x, fx, fx == MX_E2M1 ? xd - 1 : -1), dy = desc(y, fy, fy == MX_E2M1 ? yd - 2 : -1),
+            dxs = desc(xs, MX_E8M0), dys = desc(ys, MX_E8M0);
+  const int64_t M = dx.shape[xd - 2], K = dx.shape[xd - 1], N = dy.shape[yd - 1];
+  const int64_t bx = xd == 3 ? x.size(0) : 1, by = yd == 3 ? y.size(0) : 1, batch = bx > by ? bx : by;
+  if (dy.shape[yd - 2] != K || K == 0 || K % 32 != 0 || M == 0 || N == 0 || (bx != by && bx != 1 && by != 1) || bx == 0 || by == 0 ||
+      dxs.shape[xd - 2] != M || dxs.shape[xd - 1] != K / 32 || dys.shape[yd - 2] != K / 32 || dys.shape[yd - 1] != N ||
+      (xd == 3 && dxs.shape[0] != bx) || (yd == 3 && dys.shape[0] != by))
+    Py_RETURN_NONE;
+  const bool batched = xd == 3 || yd == 3;
+  if (acc.scalar_type() != at::kFloat || !acc.is_contiguous() || acc.dim() != (batched ? 3 : 2) || acc.size(-2) != M ||
+      acc.size(-1) != N || (batched && acc.size(0) != batch))
+    Py_RETURN_NONE;
+  at::Tensor out = device_empty(acc.sizes(), at::kFloat, dev);
+  mx_tensor dD = desc(acc, MX_F32), dC = desc(out, MX_F32);
+  mx_gemm_opts o = {sizeof(mx_gemm_opts), 0, MX_SCALE_2D, MX_SCALE_2D, MX_KERNEL_AUTO, 32, 0, 0};
+  const int64_t need = lib.p_mx_gemm_workspace_bytes(M, N, K, &o) * batch;
+  at::Tensor ws;
+  if (need > 0) ws = device_empty({need}, at::kByte, dev);
+  int rc;
+  {
+    NoGil nogil;
+    rc = lib.p_mx_gemm_add(&dx, &dxs, &dy, &dys, &dD, &dC, &o, need > 0 ? ws.data_ptr() : nullptr, need, stream_of(dev));
+  }
+  return rc_or(rc, out);
+}
+
 // quantize(x, dtype | str, mode, silu) -> (elements, scales), error code, or None.
 // mode: 0 "ceil", 1 "floor"; silu: x is gate | up and silu(gate) * up is what is quantised
 PyObject* py_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -359,6 +401,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     return nullptr;                                                                      \
   }
   MX_FN(mx_gemm)
+  MX_FN(mx_gemm_add)
   MX_FN(mx_gemm_workspace_bytes)
   MX_FN(mx_gemm_list)
   MX_FN(mx_gemm_list_workspace_bytes)
@@ -385,6 +428,7 @@ PyMethodDef methods[] = {
     {"bind", py_bind, METH_VARARGS, nullptr},
     {"gemm", (PyCFunction)(void (*)(void))guarded<py_gemm>, METH_FASTCALL, nullptr},
     {"gemm_list", (PyCFunction)(void (*)(void))guarded<py_gemm_list>, METH_FASTCALL, nullptr},
+    {"mma", (PyCFunction)(void (*)(void))guarded<py_mma>, METH_FASTCALL, nullptr},
     {"quantize", (PyCFunction)(void (*)(void))guarded<py_quantize>, METH_FASTCALL, nullptr},
     {"moe", (PyCFunction)(void (*)(void))guarded<py_moe>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

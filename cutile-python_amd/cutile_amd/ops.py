@@ -537,6 +537,12 @@ def mma_scaled(x: torch.Tensor, x_scale: torch.Tensor, y: torch.Tensor, y_scale:
     ``allow_mixed_dtypes`` lifts the reference's "x and y must have the same dtype" rule, which the
     CDNA4 instruction does not need.
     """
+    if kernel == "auto":
+        r = L.host().mma(x, x_scale, y, y_scale, acc, x_format, y_format, allow_mixed_dtypes)
+        if isinstance(r, torch.Tensor):
+            return r
+        if r is not None:
+            _raise_code(r)
     for name, t in (("x", x), ("y", y), ("acc", acc), ("x_scale", x_scale), ("y_scale", y_scale)):
         if t.dim() not in (2, 3):
             raise TileTypeError(f"Expect shape of `{name}` to be 2D or 3D, got {tuple(t.shape)}")

@@ -171,6 +171,15 @@ MX_API int mx_gemm(const mx_tensor* A, const mx_tensor* A_scale, const mx_tensor
             int64_t workspace_bytes, void* stream);
 
 /*
+ * C = A@B + D with D fp32, laid out like C (both contiguous): the `acc` operand of ct.mma_scaled, whose result is a new
+ * tile (src/cuda/tile/_stub.py:2198-2235).  Otherwise as mx_gemm (opts->accumulate is ignored).  A batch may be given a
+ * workspace of batch x mx_gemm_workspace_bytes: small products then run as one launch.
+ */
+MX_API int mx_gemm_add(const mx_tensor* A, const mx_tensor* A_scale, const mx_tensor* B, const mx_tensor* B_scale,
+                const mx_tensor* D, mx_tensor* C, const mx_gemm_opts* opts, void* workspace,
+                int64_t workspace_bytes, void* stream);
+
+/*
  * mx_gemm for callers that cannot allocate or hand over device scratch: code running under HIP-graph capture,
  * tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference (its launcher needs no
  * scratch; cext/tile_kernel.cpp:3874-3919 only launches).  Same operands, options, results and errors as

@@ -1,10 +1,10 @@
 """GPU parity of the pipelined 128 x 128 kernel at the edges of its dispatch: grids either side of one workgroup per CU
 (its two pipeline depths), K that ends inside a stage or a K-quad, scales read in place or from the native layout, K
-split over the workgroups."""
+split over the workgroups, and a whole batch in one launch with an addend."""
 import pytest
 import torch
 
-from mxutil import oracle_matmul, raw_operand
+from mxutil import oracle_matmul, randn_operand, raw_operand
 from oracle import mx_oracle as O
 from test_gpu_edges import _check_guarded, _guarded
 
@@ -44,3 +44,21 @@ def test_t128_splits_k(ct, dev, layout, fa, fb, M, N, K):
     a, b = raw_operand(M, K, fa, 300 + M, dev), raw_operand(N, K, fb, 400 + N, dev)
     out = _run(ct, a, b, layout, out_dtype=torch.float32)
     assert O.rel_fro(out.cpu(), oracle_matmul(a, b)) <= TOL
+
+
+@pytest.mark.parametrize("fa,fb", [(O.E4M3, O.E4M3), (O.E2M1, O.E2M1)], ids=str)
+@pytest.mark.parametrize("bx,by", [(3, 3), (1, 4), (4, 1)])
+@pytest.mark.parametrize("M,N,K", [(16, 16, 64), (128, 256, 512), (130, 70, 1056), (40, 24, 4096)])
+def test_batch_in_one_launch(ct, dev, fa, fb, bx, by, M, N, K):
+    xs = [randn_operand(M, K, fa, 500 + i, dev) for i in range(bx)]
+    ys = [randn_operand(N, K, fb, 600 + i, dev) for i in range(by)]
+    z = torch.randn((max(bx, by), M, N), generator=torch.Generator().manual_seed(7)).to(dev)
+    keep = z.clone()
+    stack = lambda v: torch.stack([t.view(torch.uint8) for t in v]).view(v[0].dtype)
+    out = ct.mma_scaled(stack([x.storage for x in xs]), stack([x.scale_t for x in xs]),
+                        stack([y.storage for y in ys]).transpose(1, 2), stack([y.scale_t for y in ys]).transpose(1, 2),
+                        z, x_format=xs[0].fmt_kw, y_format=ys[0].fmt_kw)
+    for i in range(max(bx, by)):
+        ref = oracle_matmul(xs[i % bx], ys[i % by], z[i].cpu())
+        assert O.rel_fro(out[i].cpu(), ref) <= TOL
+    assert torch.equal(z, keep)
