@@ -71,7 +71,10 @@ int plan_k_splits(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
   if (o.split_k == 1 || o.block_size != 32 || K <= 0 || M <= 0 || N <= 0) return 1;
   if (o.kernel != MX_KERNEL_AUTO && o.kernel != MX_KERNEL_MFMA_128x128 && !t256) return 1;
   if (t256 && (o.a_scale_layout != MX_SCALE_2D || o.b_scale_layout != MX_SCALE_2D || K % 512 != 0)) return 1;
-  if (o.split_k > 1) return (K % ((int64_t)512 * o.split_k) == 0) ? o.split_k : -1;   // -1: cannot honour
+  if (o.split_k > 1) {   // -1: cannot honour; a K or scale layout that has never been split runs whole
+    if (K % ((int64_t)512 * o.split_k) == 0) return o.split_k;
+    return K % 512 == 0 && o.a_scale_layout == MX_SCALE_2D && o.b_scale_layout == MX_SCALE_2D ? -1 : 1;
+  }
   if (t256) return 1;
   if (o.kernel == MX_KERNEL_AUTO && big_tile_problem(M, N)) return 1;   // big-tile kernel
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
@@ -777,7 +780,21 @@ int mx_gemm_static(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, 
     return set_error(MX_ERR_SHAPE, "mx_gemm_static: A and B must have 2 or 3 dimensions");
   int64_t M, N, K;
   problem_dims(*A, *B, M, N, K);
-  const int64_t need = mx_gemm_workspace_bytes(M, N, K, opts);
+  int64_t need = mx_gemm_workspace_bytes(M, N, K, opts);
+  mx_gemm_opts o = opts ? *opts : kDefaultOpts;
+  if (need > MX_STATIC_SCRATCH_BYTES && o.split_k == 0) {
+    // the partial sums of an automatic split are what does not fit: run it whole.  (Plain scales with a K that splits into
+    // equal slices of 512 have always been held to the buffer, and stay refused.)
+    const int S = plan_k_splits(M, N, K, o);
+    bool even = false;
+    if (K % 512 == 0 && o.a_scale_layout == MX_SCALE_2D && o.b_scale_layout == MX_SCALE_2D)
+      for (int s = S; s > 1 && !even; --s) even = K % (512 * s) == 0 && s * M * N * 4 > MX_STATIC_SCRATCH_BYTES;
+    if (S > 1 && !even) {
+      o.split_k = 1;
+      opts = &o;
+      need = mx_gemm_workspace_bytes(M, N, K, opts);
+    }
+  }
   if (need > MX_STATIC_SCRATCH_BYTES)
     return set_error(MX_ERR_WORKSPACE, "mx_gemm_static: this problem needs %lld bytes of scratch, the static buffer "
                      "holds %lld; use mx_gemm with a caller-owned workspace", (long long)need,

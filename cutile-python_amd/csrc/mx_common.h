@@ -117,10 +117,6 @@ struct GemmArgs {
   int32_t k_splits;
   int64_t as_split_stride, bs_split_stride;   // dwords
   int64_t c_split_stride;                     // elements of C
-  // grouped gate + up projection with the activation quantised in the epilogue (ping-pong kernel): W holds up_half gate
-  // rows, then up_half up rows; silu(gate) * up goes to q [slot id][up_half] (E4M3) and qs [slot id][up_half / 32]
-  uint8_t* q; uint8_t* qs;
-  int32_t up_half, scale_mode;
 };
 
 int launch_gemm_mfma(const GemmArgs& g, int kernel_id, hipStream_t stream);

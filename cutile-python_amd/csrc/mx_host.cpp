@@ -192,7 +192,8 @@ PyObject* py_gemm_list(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const auto out_t = ((THPDtype*)a[5])->scalar_type;
   if (cnt == 0 || out_code(out_t) < 0) Py_RETURN_NONE;
   std::vector<mx_tensor> A(cnt), As(cnt), B(cnt), Bs(cnt), C(cnt);
-  std::vector<at::Tensor> outs(cnt);
+  std::vector<at::Tensor> outs(cnt), keep;   // keep: the lists may change while the GIL is released
+  keep.reserve(4 * cnt);
   at::Device dev(at::kCUDA);
   int32_t la = 0, lb = 0;
   for (Py_ssize_t i = 0; i < cnt; ++i) {
@@ -202,6 +203,13 @@ PyObject* py_gemm_list(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!product(item(0), item(1), item(2), item(3), Py_None, Py_None, &p, &d)) Py_RETURN_NONE;
     if (i > 0 && (p.la != la || p.lb != lb || d != dev)) Py_RETURN_NONE;
     la = p.la; lb = p.lb; dev = d;
+    for (int k = 0; k < 4; ++k) {
+      if (THPVariable_Check(item(k))) { keep.push_back(THPVariable_Unpack(item(k))); continue; }
+      PyObject* data = PyObject_GetAttr(item(k), s_data);   // PackedScales: product() has seen a tensor here
+      if (!data) return nullptr;
+      if (THPVariable_Check(data)) keep.push_back(THPVariable_Unpack(data));
+      Py_DECREF(data);
+    }
     if (a[4] != Py_None) {
       if (!THPVariable_Check(item(4))) Py_RETURN_NONE;
       outs[i] = THPVariable_Unpack(item(4));
@@ -229,10 +237,7 @@ PyObject* py_gemm_list(PyObject*, PyObject* const* a, Py_ssize_t n) {
   PyObject* res = PyList_New(cnt);
   if (!res) return nullptr;
   for (Py_ssize_t i = 0; i < cnt; ++i) {
-    PyObject* t;
-    if (a[4] != Py_None) { t = PySequence_Fast_GET_ITEM(a[4], i); Py_INCREF(t); }
-    else t = THPVariable_Wrap(outs[i]);
-    PyList_SET_ITEM(res, i, t);
+    PyList_SET_ITEM(res, i, THPVariable_Wrap(outs[i]));   // (a tensor of Cs is the same Python object again)
   }
   return res;
 }
@@ -262,7 +267,7 @@ PyObject* py_mma(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
   const bool batched = xd == 3 || yd == 3;
   if (acc.scalar_type() != at::kFloat || !acc.is_contiguous() || acc.dim() != (batched ? 3 : 2) || acc.size(-2) != M ||
-      acc.size(-1) != N || (batched && acc.size(0) != batch))
+      acc.size(-1) != N || (batched && acc.size(0) != batch) || acc.requires_grad())   // (there the result is a clone of acc)
     Py_RETURN_NONE;
   at::Tensor out = device_empty(acc.sizes(), at::kFloat, dev);
   mx_tensor dD = desc(acc, MX_F32), dC = desc(out, MX_F32);

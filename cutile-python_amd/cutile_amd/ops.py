@@ -177,8 +177,9 @@ class _ScaleCache:
         self._entries = collections.OrderedDict()   # key -> (weakref to base, version, PackedScales, event, stream)
 
         # the same copies by scale tensor object: (id(tensor), transposed) -> (weakref to it, version, stream,
-        # PackedScales, key into _entries).  A repeated call with the same object costs a dictionary look-up this way
-        # instead of building a key from its base, shape and strides.
+        # PackedScales, key into _entries).  A repeated call with the same object saves the stream object and the base
+        # look-up this way; where it points, its extents and strides are compared all the same, since `tensor.data = ...`
+        # and the like change them without a new object or version.
         self._by_object = {}
 
     def clear(self):
@@ -190,9 +191,13 @@ class _ScaleCache:
         e = self._by_object.get((id(s), transposed))
         if e is None or e[0]() is not s or e[1] != s._version or e[2] != stream:
             return None
+        key = e[4]
+        if key[1:5] != (s.data_ptr(), s.shape, s.stride(), s.dtype):
+            return None
         with self._lock:
-            if e[4] in self._entries:
-                self._entries.move_to_end(e[4])
+            if key not in self._entries:                  # dropped in the meantime
+                return None
+            self._entries.move_to_end(key)
         return e[3]
 
     def _remember_object(self, s, transposed, version, stream, packed, key):   # under the lock

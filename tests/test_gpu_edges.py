@@ -41,3 +41,31 @@ def test_output_column_remainders(ct, dev, kernel, out_dtype, tail):
         c.fill_(2.0)
         ct.block_scaled_matmul(a.storage, a.scale_t, b.storage.T, b.scale_t.T, C=c, kernel=kernel, accumulate=True)
         _check_guarded(c, buf, ref + 2.0)
+
+
+def test_cached_scales_follow_a_tensor_whose_data_was_replaced(ct, dev):
+    """`tensor.data = other` keeps the object and its version: the cached re-layout of the old bytes must not be used."""
+    ct.clear_scale_cache()
+    a, b = randn_operand(256, 512, O.E4M3, 5, dev), randn_operand(384, 512, O.E4M3, 6, dev)
+    run = lambda: ct.block_scaled_matmul(a.storage, s, b.storage.T, bs, cache_scales=True)
+    s, bs = a.scale_t.clone(), b.scale_t.T
+    first = [run() for _ in range(3)][-1]
+    s.data = (a.scale_t.view(torch.uint8) + 1).view(torch.float8_e8m0fnu)
+    assert torch.equal(run(), first * 2)
+    ct.clear_scale_cache()
+
+
+@pytest.mark.parametrize("K", [3584, 4000])
+@pytest.mark.parametrize("packed", [False, True])
+def test_split_that_never_applied_and_static_scratch_run_whole(ct, dev, K, packed):
+    """A forced split of a K (or scale layout) that is not split runs whole instead of failing, and the static scratch
+    takes the problems whose automatic split alone would not fit into it."""
+    a, b = randn_operand(600, K, O.E4M3, 7, dev), randn_operand(1500, K, O.E4M3, 8, dev)
+    As = ct.pack_scales(a.scale_t, operand="a") if packed else a.scale_t
+    Bs = ct.pack_scales(b.scale_t, operand="b") if packed else b.scale_t.T
+    whole = ct.block_scaled_matmul(a.storage, As, b.storage.T, Bs, split_k=1)
+    if packed or K % 512:
+        forced = ct.block_scaled_matmul(a.storage, As, b.storage.T, Bs, split_k=3)
+        assert O.rel_fro(forced.cpu(), whole.cpu()) <= 1e-5   # (fp32 sums, order of the K steps at most)
+    c = ct.block_scaled_matmul(a.storage, As, b.storage.T, Bs, static_scratch=True)
+    assert O.rel_fro(c.cpu(), whole.cpu()) <= 1e-5
