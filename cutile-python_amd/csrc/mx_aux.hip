@@ -153,25 +153,150 @@ __device__ inline void quant_store(const QuantArgs& q, const QuantUnit& u, float
   if (sub == 0) q.scale[row * q.sc_ld + kb] = scale_byte;
 }
 
-// 32 / EPL lanes per 32-element block, EPL consecutive elements per lane (8: half as many threads, and the
-// per-block work -- the amax exchange, the shared exponent, the scale byte -- is spread over twice as many
-// elements; 16-byte loads also from bf16 input); every thread handles kQuantUnroll units a grid apart and
-// requests all their inputs before it processes the first (memory-level parallelism).
-constexpr int kQuantUnroll = 2;
+// General quantiser: 32 / EPL lanes per 32-element block, EPL consecutive elements per lane; any pitch, alignment and K.
 constexpr int kQuantEpl = 8;    // 16 measured no faster (58 -> 60 us on 8192^2 fp32)
 template <int EPL>
 __global__ __launch_bounds__(256) void quantize_kernel(const QuantArgs q) {
-  const int64_t nthreads = (int64_t)gridDim.x * 256;
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  QuantUnit u[kQuantUnroll];
-  float v[kQuantUnroll][EPL], w[kQuantUnroll][EPL];
+  const QuantUnit u = quant_unit<EPL>(q, (int64_t)blockIdx.x * 256 + threadIdx.x);
+  float v[EPL], w[EPL];
+  quant_load<EPL>(q, u, v, w);
+  quant_store<EPL>(q, u, v, w);
+}
+
+// The quantiser of aligned rows (whole blocks, 16-byte loads, stores of a unit in one piece), with the source type and
+// the element format known at compile time.
+//
+// Bound: one pass over the input and the codes.  The general kernel, which decides types and alignment per element
+// group and computes the integer route beside the hardware conversions, was short of loads in flight (86 vector
+// registers, two units of 16 bytes per thread) and sent each workgroup's scale bytes out in 16-byte pieces of lines that
+// other XCDs' workgroups shared: 8192 x 8192 bf16 -> E4M3 took 44 - 49 us (4.1 - 4.6 TB/s), this one 36.6 (5.5 TB/s), and
+// 8192 x 14336 of silu(gate) * up 133 us where it took 161.  Here a wave owns U * 64 consecutive
+// units, so that a workgroup writes whole lines of scale bytes, all loads of a thread are requested before the first is used,
+// and the blocks the hardware conversion does not serve (zero, subnormal, non-finite or extreme amax) are done again
+// by the general code from memory, outside of the loop.
+template <int SRC>
+__device__ __forceinline__ void quant_unpack(const v4i (&t)[SRC == MX_F32 ? 2 : 1], float (&v)[8]) {
 #pragma unroll
-  for (int i = 0; i < kQuantUnroll; ++i) {
-    u[i] = quant_unit<EPL>(q, gid + i * nthreads);
-    quant_load<EPL>(q, u[i], v[i], w[i]);
+  for (int h = 0; h < 4; ++h) {
+    if constexpr (SRC == MX_F32) {
+      v[h] = __builtin_bit_cast(float, (uint32_t)t[0][h]);   // (the cast makes a value of the element: bit_cast of the
+      v[4 + h] = __builtin_bit_cast(float, (uint32_t)t[1][h]);   // element itself reads element 0)
+    } else if constexpr (SRC == MX_BF16) {
+      v[2 * h] = __builtin_bit_cast(float, (uint32_t)t[0][h] << 16);
+      v[2 * h + 1] = __builtin_bit_cast(float, (uint32_t)t[0][h] & 0xFFFF0000u);
+    } else {
+      v[2 * h] = (float)__builtin_bit_cast(_Float16, (uint16_t)(uint32_t)t[0][h]);
+      v[2 * h + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)((uint32_t)t[0][h] >> 16));
+    }
   }
+}
+
+template <int SRC, int FMT, bool UP, int U>
+__global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
+  constexpr int NL = SRC == MX_F32 ? 2 : 1;          // 16-byte loads per unit of 8 elements
+  constexpr int ESZ = SRC == MX_F32 ? 4 : 2;
+  typedef short s2 __attribute__((ext_vector_type(2)));
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t units = (uint32_t)(q.rows * (q.K / 8)), upr = (uint32_t)(q.K / 8);   // (below 2^31: the launcher's rule)
+  const uint32_t first = ((uint32_t)blockIdx.x * 4 + wave) * (U * 64);
+  const bool flat = q.x_ld == q.K && q.xq_ld == (FMT == MX_E2M1 ? q.K / 2 : q.K) && q.sc_ld == q.K / 32;   // uniform
+  v4i t[U][NL], t2[UP ? U : 1][NL];
+  uint32_t row[U], col[U];                           // of a unit; flat: row 0, col = unit
+  bool live[U];
 #pragma unroll
-  for (int i = 0; i < kQuantUnroll; ++i) quant_store<EPL>(q, u[i], v[i], w[i]);
+  for (int u = 0; u < U; ++u) {
+    const uint32_t id = first + u * 64 + lane;
+    live[u] = id < units;
+    col[u] = live[u] ? id : 0;
+    row[u] = 0;
+    if (!flat) {
+      row[u] = col[u] / upr;
+      col[u] -= row[u] * upr;
+    }
+    const int64_t at = ((int64_t)row[u] * q.x_ld + (int64_t)col[u] * 8) * ESZ;
+#pragma unroll
+    for (int h = 0; h < NL; ++h) {
+      t[u][h] = *(const v4i*)((const uint8_t*)q.x + at + 16 * h);
+      if constexpr (UP) t2[u][h] = *(const v4i*)((const uint8_t*)q.up + at + 16 * h);
+    }
+  }
+  const bool floor_mode = q.scale_mode != 0;
+  constexpr int EMAX = FMT == MX_E4M3 ? 8 : FMT == MX_E5M2 ? 15 : 2;
+  constexpr float FMAX = FMT == MX_E4M3 ? 448.0f : 57344.0f;
+  uint32_t again = 0;                                // bit u: unit u's block takes the general route
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    float v[8];
+    quant_unpack<SRC>(t[u], v);
+    if constexpr (UP) {
+      float w[8];
+      quant_unpack<SRC>(t2[u], w);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = silu_mul_f32(v[e], w[e]);
+    }
+    uint32_t am = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t a = __builtin_bit_cast(uint32_t, v[e]) & 0x7FFFFFFFu;
+      am = a > am ? a : am;
+    }
+    // the block's other three lanes: quad permutes
+    uint32_t o = (uint32_t)__builtin_amdgcn_mov_dpp((int)am, 0xB1, 0xF, 0xF, true);   // lanes 1 0 3 2
+    am = o > am ? o : am;
+    o = (uint32_t)__builtin_amdgcn_mov_dpp((int)am, 0x4E, 0xF, 0xF, true);            // lanes 2 3 0 1
+    am = o > am ? o : am;
+    int se;
+    if (floor_mode) {
+      se = (int)(am >> 23) - 127 - EMAX;
+    } else {
+      const uint32_t tb = __builtin_bit_cast(uint32_t, fmaxf(__fdiv_rn(__builtin_bit_cast(float, am), 448.0f), 1e-12f));
+      se = (int)(tb >> 23) - 127 + ((tb & 0x7FFFFFu) ? 1 : 0);
+    }
+    const bool fast = am >= 0x00800000u && am < 0x7F800000u && se > -127 && se < 120;
+    if (live[u] && !fast) again |= 1u << u;
+    const float sc = __builtin_bit_cast(float, (uint32_t)(se + 127) << 23);
+    if (FMT != MX_E2M1 && floor_mode) {              // saturating: clamped first, which is exact
+      const float lim = __fmul_rn(FMAX, sc);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = __builtin_amdgcn_fmed3f(v[e], -lim, lim);
+    }
+    if (live[u] && fast) {
+      const int64_t block = (int64_t)row[u] * q.sc_ld + col[u] / 4;
+      if constexpr (FMT == MX_E2M1) {
+        uint32_t r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v[0], v[1], sc, 0);
+        r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, v[2], v[3], sc, 1);
+        r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, v[4], v[5], sc, 2);
+        r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, v[6], v[7], sc, 3);
+        *(uint32_t*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 4) = r;
+      } else {
+        uint32_t w[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          s2 r = {0, 0};
+          if constexpr (FMT == MX_E4M3) {
+            r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(r, v[4 * h + 0], v[4 * h + 1], sc, false);
+            r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(r, v[4 * h + 2], v[4 * h + 3], sc, true);
+          } else {
+            r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(r, v[4 * h + 0], v[4 * h + 1], sc, false);
+            r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f32(r, v[4 * h + 2], v[4 * h + 3], sc, true);
+          }
+          w[h] = __builtin_bit_cast(uint32_t, r);
+        }
+        *(uint2*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 8) = make_uint2(w[0], w[1]);
+      }
+      if ((lane & 3) == 0) q.scale[block] = (uint8_t)(se + 127);
+    }
+  }
+  // (the four lanes of a block agree on `again`: the exchange inside quant_store stays among them)
+  if (again) {
+    for (int u = 0; u < U; ++u)
+      if (again >> u & 1) {
+        const QuantUnit un = quant_unit<8>(q, (int64_t)first + u * 64 + lane);
+        float v[8], w[8];
+        quant_load<8>(q, un, v, w);
+        quant_store<8>(q, un, v, w);
+      }
+  }
 }
 
 // ================================================================================================
@@ -504,12 +629,42 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 
 }  // namespace
 
+template <int SRC, int FMT>
+static void launch_quantize_rows(const QuantArgs& q, int64_t units, hipStream_t stream) {
+  // four units per thread once that leaves every CU several waves per SIMD, else one (a single row is a few waves: the
+  // launch is all latency).  The silu form holds two inputs per unit and computes for longer: two.
+#define MX_Q(UP, U) hipLaunchKernelGGL((quantize_rows_kernel<SRC, FMT, UP, U>), dim3((unsigned)((units + 256 * U - 1) / (256 * U))), dim3(256), 0, stream, q)
+  const bool large = units >= ((int64_t)1 << 20);
+  if (q.up) { if (large) MX_Q(true, 2); else MX_Q(true, 1); }
+  else { if (large) MX_Q(false, 4); else MX_Q(false, 1); }
+#undef MX_Q
+}
+
 int launch_quantize(const QuantArgs& q, hipStream_t stream) {
   const int64_t units = q.rows * (q.Kpad / 32) * (32 / kQuantEpl);
   if (units <= 0) return MX_OK;
-  const int64_t blocks = (units + 256 * kQuantUnroll - 1) / (256 * kQuantUnroll);
+  const int64_t blocks = (units + 255) / 256;
   if (blocks > 0x7FFFFFFF) return set_error(MX_ERR_SHAPE, "quantize: tensor too large");
-  hipLaunchKernelGGL(quantize_kernel<kQuantEpl>, dim3((unsigned)blocks), dim3(256), 0, stream, q);
+  // whole blocks, rows of x at multiples of 16 bytes, a unit's codes (8 or 4 bytes) aligned
+  const int esz = q.x_dtype == MX_F32 ? 4 : 2, cb = q.fmt == MX_E2M1 ? 4 : 8;
+  const bool rows_ok = q.K % 32 == 0 && units < ((int64_t)1 << 31) && (((uintptr_t)q.x | (uintptr_t)q.up | (uintptr_t)(q.x_ld * esz)) & 15) == 0 &&
+                       (((uintptr_t)q.xq | (uintptr_t)q.xq_ld) & (cb - 1)) == 0;
+  if (rows_ok) {
+#define MX_CASE(SRC, FMT) \
+    if (q.x_dtype == SRC && q.fmt == FMT) launch_quantize_rows<SRC, FMT>(q, units, stream);
+    MX_CASE(MX_BF16, MX_E4M3)
+    MX_CASE(MX_BF16, MX_E5M2)
+    MX_CASE(MX_BF16, MX_E2M1)
+    MX_CASE(MX_F32, MX_E4M3)
+    MX_CASE(MX_F32, MX_E5M2)
+    MX_CASE(MX_F32, MX_E2M1)
+    MX_CASE(MX_F16, MX_E4M3)
+    MX_CASE(MX_F16, MX_E5M2)
+    MX_CASE(MX_F16, MX_E2M1)
+#undef MX_CASE
+  } else {
+    hipLaunchKernelGGL(quantize_kernel<kQuantEpl>, dim3((unsigned)blocks), dim3(256), 0, stream, q);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "quantize_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;

@@ -274,3 +274,38 @@ def test_quantize_nonfinite_blocks_follow_the_reference_rule(ct, dev, dt):
     codes, sb = O.block_quantize(x, 32, fmt, "ceil")
     assert np.array_equal(got_s.view(torch.uint8).cpu().numpy(), sb)
     assert np.array_equal(got_q.view(torch.uint8).cpu().numpy(), codes)
+
+
+@pytest.mark.parametrize("src", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("fmt", [O.E4M3, O.E5M2, O.E2M1])
+@pytest.mark.parametrize("mode", ["ceil", "floor"])
+@pytest.mark.parametrize("rows,K,pitch", [(3, 96, 96), (5, 2080, 2112), (1025, 8192, 8192), (1031, 8224, 8256)])
+def test_quantize_aligned_rows_match_the_general_route(ct, dev, src, fmt, mode, rows, K, pitch):
+    """The aligned-row kernel (one and four units per thread, flat and pitched rows, a remainder of its last wave)
+    against the general one, which the same values take when no row starts on 16 bytes; zero, subnormal, non-finite and
+    ordinary blocks side by side."""
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x = torch.randn((rows, pitch), generator=g, device=dev)
+    blk = x.view(-1, 32)
+    blk[::7] = 0
+    blk[3::11] *= 1e-30
+    blk[5::13, 4] = float("inf")
+    blk[6::17, 9] = float("nan")
+    blk[1::19] *= 1e4
+    x = x.to(src)[:, :K]
+    off = torch.empty(rows * (K + 1) + 8, dtype=src, device=dev)[1:1 + rows * (K + 1)].view(rows, K + 1)[:, :K]
+    off.copy_(x)
+    q, s = ct.block_quantize(x, 32, DT[fmt], scale_mode=mode)
+    q0, s0 = ct.block_quantize(off, 32, DT[fmt], scale_mode=mode)
+    assert torch.equal(s.view(torch.uint8), s0.view(torch.uint8))
+    assert torch.equal(q.view(torch.uint8), q0.view(torch.uint8))
+
+
+@pytest.mark.parametrize("rows,F", [(3, 96), (1100, 8192)])
+def test_silu_quantize_aligned_rows_match_the_general_route(ct, dev, rows, F):
+    gate_up = torch.randn((rows, 2 * F), device=dev, generator=torch.Generator(device=dev).manual_seed(3)).bfloat16()
+    off = torch.empty(rows * (2 * F + 1) + 8, dtype=torch.bfloat16, device=dev)[1:1 + rows * (2 * F + 1)].view(rows, 2 * F + 1)[:, :2 * F]
+    off.copy_(gate_up)
+    q, s = ct.silu_and_mul_quantize(gate_up)
+    q0, s0 = ct.silu_and_mul_quantize(off)
+    assert torch.equal(s.view(torch.uint8), s0.view(torch.uint8)) and torch.equal(q.view(torch.uint8), q0.view(torch.uint8))
