@@ -263,6 +263,28 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
     using OutT = std::conditional_t<kd == 1, uint16_t, float>;
     OutT* const Cp = kd == 2 ? (OutT*)(g.partial + (int64_t)split * g.M * g.N) : (OutT*)g.C + (int64_t)bz * g.c_batch;
     const int64_t ld = kd == 2 ? g.N : g.ldc;
+    // the fp32 addend (its own operand, or C): every load is requested before the first is waited for, with offsets beyond
+    // the matrix for what does not exist.  (One guarded load after another, as for the rows below that are not whole
+    // 16-byte pieces, the addend cost more than the product: six 200 x 328 x 992 took 17 us instead of 9.)
+    v4f add[kd == 0 && !GROUPED ? MT : 1][4];
+    bool added = false;
+    if constexpr (kd == 0 && !GROUPED) {
+      const float* const addend = g.acc ? g.acc + (int64_t)bz * g.c_batch : g.accumulate ? (const float*)Cp : nullptr;
+      if (addend && g.N % 4 == 0 && ld % 4 == 0 && (uintptr_t)addend % 16 == 0 && (int64_t)g.M * ld < (1 << 29)) {   // uniform
+        added = true;
+        const __amdgpu_buffer_rsrc_t rsD = make_rsrc(addend, (uint32_t)(((int64_t)(g.M - 1) * ld + g.N) * 4));
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const int m = m0 + wm0 + 16 * i + r;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int c = 32 * (j / 2) + 4 * (j % 2);
+            const uint32_t at = m < g.M && c < cols ? (uint32_t)((m * ld + n + c) * 4) : kOobOffset;
+            add[i][j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsD, at, 0, 0));
+          }
+        }
+      }
+    }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const int m = m0 + wm0 + 16 * i + r;
@@ -281,7 +303,9 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
         v4f v0 = acc[i][2 * jp], v1 = acc[i][2 * jp + 1];
         if constexpr (GROUPED) { v0 *= w; v1 *= w; }
         const int64_t off = row * ld + n + 32 * jp;
-        if (kd != 2 && g.acc) add8_edge<float>(g.acc + (int64_t)bz * g.c_batch + off, v0, v1, cols - 32 * jp);
+        if (added) {
+          if constexpr (kd == 0 && !GROUPED) { v0 += add[i][2 * jp]; v1 += add[i][2 * jp + 1]; }
+        } else if (kd != 2 && g.acc) add8_edge<float>(g.acc + (int64_t)bz * g.c_batch + off, v0, v1, cols - 32 * jp);
         else if (kd != 2 && g.accumulate) add8_edge<OutT>(Cp + off, v0, v1, cols - 32 * jp);
         store8_edge<OutT>(Cp + off, v0, v1, cols - 32 * jp);
       }
