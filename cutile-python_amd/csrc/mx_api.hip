@@ -4,10 +4,12 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <vector>
 
 #include "mx_common.h"
+#include "mx_gemm_pp.h"
 #include "mx_gemm_t128.h"
 #include "mx_stream.h"
 
@@ -853,7 +855,7 @@ int mx_gemm_list(int32_t count, const mx_tensor* A, const mx_tensor* As, const m
     items.push_back(it);
   }
   // Pass 2: one scale re-layout launch per 64 scale tensors, one persistent GEMM launch per 32 problems of one
-  // element-format pair and scale layout
+  // element-format pair
   std::vector<PackArgs> packs;
   for (const Item& it : items) {
     if (!it.simple) continue;
@@ -869,12 +871,13 @@ int mx_gemm_list(int32_t count, const mx_tensor* A, const mx_tensor* As, const m
     const T128Args& g0 = items[i].plan.g;
     for (size_t j = i; j < items.size(); ++j) {
       const T128Args& g = items[j].plan.g;
-      if (items[j].simple && !done[j] && g.a_fmt == g0.a_fmt && g.b_fmt == g0.b_fmt && g.a_plain == g0.a_plain &&
-          g.b_plain == g0.b_plain) {
+      if (items[j].simple && !done[j] && g.a_fmt == g0.a_fmt && g.b_fmt == g0.b_fmt) {
         group.push_back(g);
         done[j] = 1;
       }
     }
+    // longest products first: a workgroup's second tile is then a short one
+    std::stable_sort(group.begin(), group.end(), [](const T128Args& x, const T128Args& y) { return x.K > y.K; });
     if (int rc = launch_gemm_t128_list(group.data(), (int)group.size(), (hipStream_t)stream)) return rc;
   }
   // Pass 3: the rest (large problems for the persistent 256 x 256 kernel, skinny ones for the decode kernel,

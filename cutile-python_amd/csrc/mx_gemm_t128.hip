@@ -328,7 +328,8 @@ constexpr int kListMax = 32;
 struct ListProblem {
   const uint8_t* A; const uint8_t* B; const uint8_t* As; const uint8_t* Bs; void* C;
   int64_t lda, ldb, ldas, ldbs, ldc;
-  int32_t M, N, K, c_dtype;
+  int32_t M, N, K;
+  int16_t c_dtype, plain;              // plain: both operands' scales are read where they are
 };
 struct T128List {
   ListProblem p[kListMax];
@@ -336,7 +337,9 @@ struct T128List {
   int32_t n;
 };
 
-template <class C, bool AP, bool BP>
+// Problems whose scales are read in place and problems whose scales were re-laid share the launch: one after the other, two
+// launches of 24 problems of 96 .. 1536 took 16.6 + 10.9 us, each waiting for its own longest product.
+template <class C>
 __global__ __launch_bounds__(256, 2) void t128_list_kernel(const T128List gl) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_generic[];
   lds_u8* const smem = (lds_u8*)smem_generic;
@@ -351,7 +354,8 @@ __global__ __launch_bounds__(256, 2) void t128_list_kernel(const T128List gl) {
     g.M = q.M; g.N = q.N; g.K = q.K; g.c_dtype = q.c_dtype;
     g.k_splits = 1;
 #if defined(__HIP_DEVICE_COMPILE__)   // (the host pass, which needs the kernel's stub only, refuses the call)
-    t128_tile<C, 2, AP, BP, false>(g, smem, t - gl.first_tile[i], 0, 0);
+    if (q.plain) t128_tile<C, 2, true, true, false>(g, smem, t - gl.first_tile[i], 0, 0);
+    else t128_tile<C, 2, false, false, false>(g, smem, t - gl.first_tile[i], 0, 0);
 #endif
     // the tile's trailing (zero-fill) DMA has left the queue and every wave is done with the LDS stages before
     // the next tile's loads reuse them
@@ -378,9 +382,9 @@ int launch_one(const T128Args& g, hipStream_t stream) {
   return MX_OK;
 }
 
-template <class C, bool AP, bool BP>
+template <class C>
 int launch_list(const T128List& gl, hipStream_t stream) {
-  auto kern = t128_list_kernel<C, AP, BP>;
+  auto kern = t128_list_kernel<C>;
   constexpr int lds = 2 * C::STAGE + 2 * 4096;
   static int attr_done = 0;   // benign race: the attribute call is idempotent
   if (!attr_done) {
@@ -424,15 +428,14 @@ int t128_list_pair(const T128Args* problems, int n, hipStream_t stream) {
       ListProblem& q = gl.p[gl.n];
       q.A = g.A; q.B = g.B; q.As = g.As; q.Bs = g.Bs; q.C = g.C;
       q.lda = g.lda; q.ldb = g.ldb; q.ldas = g.ldas; q.ldbs = g.ldbs; q.ldc = g.ldc;
-      q.M = g.M; q.N = g.N; q.K = g.K; q.c_dtype = g.c_dtype;
+      q.M = g.M; q.N = g.N; q.K = g.K; q.c_dtype = (int16_t)g.c_dtype; q.plain = g.a_plain && g.b_plain;
       gl.first_tile[gl.n] = (int32_t)total;
       total += (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
       if (total > 0x7FFFFFFF) return set_error(MX_ERR_SHAPE, "gemm list: too many tiles");
       ++gl.n;
     }
     gl.first_tile[gl.n] = (int32_t)total;
-    const bool plain = problems[0].a_plain && problems[0].b_plain;
-    if (int rc = plain ? launch_list<C, true, true>(gl, stream) : launch_list<C, false, false>(gl, stream)) return rc;
+    if (int rc = launch_list<C>(gl, stream)) return rc;
   }
   return MX_OK;
 }
@@ -468,8 +471,8 @@ int launch_gemm_t128(const T128Args& g, hipStream_t stream) {
 
 int launch_gemm_t128_list(const T128Args* p, int n, hipStream_t stream) {
   for (int i = 0; i < n; ++i)
-    if (p[i].a_fmt != p[0].a_fmt || p[i].b_fmt != p[0].b_fmt || p[i].a_plain != p[0].a_plain || p[i].b_plain != p[0].b_plain)
-      return set_error(MX_ERR_INVALID, "gemm list: problems of one launch must share formats and scale layouts");
+    if (p[i].a_fmt != p[0].a_fmt || p[i].b_fmt != p[0].b_fmt || !p[i].a_plain != !p[i].b_plain)
+      return set_error(MX_ERR_INVALID, "gemm list: problems of one launch must share formats, their operands the scale layout");
 #define MX_CASE(AF, BF) \
   if (p[0].a_fmt == AF && p[0].b_fmt == BF) return t128_list_pair<AF, BF>(p, n, stream);
   MX_CASE(MX_E4M3, MX_E4M3)
