@@ -100,10 +100,15 @@ float est_t128(int64_t M, int64_t N, int64_t K, int S, bool fp4, int64_t batch =
   if (S > 1) t += 4.f + (float)S * M * N * 8 / 4e6f;
   return t;
 }
-float est_pp(int64_t M, int64_t N, int64_t K, bool fp4, bool pack) {
+float est_pp(int64_t M, int64_t N, int64_t K, bool fp4, bool pack, bool tail) {
   const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128));
-  return 8.f + st * (tiles <= 128 ? (fp4 ? 1.3f : 1.1f) : (fp4 ? 1.8f : 1.45f) * ((tiles + 255) / 256)) + (pack ? 5.f : 0.f);
+  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)), per = fp4 ? 1.8f : 1.45f;
+  const float rest = 8.f + (pack ? 5.f : 0.f);
+  if (tail) {   // the last round split S ways, its partial sums added up by a second launch
+    const int left = (int)((tiles % 256 + 7) / 8), KQ = (int)(K / 512), S = tail_splits(left, 32, KQ, fp4);
+    if (S > 1) return rest + st * per * (tiles / 256) + tail_tenths(S, left, 32, KQ, fp4) * 0.1f;
+  }
+  return rest + st * (tiles <= 128 ? (fp4 ? 1.3f : 1.1f) : per * ((tiles + 255) / 256));
 }
 float est_stream(int64_t M, int64_t N, int64_t K, int w_fmt) { return 5.f + 0.57f * stream_plan(M, N, K, w_fmt).cost; }
 
@@ -185,8 +190,9 @@ int64_t mx_packed_scale_bytes(int64_t rows, int64_t K) {
   return round256(packed_scale_dwords(rows, K) * 4);
 }
 
-int64_t mx_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, const mx_gemm_opts* opts) {
-  const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
+namespace {
+// what a product cannot do without: re-laid scales, partial sums of split-K
+int64_t gemm_workspace_min(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
   if (o.kernel == MX_KERNEL_GENERIC || o.kernel == MX_KERNEL_STREAM || o.kernel == MX_KERNEL_DECODE) return 0;
   int64_t b = 0;
   const int S = plan_k_splits(M, N, K, o);
@@ -195,14 +201,38 @@ int64_t mx_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, const mx_gemm_o
   if (!is_native(o.b_scale_layout)) b += mx_packed_scale_bytes(N, K);
   return b;
 }
-
-int64_t mx_gemm_grouped_workspace_bytes(int64_t num_slots, int64_t N, int64_t K, int64_t E,
-                                        const mx_gemm_opts* opts) {
-  const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
+// beyond that, what lets the ping-pong kernel split its last round along K (0: it would not): only for problems that it may
+// be picked for
+int64_t gemm_workspace_tail(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
+  if ((o.kernel != MX_KERNEL_AUTO && o.kernel != MX_KERNEL_MFMA_PINGPONG) || o.split_k > 1 || o.block_size != 32 || M <= 0 || N <= 0 ||
+      K <= 0)
+    return 0;
+  const int64_t t = pp_tail_bytes(M, N, K, false, true);
+  if (t == 0 || o.kernel == MX_KERNEL_MFMA_PINGPONG) return t;
+  if (M <= kStreamAutoM) return 0;
+  const bool pack = !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout);
+  for (int fp4 = 0; fp4 < 2; ++fp4)
+    if (est_pp(M, N, K, fp4, pack, true) < est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4)) return t;
+  return 0;
+}
+int64_t grouped_workspace_min(int64_t num_slots, int64_t N, int64_t K, int64_t E, const mx_gemm_opts& o) {
   if (o.kernel == MX_KERNEL_GENERIC) return 0;
   int64_t b = mx_packed_scale_bytes(num_slots, K);
   if (!is_native(o.b_scale_layout)) b += E * mx_packed_scale_bytes(N, K);
   return b;
+}
+}  // namespace
+
+int64_t mx_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, const mx_gemm_opts* opts) {
+  const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
+  return gemm_workspace_min(M, N, K, o) + gemm_workspace_tail(M, N, K, o);
+}
+
+int64_t mx_gemm_grouped_workspace_bytes(int64_t num_slots, int64_t N, int64_t K, int64_t E,
+                                        const mx_gemm_opts* opts) {
+  const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
+  const bool pp = (o.kernel == MX_KERNEL_AUTO && N > 128) || o.kernel == MX_KERNEL_MFMA_PINGPONG;
+  return grouped_workspace_min(num_slots, N, K, E, o) + (pp ? pp_tail_bytes(num_slots, N, K, false, false) : 0);
 }
 
 namespace {
@@ -415,7 +445,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       if (ok && batch > 1) {   // few long products are better off one by one with K split, large ones gain nothing
         float alone = est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4);
         if (o.kernel == MX_KERNEL_AUTO) {
-          const float pp = est_pp(M, N, K, fp4, true);
+          const float pp = est_pp(M, N, K, fp4, true, false);
           if (pp < alone) alone = pp;
           if (!fp4 && M <= kStreamAutoM && est_stream(M, N, K, B->dtype) < alone) alone = est_stream(M, N, K, B->dtype);
         }
@@ -520,7 +550,9 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     else {
       const bool fp4 = A->dtype == MX_E2M1;
       const float t128 = est_t128(M, N, K, o.split_k > 1 ? 1 : plan_k_splits(M, N, K, o), fp4);
-      const float pp = o.split_k > 1 ? 1e30f : est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout));
+      const bool room = workspace && pp_tail_bytes(M, N, K, fp4, true) > 0 &&
+                        workspace_bytes >= gemm_workspace_min(M, N, K, o) + pp_tail_bytes(M, N, K, fp4, true);
+      const float pp = o.split_k > 1 ? 1e30f : est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), room);
       const float st = may_stream ? est_stream(M, N, K, B->dtype) : 1e30f;
       kernel = st < t128 && st < pp ? MX_KERNEL_STREAM : t128 <= pp ? MX_KERNEL_MFMA_128x128 : big_tile_kernel();
     }
@@ -577,7 +609,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
 
   if (kernel == MX_KERNEL_STREAM) {
     // it uses no workspace, but a caller of MX_KERNEL_AUTO is held to what mx_gemm_workspace_bytes says, whatever is picked
-    const int64_t need = mx_gemm_workspace_bytes(M, N, K, &o);
+    const int64_t need = gemm_workspace_min(M, N, K, o);
     if (B->dtype != MX_E2M1 && need > 0 && (!workspace || workspace_bytes < need))
       return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                        (long long)workspace_bytes);
@@ -624,7 +656,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
 
   // ---- MFMA path: bring the scales into the native layout if they are not ----------------------------
   uint8_t* ws = (uint8_t*)workspace;
-  int64_t need = mx_gemm_workspace_bytes(M, N, K, &o);
+  int64_t need = gemm_workspace_min(M, N, K, o);
   if (need > 0 && (!ws || workspace_bytes < need))
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                      (long long)workspace_bytes);
@@ -759,6 +791,10 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
   g.a_fmt = A->dtype; g.b_fmt = B->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate;
   g.a_rows = M;
   g.replicas = 1;
+  if (kernel == MX_KERNEL_MFMA_PINGPONG && workspace && ((uintptr_t)workspace) % 256 == 0) {
+    const int64_t tail = pp_tail_bytes(M, N, K, A->dtype == MX_E2M1 && B->dtype == MX_E2M1, true);
+    if (tail > 0 && workspace_bytes >= need + tail) g.tail = (float*)((uint8_t*)workspace + need);
+  }
   return launch_gemm_mfma(g, kernel, (hipStream_t)stream);
 }
 }  // namespace
@@ -782,8 +818,8 @@ int mx_gemm_static(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, 
     return set_error(MX_ERR_SHAPE, "mx_gemm_static: A and B must have 2 or 3 dimensions");
   int64_t M, N, K;
   problem_dims(*A, *B, M, N, K);
-  int64_t need = mx_gemm_workspace_bytes(M, N, K, opts);
   mx_gemm_opts o = opts ? *opts : kDefaultOpts;
+  int64_t need = gemm_workspace_min(M, N, K, o);
   if (need > MX_STATIC_SCRATCH_BYTES && o.split_k == 0) {
     // the partial sums of an automatic split are what does not fit: run it whole.  (Plain scales with a K that splits into
     // equal slices of 512 have always been held to the buffer, and stay refused.)
@@ -794,7 +830,7 @@ int mx_gemm_static(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, 
     if (S > 1 && !even) {
       o.split_k = 1;
       opts = &o;
-      need = mx_gemm_workspace_bytes(M, N, K, opts);
+      need = gemm_workspace_min(M, N, K, o);
     }
   }
   if (need > MX_STATIC_SCRATCH_BYTES)
@@ -813,7 +849,7 @@ int64_t mx_gemm_list_workspace_bytes(int32_t count, const mx_tensor* A, const mx
   for (int32_t i = 0; i < count; ++i) {
     int64_t M, N, K;
     problem_dims(A[i], B[i], M, N, K);
-    need += round256(mx_gemm_workspace_bytes(M, N, K, opts));
+    need += round256(gemm_workspace_min(M, N, K, opts ? *opts : kDefaultOpts));
   }
   return need;
 }
@@ -839,7 +875,7 @@ int mx_gemm_list(int32_t count, const mx_tensor* A, const mx_tensor* As, const m
   for (int32_t i = 0; i < count; ++i) {
     int64_t M, N, K;
     problem_dims(A[i], B[i], M, N, K);
-    const int64_t b = round256(mx_gemm_workspace_bytes(M, N, K, opts));
+    const int64_t b = round256(gemm_workspace_min(M, N, K, opts ? *opts : kDefaultOpts));
     Item it = {};
     it.index = i; it.ws_off = off; it.ws_bytes = b;
     off += b;
@@ -929,11 +965,13 @@ int mx_bench_gemm(int32_t nsets, const mx_tensor* A, const mx_tensor* As, const 
   return rc;
 }
 
-int mx_gemm_grouped(const mx_tensor* A, const mx_tensor* As, const mx_tensor* W, const mx_tensor* Ws,
-                    mx_tensor* C, const float* topk_weights, const int32_t* sorted_token_ids,
-                    int64_t num_slots, const int32_t* sorted_expert_ids, int32_t tile_m,
-                    int32_t num_token_replicas, int64_t num_valid_ids, const mx_gemm_opts* opts,
-                    void* workspace, int64_t workspace_bytes, void* stream) {
+namespace {
+// slots_in_use: on the device, may be null (all num_slots); slots beyond it hold no routed row
+int gemm_grouped_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* W, const mx_tensor* Ws,
+                      mx_tensor* C, const float* topk_weights, const int32_t* sorted_token_ids,
+                      int64_t num_slots, const int32_t* slots_in_use, const int32_t* sorted_expert_ids, int32_t tile_m,
+                      int32_t num_token_replicas, int64_t num_valid_ids, const mx_gemm_opts* opts,
+                      void* workspace, int64_t workspace_bytes, void* stream) {
   const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
   if (int rc = check_tensor(A, "A", 2, 2)) return rc;
   if (int rc = check_tensor(As, "A_scale", 2, 2)) return rc;
@@ -1007,7 +1045,7 @@ int mx_gemm_grouped(const mx_tensor* A, const mx_tensor* As, const mx_tensor* W,
   }
 
   uint8_t* ws = (uint8_t*)workspace;
-  const int64_t need = mx_gemm_grouped_workspace_bytes(num_slots, N, K, E, &o);
+  const int64_t need = grouped_workspace_min(num_slots, N, K, E, o);
   if (!ws || workspace_bytes < need)
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                      (long long)workspace_bytes);
@@ -1085,7 +1123,22 @@ int mx_gemm_grouped(const mx_tensor* A, const mx_tensor* As, const mx_tensor* W,
   g.b_expert_stride = W->stride[0];
   g.bs_expert_stride = mx_packed_scale_bytes(N, K) / 4;
   g.a_rows = T;
+  g.num_slots = slots_in_use;
+  if (kernel == MX_KERNEL_MFMA_PINGPONG) {
+    const int64_t tail = pp_tail_bytes(num_slots, N, K, A->dtype == MX_E2M1 && W->dtype == MX_E2M1, !slots_in_use);
+    if (tail > 0 && workspace_bytes >= need + tail) g.tail = (float*)((uint8_t*)workspace + need);
+  }
   return launch_gemm_mfma(g, kernel, (hipStream_t)stream);
+}
+}  // namespace
+
+int mx_gemm_grouped(const mx_tensor* A, const mx_tensor* As, const mx_tensor* W, const mx_tensor* Ws,
+                    mx_tensor* C, const float* topk_weights, const int32_t* sorted_token_ids,
+                    int64_t num_slots, const int32_t* sorted_expert_ids, int32_t tile_m,
+                    int32_t num_token_replicas, int64_t num_valid_ids, const mx_gemm_opts* opts,
+                    void* workspace, int64_t workspace_bytes, void* stream) {
+  return gemm_grouped_impl(A, As, W, Ws, C, topk_weights, sorted_token_ids, num_slots, nullptr, sorted_expert_ids, tile_m,
+                           num_token_replicas, num_valid_ids, opts, workspace, workspace_bytes, stream);
 }
 
 int64_t mx_moe_align_max_slots(int64_t num_ids, int32_t num_experts, int32_t tile_m) {
@@ -1125,7 +1178,7 @@ struct MoePlan {
   int64_t T, n, E, H, F, H_out;
   bool stream;          // experts' weights streamed for a few rows each; otherwise grouped GEMMs on aligned slots
   int32_t tile_m;
-  int64_t q, qs, c3, c1, slots, max_slots, blocks, align, grouped, grouped_bytes, total;   // offsets (bytes)
+  int64_t q, qs, c3, c1, slots, in_use, max_slots, blocks, align, grouped, grouped_bytes, total;   // offsets (bytes)
 };
 // Rows per expert up to which the weights are streamed.
 constexpr int64_t kMoeStreamRows = 48;
@@ -1144,6 +1197,7 @@ MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& 
     p.max_slots = mx_moe_align_max_slots(p.n, (int32_t)p.E, p.tile_m);
     p.c1 = take(p.n * p.F * 4);
     p.slots = take(p.max_slots * 4);
+    p.in_use = take(4);
     p.blocks = take(p.max_slots / p.tile_m * 4);
     p.align = take(mx_moe_align_workspace_bytes(p.n, (int32_t)p.E));
     mx_gemm_opts g1 = kDefaultOpts, g2 = kDefaultOpts;
@@ -1249,20 +1303,23 @@ int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1,
   } else {
     int32_t* const slots = (int32_t*)(ws + p.slots);
     int32_t* const blocks = (int32_t*)(ws + p.blocks);
-    if (int rc = launch_moe_align(topk_ids, ids64, p.n, (int32_t)E, p.tile_m, slots, blocks, nullptr, p.max_slots,
+    // max_slots is what the worst routing needs; the GEMMs walk the tiles of the slots in use only (4096 tokens x 2, 8
+    // experts: 36 tile rows, not 39, so 16 rounds of 256 tiles for the first projection where there were 18)
+    int32_t* const in_use = (int32_t*)(ws + p.in_use);
+    if (int rc = launch_moe_align(topk_ids, ids64, p.n, (int32_t)E, p.tile_m, slots, blocks, in_use, p.max_slots,
                                   (int32_t*)(ws + p.align), st))
       return rc;
     mx_gemm_opts g = kDefaultOpts;
     g.b_scale_layout = o.a_scale_layout;
     mx_tensor c1 = tensor2d(ws + p.c1, MX_BF16, p.n, 2 * F, 2 * F);
-    if (int rc = mx_gemm_grouped(X, Xs, W1, W1s, &c1, nullptr, slots, p.max_slots, blocks, p.tile_m, topk, p.n, &g, ws + p.grouped,
+    if (int rc = gemm_grouped_impl(X, Xs, W1, W1s, &c1, nullptr, slots, p.max_slots, in_use, blocks, p.tile_m, topk, p.n, &g, ws + p.grouped,
                                  p.grouped_bytes, stream))
       return rc;
     mx_tensor q = tensor2d(ws + p.q, MX_E4M3, p.n, F, F), qs = tensor2d(ws + p.qs, MX_E8M0, p.n, F / 32, F / 32);
     if (int rc = mx_silu_mul_quantize(&c1, &q, &qs, scale_mode, stream)) return rc;
     g.b_scale_layout = o.b_scale_layout;
     mx_tensor c3 = tensor2d(ws + p.c3, MX_F32, p.n, H_out, H_out);
-    if (int rc = mx_gemm_grouped(&q, &qs, W2, W2s, &c3, topk_weights, slots, p.max_slots, blocks, p.tile_m, 1, p.n, &g,
+    if (int rc = gemm_grouped_impl(&q, &qs, W2, W2s, &c3, topk_weights, slots, p.max_slots, in_use, blocks, p.tile_m, 1, p.n, &g,
                                  ws + p.grouped, p.grouped_bytes, stream))
       return rc;
   }

@@ -27,6 +27,12 @@
 // while the other team is in an MFMA phase, so neither the pipeline fill nor the epilogue idles the
 // matrix pipe.  A workgroup is given more than one tile only when a tile has at least two stages and
 // a whole number of K-quads (K a multiple of 512).
+//
+// Last round: tiles that would leave most of the workgroups idle are split along K among them (SPLIT; tail_splits in
+// mx_gemm_pp.h says when), each workgroup's last tile then being some K-quads of one.  The sums leave as they lie in the
+// registers (1 KiB per store) and pp_tail_kernel adds and writes them.  The grouped form knows how many slots hold rows
+// only on the device (num_slots) and walks the tiles of those.  4096 tokens x 2 in 8 experts, 4096 x 14336 MXFP8: the first
+// projection, 18 rounds of the upper bound's 39 tile rows, 929 -> 868 us; the second, 2.25 rounds, 514 -> 413 + 17 us.
 #include <stdlib.h>
 
 #include <type_traits>
@@ -39,7 +45,9 @@ namespace {
 // KTAIL: K is not a whole number of stages (or there is a single stage): the 16-byte chunks beyond the end of K are
 // masked lane by lane at issue time.  Without it the loads take their precomputed offsets as they are, which keeps a
 // compare and a select per DMA instruction out of the memory phase.
-template <class C, typename OutT, bool GROUPED, int TEAM, bool KTAIL>
+// SPLIT: the walk may end with a K range of one more tile, whose sums go to g.tail.  (An instance of its own: the few scalars
+// more cost the whole-round products, MXFP4 8192^3 232.2 -> 234.0 us.)
+template <class C, typename OutT, bool GROUPED, bool SPLIT, int TEAM, bool KTAIL>
 __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, const int wn,
                                         const int lane, const TileWalk& walk) {
   using P = PP<C>;
@@ -56,6 +64,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   const int ksteps = (g.K + 127) / 128;
   const int nstages = (ksteps + C::KSUB - 1) / C::KSUB;
   const int KQ = (ksteps + 3) / 4;
+  constexpr int SPQ = 4 / C::KSUB;   // stages per K-quad
   const int a_groups = (g.M + 63) / 64, b_groups = (g.N + 63) / 64;
   const __amdgpu_buffer_rsrc_t rsA = make_rsrc(g.A, (uint32_t)(g.a_rows * g.lda));
 
@@ -92,8 +101,14 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   // then a vote, so a sentinel in front of valid ids does not hide them).  Such a half has nothing to multiply:
   // its fragment reads and MFMAs are skipped.
   bool skip_cur = false, skip_nxt = false;
+  int kq_nxt = KQ;   // K-quads of the tile being fetched
   auto set_fetch_tile = [&](int lid) {
-    fetch_valid = lid < walk.end;
+    fetch_valid = SPLIT ? lid != kNoTile : lid < walk.end;
+    // a tile that is split along K starts at K-quad q0: folded into the offsets, so that stages count from 0 in every tile
+    const bool part = SPLIT && fetch_valid && lid >= walk.end;
+    const int qb = part ? walk.quads & 0xFFFF : 0;
+    kq_nxt = part ? walk.quads >> 16 : KQ;
+    const uint32_t ka0 = (uint32_t)(qb * SPQ * C::A_RB), kb0 = (uint32_t)(qb * SPQ * C::B_RB);
     int m0 = 0, n0 = 0;
     if (fetch_valid) walk.origin(lid, m0, n0);
     if constexpr (GROUPED) {
@@ -126,36 +141,39 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
         ok = ok && id >= 0 && id < g.num_valid_ids;
         grow = id / g.replicas;
       }
-      a_voff[q] = ok ? (uint32_t)(grow * g.lda + a_col0) : kOobOffset;
+      a_voff[q] = ok ? (uint32_t)(grow * g.lda + a_col0) + ka0 : kOobOffset;
     }
     if constexpr (TEAM == 1) {
 #pragma unroll
       for (int q = 0; q < BL; ++q) {
         const int col = b_col(q);
         const int64_t grow = n0 + b_row0 + q * P::B_RPI;
-        b_voff[q] = (fetch_valid && grow < g.N) ? (uint32_t)(grow * g.ldb + col) : kOobOffset;
+        b_voff[q] = (fetch_valid && grow < g.N) ? (uint32_t)(grow * g.ldb + col) + kb0 : kOobOffset;
       }
     }
     // a tile that overhangs the matrix reuses the last scale group (its rows are discarded anyway)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int grp = (m0 + wm0) / 64 + u;
-      as_nxt[u] = (grp < a_groups ? grp : a_groups - 1) * KQ * 1024;
+      as_nxt[u] = ((grp < a_groups ? grp : a_groups - 1) * KQ + qb) * 1024;
     }
     const int grp = (n0 + wn0) / 64;
     bs_nxt = (GROUPED ? (int)(expert * (g.bs_expert_stride * 4)) : 0) +
-             (grp < b_groups ? grp : b_groups - 1) * KQ * 1024;
+             ((grp < b_groups ? grp : b_groups - 1) * KQ + qb) * 1024;
   };
-  // local stage sl of the fetch tile into A buffer abuf / B buffer bbuf; a stage at or beyond nstages
-  // and the 16-byte chunks beyond the end of K read nothing and zero-fill their LDS bytes
-  // (out-of-range buffer offset)
+  int kq = KQ;       // K-quads of the tile being computed
+  auto nst = [&]() { return SPLIT ? kq * SPQ : nstages; };   // its stages
+  // local stage sl of the fetch tile into A buffer abuf / B buffer bbuf; a stage at or beyond nst and the 16-byte chunks
+  // beyond the end of K read nothing and zero-fill their LDS bytes (out-of-range buffer offset).  (Walks of several tiles
+  // have two stages or more in every tile, so the first two of the next one pass as well; a tile that is split along K has
+  // whole stages only: its limits below are those of its first quad, never too small.)
   auto issue_a = [&](int sl, int abuf) {
     lds_u8* const base = smem + abuf * C::A_STAGE + wm0 * C::A_RB + wn * 1024;
     const int ka = sl * C::A_RB;
-    const int klim = sl < nstages ? Kb_a - ka : 0;   // bytes of this stage's rows that exist
+    const int klim = sl < nst() ? Kb_a - ka : 0;   // bytes of this stage's rows that exist
 #pragma unroll
     for (int q = 0; q < AL; ++q) {
-      // (without a K tail a stage at or beyond nstages is only ever requested once the walk has no further tile, and
+      // (without a K tail a stage at or beyond nst is only ever requested once the walk has no further tile, and
       // then every offset is out of range already)
       const uint32_t v = (KTAIL && a_col0 >= klim) ? kOobOffset : a_voff[q];
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (lds_void*)(base + q * 4096), 16, v, ka, 0, 0);
@@ -165,7 +183,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
     if constexpr (TEAM == 1) {
       lds_u8* const base = smem + P::B_BASE + bbuf * C::B_STAGE + wn0 * C::B_RB;
       const int kb = sl * C::B_RB;
-      const int klim = sl < nstages ? Kb_b - kb : 0;
+      const int klim = sl < nst() ? Kb_b - kb : 0;
 #pragma unroll
       for (int q = q0; q < q1; ++q) {
         const int col = b_col(q);
@@ -181,7 +199,6 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
   const int swa = swz<C::A_CPR>(r), swb = swz<C::B_CPR>(r);
-  constexpr int SPQ = 4 / C::KSUB;   // stages per K-quad
 
   // ---- output of a finished tile: lane (c, g) of tile (i, j) holds row 16 i + c, columns
   // 32 (j / 2) + 8 g + 4 (j % 2) .. + 3 (see bperm_tile_off); the accumulators are cleared for the next tile ------------------------------------
@@ -275,13 +292,18 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   };
 
   // ---- prologue: stages 0 and 1 of the first tile, scales of its K-quad 0 ---------------------------------
-  int lid = walk.first;          // tile being computed
+  // (without SPLIT the walk is the arithmetic sequence alone)
+  auto next = [&](int t) { return SPLIT ? walk.next(t) : t + walk.step; };
+  int lid = SPLIT ? walk.head() : walk.first;   // tile being computed
+  // the one before tile t: the tail follows the workgroup's tile of the last whole round
+  auto before = [&](int t) { return (SPLIT && t >= walk.end ? walk.end + ((int)blockIdx.x >> 3) : t) - walk.step; };
   set_fetch_tile(lid);
   {
     int fm0, fn0;
     walk.origin(lid, fm0, fn0);
     load_row_ids(fm0);
   }
+  kq = kq_nxt;
   issue_a(0, 0);
   issue_b(0, 0);
   issue_a(1, 1);
@@ -297,7 +319,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   auto stage = [&](auto t0c) {
     constexpr int t0 = decltype(t0c)::value;
     const int s = Q * SPQ + t0 / C::KSUB;
-    if (s >= nstages) return;
+    if (s >= nst()) return;
     // =============================== memory phase ==================================================
     if constexpr (t0 == 0) {
       // Scales of this K-quad, first in the queue of this memory phase: they have the whole phase to arrive, and
@@ -308,11 +330,11 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (t0 == 0) {
-      if (s == 0 && lid != walk.first) {
+      if (s == 0 && lid != walk.first && (!SPLIT || walk.first < walk.end)) {
         // the previous tile's output leaves while the other team is in its MFMA phase
         // (the tile index passes through an opaque move: otherwise the compiler computes the eight row
         // pointers of the stores when the tile begins and keeps them in registers through all its stages)
-        int plid = lid - walk.step;
+        int plid = before(lid);   // (always a whole tile: a split one is the last of the walk)
         asm volatile("" : "+s"(plid));
         int pm0, pn0;
         walk.origin(plid, pm0, pn0);
@@ -323,11 +345,11 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
         }
       }
     }
-    // from stage nstages - 2 on, the loads run ahead into the next tile of the walk
-    if (s + 2 == nstages) set_fetch_tile(lid + walk.step);
-    const bool wrapped = s + 2 >= nstages;
-    const int sl = wrapped ? s + 2 - nstages : s + 2;   // local stage the loads fetch
-    const int sl_eff = (wrapped && (!fetch_valid || nstages < 2)) ? nstages : sl;
+    // from stage nst - 2 on, the loads run ahead into the next tile of the walk
+    if (s + 2 == nst()) set_fetch_tile(next(lid));
+    const bool wrapped = s + 2 >= nst();
+    const int sl = wrapped ? s + 2 - nst() : s + 2;   // local stage the loads fetch
+    const int sl_eff = (wrapped && (!fetch_valid || nst() < 2)) ? nst() : sl;
     lds_u8* const atile = smem + abuf * C::A_STAGE + (wm0 + r) * C::A_RB;
     lds_u8* const btile = smem + P::B_BASE + bbuf * C::B_STAGE + (wn0 + bperm_lane_off(r)) * C::B_RB;
     issue_a(sl_eff, abuf2);
@@ -421,12 +443,13 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
     abuf2 = abuf2 == 2 ? 0 : abuf2 + 1;
     bbuf ^= 1;
   };
-  for (; lid < walk.end; lid += walk.step) {
+  for (; SPLIT ? lid != kNoTile : lid < walk.end; lid = next(lid)) {
     skip_cur = skip_nxt;
+    kq = kq_nxt;
     as_cur[0] = as_nxt[0];
     as_cur[1] = as_nxt[1];
     bs_cur = bs_nxt;
-    for (Q = 0; Q < KQ; ++Q) {
+    for (Q = 0; Q < kq; ++Q) {
       stage(std::integral_constant<int, 0>{});
       if constexpr (C::KSUB == 1) stage(std::integral_constant<int, 1>{});
       stage(std::integral_constant<int, 2>{});
@@ -435,42 +458,114 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // trailing zero-fill DMA has left the queue
   __builtin_amdgcn_sched_barrier(0);
-  {
+  if (!SPLIT || walk.tail == kNoTile) {
     int pm0, pn0;
-    walk.origin(lid - walk.step, pm0, pn0);
+    walk.origin(SPLIT ? walk.first + (walk.end - 1 - walk.first) / walk.step * walk.step : lid - walk.step, pm0, pn0);
     write_tile(pm0, pn0);
+  } else {
+    // partial sums, as the lanes hold them: 1 KiB per store instruction
+    v4f* const t = (v4f*)g.tail + ((int64_t)blockIdx.x * 8 + TEAM * 4 + wn) * 32 * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) t[(i * 4 + j) * 64] = acc[i][j];
   }
   if constexpr (TEAM == 0) asm volatile("s_barrier" ::: "memory");   // pairs with team 1's extra barrier
 }
 
-template <class C, typename OutT, bool GROUPED>
+// rows of C (slots, when grouped) that have tiles
+template <bool GROUPED>
+__device__ __forceinline__ int pp_rows(const GemmArgs& g) {
+  if constexpr (GROUPED) {
+    if (g.num_slots) {
+      const int n = *g.num_slots;
+      return n < 0 ? 0 : n < g.M ? n : g.M;
+    }
+  }
+  return g.M;
+}
+template <class C, bool GROUPED, bool SPLIT>
+__device__ __forceinline__ TileWalk pp_walk(const GemmArgs& g) {
+  const int M = pp_rows<GROUPED>(g);
+  if constexpr (SPLIT) return make_split_walk(M, g.N, g.K / 512, C::KSUB == 2);
+  else return make_tile_walk(M, g.N);
+}
+
+template <class C, typename OutT, bool GROUPED, bool SPLIT>
 __global__ __launch_bounds__(512) void gemm_pp_kernel(const GemmArgs g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_generic[];
   lds_u8* const smem = (lds_u8*)smem_generic;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
-  const TileWalk walk = make_tile_walk(g.M, g.N);
-  if (walk.first >= walk.end) return;   // cannot happen with the grids the launcher picks
   const int ksteps = (g.K + 127) / 128;
+  const TileWalk walk = pp_walk<C, GROUPED, SPLIT>(g);
+  if (walk.head() == kNoTile) return;   // uniform: nothing left for this workgroup
   // (uniform.  The MXFP4 instance keeps the one masked body: a second, unmasked one measured no faster on it.)
-  const bool ktail = C::KSUB != 1 || g.K % 128 != 0 || ksteps < 2;
+  // (a split K is a whole number of K-quads)
+  const bool ktail = C::KSUB != 1 || (!SPLIT && (g.K % 128 != 0 || ksteps < 2));
   if (ktail) {
     if (wave < 4)
-      pp_body<C, OutT, GROUPED, 0, true>(g, smem, wave, lane, walk);
+      pp_body<C, OutT, GROUPED, SPLIT, 0, true>(g, smem, wave, lane, walk);
     else
-      pp_body<C, OutT, GROUPED, 1, true>(g, smem, wave - 4, lane, walk);
+      pp_body<C, OutT, GROUPED, SPLIT, 1, true>(g, smem, wave - 4, lane, walk);
   } else if constexpr (C::KSUB == 1) {
     if (wave < 4)
-      pp_body<C, OutT, GROUPED, 0, false>(g, smem, wave, lane, walk);
+      pp_body<C, OutT, GROUPED, SPLIT, 0, false>(g, smem, wave, lane, walk);
     else
-      pp_body<C, OutT, GROUPED, 1, false>(g, smem, wave - 4, lane, walk);
+      pp_body<C, OutT, GROUPED, SPLIT, 1, false>(g, smem, wave - 4, lane, walk);
   }
 }
 
+// Adds up the partial sums of the tiles that gemm_pp_kernel split along K, in the order of their slices, and writes them.
+// Workgroup: (XCD, one of its split tiles, one wave's 128 x 64 block of it), four waves of two row tiles each.
 template <class C, typename OutT, bool GROUPED>
+__global__ __launch_bounds__(256) void pp_tail_kernel(const GemmArgs g, const int grid) {
+  const int xcd = blockIdx.x & 7, wv = (blockIdx.x >> 3) & 7, at = blockIdx.x >> 6;
+  const int lane = threadIdx.x & 63, r = lane & 15, gq = lane >> 4, w4 = threadIdx.x >> 6;
+  TileWalk walk = {};
+  walk.tiles_m = (pp_rows<GROUPED>(g) + 255) / 256;
+  walk.tiles_n = (g.N + 255) / 256;
+  const XcdShare x = xcd_share(walk.tiles_m * walk.tiles_n, grid, xcd);
+  const int rest = x.count % x.wgs, S = tail_splits(rest, x.wgs, g.K / 512, C::KSUB == 2);
+  if (S == 1 || at >= rest) return;
+  int m0, n0;
+  walk.origin(x.start + x.count - rest + at, m0, n0);
+  const int n = n0 + (wv & 3) * 64 + 8 * gq;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int i = w4 * 2 + u, m = m0 + (wv >> 2) * 128 + 16 * i + r;
+    v4f v[4] = {};
+    for (int s = 0; s < S; ++s) {
+      const int wg = (at * S + s) * 8 + xcd;
+      const v4f* const t = (const v4f*)g.tail + ((int64_t)wg * 8 + wv) * 32 * 64 + i * 4 * 64 + lane;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] += t[j * 64];
+    }
+    int64_t row = m;
+    bool ok = m < g.M;
+    float w = 1.f;
+    if constexpr (GROUPED) {
+      const int id = ok ? g.sorted_token_ids[m] : -1;
+      ok = id >= 0 && id < g.num_valid_ids;
+      row = id;
+      if (ok && g.topk_weights) w = g.topk_weights[id];
+    }
+    if (!ok) continue;
+    OutT* const p = (OutT*)g.C + row * g.ldc + n;
+#pragma unroll
+    for (int jp = 0; jp < 2; ++jp) {
+      v4f v0 = v[2 * jp], v1 = v[2 * jp + 1];
+      if constexpr (GROUPED) { v0 *= w; v1 *= w; }
+      if (g.accumulate) add8_edge<OutT>(p + 32 * jp, v0, v1, g.N - n - 32 * jp);
+      store8_edge<OutT>(p + 32 * jp, v0, v1, g.N - n - 32 * jp);
+    }
+  }
+}
+
+template <class C, typename OutT, bool GROUPED, bool SPLIT>
 int launch_pp(const GemmArgs& g, hipStream_t stream) {
-  auto kern = gemm_pp_kernel<C, OutT, GROUPED>;
+  auto kern = gemm_pp_kernel<C, OutT, GROUPED, SPLIT>;
   static int attr_done = 0;   // benign race: the attribute call is idempotent
   if (!attr_done) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -480,11 +575,17 @@ int launch_pp(const GemmArgs& g, hipStream_t stream) {
                        hipGetErrorString(e));
     attr_done = 1;
   }
-  const int64_t grid = pp_grid(g.M, g.N, g.K, C::KSUB);
+  int64_t grid = pp_grid(g.M, g.N, g.K, C::KSUB);
   if (grid <= 0) return MX_OK;
+  if (SPLIT) grid = num_cus();   // idle workgroups of a single, partly filled round take part too
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), PP<C>::LDS_BYTES, stream, g);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "gemm_pp_kernel launch: %s", hipGetErrorString(e));
+  if constexpr (SPLIT) {
+    hipLaunchKernelGGL((pp_tail_kernel<C, OutT, GROUPED>), dim3(8 * 8 * kTailMax), dim3(256), 0, stream, g, (int)grid);
+    e = hipGetLastError();
+    if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "pp_tail_kernel launch: %s", hipGetErrorString(e));
+  }
   return MX_OK;
 }
 
@@ -496,9 +597,13 @@ template <int AF, int BF>
 int launch_pp_pair(const GemmArgs& g, hipStream_t stream) {
   using C = Cfg<AF, BF, 256, 256, 2, 4>;
   const bool grouped = g.sorted_token_ids != nullptr;
-  if (g.c_dtype == MX_F32)
-    return grouped ? launch_pp<C, float, true>(g, stream) : launch_pp<C, float, false>(g, stream);
-  return grouped ? launch_pp<C, uint16_t, true>(g, stream) : launch_pp<C, uint16_t, false>(g, stream);
+  auto run = [&](auto split) {
+    constexpr bool S = decltype(split)::value;
+    if (g.c_dtype == MX_F32)
+      return grouped ? launch_pp<C, float, true, S>(g, stream) : launch_pp<C, float, false, S>(g, stream);
+    return grouped ? launch_pp<C, uint16_t, true, S>(g, stream) : launch_pp<C, uint16_t, false, S>(g, stream);
+  };
+  return g.tail ? run(std::true_type{}) : run(std::false_type{});
 }
 #if MX_PP_PAIR == 0
 template int launch_pp_pair<MX_E4M3, MX_E4M3>(const GemmArgs&, hipStream_t);

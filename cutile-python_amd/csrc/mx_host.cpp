@@ -29,6 +29,7 @@ struct Lib {
   MX_FN(mx_gemm);
   MX_FN(mx_gemm_add);
   MX_FN(mx_gemm_workspace_bytes);
+  MX_FN(mx_packed_scale_bytes);
   MX_FN(mx_gemm_list);
   MX_FN(mx_gemm_list_workspace_bytes);
   MX_FN(mx_quantize);
@@ -272,7 +273,9 @@ PyObject* py_mma(PyObject*, PyObject* const* a, Py_ssize_t n) {
   at::Tensor out = device_empty(acc.sizes(), at::kFloat, dev);
   mx_tensor dD = desc(acc, MX_F32), dC = desc(out, MX_F32);
   mx_gemm_opts o = {sizeof(mx_gemm_opts), 0, MX_SCALE_2D, MX_SCALE_2D, MX_KERNEL_AUTO, 32, 0, 0};
-  const int64_t need = lib.p_mx_gemm_workspace_bytes(M, N, K, &o) * batch;
+  // one product at a time needs its workspace once, a batch in one launch all re-laid scales at once
+  const int64_t one = lib.p_mx_gemm_workspace_bytes(M, N, K, &o),
+                all = (lib.p_mx_packed_scale_bytes(M, K) + lib.p_mx_packed_scale_bytes(N, K)) * batch, need = one > all ? one : all;
   at::Tensor ws;
   if (need > 0) ws = device_empty({need}, at::kByte, dev);
   int rc;
@@ -408,6 +411,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
   MX_FN(mx_gemm)
   MX_FN(mx_gemm_add)
   MX_FN(mx_gemm_workspace_bytes)
+  MX_FN(mx_packed_scale_bytes)
   MX_FN(mx_gemm_list)
   MX_FN(mx_gemm_list_workspace_bytes)
   MX_FN(mx_quantize)

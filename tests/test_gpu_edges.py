@@ -69,3 +69,29 @@ def test_split_that_never_applied_and_static_scratch_run_whole(ct, dev, K, packe
         assert O.rel_fro(forced.cpu(), whole.cpu()) <= 1e-5   # (fp32 sums, order of the K steps at most)
     c = ct.block_scaled_matmul(a.storage, As, b.storage.T, Bs, static_scratch=True)
     assert O.rel_fro(c.cpu(), whole.cpu()) <= 1e-5
+
+
+@pytest.mark.parametrize("fmt,K", [(O.E4M3, 2560), (O.E5M2, 4608), (O.E2M1, 4096), (O.E4M3, 14336)])
+@pytest.mark.parametrize("M,N", [(300, 260), (1000, 1030), (2800, 6200), (4097, 4096), (1000, 8000), (2500, 3300), (4000, 6400)])
+@pytest.mark.parametrize("out_dtype,accumulate", [(torch.float32, True), (torch.bfloat16, False)], ids=str)
+def test_pingpong_last_round_split_along_k(ct, dev, fmt, K, M, N, out_dtype, accumulate):
+    """Tile counts that leave the last (or only) round partly filled: one to 16 tiles per XCD beyond whole rounds (and
+    XCDs whose share leaves nothing to split beside XCDs that split), split two to eight ways into slices of unequal
+    length, ragged edges, accumulation; nothing written beside C.  The sums differ from the unsplit kernel's by the order
+    of fp32 additions."""
+    def raw(rows, seed):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        q, s = ct.block_quantize(torch.randn((rows, K), generator=g, device=dev), 32, {O.E4M3: torch.float8_e4m3fn,
+                                 O.E5M2: torch.float8_e5m2, O.E2M1: "e2m1"}[fmt], scale_mode="floor")
+        return q, s
+    (a, sa), (b, sb) = raw(M, 1), raw(N, 2)
+    kw = dict(a_format="e2m1", b_format="e2m1") if fmt == O.E2M1 else {}
+    pitch = N + 24
+    bufs = [torch.full((M + 2, pitch), 7.0, dtype=out_dtype, device=dev) for _ in range(2)]
+    for buf, kernel in zip(bufs, ("pingpong", "mfma128")):
+        c = buf[1:M + 1, :N]
+        ct.block_scaled_matmul(a, sa, b.T, sb.T, C=c, accumulate=accumulate, kernel=kernel, split_k=0 if kernel == "pingpong" else 1, **kw)
+    got, ref = bufs[0].float(), bufs[1].float()
+    rel = ((got - ref).norm() / ref[1:M + 1, :N].norm()).item()
+    assert rel <= (1e-5 if out_dtype == torch.float32 else 4e-3), rel   # (guards are equal on both sides)
+    assert (bufs[0][0] == 7).all() and (bufs[0][-1] == 7).all() and (bufs[0][:, N:] == 7).all()

@@ -21,7 +21,9 @@ def _scale(sc, dev):
 
 # T, H, F, E, topk, skew: share of the copies that go to expert 0
 CASES = [(1, 128, 128, 4, 2, 0.0), (17, 256, 128, 8, 1, 0.0), (48, 512, 256, 4, 2, 0.0), (40, 640, 384, 3, 1, 1.0),
-         (33, 1024, 256, 16, 4, 0.7), (64, 128, 640, 8, 2, 0.5), (150, 256, 128, 2, 2, 0.9), (700, 256, 256, 16, 4, 0.3)]
+         (33, 1024, 256, 16, 4, 0.7), (64, 128, 640, 8, 2, 0.5), (150, 256, 128, 2, 2, 0.9), (700, 256, 256, 16, 4, 0.3),
+         # grouped GEMMs on the slots in use, the last round of the second one split along K
+         (300, 128, 6144, 3, 2, 0.4)]
 
 
 @pytest.mark.parametrize("packed", [False, True], ids=["plain", "packed"])
