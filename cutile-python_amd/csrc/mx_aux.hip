@@ -170,7 +170,8 @@ __global__ __launch_bounds__(256) void quantize_kernel(const QuantArgs q) {
 // group and computes the integer route beside the hardware conversions, was short of loads in flight (86 vector
 // registers, two units of 16 bytes per thread) and sent each workgroup's scale bytes out in 16-byte pieces of lines that
 // other XCDs' workgroups shared: 8192 x 8192 bf16 -> E4M3 took 44 - 49 us (4.1 - 4.6 TB/s), this one 36.6 (5.5 TB/s), and
-// 8192 x 14336 of silu(gate) * up 133 us where it took 161.  Here a wave owns U * 64 consecutive
+// 8192 x 14336 of silu(gate) * up 117 us where it took 161
+// (133 with an IEEE division per element: there the vector ALUs are the bound).  Here a wave owns U * 64 consecutive
 // units, so that a workgroup writes whole lines of scale bytes, all loads of a thread are requested before the first is used,
 // and the blocks the hardware conversion does not serve (zero, subnormal, non-finite or extreme amax) are done again
 // by the general code from memory, outside of the loop.
