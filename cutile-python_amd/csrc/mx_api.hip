@@ -204,7 +204,7 @@ int64_t gemm_workspace_min(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& 
 // beyond that, what lets the ping-pong kernel split its last round along K (0: it would not): only for problems that it may
 // be picked for
 int64_t gemm_workspace_tail(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
-  if ((o.kernel != MX_KERNEL_AUTO && o.kernel != MX_KERNEL_MFMA_PINGPONG) || o.split_k > 1 || o.block_size != 32 || M <= 0 || N <= 0 ||
+  if ((o.kernel != MX_KERNEL_AUTO && o.kernel != MX_KERNEL_MFMA_PINGPONG) || o.split_k != 0 || o.block_size != 32 || M <= 0 || N <= 0 ||
       K <= 0)
     return 0;
   const int64_t t = pp_tail_bytes(M, N, K, false, true);
@@ -550,7 +550,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     else {
       const bool fp4 = A->dtype == MX_E2M1;
       const float t128 = est_t128(M, N, K, o.split_k > 1 ? 1 : plan_k_splits(M, N, K, o), fp4);
-      const bool room = workspace && pp_tail_bytes(M, N, K, fp4, true) > 0 &&
+      const bool room = workspace && o.split_k == 0 && pp_tail_bytes(M, N, K, fp4, true) > 0 &&
                         workspace_bytes >= gemm_workspace_min(M, N, K, o) + pp_tail_bytes(M, N, K, fp4, true);
       const float pp = o.split_k > 1 ? 1e30f : est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), room);
       const float st = may_stream ? est_stream(M, N, K, B->dtype) : 1e30f;
@@ -791,7 +791,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
   g.a_fmt = A->dtype; g.b_fmt = B->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate;
   g.a_rows = M;
   g.replicas = 1;
-  if (kernel == MX_KERNEL_MFMA_PINGPONG && workspace && ((uintptr_t)workspace) % 256 == 0) {
+  if (kernel == MX_KERNEL_MFMA_PINGPONG && o.split_k == 0 && workspace && ((uintptr_t)workspace) % 256 == 0) {
     const int64_t tail = pp_tail_bytes(M, N, K, A->dtype == MX_E2M1 && B->dtype == MX_E2M1, true);
     if (tail > 0 && workspace_bytes >= need + tail) g.tail = (float*)((uint8_t*)workspace + need);
   }

@@ -257,10 +257,10 @@ def _workspace(dev: torch.device, nbytes: int, stream: Optional[int] = None) -> 
     overwrite each other's scales between the re-layout launch and the GEMM launch.  While the stream is
     being captured into a graph the buffer comes fresh from the allocator (the capture's private pool) and
     is not cached: a cached one would later be reused by eager calls while replays of the graph still
-    write to it."""
+    write to it.  Neither is one of more than 16 MiB (partial sums): it goes back to the allocator with the call."""
     if nbytes <= 0:
         return None
-    if torch.cuda.is_current_stream_capturing():
+    if nbytes > 16 << 20 or torch.cuda.is_current_stream_capturing():
         return torch.empty(nbytes, dtype=torch.uint8, device=dev)
     cache = _WS_LOCAL.__dict__.setdefault("buffers", {})
     key = (dev.index, L.stream_ptr(dev) if stream is None else stream)

@@ -91,6 +91,9 @@ def test_pingpong_last_round_split_along_k(ct, dev, fmt, K, M, N, out_dtype, acc
     for buf, kernel in zip(bufs, ("pingpong", "mfma128")):
         c = buf[1:M + 1, :N]
         ct.block_scaled_matmul(a, sa, b.T, sb.T, C=c, accumulate=accumulate, kernel=kernel, split_k=0 if kernel == "pingpong" else 1, **kw)
+    if not accumulate:   # split_k = 1 forbids this split too
+        whole = ct.block_scaled_matmul(a, sa, b.T, sb.T, out_dtype=out_dtype, kernel="pingpong", split_k=1, **kw)
+        assert torch.equal(whole, bufs[1][1:M + 1, :N])
     got, ref = bufs[0].float(), bufs[1].float()
     rel = ((got - ref).norm() / ref[1:M + 1, :N].norm()).item()
     assert rel <= (1e-5 if out_dtype == torch.float32 else 4e-3), rel   # (guards are equal on both sides)
