@@ -4,7 +4,7 @@
 namespace mx {
 namespace {
 
-// Workgroup of 8 waves: kw K ranges x 8 / kw units of NT tiles.  m_tiles row tiles of 16 MT rows are neighbours in
+// Workgroup of C::WAVES waves: kw K ranges x WAVES / kw units of NT tiles.  m_tiles row tiles of 16 MT rows are neighbours in
 // dispatch order on the same XCD (workgroup ids go round-robin over 8 XCDs), so W is read from memory once.
 template <class C>
 __global__ __launch_bounds__(C::WAVES * 64) void stream_kernel(const StreamArgs a) {
@@ -95,6 +95,10 @@ __global__ __launch_bounds__(C::WAVES * 64) void stream_kernel(const StreamArgs 
   }
 }
 
+// Waves of a workgroup: with 64 rows of X a stage of FP4 weights is 16 KiB of X, of which two for each of 8 waves do not fit
+// into LDS.
+constexpr int stream_waves(int mt, int w_fmt) { return mt == 4 && w_fmt == MX_E2M1 ? 4 : 8; }
+
 template <class C>
 int launch(const StreamArgs& a, int blocks, hipStream_t stream) {
   auto kern = stream_kernel<C>;
@@ -113,14 +117,14 @@ int launch(const StreamArgs& a, int blocks, hipStream_t stream) {
 
 template <int XF, int WF, int NT, int MT>
 int launch_p(const StreamArgs& a, int blocks, hipStream_t stream) {
-  return a.ws_packed ? launch<StreamCfg<XF, WF, NT, MT, true>>(a, blocks, stream)
-                     : launch<StreamCfg<XF, WF, NT, MT, false>>(a, blocks, stream);
+  constexpr int W = stream_waves(MT, WF);
+  return a.ws_packed ? launch<StreamCfg<XF, WF, NT, MT, true, W>>(a, blocks, stream)
+                     : launch<StreamCfg<XF, WF, NT, MT, false, W>>(a, blocks, stream);
 }
 template <int XF, int WF, int NT>
 int launch_m(const StreamArgs& a, int mt, int blocks, hipStream_t stream) {
   return mt == 1 ? launch_p<XF, WF, NT, 1>(a, blocks, stream)
-         : mt == 2 || WF == MX_E2M1 ? launch_p<XF, WF, NT, 2>(a, blocks, stream)
-                                    : launch_p<XF, WF, NT, WF == MX_E2M1 ? 2 : 4>(a, blocks, stream);
+         : mt == 2 ? launch_p<XF, WF, NT, 2>(a, blocks, stream) : launch_p<XF, WF, NT, 4>(a, blocks, stream);
 }
 
 }  // namespace
@@ -130,7 +134,7 @@ bool stream_supports(int x_fmt, int w_fmt) {
          (x_fmt == MX_E5M2 && (w_fmt == MX_E5M2 || w_fmt == MX_E2M1));
 }
 
-// How the 8 waves of a workgroup split the problem: kw K ranges x 8 / kw units of nt tiles; M in tiles of 16 mt rows.  The
+// How the waves of a workgroup split the problem: kw K ranges x waves / kw units of nt tiles; M in tiles of 16 mt rows.  The
 // cost that is minimised is a wave's K-quads times what a K-step of it moves (nt tiles of W, the rows of X), plus a
 // start-up per workgroup, for every round of workgroups over the 256 CUs: X is fetched once per unit, so wide units
 // save traffic, but a second, partly filled round costs more (28672 x 8192 FP4 at 4 rows: 224 workgroups 28 us, 448
@@ -138,17 +142,21 @@ bool stream_supports(int x_fmt, int w_fmt) {
 // (tiles of a 64-row group interleave its rows, so groups are covered whole)
 StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int w_fmt) {
   StreamPlan p = {};
-  p.mt = M <= 16 ? 1 : M <= 32 || w_fmt == MX_E2M1 ? 2 : 4;
+  // FP4 weights for 33 .. 64 rows: one row tile of 64 (four waves) once the weights have 8192 rows to share out, which
+  // reads them once (28672 x 8192: 64 rows 52.6 -> 44.8 us, 48 rows 47.9 -> 41.7; 14336 x 4096, 40 rows 16.1 -> 15.0);
+  // with fewer, two tiles of 32 have the waves that it lacks (4096 x 14336, 64 rows: 17.8 against 21.5)
+  p.mt = M <= 16 ? 1 : M <= 32 ? 2 : w_fmt != MX_E2M1 ? 4 : M <= 64 && N >= 8192 ? 4 : 2;
+  const int waves = stream_waves(p.mt, w_fmt);   // (half as many waves have twice the bandwidth each)
   p.m_tiles = (int)((M + 16 * p.mt - 1) / (16 * p.mt));
   const int tiles = (int)((N + 63) / 64 * 4), KQ = (int)((K + 511) / 512);
   const float wb = w_fmt == MX_E2M1 ? 1.f : 2.f, xb = (M < 16 * p.mt ? M : 16 * p.mt) / 16.f;
   p.cost = 1e30f;
   for (int n = 4; n >= 1; n >>= 1)
-    for (int kw = 8; kw >= 1; kw >>= 1) {
+    for (int kw = waves; kw >= 1; kw >>= 1) {
       if (kw > 1 && kw > KQ) continue;
-      const int units = (tiles + n * (8 / kw) - 1) / (n * (8 / kw));
+      const int units = (tiles + n * (waves / kw) - 1) / (n * (waves / kw));
       const int64_t rounds = ((int64_t)units * p.m_tiles + 255) / 256;
-      const float t = rounds * ((KQ + kw - 1) / kw * (n * wb + xb) + 3.f);
+      const float t = rounds * ((KQ + kw - 1) / kw * (n * wb + xb) * waves / 8.f + 3.f);
       if (t < p.cost) { p.cost = t; p.nt = n; p.kw = kw; p.units = units; }
     }
   return p;

@@ -20,7 +20,7 @@ def _scales(ct, b, packed):
 @pytest.mark.parametrize("fa,fb", PAIRS, ids=str)
 @pytest.mark.parametrize("M,N,K", [(1, 16, 128), (16, 63, 384), (17, 64, 512), (32, 65, 640), (33, 130, 1024),
                                    (64, 1000, 2176), (65, 259, 1536), (130, 72, 4096), (5, 4096, 2048),
-                                   (3, 16448, 512)])
+                                   (3, 16448, 512), (33, 8192, 640), (64, 8200, 1024)])
 def test_stream_kernel(ct, dev, packed, fa, fb, M, N, K):
     a = randn_operand(M, K, fa, 7000 + M, dev)
     b = raw_operand(N, K, fb, 7100 + N, dev)
