@@ -9,6 +9,7 @@
 //   iteration s:  wait until stage s + 1 has landed; barrier (everybody's part has landed, everybody has read stage s)
 //                 issue the DMA of stage s + NS into the buffer of stage s
 //                 16 (32) MFMAs of stage s, the fragment reads of stage s + 1 between them
+// (order of the requests and what the waits count: mx_t128_schedule.h).
 // NS = 4 (128 KiB, one workgroup per CU) for grids that leave CUs with one tile, NS = 2 (64 KiB) where two workgroups share
 // a CU.  The fragment reads (64 KiB per stage at 128 bytes per clock) are as long as the MFMAs of a stage, so a CU can get
 // to about half of the MFMA rate; larger products go to the 256 x 256 kernel.
@@ -21,6 +22,7 @@
 #include "mx_gemm_pp.h"
 #include "mx_gemm_t128.h"
 #include "mx_gemm_tile.h"
+#include "mx_t128_schedule.h"
 
 namespace mx {
 namespace {
@@ -110,7 +112,9 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
   // ---- scales: 64 rows (group) x 16 bytes per wave and K-quad, by LDS-DMA SD quads ahead: waves 0, 1 fetch A's two groups,
   // 2, 3 B's.  (Each wave loading what it needs into registers is eight times as many load instructions for plain
   // scales; 1024 x 4096 x 4096 27.2 us that way.)
-  constexpr int SD = (NS + SPQ - 1) / SPQ, SSLOT = 4096;   // an earlier stage's wait then covers them
+  using Sched = T128Schedule<NS, SPQ, TL>;
+  static_assert(t128_covered<Sched>(), "a wait does not cover what is read behind it");
+  constexpr int SD = Sched::SD, SSLOT = 4096;
   lds_u8* const sbase = smem + NS * C::STAGE;
   uint32_t sco;                       // lane offset of this wave's group
   {
@@ -190,11 +194,12 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
 
   // ---- prologue ---------------------------------------------------------------------------------------------------------
 #pragma unroll
-  for (int k = 0; k < SD; ++k) load_scales(q0 + k);
-#pragma unroll
-  for (int k = 0; k < NS; ++k) issue(s0 + k, k);
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 1) * TL));
+  for (int k = 0; k < NS; ++k) {
+    if (Sched::prologue_scales(k)) load_scales(q0 + k / SPQ);
+    issue(s0 + k, k);
+    __builtin_amdgcn_sched_barrier(0);   // the waits count on this order
+  }
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(Sched::prologue_wait()));
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
@@ -215,14 +220,14 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
     const int s = Q * SPQ + t;
     if (s >= s1) return;              // uniform
     // stage s + 1 (requested NS - 1 iterations ago) has landed; younger are NS - 2 stages and the scales requested since
-    constexpr int back = NS - 2;      // iterations between
-    constexpr bool sc = back >= 1 && (SPQ == 2 || t == 1 || t == 2);
-    static_assert(NS == 2 || NS == 4, "the count above");
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(back * TL + (sc ? 1 : 0)));
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(Sched::stage_wait(t)));
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (t == 0) load_scales(Q + SD);
+    if constexpr (t == 0) {
+      load_scales(Q + SD);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     issue(s + NS, buf);
     __builtin_amdgcn_sched_barrier(0);
     const int nbuf = buf + 1 == NS ? 0 : buf + 1;

@@ -1,0 +1,63 @@
+// Order of the memory requests of the 128 x 128 kernel (mx_gemm_t128.hip) and the counted waits that follow from it.
+// Plain C++ without device code, so that the rules can be checked on the host.
+//
+// A wave requests stages of TL loads each, NS stages ahead, and one load of scales per K-quad (SPQ stages).  Its loads
+// complete in the order of the requests, so "at most n outstanding" means that all but the n youngest are in LDS.
+//   prologue: stages 0 .. NS - 1, the scales of a quad in front of its first stage; wait; stage 0 and the scales of quad 0
+//             are read
+//   stage s:  wait; barrier; at the first stage of quad Q the scales of quad Q + SD are requested, then stage s + NS; stage
+//             s + 1 is read, at the last stage of quad Q also the scales of quad Q + 1
+// The prologue's order is the one that the stages continue.  (All scales ahead of the stages, it would leave one load
+// fewer behind stage 1 than the stages' count assumes.)
+#pragma once
+
+namespace mx {
+
+template <int NS_, int SPQ_, int TL_>
+struct T128Schedule {
+  static constexpr int NS = NS_, SPQ = SPQ_, TL = TL_;
+  static constexpr int SD = (NS + SPQ - 1) / SPQ;          // quads of scales in flight
+  // scales that the prologue requests in front of stage k: those of quad k / SPQ
+  static constexpr bool prologue_scales(int k) { return k % SPQ == 0; }
+  // behind stage 0: the other stages and the scales requested between them
+  static constexpr int prologue_wait() { return (NS - 1) * TL + SD - 1; }
+  // behind stage s + 1, t = s % SPQ: NS - 2 stages, and the scales that the stages of those requests asked for
+  static constexpr int stage_wait(int t) {
+    int n = (NS - 2) * TL;
+    for (int back = 1; back <= NS - 2; ++back) n += (t + SPQ * NS - back) % SPQ == 0;
+    return n;
+  }
+};
+
+// First stage of a product of `stages` stages at which something is read that the waits do not cover, -1 if none.  -2: the
+// first reads, behind the prologue.  `scales_first`: a prologue that requests all its scales ahead of the stages.
+template <class S>
+constexpr int t128_uncovered(int stages, bool scales_first = false, int prologue_wait = S::prologue_wait()) {
+  constexpr int kMax = 64;
+  int stage_end[kMax] = {}, scales_end[kMax] = {}, issued = 0;   // loads requested up to and with the item's last one
+  if (stages + S::NS > kMax) return -3;
+  if (scales_first)
+    for (int q = 0; q < S::SD; ++q) scales_end[q] = ++issued;
+  for (int k = 0; k < S::NS; ++k) {
+    if (!scales_first && S::prologue_scales(k)) scales_end[k / S::SPQ] = ++issued;
+    stage_end[k] = issued += S::TL;
+  }
+  if (stage_end[0] > issued - prologue_wait || scales_end[0] > issued - prologue_wait) return -2;
+  for (int s = 0; s < stages; ++s) {
+    const int t = s % S::SPQ, quad = s / S::SPQ, landed = issued - S::stage_wait(t);
+    if (stage_end[s + 1] == 0 || stage_end[s + 1] > landed) return s;
+    if (t == S::SPQ - 1 && (scales_end[quad + 1] == 0 || scales_end[quad + 1] > landed)) return s;
+    if (t == 0) scales_end[quad + S::SD] = ++issued;
+    stage_end[s + S::NS] = issued += S::TL;
+  }
+  return -1;
+}
+
+template <class S>
+constexpr bool t128_covered() {
+  for (int stages = 1; stages <= 24; ++stages)
+    if (t128_uncovered<S>(stages) != -1) return false;
+  return true;
+}
+
+}  // namespace mx
