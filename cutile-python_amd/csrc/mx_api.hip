@@ -514,20 +514,26 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
 
   // what keeps the weight-streaming kernel from taking the problem (it also takes E5M2 x E2M1, which the tiled
   // kernels do not)
+  StreamArgs sa = {};
   const char* why_stream = nullptr;
   if (batched) why_stream = "batched operands";
   else if (o.block_size != 32 || As->dtype != MX_E8M0) why_stream = "it reads E8M0 scales with block 32";
-  else if (!stream_supports(A->dtype, B->dtype)) why_stream = "it takes 8-bit A with FP4 B or B of A's format";
-  else if (K < 128 || K % 128 != 0) why_stream = "K is not a multiple of 128";
-  else if ((why_stream = mfma_operand_issue(A->ptr, M, a_ld, A->stride[1], A->dtype, 1))) {}
-  else if ((why_stream = mfma_operand_issue(B->ptr, N, b_ld, B->stride[0], B->dtype, B->packed_dim == 0))) {}
+  else if (M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 30)) why_stream = "extent too large";
+  else if (A->stride[1] != 1 || B->stride[0] != 1) why_stream = "K axis is not contiguous";
+  else if (B->dtype == MX_E2M1 && B->packed_dim != 0) why_stream = "FP4 operand is not packed along K";
   else if (C->stride[1] != 1) why_stream = "C is not row-major";
-  else if (o.a_scale_layout != MX_SCALE_2D || As->stride[1] != 1 || As->stride[0] % 4 != 0 ||
-           ((uintptr_t)As->ptr) % 4 != 0)
-    why_stream = "A_scale must be the plain 2-D layout with 4-byte aligned rows";
-  else if (o.b_scale_layout != MX_SCALE_NATIVE &&
-           (o.b_scale_layout != MX_SCALE_2D || Bs->stride[0] != 1 || Bs->stride[1] % 4 != 0 || ((uintptr_t)Bs->ptr) % 4 != 0))
-    why_stream = "B_scale must be MX_SCALE_NATIVE or K-contiguous with 4-byte aligned rows";
+  else if (o.a_scale_layout != MX_SCALE_2D || As->stride[1] != 1) why_stream = "A_scale must be the plain K-contiguous layout";
+  else if (o.b_scale_layout != MX_SCALE_NATIVE && (o.b_scale_layout != MX_SCALE_2D || Bs->stride[0] != 1))
+    why_stream = "B_scale must be MX_SCALE_NATIVE or plain and K-contiguous";
+  else {
+    sa.X = (const uint8_t*)A->ptr; sa.Xs = (const uint8_t*)As->ptr;
+    sa.W = (const uint8_t*)B->ptr; sa.Ws = (const uint8_t*)Bs->ptr; sa.C = C->ptr;
+    sa.M = (int32_t)M; sa.N = (int32_t)N; sa.K = (int32_t)K;
+    sa.ldx = a_ld; sa.ldxs = As->stride[0]; sa.ldw = b_ld; sa.ldws = Bs->stride[1]; sa.ldc = C->stride[0];
+    sa.x_fmt = A->dtype; sa.w_fmt = B->dtype; sa.c_dtype = C->dtype; sa.accumulate = o.accumulate;
+    sa.ws_packed = o.b_scale_layout == MX_SCALE_NATIVE;
+    why_stream = stream_issue(sa);
+  }
 
   int kernel = o.kernel;
   if (kernel == MX_KERNEL_DECODE && K > kDecodeMaxK && M <= kDecodeMaxM && N % 16 == 0 && K % 512 == 0 && !why_stream &&
@@ -541,7 +547,8 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
         !(M <= 32 && decode_beats_stream(M, N, K) && B->dtype == MX_E2M1 && o.b_scale_layout == MX_SCALE_2D))
       kernel = MX_KERNEL_STREAM;
     else if (why) kernel = MX_KERNEL_GENERIC;
-    else if (M <= 32 && o.split_k <= 1 && A->dtype != MX_E2M1 && B->dtype == MX_E2M1 &&
+    // (a longer K streams; here that is a problem of a list, which then gets a call of its own)
+    else if (M <= 32 && (K <= kDecodeMaxK || !why_stream) && o.split_k <= 1 && A->dtype != MX_E2M1 && B->dtype == MX_E2M1 &&
              o.a_scale_layout == MX_SCALE_2D &&
              o.b_scale_layout == MX_SCALE_2D && Bs->stride[0] == 1 && As->stride[1] == 1 && K % 512 == 0 &&
              N % 16 == 0 && Bs->stride[1] % 16 == 0 && ((uintptr_t)Bs->ptr) % 16 == 0 &&
@@ -613,14 +620,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     if (B->dtype != MX_E2M1 && need > 0 && (!workspace || workspace_bytes < need))
       return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                        (long long)workspace_bytes);
-    StreamArgs d = {};
-    d.X = (const uint8_t*)A->ptr; d.Xs = (const uint8_t*)As->ptr;
-    d.W = (const uint8_t*)B->ptr; d.Ws = (const uint8_t*)Bs->ptr; d.C = C->ptr;
-    d.M = (int32_t)M; d.N = (int32_t)N; d.K = (int32_t)K;
-    d.ldx = a_ld; d.ldxs = As->stride[0]; d.ldw = b_ld; d.ldws = Bs->stride[1]; d.ldc = C->stride[0];
-    d.x_fmt = A->dtype; d.w_fmt = B->dtype; d.c_dtype = C->dtype; d.accumulate = o.accumulate;
-    d.ws_packed = o.b_scale_layout == MX_SCALE_NATIVE;
-    return launch_gemm_stream(d, (hipStream_t)stream);
+    return launch_gemm_stream(sa, (hipStream_t)stream);
   }
 
   if (kernel == MX_KERNEL_DECODE) {

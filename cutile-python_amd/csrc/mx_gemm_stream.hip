@@ -162,21 +162,26 @@ StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int w_fmt) {
   return p;
 }
 
+// Rows may overlap (a row pitch of zero is a broadcast row): the descriptors end behind the last row's last byte.
+const char* stream_issue(const StreamArgs& a) {
+  if (!stream_supports(a.x_fmt, a.w_fmt)) return "it takes 8-bit A with FP4 B or B of A's format";
+  if (a.K < 128 || a.K % 128 != 0) return "K is not a multiple of 128";
+  if ((((uintptr_t)a.X | (uintptr_t)a.W | (uintptr_t)a.ldx | (uintptr_t)a.ldw) % 16) != 0)
+    return "A and B must have 16-byte aligned rows";
+  if ((((uintptr_t)a.Xs | (uintptr_t)a.ldxs) % 4) != 0) return "A_scale must have 4-byte aligned rows";
+  if (a.ws_packed ? ((uintptr_t)a.Ws % 16) != 0 : (((uintptr_t)a.Ws | (uintptr_t)a.ldws) % 4) != 0)
+    return "B_scale must be 16-byte aligned (packed) or have 4-byte aligned rows";
+  const int64_t lim = (int64_t)1 << 31;   // lane offsets are 32-bit, and this one marks what does not exist
+  if ((int64_t)a.M * a.ldx >= lim || (int64_t)a.N * a.ldw >= lim) return "A or B spans 2 GiB or more";
+  if ((int64_t)a.M * a.ldxs >= lim || (a.ws_packed ? packed_scale_dwords(a.N, a.K) * 4 : (int64_t)a.N * a.ldws) >= lim)
+    return "A_scale or B_scale spans 2 GiB or more";
+  return nullptr;
+}
+
 int launch_gemm_stream(const StreamArgs& a0, hipStream_t stream) {
   StreamArgs a = a0;
-  if (!stream_supports(a.x_fmt, a.w_fmt))
-    return set_error(MX_ERR_DTYPE, "stream kernel: unsupported element format pair (%d, %d)", a.x_fmt, a.w_fmt);
-  if (a.M < 1 || a.N < 1 || a.K < 128 || a.K % 128 != 0)
-    return set_error(MX_ERR_SHAPE, "stream kernel: K must be a positive multiple of 128");
-  const int64_t wrow = a.w_fmt == MX_E2M1 ? a.K / 2 : a.K;
-  if ((((uintptr_t)a.X | (uintptr_t)a.W | (uintptr_t)a.ldx | (uintptr_t)a.ldw) % 16) != 0 ||
-      (((uintptr_t)a.Xs | (uintptr_t)a.ldxs) % 4) != 0 ||
-      (a.ws_packed ? ((uintptr_t)a.Ws % 16) : (((uintptr_t)a.Ws | (uintptr_t)a.ldws) % 4)) != 0)
-    return set_error(MX_ERR_LAYOUT, "stream kernel: operands must be 16-byte and scale rows 4-byte aligned");
-  const int64_t lim = (int64_t)1 << 31;
-  if ((int64_t)a.M * a.ldx >= lim || (int64_t)a.N * a.ldw >= lim || (int64_t)a.M * a.ldxs >= lim ||
-      (a.ws_packed ? packed_scale_dwords(a.N, a.K) * 4 : (int64_t)a.N * a.ldws) >= lim || wrow > a.ldw)
-    return set_error(MX_ERR_LAYOUT, "stream kernel: an operand spans 2 GiB or more");
+  if (a.M < 1 || a.N < 1) return set_error(MX_ERR_SHAPE, "stream kernel: no rows");
+  if (const char* why = stream_issue(a)) return set_error(MX_ERR_LAYOUT, "stream kernel: %s", why);
   const StreamPlan p = stream_plan(a.M, a.N, a.K, a.w_fmt);
   const int mt = p.mt, nt = p.nt;
   a.m_tiles = p.m_tiles; a.kw = p.kw; a.units = p.units;

@@ -15,6 +15,9 @@ struct StreamArgs {
   int32_t kw, m_tiles, units;
 };
 bool stream_supports(int x_fmt, int w_fmt);
+// what keeps the kernel from taking a problem whose A, A_scale and unpacked B, B_scale are K-contiguous (nullptr: nothing);
+// the launch refuses exactly these, so a dispatch that asks first never picks the kernel in vain
+const char* stream_issue(const StreamArgs& a);
 struct StreamPlan { int mt, m_tiles, nt, kw, units; float cost; };
 StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int w_fmt);
 int launch_gemm_stream(const StreamArgs& a, hipStream_t stream);

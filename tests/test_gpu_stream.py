@@ -47,3 +47,47 @@ def test_stream_kernel_ignores_scales_beyond_k(ct, dev):
     s = pad.view(torch.float8_e8m0fnu)
     c = ct.block_scaled_matmul(a.storage, s[N:, :K // 32], b.storage.T, s[:N, :K // 32].T, b_format="e2m1", kernel="stream")
     assert O.rel_fro(c.cpu(), ref) <= 1e-3
+
+
+def _spread(rows, pitch, dev):
+    """`rows` at `pitch` bytes from one another, in a buffer of their own."""
+    n, k = rows.shape
+    buf = torch.empty((n - 1) * pitch + k, dtype=torch.uint8, device=dev)
+    out = buf.as_strided((n, k), (pitch, 1))
+    out.copy_(rows.view(torch.uint8))
+    return out.view(rows.dtype)
+
+
+@pytest.mark.parametrize("M", [8, 64, 65])
+@pytest.mark.parametrize("fb,pitch", [(O.E4M3, 0), (O.E4M3, 16), (O.E2M1, 0), (O.E2M1, 16)])
+def test_rows_of_the_weights_may_overlap(ct, dev, M, fb, pitch):
+    """B as one broadcast row, or as windows that slide over one buffer, and its scales broadcast."""
+    N, K = 200, 1152
+    row = K // 2 if fb == O.E2M1 else K
+    flat = raw_operand(1, K + 32 * N, fb, 11, dev)   # (a source of valid element bytes)
+    a, s = randn_operand(M, K, O.E4M3, 12, dev), raw_operand(1, K, fb, 13, dev).scale_t
+    w = flat.storage.view(-1).as_strided((N, row), (pitch, 1))
+    codes = torch.from_numpy(flat.storage_np).view(-1).as_strided((N, row), (pitch, 1)).contiguous().numpy()
+    if fb == O.E2M1:
+        codes = O.unpack_fp4(codes)
+    scales = s.view(torch.uint8).cpu().expand(N, K // 32).contiguous().numpy()
+    ref = O.reference_matmul(a.codes, a.scales, codes.T.copy(), scales.T.copy(), O.E4M3, fb, 32)
+    for bs in (s.expand(N, K // 32).T, s.expand(N, K // 32).contiguous().T):
+        c = ct.block_scaled_matmul(a.storage, a.scale_t, w.T, bs, b_format="e2m1" if fb == O.E2M1 else None,
+                                   out_dtype=torch.float32)
+        assert O.rel_fro(c.cpu(), ref) <= 1e-3
+
+
+@pytest.mark.parametrize("M,K,fb,side", [(8, 640, O.E4M3, "b"), (33, 640, O.E2M1, "b"), (64, 1024, O.E4M3, "a"),
+                                         (8, 8704, O.E2M1, "a")])
+def test_scale_rows_that_span_2_gib(ct, dev, M, K, fb, side):
+    """Beyond the streaming kernel's 32-bit offsets: another kernel takes the problem."""
+    N = 256
+    a, b = randn_operand(M, K, O.E4M3, 21, dev), randn_operand(N, K, fb, 22, dev)
+    sa, sb = a.scale_t, b.scale_t
+    if side == "a":
+        sa = _spread(sa, (1 << 31) // M // 16 * 16 + 16, dev)
+    else:
+        sb = _spread(sb, (1 << 31) // N // 16 * 16 + 16, dev)
+    c = ct.block_scaled_matmul(a.storage, sa, b.storage.T, sb.T, b_format=b.fmt_kw, out_dtype=torch.float32)
+    assert O.rel_fro(c.cpu(), oracle_matmul(a, b)) <= 1e-3
