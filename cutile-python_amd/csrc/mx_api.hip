@@ -191,7 +191,7 @@ int64_t mx_packed_scale_bytes(int64_t rows, int64_t K) {
 }
 
 namespace {
-// what a product cannot do without: re-laid scales, partial sums of split-K
+// re-laid scales, partial sums of split-K
 int64_t gemm_workspace_min(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
   if (o.kernel == MX_KERNEL_GENERIC || o.kernel == MX_KERNEL_STREAM || o.kernel == MX_KERNEL_DECODE) return 0;
   int64_t b = 0;
@@ -200,6 +200,26 @@ int64_t gemm_workspace_min(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& 
   if (!is_native(o.a_scale_layout)) b += mx_packed_scale_bytes(M, K);
   if (!is_native(o.b_scale_layout)) b += mx_packed_scale_bytes(N, K);
   return b;
+}
+// Partial sums that a caller is held to: of a split into equal slices of 512 with plain scales, as mx_gemm_opts::split_k has it
+// (an automatic one: the most such slices within it).  Every other split is the library's own choice; where its partial
+// sums have no room the product runs whole.
+int64_t held_partial_sums(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
+  if (K % 512 != 0 || o.a_scale_layout != MX_SCALE_2D || o.b_scale_layout != MX_SCALE_2D) return 0;
+  int S = plan_k_splits(M, N, K, o);
+  while (S > 1 && K % ((int64_t)512 * S) != 0) --S;
+  return S > 1 ? round256((int64_t)S * M * N * 4) : 0;
+}
+// what mx_gemm cannot do without, and the options that a product runs under with `bytes` of workspace
+int64_t gemm_workspace_held(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
+  mx_gemm_opts whole = o;
+  whole.split_k = 1;
+  return gemm_workspace_min(M, N, K, whole) + held_partial_sums(M, N, K, o);
+}
+mx_gemm_opts opts_for_room(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o, int64_t bytes) {
+  mx_gemm_opts r = o;
+  if (bytes < gemm_workspace_min(M, N, K, o) && bytes >= gemm_workspace_held(M, N, K, o)) r.split_k = 1;
+  return r;
 }
 // beyond that, what lets the ping-pong kernel split its last round along K (0: it would not): only for problems that it may
 // be picked for
@@ -353,7 +373,7 @@ namespace {
 int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const mx_tensor* Bs, mx_tensor* C,
               const mx_gemm_opts* opts, void* workspace, int64_t workspace_bytes, void* stream, GemmPlan* plan,
               const float* acc) {
-  const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
+  mx_gemm_opts o = opts ? *opts : kDefaultOpts;
   if (int rc = check_tensor(A, "A", 2, 3)) return rc;
   if (int rc = check_tensor(B, "B", 2, 3)) return rc;
   if (int rc = check_tensor(As, "A_scale", 2, 4)) return rc;
@@ -500,6 +520,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     return MX_OK;
   }
 
+  if (!batched) o = opts_for_room(M, N, K, o, workspace ? workspace_bytes : 0);
   // ---- can the MFMA path take it? ------------------------------------------------------------------
   const char* why = nullptr;
   const int64_t a_ld = A->stride[and_ - 2], b_ld = B->stride[bnd - 1];
@@ -818,20 +839,12 @@ int mx_gemm_static(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, 
     return set_error(MX_ERR_SHAPE, "mx_gemm_static: A and B must have 2 or 3 dimensions");
   int64_t M, N, K;
   problem_dims(*A, *B, M, N, K);
-  mx_gemm_opts o = opts ? *opts : kDefaultOpts;
+  mx_gemm_opts o = opts_for_room(M, N, K, opts ? *opts : kDefaultOpts, MX_STATIC_SCRATCH_BYTES);
   int64_t need = gemm_workspace_min(M, N, K, o);
-  if (need > MX_STATIC_SCRATCH_BYTES && o.split_k == 0) {
-    // the partial sums of an automatic split are what does not fit: run it whole.  (Plain scales with a K that splits into
-    // equal slices of 512 have always been held to the buffer, and stay refused.)
-    const int S = plan_k_splits(M, N, K, o);
-    bool even = false;
-    if (K % 512 == 0 && o.a_scale_layout == MX_SCALE_2D && o.b_scale_layout == MX_SCALE_2D)
-      for (int s = S; s > 1 && !even; --s) even = K % (512 * s) == 0 && s * M * N * 4 > MX_STATIC_SCRATCH_BYTES;
-    if (S > 1 && !even) {
-      o.split_k = 1;
-      opts = &o;
-      need = gemm_workspace_min(M, N, K, o);
-    }
+  // (here an automatic split gives way to the scales beside it as well)
+  if (need > MX_STATIC_SCRATCH_BYTES && o.split_k == 0 && held_partial_sums(M, N, K, o) <= MX_STATIC_SCRATCH_BYTES) {
+    o.split_k = 1;
+    need = gemm_workspace_min(M, N, K, o);
   }
   if (need > MX_STATIC_SCRATCH_BYTES)
     return set_error(MX_ERR_WORKSPACE, "mx_gemm_static: this problem needs %lld bytes of scratch, the static buffer "
@@ -839,7 +852,7 @@ int mx_gemm_static(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, 
                      (long long)MX_STATIC_SCRATCH_BYTES);
   void* ws = nullptr;
   if (int rc = static_scratch(&ws)) return rc;
-  return mx_gemm(A, As, B, Bs, C, opts, ws, MX_STATIC_SCRATCH_BYTES, stream);
+  return mx_gemm(A, As, B, Bs, C, &o, ws, MX_STATIC_SCRATCH_BYTES, stream);
 }
 
 int64_t mx_gemm_list_workspace_bytes(int32_t count, const mx_tensor* A, const mx_tensor* B,
@@ -859,7 +872,18 @@ int mx_gemm_list(int32_t count, const mx_tensor* A, const mx_tensor* As, const m
   if (count < 0) return set_error(MX_ERR_INVALID, "mx_gemm_list: negative count");
   if (count == 0) return MX_OK;
   if (!A || !As || !B || !Bs || !C) return set_error(MX_ERR_INVALID, "mx_gemm_list: null descriptor array");
-  const int64_t need = mx_gemm_list_workspace_bytes(count, A, B, opts);
+  int64_t need = mx_gemm_list_workspace_bytes(count, A, B, opts);
+  const bool tight = (workspace ? workspace_bytes : 0) < need;   // then only what every problem is held to
+  auto slice_bytes = [&](int32_t i) {
+    int64_t M, N, K;
+    problem_dims(A[i], B[i], M, N, K);
+    const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
+    return round256(tight ? gemm_workspace_held(M, N, K, o) : gemm_workspace_min(M, N, K, o));
+  };
+  if (tight) {
+    need = 0;
+    for (int32_t i = 0; i < count; ++i) need += slice_bytes(i);
+  }
   if (need > 0 && (!workspace || workspace_bytes < need))
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                      (long long)workspace_bytes);
@@ -875,7 +899,7 @@ int mx_gemm_list(int32_t count, const mx_tensor* A, const mx_tensor* As, const m
   for (int32_t i = 0; i < count; ++i) {
     int64_t M, N, K;
     problem_dims(A[i], B[i], M, N, K);
-    const int64_t b = round256(gemm_workspace_min(M, N, K, opts ? *opts : kDefaultOpts));
+    const int64_t b = slice_bytes(i);
     Item it = {};
     it.index = i; it.ws_off = off; it.ws_bytes = b;
     off += b;

@@ -1,6 +1,7 @@
 """MX_KERNEL_AUTO never picks a kernel whose launch refuses the operands: few rows of A with weights whose rows overlap (a
-broadcast or a sliding window) or with scale rows that span 2 GiB.  On the host: where there is no device a dispatched
-launch ends in MX_ERR_LAUNCH, a refusal in MX_ERR_LAYOUT."""
+broadcast or a sliding window) or with scale rows that span 2 GiB.  And what a split along K needs is asked for only where
+the split is a contract.  On the host: where there is no device a dispatched launch ends in MX_ERR_LAUNCH, a refusal in
+MX_ERR_LAYOUT or MX_ERR_WORKSPACE."""
 import ctypes
 
 import pytest
@@ -51,3 +52,44 @@ def test_a_forced_streaming_kernel_says_what_it_cannot_take():
     assert rc == L.MX_ERR_LAYOUT and "B_scale spans 2 GiB" in message
     rc, message = _gemm(8, 256, 512, L.MX_E4M3, b_pitch=520, kernel=9)
     assert rc == L.MX_ERR_LAYOUT and "16-byte aligned rows" in message
+
+
+def _split_problem(M, N, K, layouts, split_k):
+    p = (torch.zeros(1 << 16, dtype=torch.uint8).data_ptr() + 255) // 256 * 256
+    t = (_desc(p, L.MX_E4M3, (M, K), (K, 1)), _desc(p, L.MX_E8M0, (M, K // 32), (K // 32, 1)),
+         _desc(p, L.MX_E4M3, (K, N), (1, K)), _desc(p, L.MX_E8M0, (K // 32, N), (1, K // 32)),
+         _desc(p, L.MX_F32, (M, N), (N, 1)))
+    o = L.MxGemmOpts(struct_size=32, block_size=32, split_k=split_k, a_scale_layout=layouts[0], b_scale_layout=layouts[1])
+    return p, [ctypes.byref(x) for x in t], o
+
+
+@pytest.mark.parametrize("split_k", [0, 2])
+@pytest.mark.parametrize("K,layouts", [(8192, (2, 2)), (8192, (0, 2)), (8000, (0, 0))])
+def test_an_unpromised_split_needs_no_workspace(K, layouts, split_k):
+    """Packed scales, or a K that is not whole slices of 512: with room for the scales alone the product runs whole, as one
+    call, as an entry of a list and in the static scratch."""
+    lib, (M, N) = cutile_amd.lib(), (300, 200)
+    p, t, o = _split_problem(M, N, K, layouts, split_k)
+    scales = sum(lib.mx_packed_scale_bytes(rows, K) for rows, layout in ((M, layouts[0]), (N, layouts[1])) if layout == 0)
+    assert split_k == 2 and K == 8000 or lib.mx_gemm_workspace_bytes(M, N, K, ctypes.byref(o)) > scales
+    for have in (scales, scales + 256):
+        ws = p if have else None
+        assert lib.mx_gemm(*t, ctypes.byref(o), ws, have, None) == L.MX_ERR_LAUNCH, L.last_error()
+        assert lib.mx_gemm_list(1, *t, ctypes.byref(o), ws, have, None) == L.MX_ERR_LAUNCH, L.last_error()
+    if scales:
+        assert lib.mx_gemm(*t, ctypes.byref(o), p, scales - 256, None) == L.MX_ERR_WORKSPACE
+        assert lib.mx_gemm_list(1, *t, ctypes.byref(o), p, scales - 256, None) == L.MX_ERR_WORKSPACE
+    p, t, o = _split_problem(1000, 2000, K, layouts, 2 if K == 8192 else 0)
+    if layouts != (0, 0):   # two slices of 8 MB: more than the static scratch holds
+        assert lib.mx_gemm_static(*t, ctypes.byref(o), None) == L.MX_ERR_DEVICE, L.last_error()
+
+
+@pytest.mark.parametrize("split_k", [0, 2])
+def test_a_promised_split_is_held_to_its_workspace(split_k):
+    """Plain scales and equal slices of 512: less than the partial sums need is refused."""
+    lib, (M, N, K) = cutile_amd.lib(), (300, 200, 8192)
+    p, t, o = _split_problem(M, N, K, (0, 0), split_k)
+    need = lib.mx_gemm_workspace_bytes(M, N, K, ctypes.byref(o))
+    assert lib.mx_gemm(*t, ctypes.byref(o), p, need, None) == L.MX_ERR_LAUNCH
+    assert lib.mx_gemm(*t, ctypes.byref(o), p, need - 256, None) == L.MX_ERR_WORKSPACE
+    assert lib.mx_gemm_list(1, *t, ctypes.byref(o), p, need - 256, None) == L.MX_ERR_WORKSPACE

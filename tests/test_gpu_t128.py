@@ -62,3 +62,22 @@ def test_batch_in_one_launch(ct, dev, fa, fb, bx, by, M, N, K):
         ref = oracle_matmul(xs[i % bx], ys[i % by], z[i].cpu())
         assert O.rel_fro(out[i].cpu(), ref) <= TOL
     assert torch.equal(z, keep)
+
+
+@pytest.mark.parametrize("split_k", [0, 2])
+def test_unpromised_split_without_workspace_runs_whole(ct, dev, split_k):
+    """Packed scales and no workspace at all: the bits of the unsplit product, as one call and as a list of one."""
+    from cutile_amd import _lib as L
+    M, N, K = 130, 200, 8192
+    a, b = randn_operand(M, K, O.E4M3, 31, dev), randn_operand(N, K, O.E4M3, 32, dev)
+    sa, sb = ct.pack_scales(a.scale_t, operand="a"), ct.pack_scales(b.scale_t, operand="b")
+    want = ct.block_scaled_matmul(a.storage, sa, b.storage.T, sb, split_k=1, out_dtype=torch.float32)
+    assert O.rel_fro(want.cpu(), oracle_matmul(a, b)) <= TOL
+    o = L.MxGemmOpts(struct_size=32, block_size=32, split_k=split_k, a_scale_layout=2, b_scale_layout=2)
+    for call in (ct.lib().mx_gemm, lambda *t: ct.lib().mx_gemm_list(1, *t)):
+        c = torch.zeros((M, N), device=dev)
+        t = (L.desc(a.storage, L.MX_E4M3), L.desc(a.scale_t, L.MX_E8M0), L.desc(b.storage.T, L.MX_E4M3),
+             L.desc(b.scale_t.T, L.MX_E8M0), L.desc(c, L.MX_F32))
+        t[1].ptr, t[3].ptr = sa.data.data_ptr(), sb.data.data_ptr()
+        assert call(*t, o, None, 0, L.stream_ptr(dev)) == 0, L.last_error()
+        assert torch.equal(c, want)
