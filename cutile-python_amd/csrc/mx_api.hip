@@ -1217,7 +1217,7 @@ MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& 
   p.qs = take(p.n * (p.F / 32));
   p.c3 = take(p.n * p.H_out * 4);
   if (!p.stream) {
-    p.tile_m = 256;
+    p.tile_m = o.tile_m > 0 ? o.tile_m : 256;
     p.max_slots = mx_moe_align_max_slots(p.n, (int32_t)p.E, p.tile_m);
     p.c1 = take(p.n * p.F * 4);
     p.slots = take(p.max_slots * 4);
@@ -1297,6 +1297,7 @@ int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1,
   if (!why && H_out <= 128) why = "H_out is too small";
   if (why) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: %s", why);
   const MoePlan p = moe_plan(T, topk, *W1, *W2, o);
+  if (!p.stream && p.tile_m % 128 != 0) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: tile_m is not a multiple of 128");
   if (p.n * p.F >= ((int64_t)1 << 31)) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: the activation spans 2 GiB or more");
   if (!workspace || workspace_bytes < p.total)
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)p.total, (long long)workspace_bytes);

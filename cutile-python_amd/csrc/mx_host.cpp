@@ -356,10 +356,10 @@ bool expert_scale_desc(PyObject* o, int64_t E, int64_t rows, int64_t K, const at
   return true;
 }
 
-// moe(hidden, hidden_scale, w1, w1_scale, w2, w2_scale, topk_weights, topk_ids, out_dtype, mode, w_format)
+// moe(hidden, hidden_scale, w1, w1_scale, w2, w2_scale, topk_weights, topk_ids, out_dtype, mode, w_format, tile_m)
 //   -> result, error code, or None
 PyObject* py_moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 11) { PyErr_SetString(PyExc_TypeError, "moe takes 11 arguments"); return nullptr; }
+  if (n != 12) { PyErr_SetString(PyExc_TypeError, "moe takes 12 arguments"); return nullptr; }
   for (int i : {0, 1, 2, 4, 6, 7})
     if (!THPVariable_Check(a[i])) Py_RETURN_NONE;
   const at::Tensor &X = THPVariable_Unpack(a[0]), &Xs = THPVariable_Unpack(a[1]), &W1 = THPVariable_Unpack(a[2]),
@@ -379,7 +379,10 @@ PyObject* py_moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (out_code(out_t) < 0) Py_RETURN_NONE;
   mx_tensor dX = desc(X, MX_E4M3), dXs = desc(Xs, MX_E8M0), dW1 = desc(W1, f1, f1 == MX_E2M1 ? 2 : -1),
             dW2 = desc(W2, f2, f2 == MX_E2M1 ? 2 : -1), dW1s, dW2s;
-  mx_gemm_opts o = {sizeof(mx_gemm_opts), 0, 0, 0, MX_KERNEL_AUTO, 32, 0, 0};
+  const long tile_m = PyLong_AsLong(a[11]);
+  if (tile_m == -1 && PyErr_Occurred()) PyErr_Clear();
+  if (tile_m <= 0 || tile_m > 0x7FFFFFFF) Py_RETURN_NONE;
+  mx_gemm_opts o = {sizeof(mx_gemm_opts), 0, 0, 0, MX_KERNEL_AUTO, 32, 0, (int32_t)tile_m};
   if (!expert_scale_desc(a[3], E, dW1.shape[1], dW1.shape[2], dev, &dW1s, &o.a_scale_layout) ||
       !expert_scale_desc(a[5], E, dW2.shape[1], dW2.shape[2], dev, &dW2s, &o.b_scale_layout))
     Py_RETURN_NONE;

@@ -890,11 +890,14 @@ def cutile_moe_scaled(hidden_states: torch.Tensor, hidden_scale: torch.Tensor,
     MX elements (FP4 packed along the last axis, ``w_format="e2m1"``) with scales (E, rows, K/32) or
     :class:`PackedScales`; topk_weights / topk_ids (tokens, topk).  The intermediate activation is
     re-quantised to E4M3 on the device (one fused pass) so that both GEMMs run block-scaled.  Nothing in the
-    call synchronises with the host.  Returns (tokens, H) in ``out_dtype``."""
+    call synchronises with the host.  Returns (tokens, H) in ``out_dtype``.
+
+    ``tile_m`` is the number of slots that an expert's rows are padded to (128: less padding where experts get few
+    rows).  Where they get so few that the weights are streamed there are no slots, and it has no effect."""
     if kernel == "auto" and scale_mode in ("floor", "ceil"):
-        # one library call for the whole layer (tile_m is then the library's choice: results do not depend on it)
+        # one library call for the whole layer
         r = L.host().moe(hidden_states, hidden_scale, w1, w1_scale, w2, w2_scale, topk_weights, topk_ids, out_dtype,
-                         1 if scale_mode == "floor" else 0, w_format)
+                         1 if scale_mode == "floor" else 0, w_format, tile_m)
         if isinstance(r, torch.Tensor):
             return r
         if r is not None:

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define MXGEMM_VERSION 104
+#define MXGEMM_VERSION 105
 
 /* Exported symbols (the library is built with hidden default visibility). */
 #if defined(__GNUC__)
@@ -132,7 +132,8 @@ typedef struct mx_gemm_opts {
                              partial products in a fixed order: the split-K scheme of
                              matmul_split_k_kernel, test/kernels/matmul.py:103-140, for small M x N
                              with a long K                                                        */
-  int32_t reserved;
+  int32_t tile_m;         /* mx_moe_forward only: slots per tile of the grouped GEMMs, a multiple of 128 (128-row tiles pad
+                             experts of few rows less); 0 = 256                                   */
 } mx_gemm_opts;
 
 /* Library version (MXGEMM_VERSION of the built library). */
@@ -314,8 +315,8 @@ MX_API int mx_silu_mul_quantize(const mx_tensor* gate_up, mx_tensor* xq, mx_tens
  *   topk_weights [T,topk] fp32; topk_ids [T,topk] int32 (ids64 = 0) or int64 (1), contiguous; ids outside [0, E) drop
  *   their copy.  The activation between the projections is E4M3, quantised by scale_mode as in mx_quantize.
  *   out [T,H_out] MX_F32 or MX_BF16, contiguous.
- * A few rows per expert stream the experts' weights (three launches in all); more run as alignment, grouped GEMM,
- * activation, grouped GEMM and sum.  No host synchronisation.  Returns MX_ERR_LAYOUT, with nothing enqueued, for
+ * A few rows per expert stream the experts' weights (three launches in all, no slots and hence no tile_m); more run as
+ * alignment to opts->tile_m, grouped GEMM, activation, grouped GEMM and sum.  No host synchronisation.  Returns MX_ERR_LAYOUT, with nothing enqueued, for
  * operands that only the single entry points take (generic-kernel layouts).
  */
 MX_API int64_t mx_moe_forward_workspace_bytes(int64_t T, int32_t topk, const mx_tensor* W1, const mx_tensor* W2,

@@ -93,3 +93,38 @@ def test_a_promised_split_is_held_to_its_workspace(split_k):
     assert lib.mx_gemm(*t, ctypes.byref(o), p, need, None) == L.MX_ERR_LAUNCH
     assert lib.mx_gemm(*t, ctypes.byref(o), p, need - 256, None) == L.MX_ERR_WORKSPACE
     assert lib.mx_gemm_list(1, *t, ctypes.byref(o), p, need - 256, None) == L.MX_ERR_WORKSPACE
+
+
+def test_moe_slots_follow_tile_m(monkeypatch):
+    """The grouped form of the layer aligns to the caller's tile_m (its workspace shrinks with the padding), refuses what the
+    tiled kernels cannot take, and the operator hands its tile_m over; streamed layers have no slots."""
+    lib, E, H, F = cutile_amd.lib(), 16, 512, 256
+    p = (torch.zeros(1 << 16, dtype=torch.uint8).data_ptr() + 255) // 256 * 256
+    W1, W2 = _desc(p, 0, (E, 2 * F, H), (2 * F * H, H, 1)), _desc(p, 0, (E, H, F), (H * F, F, 1))
+
+    def need(T, tile_m):
+        o = L.MxGemmOpts(struct_size=32, block_size=32, tile_m=tile_m)
+        return lib.mx_moe_forward_workspace_bytes(T, 2, ctypes.byref(W1), ctypes.byref(W2), ctypes.byref(o))
+    assert need(2000, 128) < need(2000, 256) < need(2000, 512)
+    assert need(2000, 0) == need(2000, 256)
+    assert need(64, 128) == need(64, 256) == need(64, 16)   # streamed
+
+    def forward(T, tile_m):
+        o = L.MxGemmOpts(struct_size=32, block_size=32, tile_m=tile_m)
+        X, Xs = _desc(p, 0, (T, H), (H, 1)), _desc(p, L.MX_E8M0, (T, H // 32), (H // 32, 1))
+        W1s = _desc(p, L.MX_E8M0, (E, 2 * F, H // 32), (2 * F * H // 32, H // 32, 1))
+        W2s = _desc(p, L.MX_E8M0, (E, H, F // 32), (H * F // 32, F // 32, 1))
+        out = _desc(p, L.MX_F32, (T, H), (H, 1))
+        return lib.mx_moe_forward(*(ctypes.byref(t) for t in (X, Xs, W1, W1s, W2, W2s)), p, p, 0, 2, ctypes.byref(out), 1,
+                                  ctypes.byref(o), p, 1 << 40, None)
+    assert [forward(2000, t) for t in (0, 128, 384, 512)] == [L.MX_ERR_LAUNCH] * 4
+    assert forward(2000, 64) == L.MX_ERR_LAYOUT and "tile_m" in L.last_error()
+    assert forward(64, 64) == L.MX_ERR_LAUNCH
+
+    class Host:
+        def moe(self, *args):
+            self.args = args
+            return torch.zeros(0)
+    monkeypatch.setattr(L, "_host", Host())
+    cutile_amd.cutile_moe_scaled(*[None] * 8, 128)
+    assert L._host.args[-1] == 128

@@ -55,3 +55,24 @@ def test_moe_forward(ct, dev, T, H, F, E, topk, skew, w_fmt, packed):
         err = O.rel_fro(got.float().cpu(), want)
         print(f"{T} {H} {F} {E} {topk} {w_fmt} packed={packed} {out_dtype}: {err:.2e}", flush=True)
         assert err < 2e-2
+
+
+@pytest.mark.parametrize("tile_m", [16, 128, 384, 512])
+@pytest.mark.parametrize("T,E,topk,skew", [(150, 2, 2, 0.9), (300, 5, 1, 0.2), (1100, 16, 2, 0.0)])
+def test_moe_forward_tile_m(ct, dev, T, E, topk, skew, tile_m):
+    """Slot tiles other than the default one, beyond the sizes that stream: 128-row kernel, 256-row kernel with wider slots, and
+    the single operators where no tiled kernel takes them."""
+    H, F = 256, 128
+    rng = np.random.default_rng(T)
+    hq, hs = O.block_quantize(rng.standard_normal((T, H)).astype(np.float32), 32, O.E4M3, "floor")
+    w1q, w1s = O.block_quantize((rng.standard_normal((E, 2 * F, H)) * 0.2).astype(np.float32), 32, O.E4M3, "floor")
+    w2q, w2s = O.block_quantize((rng.standard_normal((E, H, F)) * 0.2).astype(np.float32), 32, O.E4M3, "floor")
+    ids = rng.integers(0, E, (T, topk))
+    ids[rng.random((T, topk)) < skew] = 0
+    wts = rng.random((T, topk)).astype(np.float32)
+    want = O.moe_forward(hq, hs, w1q, w1s, w2q, w2s, wts, ids)
+    got = ct.cutile_moe_scaled(_elems(hq, O.E4M3, dev), _scale(hs, dev), _elems(w1q, O.E4M3, dev), _scale(w1s, dev),
+                               _elems(w2q, O.E4M3, dev), _scale(w2s, dev), torch.from_numpy(wts).to(dev),
+                               torch.from_numpy(ids).to(dev), tile_m, out_dtype=torch.float32)
+    # (tolerance as above)
+    assert O.rel_fro(got.cpu(), want) < 2e-2
