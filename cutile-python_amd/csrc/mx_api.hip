@@ -1292,6 +1292,7 @@ int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1,
   if (!why) why = weights_issue(W1, W1s, o.a_scale_layout);
   if (!why) why = weights_issue(W2, W2s, o.b_scale_layout);
   if (!why && (Xs->stride[1] != 1 || Xs->stride[0] % 4 != 0 || ((uintptr_t)Xs->ptr) % 4 != 0)) why = "X_scale rows are not contiguous and 4-byte aligned";
+  if (!why && T * Xs->stride[0] >= ((int64_t)1 << 31)) why = "X_scale spans 2 GiB or more";   // 32-bit lane offsets
   if (!why && (out->stride[1] != 1 || out->stride[0] != H_out)) why = "out is not contiguous";
   if (!why && 2 * F <= 128) why = "F is too small";
   if (!why && H_out <= 128) why = "H_out is too small";

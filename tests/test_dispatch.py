@@ -109,9 +109,9 @@ def test_moe_slots_follow_tile_m(monkeypatch):
     assert need(2000, 0) == need(2000, 256)
     assert need(64, 128) == need(64, 256) == need(64, 16)   # streamed
 
-    def forward(T, tile_m):
+    def forward(T, tile_m, xs_pitch=H // 32):
         o = L.MxGemmOpts(struct_size=32, block_size=32, tile_m=tile_m)
-        X, Xs = _desc(p, 0, (T, H), (H, 1)), _desc(p, L.MX_E8M0, (T, H // 32), (H // 32, 1))
+        X, Xs = _desc(p, 0, (T, H), (H, 1)), _desc(p, L.MX_E8M0, (T, H // 32), (xs_pitch, 1))
         W1s = _desc(p, L.MX_E8M0, (E, 2 * F, H // 32), (2 * F * H // 32, H // 32, 1))
         W2s = _desc(p, L.MX_E8M0, (E, H, F // 32), (H * F // 32, F // 32, 1))
         out = _desc(p, L.MX_F32, (T, H), (H, 1))
@@ -120,6 +120,10 @@ def test_moe_slots_follow_tile_m(monkeypatch):
     assert [forward(2000, t) for t in (0, 128, 384, 512)] == [L.MX_ERR_LAUNCH] * 4
     assert forward(2000, 64) == L.MX_ERR_LAYOUT and "tile_m" in L.last_error()
     assert forward(64, 64) == L.MX_ERR_LAUNCH
+    # scale rows that lane offsets do not reach go to the single operators, streamed or not
+    for T in (64, 2000):
+        assert forward(T, 0, ((1 << 31) - 1) // T // 4 * 4) == L.MX_ERR_LAUNCH
+        assert forward(T, 0, ((1 << 31) - 1) // T // 4 * 4 + 4) == L.MX_ERR_LAYOUT and "X_scale" in L.last_error()
 
     class Host:
         def moe(self, *args):

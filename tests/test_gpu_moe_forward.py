@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from oracle import mx_oracle as O
+from test_gpu_stream import _spread
 
 pytestmark = pytest.mark.gpu
 
@@ -55,6 +56,18 @@ def test_moe_forward(ct, dev, T, H, F, E, topk, skew, w_fmt, packed):
         err = O.rel_fro(got.float().cpu(), want)
         print(f"{T} {H} {F} {E} {topk} {w_fmt} packed={packed} {out_dtype}: {err:.2e}", flush=True)
         assert err < 2e-2
+
+
+def test_moe_forward_scale_rows_that_span_2_gib(ct, dev):
+    T, E, topk, H, F = 9, 4, 2, 256, 128
+    rng = np.random.default_rng(1)
+    q = lambda *shape: ct.block_quantize(torch.from_numpy(rng.standard_normal(shape).astype(np.float32)).to(dev), 32)
+    (x, xs), (w1, s1), (w2, s2) = q(T, H), q(E, 2 * F, H), q(E, H, F)
+    wide = _spread(xs, (1 << 32) // (T - 1) // 16 * 16, dev)
+    wt, ids = torch.rand((T, topk), device=dev), torch.from_numpy(rng.integers(0, E, (T, topk))).to(dev)
+    got, want = (ct.cutile_moe_scaled(x, s, w1, s1, w2, s2, wt, ids, out_dtype=torch.float32) for s in (wide, xs))
+    # the same products, added up in another order, then rounded to bf16 and E4M3 on the way (tolerance as above)
+    assert ((got - want).norm() / want.norm()).item() < 2e-2
 
 
 @pytest.mark.parametrize("tile_m", [16, 128, 384, 512])
