@@ -1,8 +1,9 @@
-// Measurement aid: the rate at which the matrix pipe runs the scaled MFMA instruction out of registers alone
+// Probes of the chip.  Measurement aid: the rate at which the matrix pipe runs the scaled MFMA instruction out of registers alone
 // (no LDS, no memory traffic), as a function of the operand bits.  The GEMM kernels' roofline is quoted against the
 // chip's nominal peak; this loop shows what the chip sustains on a given kind of data when nothing but the matrix
 // pipe works, which is the ceiling any schedule of the same instructions has on that data.
 #include "mx_common.h"
+#include "mx_quant.h"
 
 namespace mx {
 namespace {
@@ -40,8 +41,30 @@ __global__ __launch_bounds__(512) void mfma_rate_kernel(const v8i* __restrict__ 
   sink[blockIdx.x * 512 + t] = s;
 }
 
+// Check of rcp_rn (mx_quant.h): differ[e] += number of d in [2^(first + e), 2^(first + e + 1)) for which it is not 1 / d rounded
+// to nearest.  The fp64 quotient rounded to fp32 is: 53 bits are more than twice 24 plus one, so the two roundings of a
+// quotient are as good as one.
+__global__ __launch_bounds__(256) void rcp_check_kernel(int first, int exponents, uint32_t* __restrict__ differ) {
+  const uint32_t m = blockIdx.x * 256 + threadIdx.x;   // 2^15 x 256 threads: every significand
+  for (int e = 0; e < exponents; ++e) {
+    const float d = __builtin_bit_cast(float, (uint32_t)(127 + first + e) << 23 | m);
+    const float want = (float)(1.0 / (double)d);
+    if (__builtin_bit_cast(uint32_t, rcp_rn(d)) != __builtin_bit_cast(uint32_t, want)) atomicAdd(&differ[e], 1u);
+  }
+}
+
 }  // namespace
 }  // namespace mx
+
+extern "C" int mx_probe_rcp(int32_t first_exponent, int32_t exponents, uint32_t* differ, void* stream) {
+  using namespace mx;
+  if (!differ || first_exponent < 0 || exponents <= 0 || exponents > 128 || first_exponent > 128 - exponents)
+    return set_error(MX_ERR_INVALID, "mx_probe_rcp: null pointer or exponents outside 0 .. 127");
+  hipLaunchKernelGGL(rcp_check_kernel, dim3(1 << 15), dim3(256), 0, (hipStream_t)stream, first_exponent, exponents, differ);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "rcp_check_kernel launch: %s", hipGetErrorString(e));
+  return MX_OK;
+}
 
 extern "C" int mx_probe_mfma_rate(int32_t fmt, const void* frags, int32_t workgroups, int32_t iters, float* sink,
                                   void* stream) {

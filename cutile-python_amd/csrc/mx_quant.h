@@ -85,8 +85,8 @@ __device__ inline uint32_t encode_e2m1(const Unpacked& u, int se) {
 }
 
 // 1 / d, correctly rounded, for d in [1, 2^126): the hardware's reciprocal and one Newton step in fused arithmetic give the
-// bits of the IEEE division for every such d (compared exhaustively on MI355X, all 2^23 significands of the 126
-// exponents; from 2^126 on the result is subnormal and they do not).  3 instructions for 12.
+// bits of the IEEE division for every such d (mx_probe_rcp compares all 2^23 significands of the 126 exponents; from 2^126
+// on the result is subnormal and they do not).  3 instructions for 12.
 __device__ inline float rcp_rn(float d) {
   const float r = __builtin_amdgcn_rcpf(d);
   return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);

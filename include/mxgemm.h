@@ -356,6 +356,14 @@ MX_API int mx_pack_scales(const mx_tensor* scale, int32_t layout, int64_t rows, 
 MX_API int mx_probe_mfma_rate(int32_t fmt, const void* frags, int32_t workgroups, int32_t iters, float* sink,
                        void* stream);
 
+/*
+ * Check aid (no reference counterpart): differ[e] (uint32, on the device, set to zero by the caller) is increased by the number
+ * of fp32 values d in [2^(first_exponent + e), 2^(first_exponent + e + 1)), e < exponents, for which the reciprocal that
+ * mx_silu_mul_quantize takes in the place of a division differs from 1 / d rounded to nearest.  It is none for
+ * exponents 0 .. 125, the range that SiLU's denominator 1 + exp(-a) lies in.  Asynchronous on `stream`.
+ */
+MX_API int mx_probe_rcp(int32_t first_exponent, int32_t exponents, uint32_t* differ, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

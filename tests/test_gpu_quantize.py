@@ -309,3 +309,15 @@ def test_silu_quantize_aligned_rows_match_the_general_route(ct, dev, rows, F):
     q, s = ct.silu_and_mul_quantize(gate_up)
     q0, s0 = ct.silu_and_mul_quantize(off)
     assert torch.equal(s.view(torch.uint8), s0.view(torch.uint8)) and torch.equal(q.view(torch.uint8), q0.view(torch.uint8))
+
+
+def test_silu_reciprocal_is_the_ieee_division(ct, dev):
+    """The reciprocal that SiLU takes in the place of a division, over all fp32 denominators that it can meet (every
+    significand of the exponents 0 .. 125) -- and the exponent behind them, where it is known to differ."""
+    from cutile_amd import _lib as L
+    differ = torch.zeros(127, dtype=torch.int32, device=dev)
+    assert ct.lib().mx_probe_rcp(0, 127, differ.data_ptr(), L.stream_ptr(dev)) == 0, L.last_error()
+    counts = differ.cpu()
+    assert (counts[:126] == 0).all() and counts[126] > 0, counts
+    for first, exponents in ((-1, 1), (0, 0), (0, 129), (127, 2)):
+        assert ct.lib().mx_probe_rcp(first, exponents, differ.data_ptr(), None) == L.MX_ERR_INVALID
