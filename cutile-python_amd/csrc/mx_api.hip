@@ -1074,6 +1074,7 @@ int gemm_grouped_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* 
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                      (long long)workspace_bytes);
   if (((uintptr_t)ws) % 256 != 0) return set_error(MX_ERR_WORKSPACE, "workspace must be 256-byte aligned");
+  if (T == 0) return MX_OK;   // no slot holds a row (the kernels' descriptors end behind the last row: there has to be one)
   if (kernel == MX_KERNEL_MFMA_128x128) {
     T128Args g = {};
     g.a_plain = t128_plain_scales(As->ptr, As->stride[0], As->stride[1], T, K, A->dtype, W->dtype);

@@ -132,3 +132,19 @@ def test_moe_slots_follow_tile_m(monkeypatch):
     monkeypatch.setattr(L, "_host", Host())
     cutile_amd.cutile_moe_scaled(*[None] * 8, 128)
     assert L._host.args[-1] == 128
+
+
+@pytest.mark.parametrize("kernel,tile_m", [(0, 128), (0, 256), (2, 128), (2, 256), (3, 256), (4, 256), (6, 256)])
+def test_grouped_product_of_no_rows_launches_nothing(kernel, tile_m):
+    """Slots that are all padding over an A without rows, whose row pitch is wider than a row: a descriptor that ended behind
+    its last row would wrap around."""
+    lib, E, N, K = cutile_amd.lib(), 2, 256, 512
+    p = (torch.zeros(1 << 16, dtype=torch.uint8).data_ptr() + 255) // 256 * 256
+    W, Ws = _desc(p, 0, (E, N, K), (N * K, K, 1)), _desc(p, L.MX_E8M0, (E, N, K // 32), (N * K // 32, K // 32, 1))
+    o = L.MxGemmOpts(struct_size=32, block_size=32, kernel=kernel)
+    for T, want in ((0, L.MX_OK), (3, L.MX_ERR_LAUNCH)):
+        A, As = _desc(p, 0, (T, K), (K + 16, 1)), _desc(p, L.MX_E8M0, (T, K // 32), (K // 32, 1))
+        C = _desc(p, L.MX_F32, (T, N), (N, 1))
+        rc = lib.mx_gemm_grouped(*(ctypes.byref(t) for t in (A, As, W, Ws, C)), None, p, tile_m, p, tile_m, 1, T,
+                                 ctypes.byref(o), p, 1 << 30, None)
+        assert rc == want, L.last_error()
