@@ -133,13 +133,14 @@ bool pair_supported_by_mfma(int a, int b) {
 
 // Checks the layout preconditions of the MFMA kernels for a K-contiguous operand with `rows` rows.
 // Returns nullptr if fine, otherwise the reason.
-const char* mfma_operand_issue(const void* ptr, int64_t rows, int64_t ld_bytes, int64_t k_stride,
+const char* mfma_operand_issue(const void* ptr, int64_t rows, int64_t K, int64_t ld_bytes, int64_t k_stride,
                                int fmt, int packed_ok) {
   if (k_stride != 1) return "K axis is not contiguous";
   if (fmt == MX_E2M1 && !packed_ok) return "FP4 operand is not packed along K";
   if (((uintptr_t)ptr) % 16 != 0) return "base pointer is not 16-byte aligned";
   if (ld_bytes % 16 != 0) return "row pitch is not a multiple of 16 bytes";
-  if (rows * ld_bytes >= ((int64_t)1 << 31)) return "operand spans 2 GiB or more";
+  const int64_t row = fmt == MX_E2M1 ? K / 2 : K, lim = (int64_t)1 << 31;
+  if (rows * ld_bytes >= lim || (rows - 1) * ld_bytes + row >= lim) return "operand spans 2 GiB or more";   // (rows may overlap)
   return nullptr;
 }
 
@@ -454,8 +455,8 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       const bool fp4 = A->dtype == MX_E2M1;
       bool ok = (o.kernel == MX_KERNEL_AUTO || o.kernel == MX_KERNEL_MFMA_128x128) && o.split_k <= 1 && K > 0 &&
                 pair_supported_by_mfma(A->dtype, B->dtype) && C->stride[2] == 1 && bstride(A) % 16 == 0 && bstride(B) % 16 == 0 &&
-                !mfma_operand_issue(a2.ptr, M, a2.stride[0], a2.stride[1], A->dtype, a2.packed_dim == 1) &&
-                !mfma_operand_issue(b2.ptr, N, b2.stride[1], b2.stride[0], B->dtype, b2.packed_dim == 0) &&
+                !mfma_operand_issue(a2.ptr, M, K, a2.stride[0], a2.stride[1], A->dtype, a2.packed_dim == 1) &&
+                !mfma_operand_issue(b2.ptr, N, K, b2.stride[1], b2.stride[0], B->dtype, b2.packed_dim == 0) &&
                 M < (1 << 30) && N < (1 << 30) && K < (1 << 30);
       const bool plain = ok && t128_plain_scales(as2.ptr, as2.stride[0], as2.stride[1], M, K, A->dtype, B->dtype) &&
                          t128_plain_scales(bs2.ptr, bs2.stride[1], bs2.stride[0], N, K, A->dtype, B->dtype) &&
@@ -528,8 +529,8 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
   else if (o.block_size != 32 || As->dtype != MX_E8M0) why = "only E8M0 scales with block 32 are MFMA-native";
   else if (!pair_supported_by_mfma(A->dtype, B->dtype)) why = "element format pair not instantiated";
   else if (K == 0) why = "K is zero";
-  else if ((why = mfma_operand_issue(A->ptr, M, a_ld, A->stride[1], A->dtype, A->packed_dim == 1))) {}
-  else if ((why = mfma_operand_issue(B->ptr, N, b_ld, B->stride[0], B->dtype, B->packed_dim == 0))) {}
+  else if ((why = mfma_operand_issue(A->ptr, M, K, a_ld, A->stride[1], A->dtype, A->packed_dim == 1))) {}
+  else if ((why = mfma_operand_issue(B->ptr, N, K, b_ld, B->stride[0], B->dtype, B->packed_dim == 0))) {}
   else if (C->stride[1] != 1) why = "C is not row-major";
   else if (M >= (1 << 30) || N >= (1 << 30) || K >= (1 << 30)) why = "extent too large";
 
@@ -1030,8 +1031,8 @@ int gemm_grouped_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* 
 
   const char* why = nullptr;
   if (!pair_supported_by_mfma(A->dtype, W->dtype)) why = "element format pair not instantiated";
-  else if ((why = mfma_operand_issue(A->ptr, T, A->stride[0], A->stride[1], A->dtype, 1))) {}
-  else if ((why = mfma_operand_issue(W->ptr, N, W->stride[1], W->stride[2], W->dtype, 1))) {}
+  else if ((why = mfma_operand_issue(A->ptr, T, K, A->stride[0], A->stride[1], A->dtype, 1))) {}
+  else if ((why = mfma_operand_issue(W->ptr, N, K, W->stride[1], W->stride[2], W->dtype, 1))) {}
   else if (W->stride[0] % 16 != 0) why = "expert pitch of W is not a multiple of 16 bytes";
   else if (C->stride[1] != 1) why = "C is not row-major";
   else if (tile_m % 128 != 0) why = "tile_m is not a multiple of 128";
@@ -1278,7 +1279,7 @@ int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1,
   // every condition under which one of the steps below could refuse its operands, before anything is enqueued
   auto weights_issue = [&](const mx_tensor* W, const mx_tensor* Ws, int32_t layout) -> const char* {
     if (W->dtype == MX_E2M1 && W->packed_dim != 2) return "FP4 weights are not packed along K";
-    if (const char* why = mfma_operand_issue(W->ptr, W->shape[1], W->stride[1], W->stride[2], W->dtype, 1)) return why;
+    if (const char* why = mfma_operand_issue(W->ptr, W->shape[1], W->shape[2], W->stride[1], W->stride[2], W->dtype, 1)) return why;
     if (W->stride[0] % 16 != 0) return "expert pitch of W is not a multiple of 16 bytes";
     if (E * mx_packed_scale_bytes(W->shape[1], W->shape[2]) >= ((int64_t)1 << 31)) return "the packed scales span 2 GiB or more";
     if (layout == MX_SCALE_NATIVE) return ((uintptr_t)Ws->ptr) % 16 != 0 ? "packed scales are not 16-byte aligned" : nullptr;
@@ -1289,7 +1290,7 @@ int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1,
       return "W_scale rows are not contiguous and 4-byte aligned";
     return nullptr;
   };
-  const char* why = mfma_operand_issue(X->ptr, T, X->stride[0], X->stride[1], X->dtype, 1);
+  const char* why = mfma_operand_issue(X->ptr, T, H, X->stride[0], X->stride[1], X->dtype, 1);
   if (!why) why = weights_issue(W1, W1s, o.a_scale_layout);
   if (!why) why = weights_issue(W2, W2s, o.b_scale_layout);
   if (!why && (Xs->stride[1] != 1 || Xs->stride[0] % 4 != 0 || ((uintptr_t)Xs->ptr) % 4 != 0)) why = "X_scale rows are not contiguous and 4-byte aligned";

@@ -76,8 +76,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, lds_u8* const smem,
   }
 
   const uint8_t* Bbase = g.B + (GROUPED ? (int64_t)expert * g.b_expert_stride : 0);
-  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(g.A, (uint32_t)(g.a_rows * g.lda));
-  const __amdgpu_buffer_rsrc_t rsB = make_rsrc(Bbase, (uint32_t)((int64_t)g.N * g.ldb));
+  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(g.A, operand_bytes(g.a_rows, g.lda, Kb_a));
+  const __amdgpu_buffer_rsrc_t rsB = make_rsrc(Bbase, operand_bytes(g.N, g.ldb, Kb_b));
 
   // ---- per-thread global offsets of the 16-byte chunks this thread moves each stage -----------------
   // load q of wave w fills LDS slots [(q*NW + w)*64, +64): slot s = (row s / CPR, position s % CPR)

@@ -66,7 +66,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   const int KQ = (ksteps + 3) / 4;
   constexpr int SPQ = 4 / C::KSUB;   // stages per K-quad
   const int a_groups = (g.M + 63) / 64, b_groups = (g.N + 63) / 64;
-  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(g.A, (uint32_t)(g.a_rows * g.lda));
+  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(g.A, operand_bytes(g.a_rows, g.lda, Kb_a));
 
   // ---- load context: where the DMA and scale loads of the tile being FETCHED point --------------------
   // A: instruction q of the wave covers tile rows wm0 + (4 q + wn) * A_RPI ...; B (team 1 only):
@@ -131,7 +131,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
       expert = expert < 0 ? 0 : (expert >= g.num_experts ? g.num_experts - 1 : expert);
     }
     const uint8_t* Bbase = g.B + (GROUPED ? (int64_t)expert * g.b_expert_stride : 0);
-    rsB = make_rsrc(Bbase, (uint32_t)((int64_t)g.N * g.ldb));
+    rsB = make_rsrc(Bbase, operand_bytes(g.N, g.ldb, Kb_b));
 #pragma unroll
     for (int q = 0; q < AL; ++q) {
       int64_t grow = m0 + a_row0 + q * 4 * P::A_RPI;

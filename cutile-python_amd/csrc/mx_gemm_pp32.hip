@@ -98,7 +98,7 @@ __device__ __forceinline__ void pp32_body(const GemmArgs& g, lds_u8* const smem,
   const int nstages = ksteps;
   const int KQ = (ksteps + 3) / 4;
   const int a_groups = (g.M + 63) / 64, b_groups = (g.N + 63) / 64;
-  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(g.A, (uint32_t)(g.a_rows * g.lda));
+  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(g.A, operand_bytes(g.a_rows, g.lda, Kb_a));
 
   // ---- load context of the tile being FETCHED (see mx_gemm_pp.hip) -----------------------------------------
   uint32_t a_voff[AL], b_voff[TEAM ? BL : 1];
@@ -143,7 +143,7 @@ __device__ __forceinline__ void pp32_body(const GemmArgs& g, lds_u8* const smem,
       expert = expert < 0 ? 0 : (expert >= g.num_experts ? g.num_experts - 1 : expert);
     }
     const uint8_t* Bbase = g.B + (GROUPED ? (int64_t)expert * g.b_expert_stride : 0);
-    rsB = make_rsrc(Bbase, (uint32_t)((int64_t)g.N * g.ldb));
+    rsB = make_rsrc(Bbase, operand_bytes(g.N, g.ldb, Kb_b));
 #pragma unroll
     for (int q = 0; q < AL; ++q) {
       int64_t grow = m0 + a_row0 + q * 4 * P::A_RPI;

@@ -171,9 +171,13 @@ const char* stream_issue(const StreamArgs& a) {
   if ((((uintptr_t)a.Xs | (uintptr_t)a.ldxs) % 4) != 0) return "A_scale must have 4-byte aligned rows";
   if (a.ws_packed ? ((uintptr_t)a.Ws % 16) != 0 : (((uintptr_t)a.Ws | (uintptr_t)a.ldws) % 4) != 0)
     return "B_scale must be 16-byte aligned (packed) or have 4-byte aligned rows";
-  const int64_t lim = (int64_t)1 << 31;   // lane offsets are 32-bit, and this one marks what does not exist
-  if ((int64_t)a.M * a.ldx >= lim || (int64_t)a.N * a.ldw >= lim) return "A or B spans 2 GiB or more";
-  if ((int64_t)a.M * a.ldxs >= lim || (a.ws_packed ? packed_scale_dwords(a.N, a.K) * 4 : (int64_t)a.N * a.ldws) >= lim)
+  // lane offsets are 32-bit, and 2^31 marks what does not exist
+  auto fits = [](int64_t rows, int64_t pitch, int64_t row) {
+    return rows * pitch < (int64_t)1 << 31 && (rows - 1) * pitch + row < (int64_t)1 << 31;
+  };
+  if (!fits(a.M, a.ldx, a.K) || !fits(a.N, a.ldw, a.w_fmt == MX_E2M1 ? a.K / 2 : a.K)) return "A or B spans 2 GiB or more";
+  if (!fits(a.M, a.ldxs, a.K / 32) ||
+      !(a.ws_packed ? fits(1, 0, packed_scale_dwords(a.N, a.K) * 4) : fits(a.N, a.ldws, a.K / 32)))
     return "A_scale or B_scale spans 2 GiB or more";
   return nullptr;
 }

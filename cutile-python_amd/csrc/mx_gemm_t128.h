@@ -30,7 +30,8 @@ struct T128Args {
 // scales that the kernel reads where they are: K-contiguous rows of 4-byte aligned E8M0 bytes, K a whole number of stages
 inline bool t128_plain_scales(const void* ptr, int64_t ld, int64_t k_stride, int64_t rows, int64_t K, int a_fmt, int b_fmt) {
   const int stage = a_fmt == MX_E2M1 && b_fmt == MX_E2M1 ? 256 : 128;
-  return k_stride == 1 && K % stage == 0 && ld % 4 == 0 && ((uintptr_t)ptr) % 4 == 0 && rows * ld < ((int64_t)1 << 31);
+  return k_stride == 1 && K % stage == 0 && ld % 4 == 0 && ((uintptr_t)ptr) % 4 == 0 && rows * ld < ((int64_t)1 << 31) &&
+         (rows - 1) * ld + K / 32 < ((int64_t)1 << 31);
 }
 int launch_gemm_t128(const T128Args& g, hipStream_t stream);
 // any number of independent plain products of one element-format pair: one persistent launch per 32 of them

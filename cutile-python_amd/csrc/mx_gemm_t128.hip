@@ -62,14 +62,14 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
   const uint8_t* const Ab = g.A + (int64_t)bz * g.a_batch;
   const uint8_t* const Bb = g.B + (int64_t)bz * g.b_batch + (GROUPED ? (int64_t)expert * g.b_expert : 0);
   const int64_t a_rows = GROUPED ? g.a_rows : g.M;
-  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(Ab, (uint32_t)((a_rows - 1) * g.lda + (int64_t)g.K * C::A_EB / 8));
-  const __amdgpu_buffer_rsrc_t rsB = make_rsrc(Bb, (uint32_t)((int64_t)(g.N - 1) * g.ldb + (int64_t)g.K * C::B_EB / 8));
+  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(Ab, operand_bytes(a_rows, g.lda, (int64_t)g.K * C::A_EB / 8));
+  const __amdgpu_buffer_rsrc_t rsB = make_rsrc(Bb, operand_bytes(g.N, g.ldb, (int64_t)g.K * C::B_EB / 8));
   const __amdgpu_buffer_rsrc_t rsAs =
       make_rsrc(g.As + (int64_t)bz * g.as_batch,
-                AP ? (uint32_t)((a_rows - 1) * g.ldas + g.K / 32) : (uint32_t)(packed_scale_dwords(g.M, g.K) * 4));
+                AP ? operand_bytes(a_rows, g.ldas, g.K / 32) : (uint32_t)(packed_scale_dwords(g.M, g.K) * 4));
   const __amdgpu_buffer_rsrc_t rsBs =
       make_rsrc(g.Bs + (int64_t)bz * g.bs_batch + (GROUPED ? (int64_t)expert * g.bs_expert : 0),
-                BP ? (uint32_t)((int64_t)(g.N - 1) * g.ldbs + g.K / 32) : (uint32_t)(packed_scale_dwords(g.N, g.K) * 4));
+                BP ? operand_bytes(g.N, g.ldbs, g.K / 32) : (uint32_t)(packed_scale_dwords(g.N, g.K) * 4));
 
   // ---- DMA: instruction q of wave w fills 1 KiB of the stage: rows (q * 4 + w) * RPI ... ------------------------------
   constexpr int AL = C::A_LOADS, BL = C::B_LOADS, TL = AL + BL;

@@ -36,6 +36,12 @@ __device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* p, uint32_t bytes
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
 
+// Bytes of an operand of `rows` >= 1 rows: it ends with the last row's last byte, whether rows overlap (a broadcast row has a
+// pitch of zero) or stand apart.
+__device__ inline uint32_t operand_bytes(int64_t rows, int64_t pitch, int64_t row_bytes) {
+  return (uint32_t)((rows - 1) * pitch + row_bytes);
+}
+
 // swizzle term of a tile row: chunk c of row R lives at chunk position c ^ swz<CPR>(R)
 template <int CPR>
 __device__ inline int swz(int row) {

@@ -66,8 +66,8 @@ __global__ __launch_bounds__(256) void gemm_w4_kernel(const GemmArgs g) {
   const int H = 2 * nstages;                            // half-stages per tile (the launcher guarantees H >= 6)
   const int KQ = (nstages + 3) / 4;
   const int a_groups = (g.M + 63) / 64, b_groups = (g.N + 63) / 64;
-  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(g.A, (uint32_t)(g.a_rows * g.lda));
-  const __amdgpu_buffer_rsrc_t rsB = make_rsrc(g.B, (uint32_t)((int64_t)g.N * g.ldb));
+  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(g.A, operand_bytes(g.a_rows, g.lda, Kb));
+  const __amdgpu_buffer_rsrc_t rsB = make_rsrc(g.B, operand_bytes(g.N, g.ldb, Kb));
 
   // ---- DMA context of the tile being FETCHED: wave w loads rows 64 w .. 64 w + 63 of A and of B, instruction q
   // rows 64 w + 16 q + lane / 4, 16-byte chunk lane % 4 of the 64-byte half row (position XOR swizzle) -----------

@@ -98,3 +98,27 @@ def test_pingpong_last_round_split_along_k(ct, dev, fmt, K, M, N, out_dtype, acc
     rel = ((got - ref).norm() / ref[1:M + 1, :N].norm()).item()
     assert rel <= (1e-5 if out_dtype == torch.float32 else 4e-3), rel   # (guards are equal on both sides)
     assert (bufs[0][0] == 7).all() and (bufs[0][-1] == 7).all() and (bufs[0][:, N:] == 7).all()
+
+
+@pytest.mark.parametrize("kernel", ["mfma128", "mfma256", "mfma256w4", "pingpong", "pingpong32", "w4p", "generic"])
+@pytest.mark.parametrize("side", ["a", "b"])
+@pytest.mark.parametrize("fmt,K", [(O.E4M3, 1152), (O.E2M1, 2304), (O.E4M3, 2048)])
+def test_rows_may_overlap(ct, dev, kernel, side, fmt, K):
+    """One operand as a broadcast row, or as windows that slide over one buffer: every kernel reads its last rows to their
+    end.  (K = 2048 also split along K.)"""
+    if fmt == O.E2M1 and kernel in ("pingpong32", "w4p"):
+        pytest.skip("8-bit element formats only")
+    M, N = 300, 272
+    a, b = randn_operand(M, K, fmt, 41, dev), randn_operand(N, K, fmt, 42, dev)
+    rows, row = (M, N)[side == "b"], (K // 2 if fmt == O.E2M1 else K)
+    flat = randn_operand(1, K + 32 * max(M, N), fmt, 43, dev)
+    for pitch in (0, 16):
+        t = flat.storage.view(-1).as_strided((rows, row), (pitch, 1))
+        codes = torch.from_numpy(flat.storage_np).view(-1).as_strided((rows, row), (pitch, 1)).contiguous().numpy()
+        op = a if side == "a" else b
+        op.storage, op.codes = t, O.unpack_fp4(codes) if fmt == O.E2M1 else codes
+        ref = oracle_matmul(a, b)
+        for split_k in (0, 2) if K == 2048 and kernel.startswith("mfma") else (0,):
+            c = ct.block_scaled_matmul(a.storage, a.scale_t, b.storage.T, b.scale_t.T, a_format=a.fmt_kw, b_format=b.fmt_kw,
+                                       kernel=kernel, split_k=split_k, out_dtype=torch.float32)
+            assert O.rel_fro(c.cpu(), ref) <= TOL[torch.float32], (pitch, split_k)
