@@ -1075,7 +1075,6 @@ int gemm_grouped_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* 
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                      (long long)workspace_bytes);
   if (((uintptr_t)ws) % 256 != 0) return set_error(MX_ERR_WORKSPACE, "workspace must be 256-byte aligned");
-  if (T == 0) return MX_OK;   // no slot holds a row (the kernels' descriptors end behind the last row: there has to be one)
   if (kernel == MX_KERNEL_MFMA_128x128) {
     T128Args g = {};
     g.a_plain = t128_plain_scales(As->ptr, As->stride[0], As->stride[1], T, K, A->dtype, W->dtype);
@@ -1102,6 +1101,7 @@ int gemm_grouped_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* 
       if (int rc = make_pack_args(Ws, MX_SCALE_2D, N, K, ws, kPackB, pw)) return rc;
       g.Bs = ws;
     }
+    if (T == 0) return MX_OK;   // no slot holds a row (the descriptor of A ends behind the last one: there has to be one)
     if (!g.a_plain || pack_w)
       if (int rc = launch_pack_scales_pair(g.a_plain ? nullptr : &pa, pack_w ? &pw : nullptr, (hipStream_t)stream)) return rc;
     g.A = (const uint8_t*)A->ptr; g.B = (const uint8_t*)W->ptr; g.C = C->ptr;
@@ -1137,6 +1137,7 @@ int gemm_grouped_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* 
     if (int rc = make_pack_args(Ws, MX_SCALE_2D, N, K, ws, t32 ? kPackTile32 : kPackB, pw)) return rc;
     bs_native = (const uint32_t*)ws;
   }
+  if (T == 0) return MX_OK;   // (as above)
   if (int rc = launch_pack_scales_pair(&pa, pack_w ? &pw : nullptr, (hipStream_t)stream)) return rc;
   GemmArgs g = {};
   g.A = (const uint8_t*)A->ptr; g.B = (const uint8_t*)W->ptr; g.As = as_native; g.Bs = bs_native; g.C = C->ptr;
