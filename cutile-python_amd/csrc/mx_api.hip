@@ -521,7 +521,11 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     return MX_OK;
   }
 
-  if (!batched) o = opts_for_room(M, N, K, o, workspace ? workspace_bytes : 0);
+  int64_t ws_min = batched ? 0 : gemm_workspace_min(M, N, K, o);
+  if (ws_min > (workspace ? workspace_bytes : 0)) {
+    o = opts_for_room(M, N, K, o, workspace ? workspace_bytes : 0);
+    ws_min = gemm_workspace_min(M, N, K, o);
+  }
   // ---- can the MFMA path take it? ------------------------------------------------------------------
   const char* why = nullptr;
   const int64_t a_ld = A->stride[and_ - 2], b_ld = B->stride[bnd - 1];
@@ -580,7 +584,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       const bool fp4 = A->dtype == MX_E2M1;
       const float t128 = est_t128(M, N, K, o.split_k > 1 ? 1 : plan_k_splits(M, N, K, o), fp4);
       const bool room = workspace && o.split_k == 0 && pp_tail_bytes(M, N, K, fp4, true) > 0 &&
-                        workspace_bytes >= gemm_workspace_min(M, N, K, o) + pp_tail_bytes(M, N, K, fp4, true);
+                        workspace_bytes >= ws_min + pp_tail_bytes(M, N, K, fp4, true);
       const float pp = o.split_k > 1 ? 1e30f : est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), room);
       const float st = may_stream ? est_stream(M, N, K, B->dtype) : 1e30f;
       kernel = st < t128 && st < pp ? MX_KERNEL_STREAM : t128 <= pp ? MX_KERNEL_MFMA_128x128 : big_tile_kernel();
@@ -638,9 +642,8 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
 
   if (kernel == MX_KERNEL_STREAM) {
     // it uses no workspace, but a caller of MX_KERNEL_AUTO is held to what mx_gemm_workspace_bytes says, whatever is picked
-    const int64_t need = gemm_workspace_min(M, N, K, o);
-    if (B->dtype != MX_E2M1 && need > 0 && (!workspace || workspace_bytes < need))
-      return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
+    if (B->dtype != MX_E2M1 && ws_min > 0 && (!workspace || workspace_bytes < ws_min))
+      return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)ws_min,
                        (long long)workspace_bytes);
     return launch_gemm_stream(sa, (hipStream_t)stream);
   }
@@ -678,7 +681,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
 
   // ---- MFMA path: bring the scales into the native layout if they are not ----------------------------
   uint8_t* ws = (uint8_t*)workspace;
-  int64_t need = gemm_workspace_min(M, N, K, o);
+  const int64_t need = ws_min;
   if (need > 0 && (!ws || workspace_bytes < need))
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                      (long long)workspace_bytes);
@@ -873,18 +876,18 @@ int mx_gemm_list(int32_t count, const mx_tensor* A, const mx_tensor* As, const m
   if (count < 0) return set_error(MX_ERR_INVALID, "mx_gemm_list: negative count");
   if (count == 0) return MX_OK;
   if (!A || !As || !B || !Bs || !C) return set_error(MX_ERR_INVALID, "mx_gemm_list: null descriptor array");
-  int64_t need = mx_gemm_list_workspace_bytes(count, A, B, opts);
-  const bool tight = (workspace ? workspace_bytes : 0) < need;   // then only what every problem is held to
-  auto slice_bytes = [&](int32_t i) {
-    int64_t M, N, K;
-    problem_dims(A[i], B[i], M, N, K);
-    const mx_gemm_opts& o = opts ? *opts : kDefaultOpts;
-    return round256(tight ? gemm_workspace_held(M, N, K, o) : gemm_workspace_min(M, N, K, o));
-  };
-  if (tight) {
+  std::vector<int64_t> share(count);   // of the workspace
+  int64_t need = 0;
+  auto shares = [&](int64_t (*bytes)(int64_t, int64_t, int64_t, const mx_gemm_opts&)) {
     need = 0;
-    for (int32_t i = 0; i < count; ++i) need += slice_bytes(i);
-  }
+    for (int32_t i = 0; i < count; ++i) {
+      int64_t M, N, K;
+      problem_dims(A[i], B[i], M, N, K);
+      need += share[i] = round256(bytes(M, N, K, opts ? *opts : kDefaultOpts));
+    }
+  };
+  shares(gemm_workspace_min);
+  if ((workspace ? workspace_bytes : 0) < need) shares(gemm_workspace_held);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                      (long long)workspace_bytes);
@@ -900,7 +903,7 @@ int mx_gemm_list(int32_t count, const mx_tensor* A, const mx_tensor* As, const m
   for (int32_t i = 0; i < count; ++i) {
     int64_t M, N, K;
     problem_dims(A[i], B[i], M, N, K);
-    const int64_t b = slice_bytes(i);
+    const int64_t b = share[i];
     Item it = {};
     it.index = i; it.ws_off = off; it.ws_bytes = b;
     off += b;
@@ -1207,7 +1210,13 @@ struct MoePlan {
   int32_t tile_m;
   int64_t q, qs, c3, c1, slots, in_use, max_slots, blocks, align, grouped, grouped_bytes, total;   // offsets (bytes)
 };
-// Rows per expert up to which the weights are streamed.
+// Rows per expert up to which the weights are streamed.  us per layer, streamed | grouped with 256-slot | 128-slot tiles:
+//   16 experts of 4096 x 4096, FP8: 32 rows 218 | 269 | 278, 48 rows 276 | 276 | 285, 64 rows 336 | 283 | 298;
+//   FP4: 32 rows 139 | 182 | 181, 48 rows 173 | 188 | 194, 64 rows 238 | 193 | 205
+//   8 experts of 4096 x 14336, FP8: 16 rows 257 | 358 | 323, 32 rows 372 | 368 | 353, 48 rows 455 | 374 | 388;
+//   FP4: 32 rows 238 | 280 | 259, 48 rows 275 | 284 | 295
+// so the line is right for FP4 and for experts of middling size; of large FP8 experts the tiles are ahead from 32 rows on.
+// (64 rows: with a longer list of ids, mx_stream.h.)
 constexpr int64_t kMoeStreamRows = 48;
 
 MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& W2, const mx_gemm_opts& o) {
