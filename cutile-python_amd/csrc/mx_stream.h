@@ -23,7 +23,11 @@ StreamPlan stream_plan(int64_t M, int64_t N, int64_t K, int w_fmt);
 int launch_gemm_stream(const StreamArgs& a, hipStream_t stream);
 
 // mixture-of-experts layer at decode sizes (mx_moe.hip)
-constexpr int kMoeMaxIds = 2048;   // routed ids that a workgroup sorts out by itself
+// Routed ids that a workgroup sorts out by itself, in a list of 4 KiB of LDS.  With room for 8192 two workgroups of the FP4
+// form no longer fit on a CU and its layers take 10 - 40 % longer (8 experts of 4096 x 14336, 16 rows each: 156 -> 184 us).
+// At 64 experts the limit lies about where the two forms of the layer meet (4096 x 2048, 32 rows each, streamed | grouped
+// GEMMs: FP8 427 | 417 us, FP4 287 | 314); of more experts it ends the streaming early (64, 16 rows each: 318 | 403, 203 | 303).
+constexpr int kMoeMaxIds = 2048;
 struct MoeStreamArgs {
   const uint8_t* X; const uint8_t* Xs; const uint8_t* W; const uint8_t* Ws;
   const void* ids; const float* weights;

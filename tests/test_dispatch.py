@@ -1,6 +1,6 @@
 """MX_KERNEL_AUTO never picks a kernel whose launch refuses the operands: few rows of A with weights whose rows overlap (a
-broadcast or a sliding window) or with scale rows that span 2 GiB.  And what a split along K needs is asked for only where
-the split is a contract.  On the host: where there is no device a dispatched launch ends in MX_ERR_LAUNCH, a refusal in
+broadcast or a sliding window) or with scale rows that span 2 GiB.  What a split along K needs is asked for only where the
+split is a contract; a mixture-of-experts layer keeps to the caller's tile_m; no rows, no launch.  On the host: where there is no device a dispatched launch ends in MX_ERR_LAUNCH, a refusal in
 MX_ERR_LAYOUT or MX_ERR_WORKSPACE."""
 import ctypes
 
