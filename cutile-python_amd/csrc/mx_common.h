@@ -81,6 +81,9 @@ __device__ inline float decode_elem(uint32_t c, int fmt) {
   return fmt == MX_E4M3 ? decode_e4m3(c) : fmt == MX_E5M2 ? decode_e5m2(c) : decode_e2m1(c);
 }
 
+// Cache policy of a buffer load (its last operand) whose lines nothing reads again: non-temporal, evicted first.
+constexpr int kLoadOnce = 2;
+
 // ---- fp32 -> bf16 bits, round to nearest even (torch's .to(bfloat16)) ---------------------------
 __device__ inline uint16_t f32_to_bf16(float f) {
   uint32_t u = __builtin_bit_cast(uint32_t, f);

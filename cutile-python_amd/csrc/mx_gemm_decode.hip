@@ -85,8 +85,9 @@ __device__ inline void issue_tile_dma2(const uint8_t* W, uint32_t wbytes, const 
   for (int j = 0; j < Cf::WIW; ++j) {
     const int r0 = rbase + j * Cf::RPI;
     const uint32_t off = chunk_off ^ (uint32_t)((r0 & 15) << 4);     // byte of the row this lane fetches
+    // (non-temporal: 28672 x 8192 at 32 rows 25.7 -> 23.7 us, x 4096 at 8 rows 13.9 -> 13.3; the scales as well: no gain)
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, (lds_void*)(wdst + j * 1024), 16,
-                                             off < row_bytes ? row_off + off : kOob, wsoff + r0 * ldw, 0, 0);
+                                             off < row_bytes ? row_off + off : kOob, wsoff + r0 * ldw, 0, kLoadOnce);
   }
   if (with_scales)   // uniform per wave
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsS, (lds_void*)sdst, 16, soff, ssoff, 0, 0);
