@@ -171,7 +171,9 @@ __global__ __launch_bounds__(256) void quantize_kernel(const QuantArgs q) {
 // registers, two units of 16 bytes per thread) and sent each workgroup's scale bytes out in 16-byte pieces of lines that
 // other XCDs' workgroups shared: 8192 x 8192 bf16 -> E4M3 took 44 - 49 us (4.1 - 4.6 TB/s), this one 36.6 (5.5 TB/s), and
 // 8192 x 14336 of silu(gate) * up 117 us where it took 161
-// (133 with an IEEE division per element: there the vector ALUs are the bound).  Here a wave owns U * 64 consecutive
+// (133 with an IEEE division per element: there the vector ALUs are the bound).  The loads of large inputs are non-temporal, and so are the
+// stores of codes that exceed the L2s anyway (U > 1; smaller ones stay for the product that reads them next): 36.6 -> 34.4 us
+// (5.9 TB/s; loads alone 36.3, stores alone 36.1), 4096 x 4096 12.5 -> 11.2, 1531 x 4096 5.9 -> 5.4.  A wave owns U * 64 consecutive
 // units, so that a workgroup writes whole lines of scale bytes, all loads of a thread are requested before the first is used,
 // and the blocks the hardware conversion does not serve (zero, subnormal, non-finite or extreme amax) are done again
 // by the general code from memory, outside of the loop.
@@ -192,11 +194,20 @@ __device__ __forceinline__ void quant_unpack(const v4i (&t)[SRC == MX_F32 ? 2 : 
   }
 }
 
-template <int SRC, int FMT, bool UP, int U>
+template <int SRC, int FMT, bool UP, int U, bool ONCE>
 __global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
   constexpr int NL = SRC == MX_F32 ? 2 : 1;          // 16-byte loads per unit of 8 elements
   constexpr int ESZ = SRC == MX_F32 ? 4 : 2;
   typedef short s2 __attribute__((ext_vector_type(2)));
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  auto load = [](const v4i* p) {
+    if constexpr (ONCE) return __builtin_nontemporal_load(p);
+    else return *p;
+  };
+  auto store = [](auto v, auto* p) {
+    if constexpr (U > 1) __builtin_nontemporal_store(v, p);
+    else *p = v;
+  };
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t units = (uint32_t)(q.rows * (q.K / 8)), upr = (uint32_t)(q.K / 8);   // (below 2^31: the launcher's rule)
   const uint32_t first = ((uint32_t)blockIdx.x * 4 + wave) * (U * 64);
@@ -217,8 +228,8 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
     const int64_t at = ((int64_t)row[u] * q.x_ld + (int64_t)col[u] * 8) * ESZ;
 #pragma unroll
     for (int h = 0; h < NL; ++h) {
-      t[u][h] = *(const v4i*)((const uint8_t*)q.x + at + 16 * h);
-      if constexpr (UP) t2[u][h] = *(const v4i*)((const uint8_t*)q.up + at + 16 * h);
+      t[u][h] = load((const v4i*)((const uint8_t*)q.x + at + 16 * h));
+      if constexpr (UP) t2[u][h] = load((const v4i*)((const uint8_t*)q.up + at + 16 * h));
     }
   }
   const bool floor_mode = q.scale_mode != 0;
@@ -268,7 +279,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
         r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, v[2], v[3], sc, 1);
         r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, v[4], v[5], sc, 2);
         r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, v[6], v[7], sc, 3);
-        *(uint32_t*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 4) = r;
+        store(r, (uint32_t*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 4));
       } else {
         uint32_t w[2];
 #pragma unroll
@@ -283,7 +294,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
           }
           w[h] = __builtin_bit_cast(uint32_t, r);
         }
-        *(uint2*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 8) = make_uint2(w[0], w[1]);
+        store((u2){w[0], w[1]}, (u2*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 8));
       }
       if ((lane & 3) == 0) q.scale[block] = (uint8_t)(se + 127);
     }
@@ -634,10 +645,12 @@ template <int SRC, int FMT>
 static void launch_quantize_rows(const QuantArgs& q, int64_t units, hipStream_t stream) {
   // four units per thread once that leaves every CU several waves per SIMD, else one (a single row is a few waves: the
   // launch is all latency).  The silu form holds two inputs per unit and computes for longer: two.
-#define MX_Q(UP, U) hipLaunchKernelGGL((quantize_rows_kernel<SRC, FMT, UP, U>), dim3((unsigned)((units + 256 * U - 1) / (256 * U))), dim3(256), 0, stream, q)
-  const bool large = units >= ((int64_t)1 << 20);
-  if (q.up) { if (large) MX_Q(true, 2); else MX_Q(true, 1); }
-  else { if (large) MX_Q(false, 4); else MX_Q(false, 1); }
+  // ONCE: inputs from 4 MiB of bf16 on are loaded non-temporally; smaller ones were mostly just written and are in L2 (24 x 14336
+  // in front of a product: 15.45 us for the pair, 15.7 with non-temporal loads).
+#define MX_Q(UP, U, ONCE) hipLaunchKernelGGL((quantize_rows_kernel<SRC, FMT, UP, U, ONCE>), dim3((unsigned)((units + 256 * U - 1) / (256 * U))), dim3(256), 0, stream, q)
+  const bool large = units >= ((int64_t)1 << 20), once = units >= ((int64_t)1 << 18);
+  if (q.up) { if (large) MX_Q(true, 2, true); else MX_Q(true, 1, false); }
+  else { if (large) MX_Q(false, 4, true); else if (once) MX_Q(false, 1, true); else MX_Q(false, 1, false); }
 #undef MX_Q
 }
 
