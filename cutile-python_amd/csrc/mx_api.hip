@@ -461,7 +461,9 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       const bool plain = ok && t128_plain_scales(as2.ptr, as2.stride[0], as2.stride[1], M, K, A->dtype, B->dtype) &&
                          t128_plain_scales(bs2.ptr, bs2.stride[1], bs2.stride[0], N, K, A->dtype, B->dtype) &&
                          bstride(As) % 4 == 0 && bstride(Bs) % 4 == 0;
+      const bool any = ok && !plain && t128_any_scales(as2.stride[0], as2.stride[1], M, K) && t128_any_scales(bs2.stride[1], bs2.stride[0], N, K);
       int64_t chunk = plain ? batch : (workspace ? workspace_bytes / per : 0);
+      if (any && chunk >= 1) chunk = batch;   // (reads the scales where they are; callers are held to the workspace all the same)
       if (chunk > 32768) chunk = 32768;
       if (ok && batch > 1) {   // few long products are better off one by one with K split, large ones gain nothing
         float alone = est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4);
@@ -487,9 +489,9 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
           g.lda = a2.stride[0]; g.ldb = b2.stride[1]; g.ldas = as2.stride[0]; g.ldbs = bs2.stride[1]; g.ldc = C->stride[1];
           g.M = (int32_t)M; g.N = (int32_t)N; g.K = (int32_t)K;
           g.a_fmt = A->dtype; g.b_fmt = B->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate;
-          g.a_plain = g.b_plain = plain;
+          g.a_plain = g.b_plain = plain ? 1 : any ? kT128ScalesAny : 0;
           g.batch = (int32_t)nb; g.k_splits = 1; g.a_rows = M;
-          if (!plain) {
+          if (!g.a_plain) {
             PackArgs pa, pb;
             mx_tensor t = bs2;
             t.shape[0] = bs2.shape[1]; t.shape[1] = bs2.shape[0];
@@ -707,8 +709,12 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     const bool b_can = o.b_scale_layout == MX_SCALE_2D &&
                        t128_plain_scales(Bs->ptr, Bs->stride[1], Bs->stride[0], N, K, A->dtype, B->dtype);
     g.a_plain = a_can; g.b_plain = a_can && b_can;
-    const bool pack_a = !a_can && !is_native(o.a_scale_layout), pack_b = !g.b_plain && !is_native(o.b_scale_layout);
-    if ((!a_can && !pack_a && o.a_scale_layout != MX_SCALE_NATIVE) || (!g.b_plain && !pack_b && o.b_scale_layout != MX_SCALE_NATIVE))
+    // (in place however the rows lie: the re-layout launch costs a small product a third of its time, mx_gemm_t128.hip)
+    if (!g.b_plain && o.a_scale_layout == MX_SCALE_2D && o.b_scale_layout == MX_SCALE_2D &&
+        t128_any_scales(As->stride[0], As->stride[1], M, K) && t128_any_scales(Bs->stride[1], Bs->stride[0], N, K))
+      g.a_plain = g.b_plain = kT128ScalesAny;
+    const bool pack_a = !g.a_plain && !is_native(o.a_scale_layout), pack_b = !g.b_plain && !is_native(o.b_scale_layout);
+    if ((!g.a_plain && !pack_a && o.a_scale_layout != MX_SCALE_NATIVE) || (!g.b_plain && !pack_b && o.b_scale_layout != MX_SCALE_NATIVE))
       return set_error(MX_ERR_LAYOUT, "kernel %d reads native-layout scales of kind %d (MX_SCALE_NATIVE for the "
                        "16x16x128-instruction kernels, MX_SCALE_NATIVE32 for pingpong32 / w4p); pass the matching "
                        "layout or the plain 2-D scales", kernel, MX_SCALE_NATIVE);

@@ -5,6 +5,8 @@
 
 namespace mx {
 
+constexpr int kT128ScalesAny = 2;   // a_plain, b_plain: rows at any byte
+
 struct T128Args {
   const uint8_t* A;        // [M rows][lda bytes], K contiguous
   const uint8_t* B;        // [N rows][ldb bytes]
@@ -17,7 +19,7 @@ struct T128Args {
   float* partial;          // k_splits > 1: fp32 partial products [split][M][N]
   int32_t M, N, K;
   int32_t a_fmt, b_fmt, c_dtype, accumulate;
-  int32_t a_plain, b_plain;
+  int32_t a_plain, b_plain;            // 0, 1, or kT128ScalesAny (both)
   int32_t batch, k_splits; // 1 each unless used
   // grouped (MoE) extension; sorted_token_ids == nullptr otherwise.  M is the number of slots.
   const int32_t* sorted_token_ids;
@@ -32,6 +34,11 @@ inline bool t128_plain_scales(const void* ptr, int64_t ld, int64_t k_stride, int
   const int stage = a_fmt == MX_E2M1 && b_fmt == MX_E2M1 ? 256 : 128;
   return k_stride == 1 && K % stage == 0 && ld % 4 == 0 && ((uintptr_t)ptr) % 4 == 0 && rows * ld < ((int64_t)1 << 31) &&
          (rows - 1) * ld + K / 32 < ((int64_t)1 << 31);
+}
+// ... and rows that it fetches dword by dword (kT128ScalesAny): K-contiguous, whatever their alignment and wherever K ends
+inline bool t128_any_scales(int64_t ld, int64_t k_stride, int64_t rows, int64_t K) {
+  const int64_t lim = ((int64_t)1 << 31) - 64;   // (the last quad's window reaches beyond its row)
+  return k_stride == 1 && K >= 32 && rows * ld < lim && (rows - 1) * ld + K / 32 < lim;
 }
 int launch_gemm_t128(const T128Args& g, hipStream_t stream);
 // any number of independent plain products of one element-format pair: one persistent launch per 32 of them

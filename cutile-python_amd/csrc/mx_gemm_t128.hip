@@ -16,7 +16,11 @@
 //
 // Scales: the native layout, or (a_plain / b_plain) the caller's K-contiguous rows as they are, 16 bytes of a row per
 // K-quad, of which a lane keeps its own byte of each K-step, four in one register, which the instruction's byte select
-// walks.  That saves small products the re-layout launch in front of them.
+// walks.  That saves small products the re-layout launch in front of them.  Rows at any byte (kScaleAny: K / 32 no multiple of
+// four in a dense tensor, or a K that ends inside a stage) cannot come by DMA: a wave's lanes fetch the five aligned dwords
+// around their 16 bytes, shift them into place, clear what lies beyond K and write them to the same LDS slots, a quad
+// ahead.  Six products 200 x 328 x 992 15.6 -> 11.9 us (re-layout
+// 4.5 us and the wait for it), a list of 24 of 96 .. 1536 42.2 -> 35.6.
 #include <type_traits>
 
 #include "mx_gemm_pp.h"
@@ -27,9 +31,14 @@
 namespace mx {
 namespace {
 
-template <class C, int NS, bool AP, bool BP, bool GROUPED>
+// where an operand's scales are: native layout; plain rows that the DMA can fetch; plain rows at any byte (both operands)
+constexpr int kScaleNative = 0, kScalePlain = 1, kScaleAny = 2;
+
+template <class C, int NS, int AS, int BS, bool GROUPED>
 __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem, const int pid, const int split, const int bz) {
   constexpr int KS = C::KSUB, SPQ = 4 / KS, MT = 4, NT = 4;
+  constexpr bool AP = AS != kScaleNative, BP = BS != kScaleNative, ANY = AS == kScaleAny;
+  static_assert(ANY == (BS == kScaleAny) && !(ANY && GROUPED), "");
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, gq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
@@ -136,6 +145,36 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
       sco = row0 / 64 < (rows + 63) / 64 ? (uint32_t)(row0 / 64 * KQ * 1024 + lane * 16) : kOobOffset;
     }
   }
+  // kScaleAny: the wave's group through registers
+  __amdgpu_buffer_rsrc_t rsAny;
+  uint32_t raw[5], shift = 0;
+  if constexpr (ANY) {
+    const bool is_b = wave >= 2;
+    const uintptr_t at = (uintptr_t)(is_b ? g.Bs + (int64_t)bz * g.bs_batch : g.As + (int64_t)bz * g.as_batch);
+    const uint32_t mis = (uint32_t)(at & 3);         // whole dwords: never more than 3 bytes either side of the tensor's own
+    rsAny = make_rsrc((const void*)(at - mis), (operand_bytes(is_b ? g.N : g.M, is_b ? g.ldbs : g.ldas, g.K / 32) + mis + 3) & ~3u);
+    if (sco != kOobOffset) {
+      shift = (sco + mis) & 3;
+      sco = (sco + mis) & ~3u;
+    }
+  }
+  auto load_any = [&](int Q) {
+    const uint32_t v = Q < q1 ? sco + Q * 16 : kOobOffset;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) raw[i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsAny, v + 4 * i, 0, 0);
+  };
+  auto store_any = [&](int Q) {
+    uint32_t d[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) d[t] = __builtin_amdgcn_alignbyte(raw[t + 1], raw[t], shift);
+    if (Q == KQ - 1) {                               // uniform: the next row's bytes are not this one's scales
+      const int left = g.K / 32 - 16 * Q;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) d[t] &= left >= 4 * t + 4 ? ~0u : left <= 4 * t ? 0u : (1u << (8 * (left - 4 * t))) - 1;
+    }
+    typedef __attribute__((address_space(3))) v4i lds_w4i;
+    *(lds_w4i*)(sbase + Q % (SD + 1) * SSLOT + wave * 1024 + lane * 16) = (v4i){(int)d[0], (int)d[1], (int)d[2], (int)d[3]};
+  };
   auto load_scales = [&](int Q) {
     lds_u8* const dst = sbase + Q % (SD + 1) * SSLOT + wave * 1024;
     const uint32_t v = Q < q1 ? sco : kOobOffset;
@@ -193,14 +232,20 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
   };
 
   // ---- prologue ---------------------------------------------------------------------------------------------------------
+  if constexpr (ANY) load_any(q0);
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
-    if (Sched::prologue_scales(k)) load_scales(q0 + k / SPQ);
+    if (!ANY && Sched::prologue_scales(k)) load_scales(q0 + k / SPQ);
     issue(s0 + k, k);
     __builtin_amdgcn_sched_barrier(0);   // the waits count on this order
   }
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(Sched::prologue_wait()));
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(ANY ? Sched::any_prologue_wait() : Sched::prologue_wait()));
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (ANY) {
+    store_any(q0);
+    load_any(q0 + 1);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
   asm volatile("s_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
   read_scales(q0);
@@ -220,12 +265,17 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
     const int s = Q * SPQ + t;
     if (s >= s1) return;              // uniform
     // stage s + 1 (requested NS - 1 iterations ago) has landed; younger are NS - 2 stages and the scales requested since
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(Sched::stage_wait(t)));
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(ANY ? Sched::any_stage_wait() : Sched::stage_wait(t)));
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (t == 0) {
-      load_scales(Q + SD);
+      if constexpr (ANY) {
+        store_any(Q + 1);             // requested a quad ago; the slot was last read two quads ago
+        load_any(Q + 2);
+      } else {
+        load_scales(Q + SD);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
     issue(s + NS, buf);
@@ -321,10 +371,10 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
   else store(std::integral_constant<int, 1>{});
 }
 
-template <class C, int NS, bool AP, bool BP, bool GROUPED>
+template <class C, int NS, int AS, int BS, bool GROUPED>
 __global__ __launch_bounds__(256, NS == 2 ? 2 : 1) void t128_kernel(const T128Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_generic[];
-  t128_tile<C, NS, AP, BP, GROUPED>(g, (lds_u8*)smem_generic, blockIdx.x, blockIdx.y, blockIdx.z);
+  t128_tile<C, NS, AS, BS, GROUPED>(g, (lds_u8*)smem_generic, blockIdx.x, blockIdx.y, blockIdx.z);
   __builtin_amdgcn_s_waitcnt(0x0F70);   // the trailing zero-fill DMA has left the queue before the LDS is given back
 }
 
@@ -334,7 +384,7 @@ struct ListProblem {
   const uint8_t* A; const uint8_t* B; const uint8_t* As; const uint8_t* Bs; void* C;
   int64_t lda, ldb, ldas, ldbs, ldc;
   int32_t M, N, K;
-  int16_t c_dtype, plain;              // plain: both operands' scales are read where they are
+  int16_t c_dtype, scales;             // kScale... of both operands
 };
 struct T128List {
   ListProblem p[kListMax];
@@ -359,8 +409,9 @@ __global__ __launch_bounds__(256, 2) void t128_list_kernel(const T128List gl) {
     g.M = q.M; g.N = q.N; g.K = q.K; g.c_dtype = q.c_dtype;
     g.k_splits = 1;
 #if defined(__HIP_DEVICE_COMPILE__)   // (the host pass, which needs the kernel's stub only, refuses the call)
-    if (q.plain) t128_tile<C, 2, true, true, false>(g, smem, t - gl.first_tile[i], 0, 0);
-    else t128_tile<C, 2, false, false, false>(g, smem, t - gl.first_tile[i], 0, 0);
+    if (q.scales == kScalePlain) t128_tile<C, 2, kScalePlain, kScalePlain, false>(g, smem, t - gl.first_tile[i], 0, 0);
+    else if (q.scales == kScaleAny) t128_tile<C, 2, kScaleAny, kScaleAny, false>(g, smem, t - gl.first_tile[i], 0, 0);
+    else t128_tile<C, 2, kScaleNative, kScaleNative, false>(g, smem, t - gl.first_tile[i], 0, 0);
 #endif
     // the tile's trailing (zero-fill) DMA has left the queue and every wave is done with the LDS stages before
     // the next tile's loads reuse them
@@ -369,9 +420,9 @@ __global__ __launch_bounds__(256, 2) void t128_list_kernel(const T128List gl) {
   }
 }
 
-template <class C, int NS, bool AP, bool BP, bool GROUPED>
+template <class C, int NS, int AS, int BS, bool GROUPED>
 int launch_one(const T128Args& g, hipStream_t stream) {
-  auto kern = t128_kernel<C, NS, AP, BP, GROUPED>;
+  auto kern = t128_kernel<C, NS, AS, BS, GROUPED>;
   constexpr int lds = NS * C::STAGE + ((NS + 4 / C::KSUB - 1) / (4 / C::KSUB) + 1) * 4096;
   static int attr_done = 0;   // benign race: the attribute call is idempotent
   if (!attr_done) {
@@ -412,15 +463,18 @@ template <int AF, int BF>
 int t128_pair(const T128Args& g, hipStream_t stream) {
   using C = Cfg<AF, BF, 128, 128, 2, 2>;
   if (g.sorted_token_ids)
-    return g.a_plain ? launch_one<C, 2, true, false, true>(g, stream) : launch_one<C, 2, false, false, true>(g, stream);
+    return g.a_plain ? launch_one<C, 2, kScalePlain, kScaleNative, true>(g, stream)
+                     : launch_one<C, 2, kScaleNative, kScaleNative, true>(g, stream);
   // (A packed with B plain does not occur: the entry points re-lay B first)
-  const bool ap = g.a_plain, bp = g.b_plain && ap;
   const int64_t wgs = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.k_splits * g.batch;
-  if (wgs <= 256)
-    return bp ? launch_one<C, 4, true, true, false>(g, stream) : ap ? launch_one<C, 4, true, false, false>(g, stream)
-                                                                    : launch_one<C, 4, false, false, false>(g, stream);
-  return bp ? launch_one<C, 2, true, true, false>(g, stream) : ap ? launch_one<C, 2, true, false, false>(g, stream)
-                                                                  : launch_one<C, 2, false, false, false>(g, stream);
+  auto depth = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    if (g.a_plain == kT128ScalesAny) return launch_one<C, NS, kScaleAny, kScaleAny, false>(g, stream);
+    return !g.a_plain   ? launch_one<C, NS, kScaleNative, kScaleNative, false>(g, stream)
+           : !g.b_plain ? launch_one<C, NS, kScalePlain, kScaleNative, false>(g, stream)
+                        : launch_one<C, NS, kScalePlain, kScalePlain, false>(g, stream);
+  };
+  return wgs <= 256 ? depth(std::integral_constant<int, 4>{}) : depth(std::integral_constant<int, 2>{});
 }
 template <int AF, int BF>
 int t128_list_pair(const T128Args* problems, int n, hipStream_t stream) {
@@ -433,7 +487,7 @@ int t128_list_pair(const T128Args* problems, int n, hipStream_t stream) {
       ListProblem& q = gl.p[gl.n];
       q.A = g.A; q.B = g.B; q.As = g.As; q.Bs = g.Bs; q.C = g.C;
       q.lda = g.lda; q.ldb = g.ldb; q.ldas = g.ldas; q.ldbs = g.ldbs; q.ldc = g.ldc;
-      q.M = g.M; q.N = g.N; q.K = g.K; q.c_dtype = (int16_t)g.c_dtype; q.plain = g.a_plain && g.b_plain;
+      q.M = g.M; q.N = g.N; q.K = g.K; q.c_dtype = (int16_t)g.c_dtype; q.scales = (int16_t)(g.a_plain && g.b_plain ? g.a_plain : kScaleNative);
       gl.first_tile[gl.n] = (int32_t)total;
       total += (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
       if (total > 0x7FFFFFFF) return set_error(MX_ERR_SHAPE, "gemm list: too many tiles");

@@ -27,6 +27,10 @@ struct T128Schedule {
     for (int back = 1; back <= NS - 2; ++back) n += (t + SPQ * NS - back) % SPQ == 0;
     return n;
   }
+  // Scales that come through registers are loads whose place and number the waits leave out: of the stages' loads alone,
+  // NS - 1 (NS - 2) stages are behind stage 0 (s + 1), so a wait for all but these is never too short.
+  static constexpr int any_prologue_wait() { return (NS - 1) * TL; }
+  static constexpr int any_stage_wait() { return (NS - 2) * TL; }
 };
 
 // First stage of a product of `stages` stages at which something is read that the waits do not cover, -1 if none.  -2: the
