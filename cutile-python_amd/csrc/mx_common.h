@@ -83,6 +83,11 @@ __device__ inline float decode_elem(uint32_t c, int fmt) {
 
 // Cache policy of a buffer load (its last operand) whose lines nothing reads again: non-temporal, evicted first.
 constexpr int kLoadOnce = 2;
+// Weights of a launch that are read that way: from 96 MB on.  Two such matrices do not fit into the 256 MB Infinity Cache with
+// what lies between, so that a loop over a model's layers finds none of their lines again, and the plain policy costs 7 - 10 %
+// (28672 x 8192 FP8, 8 rows, 45 -> 40 us; FP4, 32 rows, 25.9 -> 23.7).  Smaller ones gain as much where they come from memory
+// (14336 x 4096 FP8, 8 rows, 16.1 -> 14.7) and lose more where two or three of them take turns (11.5 -> 14.3).
+constexpr int64_t kLoadOnceBytes = (int64_t)96 << 20;
 
 // ---- fp32 -> bf16 bits, round to nearest even (torch's .to(bfloat16)) ---------------------------
 __device__ inline uint16_t f32_to_bf16(float f) {

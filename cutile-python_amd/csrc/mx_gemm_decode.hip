@@ -74,7 +74,8 @@ struct DecodeCfg {
 // rbase + j * RPI ... of the tile; lane offsets: row_off = (lane / LPR) * ldw, chunk_off = the lane's 16-byte
 // chunk position already XORed with its row inside the instruction (plus the K-slice's byte offset); the
 // instruction's first row enters the swizzle as one more XOR (rbase + RPI * j and lane / LPR share no bits).
-template <int SPW>
+// ONCE: W non-temporally (28672 x 8192 at 32 rows 25.7 -> 23.7 us; the scales as well: no gain).
+template <int SPW, bool ONCE>
 __device__ inline void issue_tile_dma2(const uint8_t* W, uint32_t wbytes, const uint8_t* S, uint32_t sbytes,
                                        lds_u8* wdst, lds_u8* sdst, uint32_t row_off, uint32_t chunk_off, int rbase,
                                        uint32_t soff, int wsoff, int ldw, int ssoff, bool with_scales,
@@ -85,9 +86,8 @@ __device__ inline void issue_tile_dma2(const uint8_t* W, uint32_t wbytes, const 
   for (int j = 0; j < Cf::WIW; ++j) {
     const int r0 = rbase + j * Cf::RPI;
     const uint32_t off = chunk_off ^ (uint32_t)((r0 & 15) << 4);     // byte of the row this lane fetches
-    // (non-temporal: 28672 x 8192 at 32 rows 25.7 -> 23.7 us, x 4096 at 8 rows 13.9 -> 13.3; the scales as well: no gain)
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, (lds_void*)(wdst + j * 1024), 16,
-                                             off < row_bytes ? row_off + off : kOob, wsoff + r0 * ldw, 0, kLoadOnce);
+                                             off < row_bytes ? row_off + off : kOob, wsoff + r0 * ldw, 0, ONCE ? kLoadOnce : 0);
   }
   if (with_scales)   // uniform per wave
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsS, (lds_void*)sdst, 16, soff, ssoff, 0, 0);
@@ -110,7 +110,7 @@ __device__ inline void issue_xs_dma(const uint8_t* Xs, uint32_t bytes, lds_u8* d
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)dst, 16, voff, soff, 0, 0);
 }
 
-template <int XF, int SPW, typename OutT>
+template <int XF, int SPW, typename OutT, bool ONCE>
 __global__ __launch_bounds__(kWaves * 64) void decode_kernel(const DecodeArgs d) {
   using Cf = DecodeCfg<SPW>;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_generic[];
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(const DecodeArgs d)
   auto issue = [&](int i, int slot) {          // this wave's share of local tile i
     const int tile = t_first + i * G;
     lds_u8* const base = smem + slot * Cf::SLOT;
-    issue_tile_dma2<SPW>(d.W, wbytes, d.Ws, sbytes, base + q * (16 * Cf::SLB) + mh * Cf::WIW * 1024,
+    issue_tile_dma2<SPW, ONCE>(d.W, wbytes, d.Ws, sbytes, base + q * (16 * Cf::SLB) + mh * Cf::WIW * 1024,
                          base + Cf::W_BYTES + wave * 1024, row_off, chunk_off, mh * Cf::WIW * Cf::RPI, soff,
                          tile * 16 * (int)d.ldw, (int)d.ldw, tile * 16 * (int)d.ldws, with_scales, (uint32_t)(d.K / 2));
   };
@@ -333,10 +333,10 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(const DecodeArgs d)
   if (wave < 2) reduce_store(t_count - 1);
 }
 
-template <int XF, int SPW, typename OutT>
+template <int XF, int SPW, typename OutT, bool ONCE>
 int launch_decode_k(const DecodeArgs& d, int grid, hipStream_t stream) {
   using Cf = DecodeCfg<SPW>;
-  auto kern = decode_kernel<XF, SPW, OutT>;
+  auto kern = decode_kernel<XF, SPW, OutT, ONCE>;
   static int attr_done = 0;   // benign race: the attribute call is idempotent
   if (!attr_done) {
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cf::LDS_BYTES);
@@ -350,13 +350,13 @@ int launch_decode_k(const DecodeArgs& d, int grid, hipStream_t stream) {
   return MX_OK;
 }
 
-template <int XF>
+template <int XF, bool ONCE>
 int launch_decode_x(const DecodeArgs& d, int grid, hipStream_t stream) {
   if (d.K > 4096)
-    return d.c_dtype == MX_F32 ? launch_decode_k<XF, 16, float>(d, grid, stream)
-                               : launch_decode_k<XF, 16, uint16_t>(d, grid, stream);
-  return d.c_dtype == MX_F32 ? launch_decode_k<XF, 8, float>(d, grid, stream)
-                             : launch_decode_k<XF, 8, uint16_t>(d, grid, stream);
+    return d.c_dtype == MX_F32 ? launch_decode_k<XF, 16, float, ONCE>(d, grid, stream)
+                               : launch_decode_k<XF, 16, uint16_t, ONCE>(d, grid, stream);
+  return d.c_dtype == MX_F32 ? launch_decode_k<XF, 8, float, ONCE>(d, grid, stream)
+                             : launch_decode_k<XF, 8, uint16_t, ONCE>(d, grid, stream);
 }
 
 }  // namespace
@@ -378,7 +378,9 @@ int launch_gemm_decode(const DecodeArgs& d, hipStream_t stream) {
   const int tiles = d.N / 16;
   const int grid = tiles < 256 ? tiles : 256;
   if (grid == 0) return MX_OK;
-  return d.x_fmt == MX_E4M3 ? launch_decode_x<MX_E4M3>(d, grid, stream) : launch_decode_x<MX_E5M2>(d, grid, stream);
+  if (d.N * d.ldw >= kLoadOnceBytes)
+    return d.x_fmt == MX_E4M3 ? launch_decode_x<MX_E4M3, true>(d, grid, stream) : launch_decode_x<MX_E5M2, true>(d, grid, stream);
+  return d.x_fmt == MX_E4M3 ? launch_decode_x<MX_E4M3, false>(d, grid, stream) : launch_decode_x<MX_E5M2, false>(d, grid, stream);
 }
 
 }  // namespace mx

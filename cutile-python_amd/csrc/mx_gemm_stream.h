@@ -29,7 +29,8 @@
 namespace mx {
 
 // UP: the four tiles of a wave are 32 rows of the gate half of W and the 32 rows of the up half that belong to them.
-template <int XF_, int WF_, int NT_, int MT_, bool PACKED_, int WAVES_ = 8, bool UP_ = false>
+// ONCE: W is read non-temporally (kLoadOnceBytes).
+template <int XF_, int WF_, int NT_, int MT_, bool PACKED_, int WAVES_ = 8, bool UP_ = false, bool ONCE_ = false>
 struct StreamCfg {
   static constexpr int XF = XF_, WF = WF_, NT = NT_, MT = MT_, WAVES = WAVES_;
   static constexpr bool PACKED = PACKED_, UP = UP_;
@@ -38,10 +39,12 @@ struct StreamCfg {
   static constexpr int SPQ = 4 / SK;                      // stages per K-quad
   static constexpr int WEB = WF == MX_E2M1 ? 4 : 8;
   static constexpr int L = 2 * MT * SK + 2 * NT;          // load instructions per stage
-  // W is read non-temporally where a wave streams whole 64-row groups: 8 experts of 4096 x 14336, 12 rows each, up + down
-  // projection FP8 257 -> 226 us (5.7 -> 6.4 TB/s), FP4 149 -> 136; 28672 x 8192 FP8, 16 rows 45.2 -> 40.9.  Narrow units (one
-  // or two tiles, which split K over more waves) gain nothing, and 4096 x 14336 FP8 at 24 rows loses: 18.1 -> 19.9.
-  static constexpr int W_POLICY = NT == 4 ? kLoadOnce : 0;
+  // For units of whole 64-row groups: 8 experts of 4096 x 14336, 12 rows each, up + down projection FP8 257 -> 226 us (5.7 -> 6.4
+  // TB/s), FP4 149 -> 136; 28672 x 8192 FP8, 16 rows 45.2 -> 40.9.  Narrow units (one or two tiles, which split K over more
+  // waves) gain nothing, and 4096 x 14336 FP8 at 24 rows loses: 18.1 -> 19.9.  (Instances of their own: both kinds of load in
+  // one kernel cost small layers 5 % in instruction fetches.)
+  static constexpr int W_POLICY = ONCE_ ? kLoadOnce : 0;
+  static_assert(!ONCE_ || NT == 4, "");
   static constexpr int NSC = MT + NSW;      // scale load instructions per K-quad
   static constexpr int XSLOT = MT * SK * 2048;            // LDS bytes of one stage of X
   // tiles of W re-sorted at a time (one where that lets two workgroups of four waves share a CU's LDS)
