@@ -87,28 +87,32 @@ int plan_k_splits(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
 
 
 // What MX_KERNEL_AUTO weighs beyond kStreamAutoM rows: estimated time (us) of a product on the kernels that can run it.
-// Fitted to measurements of 96 .. 4096 rows x 512 .. 17456 columns x 512 .. 9216 (stages of 128 bytes of a row):
-//   128 x 128 tiles: 0.62 us per stage with one tile on a CU (1024 x 4096 x 4096 24.6 us, 2048 x 2048 x 8192 45 us), 0.97
-//     with two (2048 x 4096 x 4096 36.7 us); FP4 x FP4 0.68 / 1.2.  Split along K: the partial sums are written and read.
-//   256 x 256 tiles: 1.1 us per stage when they leave half of the CUs idle, else 1.45 (1531 x 14336 x 4096: two rounds, 92 us;
-//     4009 x 3171 x 3072: one, 44 us); FP4 1.3 / 1.8; it needs re-laid scales.
+// Fitted to measurements of 96 .. 4096 rows x 512 .. 28672 columns x 512 .. 9216 (stages of 128 bytes of a row, launches
+// back to back, MXFP8; FP4 x FP4 has constants of its own):
+//   128 x 128 tiles: 0.62 us per stage with one tile on a CU (1024 x 4096 x 4096 24.6 us, 2048 x 2048 x 8192 45 us), then by
+//     their number (2048 x 4096 x 4096 40, 1531 x 14336 x 4096 95).  Split along K: the partial sums are written and read.
+//   256 x 256 tiles: a round's length and, as the clock falls the busier the chip is, its share of tiles (4096^3, one full
+//     round, 50; 2048 x 4096 x 4096, half of one, 44; 1531 x 14336 x 4096, 1.31 rounds, 86); it needs re-laid scales.
+//   192 x 256 tiles: a round of them is 18 % shorter for 25 % fewer rows (more of a stage is not MFMA), which pays where it
+//     fills rounds that 256 rows leave half empty (1531 x 14336 x 4096, 1.75 rounds, 77; 3000 x 4096 x 4096 42 against 45;
+//     but 4096 x 14336 x 4096 187 against 175).
 //   streaming: 0.57 us per unit of its own cost estimate (256 x 14336 x 4096 40 us, 1024 x 4096 x 8192 60 us).
 float est_t128(int64_t M, int64_t N, int64_t K, int S, bool fp4, int64_t batch = 1) {
   const int64_t wgs = ((M + 127) / 128) * ((N + 127) / 128) * S * batch;
-  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)) / S;
-  float t = 5.f + st * (wgs <= 256 ? (fp4 ? 0.68f : 0.62f) : (fp4 ? 1.2f : 0.97f) * ((wgs + 511) / 512));
+  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)) / S, fill = wgs < 435 ? 0.85f : wgs / 512.f;
+  float t = 5.f + st * (wgs <= 256 ? (fp4 ? 0.68f : 0.62f) : 0.1f + (fp4 ? 1.25f : 1.05f) * fill);
   if (S > 1) t += 4.f + (float)S * M * N * 8 / 4e6f;
   return t;
 }
-float est_pp(int64_t M, int64_t N, int64_t K, bool fp4, bool pack, bool tail) {
-  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)), per = fp4 ? 1.8f : 1.45f;
-  const float rest = 8.f + (pack ? 5.f : 0.f);
+float est_pp(int64_t M, int64_t N, int64_t K, bool fp4, bool pack, bool tail, int rows = 256) {
+  const int64_t tiles = ((M + rows - 1) / rows) * ((N + 255) / 256);
+  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)), rest = 6.f + (pack ? 5.f : 0.f);
+  const float round = rows == 256 ? (fp4 ? 1.14f : 0.95f) : (fp4 ? 0.80f : 0.79f), full = rows == 256 ? (fp4 ? 0.75f : 0.47f) : (fp4 ? 0.70f : 0.35f);
   if (tail) {   // the last round split S ways, its partial sums added up by a second launch
     const int left = (int)((tiles % 256 + 7) / 8), KQ = (int)(K / 512), S = tail_splits(left, 32, KQ, fp4);
-    if (S > 1) return rest + st * per * (tiles / 256) + tail_tenths(S, left, 32, KQ, fp4) * 0.1f;
+    if (S > 1) return rest + st * (round + full) * (tiles / 256) + tail_tenths(S, left, 32, KQ, fp4) * 0.1f;
   }
-  return rest + st * (tiles <= 128 ? (fp4 ? 1.3f : 1.1f) : per * ((tiles + 255) / 256));
+  return rest + st * (round * ((tiles + 255) / 256) + full * tiles / 256);
 }
 float est_stream(int64_t M, int64_t N, int64_t K, int w_fmt) { return 5.f + 0.57f * stream_plan(M, N, K, w_fmt).cost; }
 
@@ -563,7 +567,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     why_stream = stream_issue(sa);
   }
 
-  int kernel = o.kernel;
+  int kernel = o.kernel, tile_rows = 256;
   if (kernel == MX_KERNEL_DECODE && K > kDecodeMaxK && M <= kDecodeMaxM && N % 16 == 0 && K % 512 == 0 && !why_stream &&
       o.b_scale_layout == MX_SCALE_2D && B->dtype == MX_E2M1)
     kernel = MX_KERNEL_STREAM;   // beyond what the decode kernel keeps of X in registers
@@ -587,7 +591,11 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       const float t128 = est_t128(M, N, K, o.split_k > 1 ? 1 : plan_k_splits(M, N, K, o), fp4);
       const bool room = workspace && o.split_k == 0 && pp_tail_bytes(M, N, K, fp4, true) > 0 &&
                         workspace_bytes >= ws_min + pp_tail_bytes(M, N, K, fp4, true);
-      const float pp = o.split_k > 1 ? 1e30f : est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), room);
+      float pp = o.split_k > 1 ? 1e30f : est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), room);
+      if (o.split_k <= 1) {
+        const float pp192 = est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), false, 192);
+        if (big_tile_kernel() == MX_KERNEL_MFMA_PINGPONG && pp192 < pp) { pp = pp192; tile_rows = 192; }
+      }
       const float st = may_stream ? est_stream(M, N, K, B->dtype) : 1e30f;
       kernel = st < t128 && st < pp ? MX_KERNEL_STREAM : t128 <= pp ? MX_KERNEL_MFMA_128x128 : big_tile_kernel();
     }
@@ -822,9 +830,10 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
   g.a_fmt = A->dtype; g.b_fmt = B->dtype; g.c_dtype = C->dtype; g.accumulate = o.accumulate;
   g.a_rows = M;
   g.replicas = 1;
+  g.tile_rows = tile_rows;
   if (kernel == MX_KERNEL_MFMA_PINGPONG && o.split_k == 0 && workspace && ((uintptr_t)workspace) % 256 == 0) {
     const int64_t tail = pp_tail_bytes(M, N, K, A->dtype == MX_E2M1 && B->dtype == MX_E2M1, true);
-    if (tail > 0 && workspace_bytes >= need + tail) g.tail = (float*)((uint8_t*)workspace + need);
+    if (tail > 0 && tile_rows == 256 && workspace_bytes >= need + tail) g.tail = (float*)((uint8_t*)workspace + need);
   }
   return launch_gemm_mfma(g, kernel, (hipStream_t)stream);
 }

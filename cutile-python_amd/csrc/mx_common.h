@@ -121,6 +121,7 @@ struct GemmArgs {
   int64_t bs_expert_stride;  // dwords between experts in Bs
   int64_t a_rows;            // rows of the A tensor (for the buffer descriptor)
   const int32_t* num_slots;  // grouped, may be null: slots in use (on the device); tiles beyond them are not walked
+  int32_t tile_rows;         // ping-pong kernel, plain products: 192, else 256
   float* tail;               // ping-pong kernel, may be null: partial sums of tiles split along K (pp_tail_bytes)
   // split-K (one-tile kernels only): K is the slice length, slice i reads the scales / writes the partial
   // output i strides further on

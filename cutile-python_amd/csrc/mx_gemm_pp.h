@@ -10,13 +10,12 @@ constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 
 template <class C>
 struct PP {
-  static_assert(C::BM == 256 && C::BN == 256, "ping-pong kernel is 256 x 256");
+  static_assert((C::BM == 256 || C::BM == 192) && C::BN == 256, "ping-pong kernel is 256 (192) x 256");
   static constexpr int A_BUFS = 3, B_BUFS = 2;
-  static constexpr int A_HALF = 128 * C::A_RB;              // bytes of one team's rows in an A buffer
   static constexpr int B_BASE = A_BUFS * C::A_STAGE;
   static constexpr int LDS_BYTES = B_BASE + B_BUFS * C::B_STAGE;
   static constexpr int A_RPI = 64 / C::A_CPR, B_RPI = 64 / C::B_CPR;   // rows per DMA instruction
-  static constexpr int AL = 128 / A_RPI / 4;                // A loads per wave and stage
+  static constexpr int AL = C::WTM / A_RPI / 4;              // A loads per wave and stage
   static constexpr int BL = 64 / B_RPI;                     // B loads per team-1 wave and stage
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 };
@@ -30,13 +29,14 @@ struct TileWalk {
   int first, step, end, tiles_m, tiles_n;
   int tail = kNoTile;
   int quads = 0;   // of the tail: first K-quad | number << 16
+  template <int ROWS = 256>   // of a tile
   __device__ void origin(int lid, int& m0, int& n0) const {
     constexpr int GM = 4;   // measured: 4 rows is 1 - 3 % faster than 8 (2, 3, 6, 16 are slower than either)
     const int in_group = GM * tiles_n;
     const int gid = lid / in_group, first_m = gid * GM;
     const int gsz = (tiles_m - first_m) < GM ? (tiles_m - first_m) : GM;
     const int in = lid % in_group;
-    m0 = (first_m + in % gsz) * 256;
+    m0 = (first_m + in % gsz) * ROWS;
     n0 = (in / gsz) * 256;
   }
   // the walk including the tail tile: kNoTile after the last one
@@ -72,9 +72,9 @@ __host__ __device__ inline int tail_splits(int rest, int wgs, int KQ, bool fp4) 
   return S;
 }
 
-__device__ inline TileWalk make_tile_walk(int M, int N) {
+__device__ inline TileWalk make_tile_walk(int M, int N, int rows = 256) {
   TileWalk walk;
-  walk.tiles_m = (M + 255) / 256;
+  walk.tiles_m = (M + rows - 1) / rows;
   walk.tiles_n = (N + 255) / 256;
   const XcdShare x = xcd_share(walk.tiles_m * walk.tiles_n, gridDim.x, blockIdx.x & 7);
   walk.step = x.wgs;
@@ -111,8 +111,8 @@ inline int num_cus() {
 
 // grid of a persistent ping-pong launch: one workgroup per CU walking several tiles when the stage pipeline can
 // run across tile boundaries (at least two stages per tile, whole K-quads); otherwise one workgroup per tile
-inline int64_t pp_grid(int M, int N, int K, int ksub) {
-  const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
+inline int64_t pp_grid(int M, int N, int K, int ksub, int rows = 256) {
+  const int64_t tiles = (int64_t)((M + rows - 1) / rows) * ((N + 255) / 256);
   const int ksteps = (K + 127) / 128;
   const int nstages = (ksteps + ksub - 1) / ksub;
   const bool can_walk = nstages >= 2 && ksteps % 4 == 0;

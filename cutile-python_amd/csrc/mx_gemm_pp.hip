@@ -56,8 +56,11 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   // 8 MFMAs ahead of their use.  Two measured best (four: 1.5 % slower on MXFP8, 5 % on the grouped
   // variant: the longer memory phase costs more than the later reads)
   constexpr int EARLY = 2;
+  constexpr int MT = C::MT;          // A tiles of a wave: 8 (6 with tiles of 192 rows)
   const int r = lane & 15, gq = lane >> 4;
-  constexpr int wm0 = TEAM * 128;
+  constexpr int wm0 = TEAM * C::WTM;
+  constexpr int at0 = wm0 % 64 / 16; // the first one's place in its 64-row scale group
+  static_assert(MT == 8 || !(GROUPED || SPLIT), "");
   const int wn0 = wn * 64;
 
   const int Kb_a = g.K * C::A_EB / 8, Kb_b = g.K * C::B_EB / 8;
@@ -110,7 +113,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
     kq_nxt = part ? walk.quads >> 16 : KQ;
     const uint32_t ka0 = (uint32_t)(qb * SPQ * C::A_RB), kb0 = (uint32_t)(qb * SPQ * C::B_RB);
     int m0 = 0, n0 = 0;
-    if (fetch_valid) walk.origin(lid, m0, n0);
+    if (fetch_valid) walk.origin<C::BM>(lid, m0, n0);
     if constexpr (GROUPED) {
       skip_nxt = false;
       if (fetch_valid) {
@@ -193,9 +196,9 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
     }
   };
 
-  v4f acc[8][4];
+  v4f acc[MT][4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
   const int swa = swz<C::A_CPR>(r), swb = swz<C::B_CPR>(r);
@@ -211,10 +214,10 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   auto write_tile = [&](int m0, int n0) {
     if constexpr (!GROUPED) {
       // interior tile, plain store: one address per lane, everything else immediate offsets
-      if (m0 + 256 <= g.M && n0 + 256 <= g.N && vec8_ok && !accumulate) {
+      if (m0 + C::BM <= g.M && n0 + 256 <= g.N && vec8_ok && !accumulate) {
         OutT* p = Cp + (int64_t)(m0 + wm0 + r) * g.ldc + (n0 + wn0 + 8 * gq);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < MT; ++i) {
 #pragma unroll
           for (int jp = 0; jp < 2; ++jp) {
             store8_full<OutT>(p + 32 * jp, acc[i][2 * jp], acc[i][2 * jp + 1]);
@@ -232,7 +235,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
       OutT* p = Cp + (int64_t)(m0 + wm0 + r) * g.ldc + (n0 + wn0 + 8 * gq);
       const int rows = g.M - (m0 + wm0 + r), cols = g.N - (n0 + wn0 + 8 * gq);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < MT; ++i) {
         if (16 * i < rows) {
 #pragma unroll
           for (int jp = 0; jp < 2; ++jp) {
@@ -256,7 +259,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
         if (eid[u] >= 0 && eid[u] < g.num_valid_ids) ewt[u] = g.topk_weights[eid[u]];
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < MT; ++i) {
       const int src = (16 * (i & 3) + r) * 4;
       const int id = __builtin_amdgcn_ds_bpermute(src, eid[i >> 2]);
       const bool ok = id >= 0 && id < g.num_valid_ids;
@@ -300,7 +303,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   set_fetch_tile(lid);
   {
     int fm0, fn0;
-    walk.origin(lid, fm0, fn0);
+    walk.origin<C::BM>(lid, fm0, fn0);
     load_row_ids(fm0);
   }
   kq = kq_nxt;
@@ -337,10 +340,10 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
         int plid = before(lid);   // (always a whole tile: a split one is the last of the walk)
         asm volatile("" : "+s"(plid));
         int pm0, pn0;
-        walk.origin(plid, pm0, pn0);
+        walk.origin<C::BM>(plid, pm0, pn0);
         write_tile(pm0, pn0);
         if constexpr (GROUPED) {
-          walk.origin(lid, pm0, pn0);
+          walk.origin<C::BM>(lid, pm0, pn0);
           load_row_ids(pm0);
         }
       }
@@ -353,7 +356,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
     lds_u8* const atile = smem + abuf * C::A_STAGE + (wm0 + r) * C::A_RB;
     lds_u8* const btile = smem + P::B_BASE + bbuf * C::B_STAGE + (wn0 + bperm_lane_off(r)) * C::B_RB;
     issue_a(sl_eff, abuf2);
-    v8i bf[C::KSUB][4], af[C::KSUB][8];
+    v8i bf[C::KSUB][4], af[C::KSUB][MT];
     if (!(GROUPED && skip_cur)) {
       // B tiles 0, 1 (rows 0 .. 31 of the wave's 64), then tiles 2, 3, then the early A tiles: LDS returns reads in
       // order, so the DMA that refills the first half of the B rows can go as soon as the first group is back
@@ -408,8 +411,8 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
         for (int i = i0; i < i0 + n; ++i) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            acc[i][j] = mfma_scaled<C::BF, C::AF>(bf[kk][j], af[kk][i], acc[i][j], j, sb[t0 + kk], i % 4,
-                                                  sa[i / 4][t0 + kk]);
+            acc[i][j] = mfma_scaled<C::BF, C::AF>(bf[kk][j], af[kk][i], acc[i][j], j, sb[t0 + kk], (at0 + i) % 4,
+                                                  sa[(at0 + i) / 4][t0 + kk]);
           }
         }
       }
@@ -418,7 +421,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
     // A tiles below EARLY were read in the memory phase; the rest is read EARLY * 4 MFMAs ahead of use
     if (!(GROUPED && skip_cur)) {
 #pragma unroll
-      for (int ip = 0; ip < 8; ip += 2) {
+      for (int ip = 0; ip < MT; ip += 2) {
         if (ip == 0) {
           // the phase opens with MFMAs, not with LDS read issue: the matrix pipe restarts that much sooner after the
           // hand-over, and the reads issue while the first MFMAs run
@@ -427,7 +430,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
           mfma_pair(1, 1);
           continue;
         }
-        if (ip + EARLY < 8) read_pair(ip + EARLY);
+        if (ip + EARLY < MT) read_pair(ip + EARLY);
         mfma_pair(ip);
       }
     }
@@ -460,13 +463,13 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   __builtin_amdgcn_sched_barrier(0);
   if (!SPLIT || walk.tail == kNoTile) {
     int pm0, pn0;
-    walk.origin(SPLIT ? walk.first + (walk.end - 1 - walk.first) / walk.step * walk.step : lid - walk.step, pm0, pn0);
+    walk.origin<C::BM>(SPLIT ? walk.first + (walk.end - 1 - walk.first) / walk.step * walk.step : lid - walk.step, pm0, pn0);
     write_tile(pm0, pn0);
   } else {
     // partial sums, as the lanes hold them: 1 KiB per store instruction
     v4f* const t = (v4f*)g.tail + ((int64_t)blockIdx.x * 8 + TEAM * 4 + wn) * 32 * 64 + lane;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) t[(i * 4 + j) * 64] = acc[i][j];
   }
@@ -488,7 +491,7 @@ template <class C, bool GROUPED, bool SPLIT>
 __device__ __forceinline__ TileWalk pp_walk(const GemmArgs& g) {
   const int M = pp_rows<GROUPED>(g);
   if constexpr (SPLIT) return make_split_walk(M, g.N, g.K / 512, C::KSUB == 2);
-  else return make_tile_walk(M, g.N);
+  else return make_tile_walk(M, g.N, C::BM);
 }
 
 template <class C, typename OutT, bool GROUPED, bool SPLIT>
@@ -575,7 +578,7 @@ int launch_pp(const GemmArgs& g, hipStream_t stream) {
                        hipGetErrorString(e));
     attr_done = 1;
   }
-  int64_t grid = pp_grid(g.M, g.N, g.K, C::KSUB);
+  int64_t grid = pp_grid(g.M, g.N, g.K, C::KSUB, C::BM);
   if (grid <= 0) return MX_OK;
   if (SPLIT) grid = num_cus();   // idle workgroups of a single, partly filled round take part too
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), PP<C>::LDS_BYTES, stream, g);
@@ -603,6 +606,10 @@ int launch_pp_pair(const GemmArgs& g, hipStream_t stream) {
       return grouped ? launch_pp<C, float, true, S>(g, stream) : launch_pp<C, float, false, S>(g, stream);
     return grouped ? launch_pp<C, uint16_t, true, S>(g, stream) : launch_pp<C, uint16_t, false, S>(g, stream);
   };
+  if (g.tile_rows == 192 && !grouped) {
+    using C192 = Cfg<AF, BF, 192, 256, 2, 4>;
+    return g.c_dtype == MX_F32 ? launch_pp<C192, float, false, false>(g, stream) : launch_pp<C192, uint16_t, false, false>(g, stream);
+  }
   return g.tail ? run(std::true_type{}) : run(std::false_type{});
 }
 #if MX_PP_PAIR == 0
