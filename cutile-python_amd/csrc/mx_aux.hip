@@ -642,7 +642,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 }  // namespace
 
 template <int SRC, int FMT>
-static void launch_quantize_rows(const QuantArgs& q, int64_t units, hipStream_t stream) {
+static hipError_t launch_quantize_rows(const QuantArgs& q, int64_t units, hipStream_t stream) {
   // four units per thread once that leaves every CU several waves per SIMD, else one (a single row is a few waves: the
   // launch is all latency).  The silu form holds two inputs per unit and computes for longer: two.
   // ONCE: the input is loaded non-temporally.  Where it comes from memory that is as fast or faster at every size; where it was
@@ -650,7 +650,7 @@ static void launch_quantize_rows(const QuantArgs& q, int64_t units, hipStream_t 
   // 30.2 -> 33.7 us) and below 8 MB (24 x 14336 in front of a product: 15.45 us for the pair, 15.7; 244 x 13440 39.0, 39.3).  So:
   // inputs of 8 .. 16 MB (bf16; 1531 x 4096 5.9 -> 5.4 us, with the product behind it 101 -> 98.4), and those that the cache
   // cannot hold.
-#define MX_Q(UP, U, ONCE) hipLaunchKernelGGL((quantize_rows_kernel<SRC, FMT, UP, U, ONCE>), dim3((unsigned)((units + 256 * U - 1) / (256 * U))), dim3(256), 0, stream, q)
+#define MX_Q(UP, U, ONCE) return launch_kernel(quantize_rows_kernel<SRC, FMT, UP, U, ONCE>, dim3((unsigned)((units + 256 * U - 1) / (256 * U))), dim3(256), 0, stream, q)
   const bool large = units >= ((int64_t)1 << 20), mid = units >= ((int64_t)1 << 19);
   const bool beyond = units * 8 * (SRC == MX_F32 ? 4 : 2) >= kLoadOnceBytes;
   if (q.up) { if (large) MX_Q(true, 2, false); else MX_Q(true, 1, false); }
@@ -668,9 +668,10 @@ int launch_quantize(const QuantArgs& q, hipStream_t stream) {
   const int esz = q.x_dtype == MX_F32 ? 4 : 2, cb = q.fmt == MX_E2M1 ? 4 : 8;
   const bool rows_ok = q.K % 32 == 0 && units < ((int64_t)1 << 31) && (((uintptr_t)q.x | (uintptr_t)q.up | (uintptr_t)(q.x_ld * esz)) & 15) == 0 &&
                        (((uintptr_t)q.xq | (uintptr_t)q.xq_ld) & (cb - 1)) == 0;
+  hipError_t e = hipSuccess;
   if (rows_ok) {
 #define MX_CASE(SRC, FMT) \
-    if (q.x_dtype == SRC && q.fmt == FMT) launch_quantize_rows<SRC, FMT>(q, units, stream);
+    if (q.x_dtype == SRC && q.fmt == FMT) e = launch_quantize_rows<SRC, FMT>(q, units, stream);
     MX_CASE(MX_BF16, MX_E4M3)
     MX_CASE(MX_BF16, MX_E5M2)
     MX_CASE(MX_BF16, MX_E2M1)
@@ -682,9 +683,8 @@ int launch_quantize(const QuantArgs& q, hipStream_t stream) {
     MX_CASE(MX_F16, MX_E2M1)
 #undef MX_CASE
   } else {
-    hipLaunchKernelGGL(quantize_kernel<kQuantEpl>, dim3((unsigned)blocks), dim3(256), 0, stream, q);
+    e = launch_kernel(quantize_kernel<kQuantEpl>, dim3((unsigned)blocks), dim3(256), 0, stream, q);
   }
-  hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "quantize_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }
@@ -705,8 +705,7 @@ int launch_pack_scales_pair(const PackArgs* a, const PackArgs* b, hipStream_t st
   const int64_t total = blocks[0] + blocks[1];
   if (total > 0x7FFFFFFF) return set_error(MX_ERR_SHAPE, "pack_scales: tensor too large");
   pp.blocks0 = (int32_t)blocks[0];
-  hipLaunchKernelGGL(pack_scales_kernel, dim3((unsigned)total), dim3(256), 0, stream, pp);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(pack_scales_kernel, dim3((unsigned)total), dim3(256), 0, stream, pp);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "pack_scales_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }
@@ -728,8 +727,7 @@ int launch_pack_scales_list(const PackArgs* list, int n, hipStream_t stream) {
     }
     if (pl.n == 0) continue;
     pl.first_block[pl.n] = (int32_t)total;
-    hipLaunchKernelGGL(pack_scales_list_kernel, dim3((unsigned)total), dim3(256), 0, stream, pl);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_kernel(pack_scales_list_kernel, dim3((unsigned)total), dim3(256), 0, stream, pl);
     if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "pack_scales_list_kernel launch: %s", hipGetErrorString(e));
   }
   return MX_OK;
@@ -743,9 +741,8 @@ int launch_splitk_reduce(const float* partials, int splits, int64_t M, int64_t N
                          int c_dtype, int accumulate, hipStream_t stream) {
   const int64_t threads = M * ((N + 3) / 4);
   if (threads <= 0) return MX_OK;
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, partials,
-                     splits, M, N, C, ldc, c_dtype, accumulate);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(splitk_reduce_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, partials,
+                               splits, M, N, C, ldc, c_dtype, accumulate);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "splitk_reduce_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }
@@ -785,14 +782,12 @@ int launch_moe_align(const void* ids, int ids64, int64_t num_ids, int32_t num_ex
     attr_done = 1;
   }
   if (blocks > 1) {
-    hipLaunchKernelGGL(moe_hist_kernel, dim3((unsigned)blocks), dim3(kAlignThreads), (size_t)num_experts * sizeof(int32_t),
-                       stream, topk_ids, id_shift, num_ids, num_experts, chunk, counts);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_kernel(moe_hist_kernel, dim3((unsigned)blocks), dim3(kAlignThreads), (size_t)num_experts * sizeof(int32_t),
+                                 stream, topk_ids, id_shift, num_ids, num_experts, chunk, counts);
     if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_hist_kernel launch: %s", hipGetErrorString(e));
   }
-  hipLaunchKernelGGL(moe_place_kernel, dim3((unsigned)blocks), dim3(kAlignThreads), lds, stream, topk_ids, id_shift, num_ids,
-                     num_experts, tile_m, chunk, counts, sorted_token_ids, sorted_expert_ids, num_slots_out, max_slots);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(moe_place_kernel, dim3((unsigned)blocks), dim3(kAlignThreads), lds, stream, topk_ids, id_shift, num_ids,
+                               num_experts, tile_m, chunk, counts, sorted_token_ids, sorted_expert_ids, num_slots_out, max_slots);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_place_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }

@@ -344,8 +344,7 @@ int launch_decode_k(const DecodeArgs& d, int grid, hipStream_t stream) {
       return set_error(MX_ERR_LAUNCH, "hipFuncSetAttribute(%d bytes LDS): %s", Cf::LDS_BYTES, hipGetErrorString(e));
     attr_done = 1;
   }
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(kWaves * 64), Cf::LDS_BYTES, stream, d);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(kern, dim3(grid), dim3(kWaves * 64), Cf::LDS_BYTES, stream, d);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "decode_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }

@@ -98,8 +98,7 @@ int launch_gemm_generic(const GenericArgs& g, hipStream_t stream) {
   const int64_t gy = (rows + 15) / 16;
   if (gy > 65535) return set_error(MX_ERR_SHAPE, "generic kernel: too many rows (%lld)", (long long)rows);
   dim3 grid((unsigned)((g.N + 15) / 16), (unsigned)gy, (unsigned)g.batch);
-  hipLaunchKernelGGL(generic_kernel, grid, dim3(256), 0, stream, g);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(generic_kernel, grid, dim3(256), 0, stream, g);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "generic_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }

@@ -270,9 +270,8 @@ int launch_one(const GemmArgs& g, hipStream_t stream) {
   }
   const int64_t tiles = (int64_t)((g.M + C::BM - 1) / C::BM) * ((g.N + C::BN - 1) / C::BN);
   if (tiles <= 0) return MX_OK;
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)(g.k_splits > 1 ? g.k_splits : 1)), dim3(C::NT),
-                     C::LDS_BYTES, stream, g);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(kern, dim3((unsigned)tiles, (unsigned)(g.k_splits > 1 ? g.k_splits : 1)), dim3(C::NT),
+                               C::LDS_BYTES, stream, g);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "gemm_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }

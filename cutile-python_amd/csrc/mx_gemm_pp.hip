@@ -581,12 +581,10 @@ int launch_pp(const GemmArgs& g, hipStream_t stream) {
   int64_t grid = pp_grid(g.M, g.N, g.K, C::KSUB, C::BM);
   if (grid <= 0) return MX_OK;
   if (SPLIT) grid = num_cus();   // idle workgroups of a single, partly filled round take part too
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), PP<C>::LDS_BYTES, stream, g);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(kern, dim3((unsigned)grid), dim3(512), PP<C>::LDS_BYTES, stream, g);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "gemm_pp_kernel launch: %s", hipGetErrorString(e));
   if constexpr (SPLIT) {
-    hipLaunchKernelGGL((pp_tail_kernel<C, OutT, GROUPED>), dim3(8 * 8 * kTailMax), dim3(256), 0, stream, g, (int)grid);
-    e = hipGetLastError();
+    e = launch_kernel(pp_tail_kernel<C, OutT, GROUPED>, dim3(8 * 8 * kTailMax), dim3(256), 0, stream, g, (int)grid);
     if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "pp_tail_kernel launch: %s", hipGetErrorString(e));
   }
   return MX_OK;

@@ -423,8 +423,7 @@ int launch_pp32(const GemmArgs& g, hipStream_t stream) {
   }
   const int64_t grid = pp_grid(g.M, g.N, g.K, C::KSUB);
   if (grid <= 0) return MX_OK;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), PP<C>::LDS_BYTES, stream, g);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(kern, dim3((unsigned)grid), dim3(512), PP<C>::LDS_BYTES, stream, g);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "gemm_pp32_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }

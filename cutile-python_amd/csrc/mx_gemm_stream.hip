@@ -109,8 +109,7 @@ int launch(const StreamArgs& a, int blocks, hipStream_t stream) {
       return set_error(MX_ERR_LAUNCH, "hipFuncSetAttribute(%d bytes LDS): %s", C::LDS_BYTES, hipGetErrorString(e));
     attr_done = 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::WAVES * 64), C::LDS_BYTES, stream, a);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(kern, dim3((unsigned)blocks), dim3(C::WAVES * 64), C::LDS_BYTES, stream, a);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "stream_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }

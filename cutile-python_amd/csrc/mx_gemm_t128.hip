@@ -432,8 +432,7 @@ int launch_one(const T128Args& g, hipStream_t stream) {
   }
   const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
   if (tiles <= 0) return MX_OK;
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)g.k_splits, (unsigned)g.batch), dim3(256), lds, stream, g);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(kern, dim3((unsigned)tiles, (unsigned)g.k_splits, (unsigned)g.batch), dim3(256), lds, stream, g);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "t128_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }
@@ -450,8 +449,7 @@ int launch_list(const T128List& gl, hipStream_t stream) {
   }
   const int total = gl.first_tile[gl.n];
   if (total <= 0) return MX_OK;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(total < 512 ? total : 512)), dim3(256), lds, stream, gl);   // two per CU
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(kern, dim3((unsigned)(total < 512 ? total : 512)), dim3(256), lds, stream, gl);   // two per CU
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "t128_list_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }

@@ -298,8 +298,7 @@ int launch_w4(const GemmArgs& g, hipStream_t stream) {
   const int64_t tiles = (int64_t)((g.M + 255) / 256) * ((g.N + 255) / 256);
   if (tiles <= 0) return MX_OK;
   const int64_t grid = tiles > num_cus() ? num_cus() : tiles;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), kLds, stream, g);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(kern, dim3((unsigned)grid), dim3(256), kLds, stream, g);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "gemm_w4_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }

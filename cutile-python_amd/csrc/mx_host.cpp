@@ -12,8 +12,11 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <ATen/Context.h>
 #include <ATen/Functions.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/empty.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
@@ -113,7 +116,12 @@ bool scale_desc(PyObject* o, int64_t rows, int64_t K, bool is_b, const at::Devic
   return ok;
 }
 
+// at::empty without the dispatcher (0.47 instead of 0.72 us; a call allocates up to three tensors, a list one per problem),
+// unless something has asked to see factory calls (dispatch modes, functorch) or to have new memory filled.
 inline at::Tensor device_empty(at::IntArrayRef shape, at::ScalarType t, const at::Device& dev) {
+  const c10::impl::LocalDispatchKeySet tls = c10::impl::tls_local_dispatch_key_set();
+  if ((tls.included_ - c10::default_included_set).empty() && !at::globalContext().deterministicAlgorithms())
+    return at::detail::empty_cuda(shape, t, dev, std::nullopt);
   return at::empty(shape, at::TensorOptions().dtype(t).device(dev));
 }
 

@@ -190,8 +190,7 @@ int launch(const MoeStreamArgs& a, int blocks, hipStream_t stream) {
     if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "hipFuncSetAttribute(%d bytes LDS): %s", lds, hipGetErrorString(e));
     attr_done = 1;
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(C::WAVES * 64), lds, stream, a);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(kern, dim3((unsigned)blocks), dim3(C::WAVES * 64), lds, stream, a);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_stream_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }
@@ -240,9 +239,8 @@ int launch_moe_combine(const float* c, const void* ids, int ids64, int E, int64_
                        int out_dtype, hipStream_t stream) {
   const int64_t threads = T * ((H + 3) / 4);
   if (threads <= 0) return MX_OK;
-  hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, c, ids, ids64, E, T,
-                     topk, H, out, out_dtype);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_kernel(moe_combine_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, c, ids, ids64, E, T,
+                               topk, H, out, out_dtype);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_combine_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }
