@@ -171,9 +171,8 @@ __global__ __launch_bounds__(256) void quantize_kernel(const QuantArgs q) {
 // registers, two units of 16 bytes per thread) and sent each workgroup's scale bytes out in 16-byte pieces of lines that
 // other XCDs' workgroups shared: 8192 x 8192 bf16 -> E4M3 took 44 - 49 us (4.1 - 4.6 TB/s), this one 36.6 (5.5 TB/s), and
 // 8192 x 14336 of silu(gate) * up 117 us where it took 161
-// (133 with an IEEE division per element: there the vector ALUs are the bound).  Codes that exceed the L2s anyway (U > 1) are
-// stored and inputs that exceed the Infinity Cache loaded non-temporally: 8192 x 8192 36.6 -> 33.6 us (6.0 TB/s; stores
-// alone 35.7), 8192 x 4096 20.0 -> 16.4.  (The silu form gains nothing, and its codes are read next.)  A wave owns U * 64 consecutive
+// (133 with an IEEE division per element: there the vector ALUs are the bound).  Inputs that the Infinity Cache cannot hold
+// are loaded and their codes stored non-temporally: 8192 x 8192 36.6 -> 33.6 us (6.0 TB/s).  A wave owns U * 64 consecutive
 // units, so that a workgroup writes whole lines of scale bytes, all loads of a thread are requested before the first is used,
 // and the blocks the hardware conversion does not serve (zero, subnormal, non-finite or extreme amax) are done again
 // by the general code from memory, outside of the loop.
@@ -205,7 +204,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
     else return *p;
   };
   auto store = [](auto v, auto* p) {
-    if constexpr (U > 1 && !UP) __builtin_nontemporal_store(v, p);
+    if constexpr (ONCE) __builtin_nontemporal_store(v, p);
     else *p = v;
   };
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -645,17 +644,16 @@ template <int SRC, int FMT>
 static hipError_t launch_quantize_rows(const QuantArgs& q, int64_t units, hipStream_t stream) {
   // four units per thread once that leaves every CU several waves per SIMD, else one (a single row is a few waves: the
   // launch is all latency).  The silu form holds two inputs per unit and computes for longer: two.
-  // ONCE: the input is loaded non-temporally.  Where it comes from memory that is as fast or faster at every size; where it was
-  // just written and is still in the Infinity Cache (256 MB) it is slower from 16 MB on (8192^2, the same input every time,
-  // 30.2 -> 33.7 us) and below 8 MB (24 x 14336 in front of a product: 15.45 us for the pair, 15.7; 244 x 13440 39.0, 39.3).  So:
-  // inputs of 8 .. 16 MB (bf16; 1531 x 4096 5.9 -> 5.4 us, with the product behind it 101 -> 98.4), and those that the cache
-  // cannot hold.
+  // ONCE: loaded and stored non-temporally, from 96 MB of input on.  Smaller ones gain as much by themselves (4096^2 12.5 -> 11.2 us)
+  // where they come from memory, but an input that was just written is slower (8192^2, the same one every time, 30.2 -> 33.7;
+  // in front of a product 3973 x 2048 24.1 -> 25.2 for the pair), and so is the product that reads the codes next (1257 x 7808
+  // in front of 2816 columns 45.1 -> 48.3).
 #define MX_Q(UP, U, ONCE) return launch_kernel(quantize_rows_kernel<SRC, FMT, UP, U, ONCE>, dim3((unsigned)((units + 256 * U - 1) / (256 * U))), dim3(256), 0, stream, q)
-  const bool large = units >= ((int64_t)1 << 20), mid = units >= ((int64_t)1 << 19);
+  const bool large = units >= ((int64_t)1 << 20);
   const bool beyond = units * 8 * (SRC == MX_F32 ? 4 : 2) >= kLoadOnceBytes;
   if (q.up) { if (large) MX_Q(true, 2, false); else MX_Q(true, 1, false); }
   else if (large) { if (beyond) MX_Q(false, 4, true); else MX_Q(false, 4, false); }
-  else { if (mid) MX_Q(false, 1, true); else MX_Q(false, 1, false); }
+  else MX_Q(false, 1, false);
 #undef MX_Q
 }
 
