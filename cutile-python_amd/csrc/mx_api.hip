@@ -89,20 +89,50 @@ int plan_k_splits(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
 // What MX_KERNEL_AUTO weighs beyond kStreamAutoM rows: estimated time (us) of a product on the kernels that can run it.
 // Fitted to measurements of 96 .. 4096 rows x 512 .. 28672 columns x 512 .. 9216 (stages of 128 bytes of a row, launches
 // back to back, MXFP8; FP4 x FP4 has constants of its own):
-//   128 x 128 tiles: 0.62 us per stage with one tile on a CU (1024 x 4096 x 4096 24.6 us, 2048 x 2048 x 8192 45 us), then by
-//     their number (2048 x 4096 x 4096 40, 1531 x 14336 x 4096 95).  Split along K: the partial sums are written and read.
+//   64 x 64 and 128 x 128 tiles (mx_gemm_t128.hip picks by their number): a stage of 64 x 64 tiles 0.25 us with one on a CU
+//     (1024 x 1024 x 4096 13.4 us), 0.36 with two (512 x 4096 x 4096 17.1); of 128 x 128 ones 0.62 with one on a CU (2048 x
+//     2048 x 8192 45 us), then by their number (2048 x 4096 x 4096 40, 1531 x 14336 x 4096 95).  Split along K: the partial
+//     sums are written and read by a second launch.
 //   256 x 256 tiles: a round's length and, as the clock falls the busier the chip is, its share of tiles (4096^3, one full
 //     round, 50; 2048 x 4096 x 4096, half of one, 44; 1531 x 14336 x 4096, 1.31 rounds, 86); it needs re-laid scales.
 //   192 x 256 tiles: a round of them is 18 % shorter for 25 % fewer rows (more of a stage is not MFMA), which pays where it
 //     fills rounds that 256 rows leave half empty (1531 x 14336 x 4096, 1.75 rounds, 77; 3000 x 4096 x 4096 42 against 45;
 //     but 4096 x 14336 x 4096 187 against 175).
-//   streaming: 0.57 us per unit of its own cost estimate (256 x 14336 x 4096 40 us, 1024 x 4096 x 8192 60 us).
-float est_t128(int64_t M, int64_t N, int64_t K, int S, bool fp4, int64_t batch = 1) {
-  const int64_t wgs = ((M + 127) / 128) * ((N + 127) / 128) * S * batch;
-  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)) / S, fill = wgs < 435 ? 0.85f : wgs / 512.f;
-  float t = 5.f + st * (wgs <= 256 ? (fp4 ? 0.68f : 0.62f) : 0.1f + (fp4 ? 1.25f : 1.05f) * fill);
-  if (S > 1) t += 4.f + (float)S * M * N * 8 / 4e6f;
-  return t;
+//   streaming: 0.5 .. 0.75 us per unit of its own cost estimate (64 x 4096 x 4096 9.4 us, 128 x 4096 x 8192 15.2, FP4 weights
+//     12.1), or the time that reading the weights takes, longer the more row tiles share them (14336 x 8192, 64, 128, 256 rows:
+//     28.6, 47, 83 us).  33 .. 64 rows: 64 x 64 tiles are faster for K up to 1024 (64 x 4096 x 1024 6.3 us against 7.8) and
+//     for many columns (64 x 28672 x 2048 12.7 against 15.4), streaming for few and long ones (64 x 4096 x 4096 12.3 against 9.4).
+float est_t128_split(int64_t M, int64_t N, int64_t K, int S, bool fp4, int64_t batch, bool fp4_b) {
+  const int64_t small = t128_small_tiles(M, N) * S * batch, wgs = ((M + 127) / 128) * ((N + 127) / 128) * S * batch;
+  const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)) / S;
+  float stage;
+  if (small <= kT128SmallTiles) stage = small <= 256 ? (fp4 ? 0.33f : 0.25f) : (fp4 ? 0.43f : 0.36f);
+  else if (wgs <= 256) stage = fp4 ? 0.68f : 0.62f;
+  else stage = 0.1f + (fp4 ? 1.25f : 1.05f) * (wgs < 435 ? 0.85f : wgs / 512.f);
+  float t = 4.5f + st * stage;
+  if (small <= kT128SmallTiles) {   // many columns for few rows: the time that reading B takes
+    const float b = (float)N * K * (fp4_b ? 0.5f : 1.f) * batch;
+    const float read = 1.3f + b / (b < 96e6f ? 4.8e6f : 3.8e6f);
+    if (read > t) t = read;
+  }
+  return t + (S > 1 ? 3.f + (float)S * M * N * 8 / 4e6f : 0.f);
+}
+// Of the ways to split K that there is room for (up to S; automatic splits only) the best one: none, all, or as many as give
+// every CU one or two 64 x 64 tiles.
+int t128_splits(int64_t M, int64_t N, int64_t K, int S, bool fp4, bool fp4_b) {
+  if (S <= 1) return 1;
+  const int64_t w = t128_small_tiles(M, N);
+  int best = 1;
+  float us = est_t128_split(M, N, K, 1, fp4, 1, fp4_b);
+  for (const int64_t s : {(int64_t)S, 256 / w, 512 / w}) {
+    if (s < 2 || s > S) continue;
+    const float t = est_t128_split(M, N, K, (int)s, fp4, 1, fp4_b);
+    if (t < us) { us = t; best = (int)s; }
+  }
+  return best;
+}
+float est_t128(int64_t M, int64_t N, int64_t K, int S, bool fp4, bool fp4_b, int64_t batch = 1) {
+  return est_t128_split(M, N, K, batch == 1 ? t128_splits(M, N, K, S, fp4, fp4_b) : 1, fp4, batch, fp4_b);
 }
 float est_pp(int64_t M, int64_t N, int64_t K, bool fp4, bool pack, bool tail, int rows = 256) {
   const int64_t tiles = ((M + rows - 1) / rows) * ((N + 255) / 256);
@@ -114,7 +144,17 @@ float est_pp(int64_t M, int64_t N, int64_t K, bool fp4, bool pack, bool tail, in
   }
   return rest + st * (round * ((tiles + 255) / 256) + full * tiles / 256);
 }
-float est_stream(int64_t M, int64_t N, int64_t K, int w_fmt) { return 5.f + 0.57f * stream_plan(M, N, K, w_fmt).cost; }
+float est_stream(int64_t M, int64_t N, int64_t K, int w_fmt) {
+  const StreamPlan p = stream_plan(M, N, K, w_fmt);
+  const bool fp4 = w_fmt == MX_E2M1;
+  // (the plan's cost is that of its longest wave: where K-quads do not divide evenly, most waves are shorter)
+  const int64_t KQ = (K + 511) / 512;
+  const float rounds = (float)(((int64_t)p.units * p.m_tiles + 255) / 256) * 3.f;
+  const float cost = rounds + (p.cost - rounds) * ((float)KQ / p.kw) / (float)((KQ + p.kw - 1) / p.kw);
+  const float t = !fp4 ? 3.f + 0.55f * cost : p.mt == 4 ? 3.2f + 0.75f * cost : 2.6f + 0.5f * cost;
+  const float read = 1.3f + (float)N * K * (fp4 ? 0.5f : 1.f) / 4.2e6f * (0.3f + 0.7f * p.m_tiles);
+  return t > read ? t : read;
+}
 
 int check_tensor(const mx_tensor* t, const char* name, int min_nd, int max_nd) {
   if (!t) return set_error(MX_ERR_INVALID, "%s: null descriptor", name);
@@ -237,7 +277,7 @@ int64_t gemm_workspace_tail(int64_t M, int64_t N, int64_t K, const mx_gemm_opts&
   if (M <= kStreamAutoM) return 0;
   const bool pack = !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout);
   for (int fp4 = 0; fp4 < 2; ++fp4)
-    if (est_pp(M, N, K, fp4, pack, true) < est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4)) return t;
+    if (est_pp(M, N, K, fp4, pack, true) < est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4, fp4)) return t;
   return 0;
 }
 int64_t grouped_workspace_min(int64_t num_slots, int64_t N, int64_t K, int64_t E, const mx_gemm_opts& o) {
@@ -470,13 +510,13 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       if (any && chunk >= 1) chunk = batch;   // (reads the scales where they are; callers are held to the workspace all the same)
       if (chunk > 32768) chunk = 32768;
       if (ok && batch > 1) {   // few long products are better off one by one with K split, large ones gain nothing
-        float alone = est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4);
+        float alone = est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4, B->dtype == MX_E2M1);
         if (o.kernel == MX_KERNEL_AUTO) {
           const float pp = est_pp(M, N, K, fp4, true, false);
           if (pp < alone) alone = pp;
           if (!fp4 && M <= kStreamAutoM && est_stream(M, N, K, B->dtype) < alone) alone = est_stream(M, N, K, B->dtype);
         }
-        ok = est_t128(M, N, K, 1, fp4, batch) <= batch * alone;
+        ok = est_t128(M, N, K, 1, fp4, B->dtype == MX_E2M1, batch) <= batch * alone;
       }
       if (!plain && workspace && ((uintptr_t)workspace) % 256 != 0) ok = false;
       if (ok && chunk >= 1) {
@@ -575,7 +615,11 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     if (why_stream) return set_error(MX_ERR_LAYOUT, "the streaming kernel cannot run this problem: %s", why_stream);
   } else if (kernel == MX_KERNEL_AUTO) {
     const bool may_stream = !plan && !why_stream && o.split_k <= 1;
-    if (may_stream && (why || M <= kStreamAutoM) &&
+    // (a call that would need the workspace on the tiled kernel and has none streams as it always did)
+    const bool tiles = may_stream && !why && M > 32 && M <= kStreamAutoM && (ws_min == 0 || (workspace && workspace_bytes >= ws_min && ((uintptr_t)workspace) % 256 == 0)) &&
+                       est_t128(M, N, K, plan_k_splits(M, N, K, o), A->dtype == MX_E2M1, B->dtype == MX_E2M1) <
+                           est_stream(M, N, K, B->dtype);
+    if (may_stream && (why || (M <= kStreamAutoM && !tiles)) &&
         !(M <= 32 && decode_beats_stream(M, N, K) && B->dtype == MX_E2M1 && o.b_scale_layout == MX_SCALE_2D))
       kernel = MX_KERNEL_STREAM;
     else if (why) kernel = MX_KERNEL_GENERIC;
@@ -588,7 +632,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       kernel = MX_KERNEL_DECODE;
     else {
       const bool fp4 = A->dtype == MX_E2M1;
-      const float t128 = est_t128(M, N, K, o.split_k > 1 ? 1 : plan_k_splits(M, N, K, o), fp4);
+      const float t128 = est_t128(M, N, K, o.split_k > 1 ? 1 : plan_k_splits(M, N, K, o), fp4, B->dtype == MX_E2M1);
       const bool room = workspace && o.split_k == 0 && pp_tail_bytes(M, N, K, fp4, true) > 0 &&
                         workspace_bytes >= ws_min + pp_tail_bytes(M, N, K, fp4, true);
       float pp = o.split_k > 1 ? 1e30f : est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), room);
@@ -708,6 +752,7 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
                        512 * o.split_k);
   }
   if (S > 1 && plan) return kPlanNotSimple;
+  if (kernel == MX_KERNEL_MFMA_128x128 && o.split_k == 0) S = t128_splits(M, N, K, S, A->dtype == MX_E2M1, B->dtype == MX_E2M1);
   if (S > 1 && acc) return kAccNeedsCopy;
   if (kernel == MX_KERNEL_MFMA_128x128) {
     // scales are read where they are if the kernel can (A alone, or A and B), else re-laid first

@@ -40,6 +40,10 @@ inline bool t128_any_scales(int64_t ld, int64_t k_stride, int64_t rows, int64_t 
   const int64_t lim = ((int64_t)1 << 31) - 64;   // (the last quad's window reaches beyond its row)
   return k_stride == 1 && K >= 32 && rows * ld < lim && (rows - 1) * ld + K / 32 < lim;
 }
+// 64 x 64 tiles of a product; up to kT128SmallTiles workgroups (two for every CU) of them run instead of 128 x 128 ones
+// (measured either side in mx_gemm_t128.hip)
+constexpr int64_t kT128SmallTiles = 512;
+inline int64_t t128_small_tiles(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 63) / 64); }
 int launch_gemm_t128(const T128Args& g, hipStream_t stream);
 // any number of independent plain products of one element-format pair: one persistent launch per 32 of them
 int launch_gemm_t128_list(const T128Args* problems, int n, hipStream_t stream);

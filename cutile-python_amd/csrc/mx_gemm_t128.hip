@@ -10,6 +10,11 @@
 //                 issue the DMA of stage s + NS into the buffer of stage s
 //                 16 (32) MFMAs of stage s, the fragment reads of stage s + 1 between them
 // (order of the requests and what the waits count: mx_t128_schedule.h).
+// 64 x 64 tiles (four waves of 32 x 32, eight stages in flight or four) take products that leave CUs idle: a stage is 0.25 us
+// instead of 0.62, and there are four times as many workgroups.  Six products 200 x 328 x 992 with an addend 10.7 -> 7.0 us,
+// 1024 x 1024 x 4096 21.4 -> 13.4 (19.2 with K split four ways), 256 x 4096 x 8192 22.7 (split) -> 20.5; with two workgroups
+// on a CU 512 x 4096 x 4096 22.4 -> 17.1; beyond that the larger tile reads less (1200 x 2048 x 2048 14.6 against 15.7).
+//
 // NS = 4 (128 KiB, one workgroup per CU) for grids that leave CUs with one tile, NS = 2 (64 KiB) where two workgroups share
 // a CU.  The fragment reads (64 KiB per stage at 128 bytes per clock) are as long as the MFMAs of a stage, so a CU can get
 // to about half of the MFMA rate; larger products go to the 256 x 256 kernel.
@@ -36,15 +41,15 @@ constexpr int kScaleNative = 0, kScalePlain = 1, kScaleAny = 2;
 
 template <class C, int NS, int AS, int BS, bool GROUPED>
 __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem, const int pid, const int split, const int bz) {
-  constexpr int KS = C::KSUB, SPQ = 4 / KS, MT = 4, NT = 4;
+  constexpr int KS = C::KSUB, SPQ = 4 / KS, MT = C::MT, NT = C::NTL;
   constexpr bool AP = AS != kScaleNative, BP = BS != kScaleNative, ANY = AS == kScaleAny;
-  static_assert(ANY == (BS == kScaleAny) && !(ANY && GROUPED), "");
+  static_assert(ANY == (BS == kScaleAny) && !(ANY && GROUPED) && MT == NT && (C::BM == 128 || !GROUPED), "");
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, gq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
+  const int wm0 = (wave >> 1) * C::WTM, wn0 = (wave & 1) * C::WTN;
 
   // ---- tile of C: XCD-aware, then grouped along M (as in mx_gemm_mfma.hip) ------------------------------------------
-  const int tiles_m = (g.M + 127) / 128, tiles_n = (g.N + 127) / 128;
+  const int tiles_m = (g.M + C::BM - 1) / C::BM, tiles_n = (g.N + C::BN - 1) / C::BN;
   int m0, n0;
   {
     const int total = tiles_m * tiles_n;
@@ -55,8 +60,8 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
     const int gid = lid / in_group, first_m = gid * GM;
     const int gsz = (tiles_m - first_m) < GM ? (tiles_m - first_m) : GM;
     const int in = lid % in_group;
-    m0 = (first_m + in % gsz) * 128;
-    n0 = (in / gsz) * 128;
+    m0 = (first_m + in % gsz) * C::BM;
+    n0 = (in / gsz) * C::BN;
   }
   int expert = 0;
   if constexpr (GROUPED) {
@@ -130,7 +135,9 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
     const bool is_b = wave >= 2;
     const int row0 = (is_b ? n0 : m0) + 64 * (wave & 1), rows = is_b ? g.N : g.M;
     const bool plain = is_b ? BP : AP;
-    if (plain) {
+    if (C::BM == 64 && (wave & 1)) {   // one group per operand
+      sco = kOobOffset;
+    } else if (plain) {
       int64_t row = row0 + lane;
       bool ok = row < rows;
       if constexpr (GROUPED) {
@@ -181,7 +188,7 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
     if (wave < 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsAs, (lds_void*)dst, 16, v, Q * (AP ? 16 : 1024), 0, 0);
     else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsBs, (lds_void*)dst, 16, v, Q * (BP ? 16 : 1024), 0, 0);
   };
-  int sa[4], sb[4], san[4], sbn[4];   // plain: register = tile, byte = K-step; packed: register = K-step, byte = tile
+  int sa[4] = {}, sb[4] = {}, san[4] = {}, sbn[4] = {};   // plain: register = tile, byte = K-step; packed: register = K-step, byte = tile
   // plain: the lane's byte gq of each of a row's four dwords
   const uint32_t sel = 0x0c0c0400u + (uint32_t)gq * 0x0101u;
   auto own = [&](const v4i v) {
@@ -189,23 +196,24 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
     return (int)(lo | (hi << 16));
   };
   auto read_scales = [&](int Q) {
-    lds_u8* const ta = sbase + Q % (SD + 1) * SSLOT + wm0 * 16;
-    lds_u8* const tb = sbase + Q % (SD + 1) * SSLOT + 2048 + wn0 * 16;
+    lds_u8* const ta = sbase + Q % (SD + 1) * SSLOT + (AP ? wm0 : wm0 / 64 * 64) * 16;
+    lds_u8* const tb = sbase + Q % (SD + 1) * SSLOT + 2048 + (BP ? wn0 : wn0 / 64 * 64) * 16;
+    // (packed: a register holds the group's four tiles of a K-step; a wave of 32 rows has the first or the last two)
     if constexpr (AP) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) san[i] = own(*(lds_v4i*)(ta + (16 * i + r) * 16));
+      for (int i = 0; i < MT; ++i) san[i] = own(*(lds_v4i*)(ta + (16 * i + r) * 16));
     } else {
       const v4i v = *(lds_v4i*)(ta + lane * 16);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) san[i] = v[i];
+      for (int i = 0; i < 4; ++i) san[i] = MT == 4 ? v[i] : (int)((uint32_t)v[i] >> (wm0 / 2));
     }
     if constexpr (BP) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) sbn[j] = own(*(lds_v4i*)(tb + bperm_row(j, r) * 16));
+      for (int j = 0; j < NT; ++j) sbn[j] = own(*(lds_v4i*)(tb + bperm_row(j, r) * 16));
     } else {
       const v4i v = *(lds_v4i*)(tb + lane * 16);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) sbn[j] = v[j];
+      for (int j = 0; j < 4; ++j) sbn[j] = NT == 4 ? v[j] : (int)((uint32_t)v[j] >> (wn0 / 2));
     }
   };
   auto take_scales = [&]() {
@@ -230,6 +238,41 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk) bf[decltype(set)::value][kk][j] = load_frag<C::B_RB, C::B_EB>(t, bperm_tile_off(j), kk, gq, swb);
   };
+
+  // the fp32 addend (its own operand, or C): every load is requested before the first is waited for, with offsets beyond
+  // the matrix for what does not exist.  (One guarded load after another, as for the rows below that are not whole
+  // 16-byte pieces, the addend cost more than the product: six 200 x 328 x 992 took 17 us instead of 9.)  Tiles of 64 have
+  // the registers to request it ahead of everything else.
+  constexpr bool EARLY_ADD = C::BM == 64;
+  const int n = n0 + wn0 + 8 * gq;
+  const int cols = g.N - n;
+  v4f add[GROUPED ? 1 : MT][NT];
+  bool added = false;
+  auto load_addend = [&]() {
+    if constexpr (!GROUPED) {
+      const float* const addend = g.acc ? g.acc + (int64_t)bz * g.c_batch
+                                  : g.accumulate ? (const float*)g.C + (int64_t)bz * g.c_batch : nullptr;
+      const int64_t ld = g.ldc;
+      if (addend && g.N % 4 == 0 && ld % 4 == 0 && (uintptr_t)addend % 16 == 0 && (int64_t)g.M * ld < (1 << 29)) {   // uniform
+        added = true;
+        const __amdgpu_buffer_rsrc_t rsD = make_rsrc(addend, (uint32_t)(((int64_t)(g.M - 1) * ld + g.N) * 4));
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          const int m = m0 + wm0 + 16 * i + r;
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+            const int c = 32 * (j / 2) + 4 * (j % 2);
+            const uint32_t at = m < g.M && c < cols ? (uint32_t)((m * ld + n + c) * 4) : kOobOffset;
+            add[i][j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsD, at, 0, 0));
+          }
+        }
+      }
+    }
+  };
+  if constexpr (EARLY_ADD) {
+    if (g.c_dtype == MX_F32 && g.k_splits <= 1) load_addend();
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   // ---- prologue ---------------------------------------------------------------------------------------------------------
   if constexpr (ANY) load_any(q0);
@@ -311,35 +354,12 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
   }
 
   // ---- epilogue: lane (r, gq) of tile pair (2 jp, 2 jp + 1) holds row 16 i + r, columns 32 jp + 8 gq .. + 7 -------------
-  const int n = n0 + wn0 + 8 * gq;
-  const int cols = g.N - n;
   auto store = [&](auto kind) {        // 0: fp32, 1: bf16, 2: fp32 partial product of a split
     constexpr int kd = decltype(kind)::value;
     using OutT = std::conditional_t<kd == 1, uint16_t, float>;
     OutT* const Cp = kd == 2 ? (OutT*)(g.partial + (int64_t)split * g.M * g.N) : (OutT*)g.C + (int64_t)bz * g.c_batch;
     const int64_t ld = kd == 2 ? g.N : g.ldc;
-    // the fp32 addend (its own operand, or C): every load is requested before the first is waited for, with offsets beyond
-    // the matrix for what does not exist.  (One guarded load after another, as for the rows below that are not whole
-    // 16-byte pieces, the addend cost more than the product: six 200 x 328 x 992 took 17 us instead of 9.)
-    v4f add[kd == 0 && !GROUPED ? MT : 1][4];
-    bool added = false;
-    if constexpr (kd == 0 && !GROUPED) {
-      const float* const addend = g.acc ? g.acc + (int64_t)bz * g.c_batch : g.accumulate ? (const float*)Cp : nullptr;
-      if (addend && g.N % 4 == 0 && ld % 4 == 0 && (uintptr_t)addend % 16 == 0 && (int64_t)g.M * ld < (1 << 29)) {   // uniform
-        added = true;
-        const __amdgpu_buffer_rsrc_t rsD = make_rsrc(addend, (uint32_t)(((int64_t)(g.M - 1) * ld + g.N) * 4));
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-          const int m = m0 + wm0 + 16 * i + r;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int c = 32 * (j / 2) + 4 * (j % 2);
-            const uint32_t at = m < g.M && c < cols ? (uint32_t)((m * ld + n + c) * 4) : kOobOffset;
-            add[i][j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rsD, at, 0, 0));
-          }
-        }
-      }
-    }
+    if constexpr (kd == 0 && !GROUPED && !EARLY_ADD) load_addend();
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const int m = m0 + wm0 + 16 * i + r;
@@ -354,11 +374,11 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
       }
       if (!ok) continue;
 #pragma unroll
-      for (int jp = 0; jp < 2; ++jp) {
+      for (int jp = 0; jp < NT / 2; ++jp) {
         v4f v0 = acc[i][2 * jp], v1 = acc[i][2 * jp + 1];
         if constexpr (GROUPED) { v0 *= w; v1 *= w; }
         const int64_t off = row * ld + n + 32 * jp;
-        if (added) {
+        if (kd == 0 && added) {
           if constexpr (kd == 0 && !GROUPED) { v0 += add[i][2 * jp]; v1 += add[i][2 * jp + 1]; }
         } else if (kd != 2 && g.acc) add8_edge<float>(g.acc + (int64_t)bz * g.c_batch + off, v0, v1, cols - 32 * jp);
         else if (kd != 2 && g.accumulate) add8_edge<OutT>(Cp + off, v0, v1, cols - 32 * jp);
@@ -372,7 +392,7 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
 }
 
 template <class C, int NS, int AS, int BS, bool GROUPED>
-__global__ __launch_bounds__(256, NS == 2 ? 2 : 1) void t128_kernel(const T128Args g) {
+__global__ __launch_bounds__(256, NS == 2 || (C::BM == 64 && NS == 4) ? 2 : 1) void t128_kernel(const T128Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_generic[];
   t128_tile<C, NS, AS, BS, GROUPED>(g, (lds_u8*)smem_generic, blockIdx.x, blockIdx.y, blockIdx.z);
   __builtin_amdgcn_s_waitcnt(0x0F70);   // the trailing zero-fill DMA has left the queue before the LDS is given back
@@ -430,7 +450,7 @@ int launch_one(const T128Args& g, hipStream_t stream) {
     if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "hipFuncSetAttribute(%d bytes LDS): %s", lds, hipGetErrorString(e));
     attr_done = 1;
   }
-  const int64_t tiles = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128);
+  const int64_t tiles = (int64_t)((g.M + C::BM - 1) / C::BM) * ((g.N + C::BN - 1) / C::BN);
   if (tiles <= 0) return MX_OK;
   hipError_t e = launch_kernel(kern, dim3((unsigned)tiles, (unsigned)g.k_splits, (unsigned)g.batch), dim3(256), lds, stream, g);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "t128_kernel launch: %s", hipGetErrorString(e));
@@ -465,14 +485,20 @@ int t128_pair(const T128Args& g, hipStream_t stream) {
                      : launch_one<C, 2, kScaleNative, kScaleNative, true>(g, stream);
   // (A packed with B plain does not occur: the entry points re-lay B first)
   const int64_t wgs = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * g.k_splits * g.batch;
-  auto depth = [&](auto ns) {
+  auto depth = [&](auto cfg, auto ns) {
+    using D = decltype(cfg);
     constexpr int NS = decltype(ns)::value;
-    if (g.a_plain == kT128ScalesAny) return launch_one<C, NS, kScaleAny, kScaleAny, false>(g, stream);
-    return !g.a_plain   ? launch_one<C, NS, kScaleNative, kScaleNative, false>(g, stream)
-           : !g.b_plain ? launch_one<C, NS, kScalePlain, kScaleNative, false>(g, stream)
-                        : launch_one<C, NS, kScalePlain, kScalePlain, false>(g, stream);
+    if (g.a_plain == kT128ScalesAny) return launch_one<D, NS, kScaleAny, kScaleAny, false>(g, stream);
+    return !g.a_plain   ? launch_one<D, NS, kScaleNative, kScaleNative, false>(g, stream)
+           : !g.b_plain ? launch_one<D, NS, kScalePlain, kScaleNative, false>(g, stream)
+                        : launch_one<D, NS, kScalePlain, kScalePlain, false>(g, stream);
   };
-  return wgs <= 256 ? depth(std::integral_constant<int, 4>{}) : depth(std::integral_constant<int, 2>{});
+  const int64_t small = t128_small_tiles(g.M, g.N) * g.k_splits * g.batch;
+  if (small <= kT128SmallTiles) {
+    using S = Cfg<AF, BF, 64, 64, 2, 2>;
+    return small <= 256 ? depth(S{}, std::integral_constant<int, 8>{}) : depth(S{}, std::integral_constant<int, 4>{});
+  }
+  return wgs <= 256 ? depth(C{}, std::integral_constant<int, 4>{}) : depth(C{}, std::integral_constant<int, 2>{});
 }
 template <int AF, int BF>
 int t128_list_pair(const T128Args* problems, int n, hipStream_t stream) {

@@ -27,7 +27,7 @@ struct Cfg {
   static constexpr int A_LOADS = BM * A_CPR / NT, B_LOADS = BN * B_CPR / NT;
   static constexpr int WTM = BM / WGM, WTN = BN / WGN;   // wave tile
   static constexpr int MT = WTM / 16, NTL = WTN / 16;    // 16x16 MFMA tiles per wave
-  static_assert(BM % 64 == 0 && WTM % 32 == 0 && WTN % 64 == 0, "tiles must cover whole 64-row scale groups");
+  static_assert(BM % 64 == 0 && WTM % 32 == 0 && BN % 64 == 0 && WTN % 32 == 0, "tiles must cover whole 64-row scale groups");
   static_assert((BM * A_CPR) % NT == 0 && (BN * B_CPR) % NT == 0, "loads must divide evenly");
   static_assert(A_CPR == 8 || A_CPR == 4, "row is 64 or 128 bytes");
 };
