@@ -1270,19 +1270,24 @@ struct MoePlan {
   int32_t tile_m;
   int64_t q, qs, c3, c1, slots, in_use, max_slots, blocks, align, grouped, grouped_bytes, total;   // offsets (bytes)
 };
-// Rows per expert up to which the weights are streamed.  us per layer, streamed | grouped with 256-slot | 128-slot tiles:
-//   16 experts of 4096 x 4096, FP8: 32 rows 218 | 269 | 278, 48 rows 276 | 276 | 285, 64 rows 336 | 283 | 298;
-//   FP4: 32 rows 139 | 182 | 181, 48 rows 173 | 188 | 194, 64 rows 238 | 193 | 205
-//   8 experts of 4096 x 14336, FP8: 16 rows 257 | 358 | 323, 32 rows 372 | 368 | 353, 48 rows 455 | 374 | 388;
-//   FP4: 32 rows 238 | 280 | 259, 48 rows 275 | 284 | 295
-// so the line is right for FP4 and for experts of middling size; of large FP8 experts the tiles are ahead from 32 rows on.
+// Rows per expert up to which the weights are streamed.  us per layer, streamed | grouped with 256-slot tiles:
+//   16 experts of 4096 x 4096, FP8: 32 rows 218 | 266, 48 rows 276 | 273, 64 rows 336 | 283; FP4: 32 rows 139 | 183, 48 rows
+//   173 | 187, 64 rows 238 | 193
+//   8 experts of 4096 x 14336, FP8: 16 rows 231 | 358, 32 rows 372 | 366, 48 rows 453 | 373; FP4: 32 rows 239 | 282, 48 rows
+//   274 | 286
+//   64 experts of 3584 x 1024, FP8: 32 rows 223 | 248
+// (128-slot and 64-slot tiles are slower than one or the other everywhere.)  Beyond 32 rows an expert's weights are read once
+// more; against that stand the tiles' extra passes, some 40 us whatever the size: from 1 GB of weights on the tiles are ahead
+// (34 rows: 1.41 GB 393 | 366, 0.81 GB 231 | 264).
 // (64 rows: with a longer list of ids, mx_stream.h.)
-constexpr int64_t kMoeStreamRows = 48;
+constexpr int64_t kMoeStreamRows = 48, kMoeStreamTwiceBytes = 1000000000;
 
 MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& W2, const mx_gemm_opts& o) {
   MoePlan p = {};
   p.T = T; p.n = T * topk; p.E = W1.shape[0]; p.H = W1.shape[2]; p.F = W1.shape[1] / 2; p.H_out = W2.shape[1];
-  p.stream = p.n <= kMoeMaxIds && p.n <= p.E * kMoeStreamRows && p.H % 128 == 0 && p.F % 128 == 0;
+  const int64_t weights = p.E * (2 * p.F * p.H + p.H_out * p.F) / (W1.dtype == MX_E2M1 ? 2 : 1);   // bytes
+  const int64_t rows = weights > kMoeStreamTwiceBytes ? 32 : kMoeStreamRows;
+  p.stream = p.n <= kMoeMaxIds && p.n <= p.E * rows && p.H % 128 == 0 && p.F % 128 == 0;
   int64_t off = 0;
   auto take = [&](int64_t bytes) { const int64_t at = off; off += round256(bytes); return at; };
   p.q = take(p.n * p.F);
