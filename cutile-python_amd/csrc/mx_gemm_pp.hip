@@ -77,9 +77,8 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   uint32_t a_voff[AL], b_voff[TEAM ? BL : 1];
   const int a_row0 = wm0 + wn * P::A_RPI + lane / C::A_CPR;
   const int a_col0 = ((lane % C::A_CPR) ^ swz<C::A_CPR>(a_row0)) * 16;
-  const int b_row0 = wn0 + lane / C::B_CPR;
   // swizzled byte column of DMA instruction q (rows b_row0 + q * B_RPI ...)
-  auto b_col = [&](int q) { return ((lane % C::B_CPR) ^ swz_bperm<C::B_CPR>(lane / C::B_CPR + q * P::B_RPI)) * 16; };
+  auto b_col = [&](int q, int lane) { return ((lane % C::B_CPR) ^ swz_bperm<C::B_CPR>(lane / C::B_CPR + q * P::B_RPI)) * 16; };
   __amdgpu_buffer_rsrc_t rsB;
   // ---- scales (native layout, mx_common.h): 16 bytes per (64-row group, K-quad, lane), dword t = K-step t of the
   // quad, byte = 16-row tile of the group (B: in the bperm_row order of the fragments).  A K-quad needs the team's
@@ -104,6 +103,35 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   // then a vote, so a sentinel in front of valid ids does not hide them).  Such a half has nothing to multiply:
   // its fragment reads and MFMAs are skipped.
   bool skip_cur = false, skip_nxt = false;
+  // grouped: routed-slot ids of the team's 128 rows, two per lane (lane l: rows l and 64 + l; -1 where there is no slot): of
+  // the tile to be fetched next, then again of the tile being computed, whose output they place.  They and the expert are
+  // requested a stage or more before the tile's first loads are set up (each DMA instruction's rows read their own ids in that
+  // memory phase before, one after the other, while both teams waited).  With the walk by experts (ExpertRuns) the layer of
+  // 4096 tokens, 8 experts, top 2, 4096 x 14336 takes 1400 us instead of 1445; the ids alone gave 0.5 % of it.
+  int eid[2] = {-1, -1}, expert_nxt = 0;
+  // grouped: origin of the tile being computed, being fetched; the columns of the one written next (the last one computed)
+  int n_out = 0, m_cur = 0, n_cur = 0, m_nxt = 0, n_nxt = 0;
+  ExpertRuns runs = {g.sorted_expert_ids, g.tile_m, walk.tiles_m, walk.tiles_n};
+  auto load_row_ids = [&](bool valid, int m0) {
+    int l = lane;
+    asm volatile("" : "+v"(l));   // (nothing of this is kept in registers from one tile to the next)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int m = m0 + wm0 + 64 * u + l;
+      eid[u] = valid && m < g.M ? g.sorted_token_ids[m] : -1;
+    }
+  };
+  auto request_tile = [&](int lid) {   // ahead of set_fetch_tile
+    if constexpr (GROUPED) {
+      const bool valid = SPLIT ? lid != kNoTile : lid < walk.end;
+      m_nxt = n_nxt = 0;
+      if (valid) runs.origin(lid, m_nxt, n_nxt);
+      load_row_ids(valid, m_nxt);
+      int tile_m = g.tile_m;
+      asm volatile("" : "+s"(tile_m));
+      expert_nxt = g.sorted_expert_ids[m_nxt / tile_m];
+    }
+  };
   int kq_nxt = KQ;   // K-quads of the tile being fetched
   auto set_fetch_tile = [&](int lid) {
     fetch_valid = SPLIT ? lid != kNoTile : lid < walk.end;
@@ -112,44 +140,49 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
     const int qb = part ? walk.quads & 0xFFFF : 0;
     kq_nxt = part ? walk.quads >> 16 : KQ;
     const uint32_t ka0 = (uint32_t)(qb * SPQ * C::A_RB), kb0 = (uint32_t)(qb * SPQ * C::B_RB);
-    int m0 = 0, n0 = 0;
-    if (fetch_valid) walk.origin<C::BM>(lid, m0, n0);
+    int m0 = m_nxt, n0 = n_nxt;
+    if (!GROUPED && fetch_valid) walk.origin<C::BM>(lid, m0, n0);
+    int ln = lane;
+    if constexpr (GROUPED) asm volatile("" : "+v"(ln));   // (as in load_row_ids)
+    const int row = wn * P::A_RPI + ln / C::A_CPR;   // of the team's 128
+    const int a_col0 = ((ln % C::A_CPR) ^ swz<C::A_CPR>(wm0 + row)) * 16, b_row0 = wn0 + ln / C::B_CPR;
+    uint32_t row_off[2];   // grouped: where the rows of eid begin in A
     if constexpr (GROUPED) {
-      skip_nxt = false;
-      if (fetch_valid) {
-        bool any = false;
+      bool any = false;
+      int replicas = g.replicas;
+      asm volatile("" : "+s"(replicas));
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int m = m0 + wm0 + 64 * u + lane;
-          const int id = m < g.M ? g.sorted_token_ids[m] : -1;
-          any = any || (id >= 0 && id < g.num_valid_ids);
-        }
-        skip_nxt = __builtin_amdgcn_ballot_w64(any) == 0;
+      for (int u = 0; u < 2; ++u) {
+        const int id = eid[u];
+        const bool ok = id >= 0 && id < g.num_valid_ids;
+        any = any || ok;
+        row_off[u] = ok ? (uint32_t)((int64_t)(id / replicas) * g.lda) : kOobOffset;
       }
+      skip_nxt = __builtin_amdgcn_ballot_w64(any) == 0;
     }
     int expert = 0;
     if constexpr (GROUPED) {
       // an id outside [0, experts) would move the descriptor's base past W, where the range check no longer helps
-      expert = g.sorted_expert_ids[m0 / g.tile_m];
+      expert = __builtin_amdgcn_readfirstlane(expert_nxt);
       expert = expert < 0 ? 0 : (expert >= g.num_experts ? g.num_experts - 1 : expert);
     }
     const uint8_t* Bbase = g.B + (GROUPED ? (int64_t)expert * g.b_expert_stride : 0);
     rsB = make_rsrc(Bbase, operand_bytes(g.N, g.ldb, Kb_b));
 #pragma unroll
     for (int q = 0; q < AL; ++q) {
-      int64_t grow = m0 + a_row0 + q * 4 * P::A_RPI;
-      bool ok = fetch_valid && grow < g.M;
       if constexpr (GROUPED) {
-        const int id = ok ? g.sorted_token_ids[grow] : 0x7FFFFFFF;
-        ok = ok && id >= 0 && id < g.num_valid_ids;
-        grow = id / g.replicas;
+        // (the team's row of instruction q: all of them lie in one half of the 128 when q is known)
+        const uint32_t off = __builtin_amdgcn_ds_bpermute(((row + q * 4 * P::A_RPI) & 63) * 4, row_off[q * 4 * P::A_RPI / 64]);
+        a_voff[q] = off == kOobOffset ? off : off + a_col0 + ka0;
+      } else {
+        const int64_t grow = m0 + wm0 + row + q * 4 * P::A_RPI;
+        a_voff[q] = fetch_valid && grow < g.M ? (uint32_t)(grow * g.lda + a_col0) + ka0 : kOobOffset;
       }
-      a_voff[q] = ok ? (uint32_t)(grow * g.lda + a_col0) + ka0 : kOobOffset;
     }
     if constexpr (TEAM == 1) {
 #pragma unroll
       for (int q = 0; q < BL; ++q) {
-        const int col = b_col(q);
+        const int col = b_col(q, ln);
         const int64_t grow = n0 + b_row0 + q * P::B_RPI;
         b_voff[q] = (fetch_valid && grow < g.N) ? (uint32_t)(grow * g.ldb + col) + kb0 : kOobOffset;
       }
@@ -189,7 +222,7 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
       const int klim = sl < nst() ? Kb_b - kb : 0;
 #pragma unroll
       for (int q = q0; q < q1; ++q) {
-        const int col = b_col(q);
+        const int col = b_col(q, lane);
         const uint32_t v = (KTAIL && col >= klim) ? kOobOffset : b_voff[q];
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (lds_void*)(base + q * 1024), 16, v, kb, 0, 0);
       }
@@ -210,7 +243,6 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   // the lane's 8 consecutive outputs of a tile pair as 16-byte stores: every row start 16-byte aligned
   const bool vec8_ok = ((g.ldc * (int64_t)sizeof(OutT)) % 16 == 0) && (((uintptr_t)g.C) % 16 == 0);
   const bool accumulate = g.accumulate != 0;
-  int eid[2] = {-1, -1};
   auto write_tile = [&](int m0, int n0) {
     if constexpr (!GROUPED) {
       // interior tile, plain store: one address per lane, everything else immediate offsets
@@ -283,29 +315,14 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
       for (int j = 0; j < 4; ++j) acc[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
     }
   };
-  // grouped: the routed-slot ids of the team's 128 rows of the tile at m0, two per lane
-  auto load_row_ids = [&](int m0) {
-    if constexpr (GROUPED) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int m = m0 + wm0 + 64 * u + lane;
-        eid[u] = m < g.M ? g.sorted_token_ids[m] : -1;
-      }
-    }
-  };
-
   // ---- prologue: stages 0 and 1 of the first tile, scales of its K-quad 0 ---------------------------------
   // (without SPLIT the walk is the arithmetic sequence alone)
   auto next = [&](int t) { return SPLIT ? walk.next(t) : t + walk.step; };
   int lid = SPLIT ? walk.head() : walk.first;   // tile being computed
   // the one before tile t: the tail follows the workgroup's tile of the last whole round
   auto before = [&](int t) { return (SPLIT && t >= walk.end ? walk.end + ((int)blockIdx.x >> 3) : t) - walk.step; };
+  request_tile(lid);
   set_fetch_tile(lid);
-  {
-    int fm0, fn0;
-    walk.origin<C::BM>(lid, fm0, fn0);
-    load_row_ids(fm0);
-  }
   kq = kq_nxt;
   issue_a(0, 0);
   issue_b(0, 0);
@@ -339,17 +356,15 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
         // pointers of the stores when the tile begins and keeps them in registers through all its stages)
         int plid = before(lid);   // (always a whole tile: a split one is the last of the walk)
         asm volatile("" : "+s"(plid));
-        int pm0, pn0;
-        walk.origin<C::BM>(plid, pm0, pn0);
+        int pm0 = 0, pn0 = n_out;   // (grouped rows are placed by their ids)
+        if constexpr (!GROUPED) walk.origin<C::BM>(plid, pm0, pn0);
         write_tile(pm0, pn0);
-        if constexpr (GROUPED) {
-          walk.origin<C::BM>(lid, pm0, pn0);
-          load_row_ids(pm0);
-        }
       }
     }
+    if (GROUPED && t0 == 0 && Q == (nst() > 3 ? (nst() - 3) / SPQ : 0)) request_tile(next(lid));
     // from stage nst - 2 on, the loads run ahead into the next tile of the walk
     if (s + 2 == nst()) set_fetch_tile(next(lid));
+    if (GROUPED && s + 1 == nst()) load_row_ids(true, m_cur);
     const bool wrapped = s + 2 >= nst();
     const int sl = wrapped ? s + 2 - nst() : s + 2;   // local stage the loads fetch
     const int sl_eff = (wrapped && (!fetch_valid || nst() < 2)) ? nst() : sl;
@@ -448,6 +463,8 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   };
   for (; SPLIT ? lid != kNoTile : lid < walk.end; lid = next(lid)) {
     skip_cur = skip_nxt;
+    n_out = n_cur;
+    m_cur = m_nxt; n_cur = n_nxt;
     kq = kq_nxt;
     as_cur[0] = as_nxt[0];
     as_cur[1] = as_nxt[1];
@@ -462,8 +479,8 @@ __device__ __forceinline__ void pp_body(const GemmArgs& g, lds_u8* const smem, c
   __builtin_amdgcn_s_waitcnt(0x0F70);   // trailing zero-fill DMA has left the queue
   __builtin_amdgcn_sched_barrier(0);
   if (!SPLIT || walk.tail == kNoTile) {
-    int pm0, pn0;
-    walk.origin<C::BM>(SPLIT ? walk.first + (walk.end - 1 - walk.first) / walk.step * walk.step : lid - walk.step, pm0, pn0);
+    int pm0 = m_cur, pn0 = n_cur;
+    if constexpr (!GROUPED) walk.origin<C::BM>(SPLIT ? walk.first + (walk.end - 1 - walk.first) / walk.step * walk.step : lid - walk.step, pm0, pn0);
     write_tile(pm0, pn0);
   } else {
     // partial sums, as the lanes hold them: 1 KiB per store instruction
@@ -533,7 +550,12 @@ __global__ __launch_bounds__(256) void pp_tail_kernel(const GemmArgs g, const in
   const int rest = x.count % x.wgs, S = tail_splits(rest, x.wgs, g.K / 512, C::KSUB == 2);
   if (S == 1 || at >= rest) return;
   int m0, n0;
-  walk.origin(x.start + x.count - rest + at, m0, n0);
+  if constexpr (GROUPED) {
+    ExpertRuns runs = {g.sorted_expert_ids, g.tile_m, walk.tiles_m, walk.tiles_n};
+    runs.origin(x.start + x.count - rest + at, m0, n0);
+  } else {
+    walk.origin(x.start + x.count - rest + at, m0, n0);
+  }
   const int n = n0 + (wv & 3) * 64 + 8 * gq;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
