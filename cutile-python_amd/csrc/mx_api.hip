@@ -505,7 +505,8 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       const bool plain = ok && t128_plain_scales(as2.ptr, as2.stride[0], as2.stride[1], M, K, A->dtype, B->dtype) &&
                          t128_plain_scales(bs2.ptr, bs2.stride[1], bs2.stride[0], N, K, A->dtype, B->dtype) &&
                          bstride(As) % 4 == 0 && bstride(Bs) % 4 == 0;
-      const bool any = ok && !plain && t128_any_scales(as2.stride[0], as2.stride[1], M, K) && t128_any_scales(bs2.stride[1], bs2.stride[0], N, K);
+      const bool any = ok && !plain && t128_any_pays(M, N, K, batch, A->dtype == MX_E2M1 && B->dtype == MX_E2M1) &&
+                       t128_any_scales(as2.stride[0], as2.stride[1], M, K) && t128_any_scales(bs2.stride[1], bs2.stride[0], N, K);
       int64_t chunk = plain ? batch : (workspace ? workspace_bytes / per : 0);
       if (any && chunk >= 1) chunk = batch;   // (reads the scales where they are; callers are held to the workspace all the same)
       if (chunk > 32768) chunk = 32768;
@@ -762,8 +763,9 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
     const bool b_can = o.b_scale_layout == MX_SCALE_2D &&
                        t128_plain_scales(Bs->ptr, Bs->stride[1], Bs->stride[0], N, K, A->dtype, B->dtype);
     g.a_plain = a_can; g.b_plain = a_can && b_can;
-    // (in place however the rows lie: the re-layout launch costs a small product a third of its time, mx_gemm_t128.hip)
+    // (in place however the rows lie, where that pays: the re-layout launch costs a small product a third of its time)
     if (!g.b_plain && o.a_scale_layout == MX_SCALE_2D && o.b_scale_layout == MX_SCALE_2D &&
+        t128_any_pays(M, N, K, 1, A->dtype == MX_E2M1 && B->dtype == MX_E2M1) &&
         t128_any_scales(As->stride[0], As->stride[1], M, K) && t128_any_scales(Bs->stride[1], Bs->stride[0], N, K))
       g.a_plain = g.b_plain = kT128ScalesAny;
     const bool pack_a = !g.a_plain && !is_native(o.a_scale_layout), pack_b = !g.b_plain && !is_native(o.b_scale_layout);

@@ -40,6 +40,14 @@ inline bool t128_any_scales(int64_t ld, int64_t k_stride, int64_t rows, int64_t 
   const int64_t lim = ((int64_t)1 << 31) - 64;   // (the last quad's window reaches beyond its row)
   return k_stride == 1 && K >= 32 && rows * ld < lim && (rows - 1) * ld + K / 32 < lim;
 }
+// ... where that is the faster way: it costs every stage of every tile, the re-layout launch costs a call 3 .. 4 us.  MXFP8 (any | re-
+// laid first): 1024 x 1024 x 5440 18.9 | 21.6 us, 2048 x 2048 x 5440 35.1 | 36.0, 3072 x 1500 x 4000 (9216 stages) 41.6 | 41.3, x 5440
+// 51.7 | 47.0, 5653 x 944 x 5440 49.2 | 46.9; MXFP4: 2048 x 2048 x 5440 25.7 | 26.4, 3072 x 1500 x 4000 (4608) 28.7 | 29.4, x 5440
+// 35.0 | 33.7.
+inline bool t128_any_pays(int64_t M, int64_t N, int64_t K, int64_t batch, bool fp4) {
+  const int64_t stages = (K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128);
+  return ((M + 127) / 128) * ((N + 127) / 128) * batch * stages <= (fp4 ? 4800 : 10000);
+}
 // 64 x 64 tiles of a product; up to kT128SmallTiles workgroups (two for every CU) of them run instead of 128 x 128 ones
 // (measured either side in mx_gemm_t128.hip)
 constexpr int64_t kT128SmallTiles = 512;

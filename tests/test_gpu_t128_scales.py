@@ -35,6 +35,17 @@ def test_rows_at_any_byte(ct, dev, fa, fb, M, N, K, oa, pa, ob, pb):
     assert O.rel_fro(out.cpu(), oracle_matmul(a, b)) <= TOL
 
 
+@pytest.mark.parametrize("fa,fb", PAIRS, ids=str)
+@pytest.mark.parametrize("K", [4000, 4384])   # the last that is read in place, the first that is re-laid (288 tiles)
+def test_either_side_of_the_line(ct, dev, fa, fb, K):
+    M, N = 2177, 1930
+    a, b = raw_operand(M, K, fa, 1300 + K, dev), raw_operand(N, K, fb, 1400 + K, dev)
+    run = lambda sa, sb: ct.block_scaled_matmul(a.storage, sa, b.storage.T, sb, a_format=a.fmt_kw, b_format=b.fmt_kw,
+                                                kernel="mfma128", out_dtype=torch.float32)
+    out = run(_placed(a.scale_t, 1, 0), _placed(b.scale_t, 3, 5).T)
+    assert torch.equal(out, run(ct.pack_scales(a.scale_t, operand="a"), ct.pack_scales(b.scale_t, operand="b")))
+
+
 @pytest.mark.parametrize("fmt", [O.E4M3, O.E2M1])
 def test_in_lists_and_batches(ct, dev, fmt):
     shapes = [(96, 200, 96), (128, 128, 512), (300, 64, 1056), (33, 130, 32), (257, 129, 992)]
