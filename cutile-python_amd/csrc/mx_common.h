@@ -88,6 +88,9 @@ constexpr int kLoadOnce = 2;
 // (28672 x 8192 FP8, 8 rows, 45 -> 40 us; FP4, 32 rows, 25.9 -> 23.7).  Smaller ones gain as much where they come from memory
 // (14336 x 4096 FP8, 8 rows, 16.1 -> 14.7) and lose more where two or three of them take turns (11.5 -> 14.3).
 constexpr int64_t kLoadOnceBytes = (int64_t)96 << 20;
+// ... of W: rows of whole 128-byte lines only.  A line that two rows share is asked for by two waves, the second time
+// after it has gone (25600 x 11392 MXFP4, rows of 44.5 lines: 33 rows 51.0 -> 52.6 us, 8 rows 38.9 -> 39.3).
+inline bool load_once(int64_t bytes, int64_t ldw) { return bytes >= kLoadOnceBytes && ldw % 128 == 0; }
 
 // ---- fp32 -> bf16 bits, round to nearest even (torch's .to(bfloat16)) ---------------------------
 __device__ inline uint16_t f32_to_bf16(float f) {

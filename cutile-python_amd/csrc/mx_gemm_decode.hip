@@ -377,7 +377,7 @@ int launch_gemm_decode(const DecodeArgs& d, hipStream_t stream) {
   const int tiles = d.N / 16;
   const int grid = tiles < 256 ? tiles : 256;
   if (grid == 0) return MX_OK;
-  if (d.N * d.ldw >= kLoadOnceBytes)
+  if (load_once(d.N * d.ldw, d.ldw))
     return d.x_fmt == MX_E4M3 ? launch_decode_x<MX_E4M3, true>(d, grid, stream) : launch_decode_x<MX_E5M2, true>(d, grid, stream);
   return d.x_fmt == MX_E4M3 ? launch_decode_x<MX_E4M3, false>(d, grid, stream) : launch_decode_x<MX_E5M2, false>(d, grid, stream);
 }

@@ -118,7 +118,7 @@ template <int XF, int WF, int NT, int MT>
 int launch_p(const StreamArgs& a, int blocks, hipStream_t stream) {
   constexpr int W = stream_waves(MT, WF);
   if constexpr (NT == 4)
-    if (a.N * a.ldw >= kLoadOnceBytes)
+    if (load_once(a.N * a.ldw, a.ldw))
       return a.ws_packed ? launch<StreamCfg<XF, WF, NT, MT, true, W, false, true>>(a, blocks, stream)
                          : launch<StreamCfg<XF, WF, NT, MT, false, W, false, true>>(a, blocks, stream);
   return a.ws_packed ? launch<StreamCfg<XF, WF, NT, MT, true, W>>(a, blocks, stream)
