@@ -90,9 +90,11 @@ int plan_k_splits(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
 // Fitted to measurements of 96 .. 4096 rows x 512 .. 28672 columns x 512 .. 9216 (stages of 128 bytes of a row, launches
 // back to back, MXFP8; FP4 x FP4 has constants of its own):
 //   64 x 64 and 128 x 128 tiles (mx_gemm_t128.hip picks by their number): a stage of 64 x 64 tiles 0.25 us with one on a CU
-//     (1024 x 1024 x 4096 13.4 us), 0.36 with two (512 x 4096 x 4096 17.1); of 128 x 128 ones 0.62 with one on a CU (2048 x
-//     2048 x 8192 45 us), then by their number (2048 x 4096 x 4096 40, 1531 x 14336 x 4096 95).  Split along K: the partial
-//     sums are written and read by a second launch.
+//     (1024 x 1024 x 4096 13.4 us), 0.42 with two (512 x 4096 x 4096 17.1, 335 x 2896 x 6144 24.3, x 12288 45.5); of 128 x 128
+//     ones 0.53 with one on every other CU (335 x 2896 x 12288 in two slices 36.5), 0.62 with one on each (2048 x 2048 x 8192
+//     45), then by their number (2048 x 4096 x 4096 40, 1531 x 14336 x 4096 95).  Split along K: the partial sums are written
+//     and read by a second launch (335 x 2896 x 6144 in 1, 2, 3, 6, 12 slices 24.3, 24.3, 21.5, 23.4, 32.3 us; 128 x 1024 x
+//     12288 in 1, 4, 6, 12: 28.4, 15.7, 15.0, 17.2).
 //   256 x 256 tiles: a round's length and, as the clock falls the busier the chip is, its share of tiles (4096^3, one full
 //     round, 50; 2048 x 4096 x 4096, half of one, 44; 1531 x 14336 x 4096, 1.31 rounds, 86); it needs re-laid scales.
 //   192 x 256 tiles: a round of them is 18 % shorter for 25 % fewer rows (more of a stage is not MFMA), which pays where it
@@ -106,8 +108,8 @@ float est_t128_split(int64_t M, int64_t N, int64_t K, int S, bool fp4, int64_t b
   const int64_t small = t128_small_tiles(M, N) * S * batch, wgs = ((M + 127) / 128) * ((N + 127) / 128) * S * batch;
   const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)) / S;
   float stage;
-  if (small <= kT128SmallTiles) stage = small <= 256 ? (fp4 ? 0.33f : 0.25f) : (fp4 ? 0.43f : 0.36f);
-  else if (wgs <= 256) stage = fp4 ? 0.68f : 0.62f;
+  if (small <= kT128SmallTiles) stage = small <= 256 ? (fp4 ? 0.33f : 0.25f) : (fp4 ? 0.47f : 0.42f);
+  else if (wgs <= 256) stage = 0.42f + (fp4 ? 0.26f : 0.20f) * wgs / 256;
   else stage = 0.1f + (fp4 ? 1.25f : 1.05f) * (wgs < 435 ? 0.85f : wgs / 512.f);
   float t = 4.5f + st * stage;
   if (small <= kT128SmallTiles) {   // many columns for few rows: the time that reading B takes
@@ -115,7 +117,7 @@ float est_t128_split(int64_t M, int64_t N, int64_t K, int S, bool fp4, int64_t b
     const float read = 1.3f + b / (b < 96e6f ? 4.8e6f : 3.8e6f);
     if (read > t) t = read;
   }
-  return t + (S > 1 ? 3.f + (float)S * M * N * 8 / 4e6f : 0.f);
+  return t + (S > 1 ? 3.f + 0.25f * S + (float)S * M * N * 8 / 5.5e6f : 0.f);
 }
 // Of the ways to split K that there is room for (up to S; automatic splits only) the best one: none, all, or as many as give
 // every CU one or two 64 x 64 tiles.
