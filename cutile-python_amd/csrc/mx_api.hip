@@ -90,7 +90,8 @@ int plan_k_splits(int64_t M, int64_t N, int64_t K, const mx_gemm_opts& o) {
 // Fitted to measurements of 96 .. 4096 rows x 512 .. 28672 columns x 512 .. 9216 (stages of 128 bytes of a row, launches
 // back to back, MXFP8; FP4 x FP4 has constants of its own):
 //   64 x 64 and 128 x 128 tiles (mx_gemm_t128.hip picks by their number): a stage of 64 x 64 tiles 0.25 us with one on a CU
-//     (1024 x 1024 x 4096 13.4 us), 0.42 with two (512 x 4096 x 4096 17.1, 335 x 2896 x 6144 24.3, x 12288 45.5); of 128 x 128
+//     (1024 x 1024 x 4096 13.4 us), 0.42 with two (512 x 4096 x 4096 17.1, 335 x 2896 x 6144 24.3, x 12288 45.5), 0.21
+//     and 0.32 with FP4 weights (221 x 4096 x 1408 6.7, 221 x 7424 x 1408 7.8, 200 x 8192 x 2048 9.4); of 128 x 128
 //     ones 0.53 with one on every other CU (335 x 2896 x 12288 in two slices 36.5), 0.62 with one on each (2048 x 2048 x 8192
 //     45), then by their number (2048 x 4096 x 4096 40, 1531 x 14336 x 4096 95).  Split along K: the partial sums are written
 //     and read by a second launch (335 x 2896 x 6144 in 1, 2, 3, 6, 12 slices 24.3, 24.3, 21.5, 23.4, 32.3 us; 128 x 1024 x
@@ -108,7 +109,7 @@ float est_t128_split(int64_t M, int64_t N, int64_t K, int S, bool fp4, int64_t b
   const int64_t small = t128_small_tiles(M, N) * S * batch, wgs = ((M + 127) / 128) * ((N + 127) / 128) * S * batch;
   const float st = (float)((K + (fp4 ? 255 : 127)) / (fp4 ? 256 : 128)) / S;
   float stage;
-  if (small <= kT128SmallTiles) stage = small <= 256 ? (fp4 ? 0.33f : 0.25f) : (fp4 ? 0.47f : 0.42f);
+  if (small <= kT128SmallTiles) stage = small <= 256 ? (fp4 ? 0.33f : fp4_b ? 0.21f : 0.25f) : (fp4 ? 0.47f : fp4_b ? 0.32f : 0.42f);
   else if (wgs <= 256) stage = 0.42f + (fp4 ? 0.26f : 0.20f) * wgs / 256;
   else stage = 0.1f + (fp4 ? 1.25f : 1.05f) * (wgs < 435 ? 0.85f : wgs / 512.f);
   float t = 4.5f + st * stage;
