@@ -1,6 +1,7 @@
 // Memory-bound helpers around the block-scaled GEMM: MX quantisation, native scale re-layout and the
 // MoE slot alignment.  All integer / byte work; results must be bit-exact.
 #include "mx_common.h"
+#include "mx_load_once.h"
 #include "mx_quant.h"
 
 namespace mx {
@@ -193,6 +194,7 @@ __device__ __forceinline__ void quant_unpack(const v4i (&t)[SRC == MX_F32 ? 2 : 
   }
 }
 
+// ONCE: the input is loaded non-temporally (mx_load_once.h); the codes are stored as ever, for the product that reads them next.
 template <int SRC, int FMT, bool UP, int U, bool ONCE>
 __global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
   constexpr int NL = SRC == MX_F32 ? 2 : 1;          // 16-byte loads per unit of 8 elements
@@ -202,10 +204,6 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
   auto load = [](const v4i* p) {
     if constexpr (ONCE) return __builtin_nontemporal_load(p);
     else return *p;
-  };
-  auto store = [](auto v, auto* p) {
-    if constexpr (ONCE) __builtin_nontemporal_store(v, p);
-    else *p = v;
   };
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t units = (uint32_t)(q.rows * (q.K / 8)), upr = (uint32_t)(q.K / 8);   // (below 2^31: the launcher's rule)
@@ -278,7 +276,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
         r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, v[2], v[3], sc, 1);
         r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, v[4], v[5], sc, 2);
         r = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r, v[6], v[7], sc, 3);
-        store(r, (uint32_t*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 4));
+        *(uint32_t*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 4) = r;
       } else {
         uint32_t w[2];
 #pragma unroll
@@ -293,7 +291,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const QuantArgs q) {
           }
           w[h] = __builtin_bit_cast(uint32_t, r);
         }
-        store((u2){w[0], w[1]}, (u2*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 8));
+        *(u2*)(q.xq + (int64_t)row[u] * q.xq_ld + (int64_t)col[u] * 8) = (u2){w[0], w[1]};
       }
       if ((lane & 3) == 0) q.scale[block] = (uint8_t)(se + 127);
     }
@@ -644,15 +642,10 @@ template <int SRC, int FMT>
 static hipError_t launch_quantize_rows(const QuantArgs& q, int64_t units, hipStream_t stream) {
   // four units per thread once that leaves every CU several waves per SIMD, else one (a single row is a few waves: the
   // launch is all latency).  The silu form holds two inputs per unit and computes for longer: two.
-  // ONCE: loaded and stored non-temporally, from 96 MB of input on.  Smaller ones gain as much by themselves (4096^2 12.5 -> 11.2 us)
-  // where they come from memory, but an input that was just written is slower (8192^2, the same one every time, 30.2 -> 33.7;
-  // in front of a product 3973 x 2048 24.1 -> 25.2 for the pair), and so is the product that reads the codes next (1257 x 7808
-  // in front of 2816 columns 45.1 -> 48.3).
 #define MX_Q(UP, U, ONCE) return launch_kernel(quantize_rows_kernel<SRC, FMT, UP, U, ONCE>, dim3((unsigned)((units + 256 * U - 1) / (256 * U))), dim3(256), 0, stream, q)
   const bool large = units >= ((int64_t)1 << 20);
-  const bool beyond = units * 8 * (SRC == MX_F32 ? 4 : 2) >= kLoadOnceBytes;
   if (q.up) { if (large) MX_Q(true, 2, false); else MX_Q(true, 1, false); }
-  else if (large) { if (beyond) MX_Q(false, 4, true); else MX_Q(false, 4, false); }
+  else if (large) { if (quantize_loads_once(units * 8)) MX_Q(false, 4, true); else MX_Q(false, 4, false); }
   else MX_Q(false, 1, false);
 #undef MX_Q
 }

@@ -1,0 +1,33 @@
+"""The sizes from which a kernel reads an operand past the caches (csrc/mx_load_once.h), on the host."""
+import pathlib
+import subprocess
+
+import pytest
+
+CSRC = pathlib.Path(__file__).resolve().parent.parent / "cutile-python_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def evaluate(tmp_path_factory):
+    """Values of C++ expressions over the header."""
+    d = tmp_path_factory.mktemp("load_once")
+
+    def run(*expressions):
+        body = "".join(f'std::printf("%d\\n", (int)({e}));' for e in expressions)
+        (d / "p.cpp").write_text('#include <cstdio>\n#include "mx_load_once.h"\nusing namespace mx;\nint main() { %s }\n' % body)
+        subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", f"-I{CSRC}", "-o", str(d / "p"), str(d / "p.cpp")], check=True)
+        return [int(v) for v in subprocess.run([str(d / "p")], check=True, capture_output=True, text=True).stdout.split()]
+    return run
+
+
+def test_quantiser_input(evaluate):
+    """The line is a number of elements: 32-bit input between 96 and 192 MB is slower that way, with a product behind and
+    without one."""
+    mi = 1 << 20
+    assert evaluate(f"quantize_loads_once({48 * mi})", f"quantize_loads_once({48 * mi} - 8)", "quantize_loads_once(3072LL * 8192)",
+                    "quantize_loads_once(8192LL * 8192)") == [1, 0, 0, 1]
+
+
+def test_quantiser_stores_its_codes_for_whoever_reads_next():
+    """A product reads the codes behind the quantiser: no store of theirs is non-temporal."""
+    assert "nontemporal_store" not in (CSRC / "mx_aux.hip").read_text()
