@@ -81,16 +81,8 @@ __device__ inline float decode_elem(uint32_t c, int fmt) {
   return fmt == MX_E4M3 ? decode_e4m3(c) : fmt == MX_E5M2 ? decode_e5m2(c) : decode_e2m1(c);
 }
 
-// Cache policy of a buffer load (its last operand) whose lines nothing reads again: non-temporal, evicted first.
+// Cache policy of a buffer load (its last operand) whose lines nothing reads again: non-temporal, evicted first (where: mx_load_once.h).
 constexpr int kLoadOnce = 2;
-// Weights of a launch that are read that way: from 96 MB on.  Two such matrices do not fit into the 256 MB Infinity Cache with
-// what lies between, so that a loop over a model's layers finds none of their lines again, and the plain policy costs 7 - 10 %
-// (28672 x 8192 FP8, 8 rows, 45 -> 40 us; FP4, 32 rows, 25.9 -> 23.7).  Smaller ones gain as much where they come from memory
-// (14336 x 4096 FP8, 8 rows, 16.1 -> 14.7) and lose more where two or three of them take turns (11.5 -> 14.3).
-constexpr int64_t kLoadOnceBytes = (int64_t)96 << 20;
-// ... of W: rows of whole 128-byte lines only.  A line that two rows share is asked for by two waves, the second time
-// after it has gone (25600 x 11392 MXFP4, rows of 44.5 lines: 33 rows 51.0 -> 52.6 us, 8 rows 38.9 -> 39.3).
-inline bool load_once(int64_t bytes, int64_t ldw) { return bytes >= kLoadOnceBytes && ldw % 128 == 0; }
 
 // ---- fp32 -> bf16 bits, round to nearest even (torch's .to(bfloat16)) ---------------------------
 __device__ inline uint16_t f32_to_bf16(float f) {

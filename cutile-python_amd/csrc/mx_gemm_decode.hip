@@ -22,6 +22,7 @@
 #include <stdlib.h>
 
 #include "mx_common.h"
+#include "mx_load_once.h"
 
 namespace mx {
 namespace {
@@ -377,7 +378,7 @@ int launch_gemm_decode(const DecodeArgs& d, hipStream_t stream) {
   const int tiles = d.N / 16;
   const int grid = tiles < 256 ? tiles : 256;
   if (grid == 0) return MX_OK;
-  if (load_once(d.N * d.ldw, d.ldw))
+  if (weights_load_once(d.N, d.K / 2, d.ldw))
     return d.x_fmt == MX_E4M3 ? launch_decode_x<MX_E4M3, true>(d, grid, stream) : launch_decode_x<MX_E5M2, true>(d, grid, stream);
   return d.x_fmt == MX_E4M3 ? launch_decode_x<MX_E4M3, false>(d, grid, stream) : launch_decode_x<MX_E5M2, false>(d, grid, stream);
 }

@@ -24,12 +24,13 @@
 
 #include "mx_gemm_pp.h"   // vmcnt_imm
 #include "mx_gemm_tile.h"
+#include "mx_load_once.h"
 #include "mx_stream.h"
 
 namespace mx {
 
 // UP: the four tiles of a wave are 32 rows of the gate half of W and the 32 rows of the up half that belong to them.
-// ONCE: W is read non-temporally (kLoadOnceBytes).
+// ONCE: W is read non-temporally (stream_loads_once).
 template <int XF_, int WF_, int NT_, int MT_, bool PACKED_, int WAVES_ = 8, bool UP_ = false, bool ONCE_ = false>
 struct StreamCfg {
   static constexpr int XF = XF_, WF = WF_, NT = NT_, MT = MT_, WAVES = WAVES_;

@@ -118,7 +118,7 @@ template <int XF, int WF, int NT, int MT>
 int launch_p(const StreamArgs& a, int blocks, hipStream_t stream) {
   constexpr int W = stream_waves(MT, WF);
   if constexpr (NT == 4)
-    if (load_once(a.N * a.ldw, a.ldw))
+    if (stream_loads_once(a.N, WF == MX_E2M1 ? a.K / 2 : a.K, a.ldw, (uint64_t)a.W, a.m_tiles))
       return a.ws_packed ? launch<StreamCfg<XF, WF, NT, MT, true, W, false, true>>(a, blocks, stream)
                          : launch<StreamCfg<XF, WF, NT, MT, false, W, false, true>>(a, blocks, stream);
   return a.ws_packed ? launch<StreamCfg<XF, WF, NT, MT, true, W>>(a, blocks, stream)

@@ -199,7 +199,8 @@ template <int WF, bool PACKED, bool UP>
 int launch_mt(const MoeStreamArgs& a, int mt, int blocks, hipStream_t stream) {
   // (experts that no id names are not read; from 20 rows per expert on some have more than a pass takes, and read W again: 32
   // experts of 1536 x 2048, 30 rows each, 105.6 us, 109.5 non-temporally)
-  if (a.n_ids <= (int64_t)a.E * 20 && load_once((int64_t)(a.n_ids < a.E ? a.n_ids : a.E) * a.N * a.ldw, a.ldw))
+  const int64_t rows = (int64_t)(a.n_ids < a.E ? a.n_ids : a.E) * a.N;
+  if (a.n_ids <= (int64_t)a.E * 20 && stream_loads_once(rows, WF == MX_E2M1 ? a.K / 2 : a.K, a.ldw, (uint64_t)a.W | (uint64_t)a.w_es, 1))
     return mt == 1 ? launch<StreamCfg<MX_E4M3, WF, 4, 1, PACKED, 4, UP, true>>(a, blocks, stream)
                    : launch<StreamCfg<MX_E4M3, WF, 4, 2, PACKED, 4, UP, true>>(a, blocks, stream);
   return mt == 1 ? launch<StreamCfg<MX_E4M3, WF, 4, 1, PACKED, 4, UP>>(a, blocks, stream)

@@ -31,3 +31,13 @@ def test_quantiser_input(evaluate):
 def test_quantiser_stores_its_codes_for_whoever_reads_next():
     """A product reads the codes behind the quantiser: no store of theirs is non-temporal."""
     assert "nontemporal_store" not in (CSRC / "mx_aux.hip").read_text()
+
+
+def test_streamed_weights(evaluate):
+    """Whole lines that one workgroup alone reads, 96 MB of them: not behind several row tiles, not from inside a line, not a view
+    or a broadcast that spans as much and reads less."""
+    big = 12288, 8192, 8192   # rows, bytes read of a row, pitch: 96 MB
+    call = lambda rows, row, pitch, at=0, tiles=1: f"stream_loads_once({rows}, {row}, {pitch}, {at}, {tiles})"
+    assert evaluate(call(*big), call(*big, 128), call(12288, 8192, 8192 + 128), call(25000, 4096, 4096)) == [1] * 4
+    assert evaluate(call(12287, 8192, 8192), call(*big, 0, 2), call(*big, 16), call(*big, 64), call(*big, 0x1000 | 8192 + 16),
+                    call(12288, 8192, 8192 + 64), call(14336, 4096, 8192), call(1 << 20, 8192, 0)) == [0] * 8
