@@ -41,3 +41,13 @@ def test_streamed_weights(evaluate):
     assert evaluate(call(*big), call(*big, 128), call(12288, 8192, 8192 + 128), call(25000, 4096, 4096)) == [1] * 4
     assert evaluate(call(12287, 8192, 8192), call(*big, 0, 2), call(*big, 16), call(*big, 64), call(*big, 0x1000 | 8192 + 16),
                     call(12288, 8192, 8192 + 64), call(14336, 4096, 8192), call(1 << 20, 8192, 0)) == [0] * 8
+
+
+def test_shapes_of_the_gpu_tests_reach_the_non_temporal_instances(evaluate):
+    import test_gpu_load_once as g
+    byte = lambda fmt, k: k // 2 if fmt == "e2m1" else k
+    assert evaluate(*[f"stream_loads_once({n}, {byte(f, g.STREAM_K)}, {byte(f, g.STREAM_K)}, 0, 1)" for f, n in g.STREAM_N.items()],
+                    *[f"weights_load_once({n}, {k // 2}, {k // 2})" for n, k in g.DECODE_NK],
+                    *[f"stream_loads_once({min(t * g.MOE_TOPK, e) * rows}LL, {byte(f, k)}, {byte(f, k)}, 0, 1)"
+                      for f, e in g.MOE_E.items() for t in g.MOE_T for rows, k in ((2 * g.MOE_F, g.MOE_H), (g.MOE_OUT, g.MOE_F))]
+                    ) == [1] * (len(g.STREAM_N) + len(g.DECODE_NK) + 4 * len(g.MOE_T))
