@@ -1276,14 +1276,19 @@ struct MoePlan {
   int64_t q, qs, c3, c1, slots, in_use, max_slots, blocks, align, grouped, grouped_bytes, total;   // offsets (bytes)
 };
 // Rows per expert up to which the weights are streamed.  us per layer, streamed | grouped with 256-slot tiles:
-//   16 experts of 4096 x 4096, FP8: 32 rows 218 | 266, 48 rows 276 | 273, 64 rows 336 | 283; FP4: 32 rows 139 | 183, 48 rows
-//   173 | 187, 64 rows 238 | 193
-//   8 experts of 4096 x 14336, FP8: 16 rows 231 | 358, 32 rows 372 | 366, 48 rows 453 | 373; FP4: 32 rows 239 | 282, 48 rows
-//   274 | 286
+//   16 experts of 4096 x 4096, FP8: 32 rows 218 | 266, 64 rows 336 | 283; FP4: 32 rows 139 | 183, 48 rows 173 | 187, 64 rows
+//   238 | 193
+//   8 experts of 4096 x 14336, FP8: 16 rows 231 | 358, 32 rows 372 | 366; FP4: 32 rows 239 | 282, 48 rows 274 | 286
 //   64 experts of 3584 x 1024, FP8: 32 rows 223 | 248
 // (128-slot and 64-slot tiles are slower than one or the other everywhere.)  Beyond 32 rows an expert's weights are read once
-// more; against that stand the tiles' extra passes, some 40 us whatever the size: from 1 GB of weights on the tiles are ahead
-// (34 rows: 1.41 GB 393 | 366, 0.81 GB 231 | 264).
+// more; against that stand the tiles' extra passes, some 40 us whatever the size.  33, 40 and 48 rows:
+//   0.81 GB: 8 experts 226 | 282, 245 | 284, 262 | 286; 16 experts 234 | 254, 252 | 257, 269 | 261
+//   0.96 GB: 8 experts 260 | 303, 310 | 305, 315 | 310
+//   1.06 GB: 8 experts 294 | 307, 311 | 309, 389 | 314;  1.11 GB: 16 experts 289 | 286, 358 | 290, 374 | 294, 32 experts 294 |
+//     314, 368 | 320, 384 | 325
+//   1.21 GB: 8 experts 289 | 318 (34 rows 336 | 321), 360 | 321, 392 | 327;  1.41 GB: 8 experts 357 | 360 (34 rows 384 | 362), 416 | 365,
+//     455 | 369; FP4, 16 experts 421 | 430, 505 | 437, 516 | 442
+// so that the tiles are ahead from 1 GB of weights on, at 33 rows not yet everywhere.
 // (64 rows: with a longer list of ids, mx_stream.h.)
 constexpr int64_t kMoeStreamRows = 48, kMoeStreamTwiceBytes = 1000000000;
 

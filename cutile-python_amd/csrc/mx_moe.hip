@@ -197,10 +197,13 @@ int launch(const MoeStreamArgs& a, int blocks, hipStream_t stream) {
 
 template <int WF, bool PACKED, bool UP>
 int launch_mt(const MoeStreamArgs& a, int mt, int blocks, hipStream_t stream) {
-  // (experts that no id names are not read; from 20 rows per expert on some have more than a pass takes, and read W again: 32
-  // experts of 1536 x 2048, 30 rows each, 105.6 us, 109.5 non-temporally)
+  // Non-temporal weights up to 24 rows per expert (experts that no id names are not read): beyond, experts get more rows than a
+  // pass takes and read W again.  us per layer, plain | non-temporal, rows per expert 22, 24, 28, 32: 16 experts of 4096 x 4096
+  // FP8 161 | 142, 179 | 171, 192 | 191, 216 | 227; 8 of 4096 x 14336 FP4 157 | 149, 182 | 180, 184 | 183, 214 | 227, FP8 257 |
+  // 234, 284 | 276, 293 | 278, 353 | 348; 32 of 2048 x 2048 FP8 24, 28, 32 rows 103.6 | 99, 117.4 | 119.3, 126 | 135; 64 of them FP4
+  // 140 | 138, 146 | 149, 166 | 173.
   const int64_t rows = (int64_t)(a.n_ids < a.E ? a.n_ids : a.E) * a.N;
-  if (a.n_ids <= (int64_t)a.E * 20 && stream_loads_once(rows, WF == MX_E2M1 ? a.K / 2 : a.K, a.ldw, (uint64_t)a.W | (uint64_t)a.w_es, 1))
+  if (a.n_ids <= (int64_t)a.E * 24 && stream_loads_once(rows, WF == MX_E2M1 ? a.K / 2 : a.K, a.ldw, (uint64_t)a.W | (uint64_t)a.w_es, 1))
     return mt == 1 ? launch<StreamCfg<MX_E4M3, WF, 4, 1, PACKED, 4, UP, true>>(a, blocks, stream)
                    : launch<StreamCfg<MX_E4M3, WF, 4, 2, PACKED, 4, UP, true>>(a, blocks, stream);
   return mt == 1 ? launch<StreamCfg<MX_E4M3, WF, 4, 1, PACKED, 4, UP>>(a, blocks, stream)
