@@ -154,7 +154,7 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
   }
   // kScaleAny: the wave's group through registers
   __amdgpu_buffer_rsrc_t rsAny;
-  uint32_t raw[5], shift = 0;
+  uint32_t raw[Sched::kAnyLoads], shift = 0;
   if constexpr (ANY) {
     const bool is_b = wave >= 2;
     const uintptr_t at = (uintptr_t)(is_b ? g.Bs + (int64_t)bz * g.bs_batch : g.As + (int64_t)bz * g.as_batch);
@@ -168,7 +168,7 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
   auto load_any = [&](int Q) {
     const uint32_t v = Q < q1 ? sco + Q * 16 : kOobOffset;
 #pragma unroll
-    for (int i = 0; i < 5; ++i) raw[i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsAny, v + 4 * i, 0, 0);
+    for (int i = 0; i < Sched::kAnyLoads; ++i) raw[i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsAny, v + 4 * i, 0, 0);
   };
   auto store_any = [&](int Q) {
     uint32_t d[4];

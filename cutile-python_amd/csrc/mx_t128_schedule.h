@@ -9,6 +9,9 @@
 //             s + 1 is read, at the last stage of quad Q also the scales of quad Q + 1
 // The prologue's order is the one that the stages continue.  (All scales ahead of the stages, it would leave one load
 // fewer behind stage 1 than the stages' count assumes.)
+// Scales at any byte come through registers: a quad's kAnyLoads loads are requested into them where the loads of scales above
+// have their place, one quad ahead, and go to LDS a quad later, behind the barrier of that quad's first stage; all waves read them
+// at its last stage.  (The register contents are waited for by their own use.)
 #pragma once
 
 namespace mx {
@@ -29,6 +32,7 @@ struct T128Schedule {
   }
   // Scales that come through registers are loads whose place and number the waits leave out: of the stages' loads alone,
   // NS - 1 (NS - 2) stages are behind stage 0 (s + 1), so a wait for all but these is never too short.
+  static constexpr int kAnyLoads = 5;
   static constexpr int any_prologue_wait() { return (NS - 1) * TL; }
   static constexpr int any_stage_wait() { return (NS - 2) * TL; }
 };
@@ -57,10 +61,47 @@ constexpr int t128_uncovered(int stages, bool scales_first = false, int prologue
   return -1;
 }
 
+// The same for scales at any byte; -4: a wave reads a quad's scales that another may not have written yet.  `loads`: of a quad's kAnyLoads
+// those still among the requests that a wait counts; `ahead`: of the first quad's those that lie ahead of stage 0.
+template <class S>
+constexpr int t128_any_uncovered(int stages, int loads = S::kAnyLoads, int ahead = S::kAnyLoads, int prologue_wait = S::any_prologue_wait(),
+                                 int stage_wait = S::any_stage_wait()) {
+  constexpr int kMax = 64;
+  int stage_end[kMax] = {}, issued = 0, barriers = 0;
+  int written[kMax] = {};                                // barriers ahead of it, + 1
+  if (stages + S::NS > kMax) return -3;
+  if (ahead > loads) ahead = loads;
+  issued += ahead;
+  for (int k = 0; k < S::NS; ++k) {
+    stage_end[k] = issued += S::TL;
+    if (k == 0) issued += loads - ahead;
+  }
+  if (stage_end[0] > issued - prologue_wait) return -2;
+  written[0] = barriers + 1;
+  issued += loads;                                       // quad 1
+  ++barriers;                                            // quad 0 is read behind it
+  for (int s = 0; s < stages; ++s) {
+    const int t = s % S::SPQ, quad = s / S::SPQ;
+    if (stage_end[s + 1] == 0 || stage_end[s + 1] > issued - stage_wait) return s;
+    ++barriers;
+    if (t == 0) {
+      written[quad + 1] = barriers + 1;
+      issued += loads;                                   // quad + 2
+    }
+    stage_end[s + S::NS] = issued += S::TL;
+    if (t == S::SPQ - 1 && written[quad + 1] >= barriers + 1) return -4;
+  }
+  return -1;
+}
+
 template <class S>
 constexpr bool t128_covered() {
-  for (int stages = 1; stages <= 24; ++stages)
+  for (int stages = 1; stages <= 24; ++stages) {
     if (t128_uncovered<S>(stages) != -1) return false;
+    for (int loads = 0; loads <= S::kAnyLoads; ++loads)
+      for (int ahead = 0; ahead <= loads; ++ahead)
+        if (t128_any_uncovered<S>(stages, loads, ahead) != -1) return false;
+  }
   return true;
 }
 
