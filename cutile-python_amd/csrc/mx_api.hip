@@ -147,6 +147,13 @@ float est_pp(int64_t M, int64_t N, int64_t K, bool fp4, bool pack, bool tail, in
   }
   return rest + st * (round * ((tiles + 255) / 256) + full * tiles / 256);
 }
+// rows of the ping-pong kernel's tiles under MX_KERNEL_AUTO, and what they take; tail: there is room to split the last round of 256-row
+// tiles (the 192-row form never splits)
+struct PpRows { int rows; float us; };
+PpRows pp_rows(int64_t M, int64_t N, int64_t K, bool fp4, bool pack, bool tail) {
+  const float us = est_pp(M, N, K, fp4, pack, tail), us192 = est_pp(M, N, K, fp4, pack, false, 192);
+  return us192 < us ? PpRows{192, us192} : PpRows{256, us};
+}
 float est_stream(int64_t M, int64_t N, int64_t K, int w_fmt) {
   const StreamPlan p = stream_plan(M, N, K, w_fmt);
   const bool fp4 = w_fmt == MX_E2M1;
@@ -279,8 +286,12 @@ int64_t gemm_workspace_tail(int64_t M, int64_t N, int64_t K, const mx_gemm_opts&
   if (t == 0 || o.kernel == MX_KERNEL_MFMA_PINGPONG) return t;
   if (M <= kStreamAutoM) return 0;
   const bool pack = !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout);
-  for (int fp4 = 0; fp4 < 2; ++fp4)
-    if (est_pp(M, N, K, fp4, pack, true) < est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4, fp4)) return t;
+  for (int fp4 = 0; fp4 < 2; ++fp4) {
+    const PpRows with = pp_rows(M, N, K, fp4, pack, true);
+    // (192 rows with room and without it: nothing is split)
+    if (with.rows == 192 && pp_rows(M, N, K, fp4, pack, false).rows == 192) continue;
+    if (with.us < est_t128(M, N, K, plan_k_splits(M, N, K, o), fp4, fp4)) return t;
+  }
   return 0;
 }
 int64_t grouped_workspace_min(int64_t num_slots, int64_t N, int64_t K, int64_t E, const mx_gemm_opts& o) {
@@ -639,11 +650,9 @@ int gemm_impl(const mx_tensor* A, const mx_tensor* As, const mx_tensor* B, const
       const float t128 = est_t128(M, N, K, o.split_k > 1 ? 1 : plan_k_splits(M, N, K, o), fp4, B->dtype == MX_E2M1);
       const bool room = workspace && o.split_k == 0 && pp_tail_bytes(M, N, K, fp4, true) > 0 &&
                         workspace_bytes >= ws_min + pp_tail_bytes(M, N, K, fp4, true);
-      float pp = o.split_k > 1 ? 1e30f : est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), room);
-      if (o.split_k <= 1) {
-        const float pp192 = est_pp(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), false, 192);
-        if (big_tile_kernel() == MX_KERNEL_MFMA_PINGPONG && pp192 < pp) { pp = pp192; tile_rows = 192; }
-      }
+      const PpRows p = pp_rows(M, N, K, fp4, !is_native(o.a_scale_layout) || !is_native(o.b_scale_layout), room);
+      const float pp = o.split_k > 1 ? 1e30f : p.us;
+      if (o.split_k <= 1) tile_rows = p.rows;
       const float st = may_stream ? est_stream(M, N, K, B->dtype) : 1e30f;
       kernel = st < t128 && st < pp ? MX_KERNEL_STREAM : t128 <= pp ? MX_KERNEL_MFMA_128x128 : big_tile_kernel();
     }

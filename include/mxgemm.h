@@ -156,6 +156,8 @@ MX_API int mx_device_check(void);
  * with less, down to what the scales and split-K need, or with split_k = 1 the round runs unsplit.
  * Optional are also the partial sums of a split along K other than into equal slices of 512 with plain scales (native scales,
  * another K): without room for them the product runs whole.  mx_gemm_list asks in the same way for every problem's share.
+ * The answer goes by the sizes alone: scales whose rows a kernel then reads where they are, and a format that takes another
+ * kernel, still count.
  */
 MX_API int64_t mx_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, const mx_gemm_opts* opts);
 

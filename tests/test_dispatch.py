@@ -95,6 +95,19 @@ def test_a_promised_split_is_held_to_its_workspace(split_k):
     assert lib.mx_gemm_list(1, *t, ctypes.byref(o), p, need - 256, None) == L.MX_ERR_WORKSPACE
 
 
+@pytest.mark.parametrize("M,N,K", [(6319, 3444, 9216), (1554, 13416, 10240), (759, 26481, 7680), (9970, 7006, 4096)])
+@pytest.mark.parametrize("layouts", [(0, 0), (0, 2), (2, 2)])
+def test_no_room_is_asked_for_a_split_that_192_row_tiles_do_not_make(M, N, K, layouts):
+    """MX_KERNEL_AUTO takes 192-row tiles here, with room for the split last round of 256-row tiles and without; the forced kernel,
+    which keeps to 256 rows, is given the room as before."""
+    lib = cutile_amd.lib()
+    scales = sum(lib.mx_packed_scale_bytes(rows, K) for rows, layout in ((M, layouts[0]), (N, layouts[1])) if layout == 0)
+    need = lambda **kw: lib.mx_gemm_workspace_bytes(M, N, K, ctypes.byref(
+        L.MxGemmOpts(struct_size=32, block_size=32, a_scale_layout=layouts[0], b_scale_layout=layouts[1], **kw)))
+    assert need() == need(split_k=1) == scales
+    assert need(kernel=L.MX_KERNEL_MFMA_PINGPONG) > scales
+
+
 def test_moe_slots_follow_tile_m(monkeypatch):
     """The grouped form of the layer aligns to the caller's tile_m (its workspace shrinks with the padding), refuses what the
     tiled kernels cannot take, and the operator hands its tile_m over; streamed layers have no slots."""
