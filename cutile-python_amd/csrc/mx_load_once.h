@@ -22,8 +22,9 @@ inline bool quantize_loads_once(int64_t elements) { return elements >= kQuantize
 // Weights: from 96 MB a launch on.  Two such matrices do not fit into the 256 MB Infinity Cache with what lies between, so that a
 // loop over a model's layers finds none of their lines again, and the plain policy costs 7 - 10 % (28672 x 8192 FP8, 8 rows,
 // 45 -> 40 us; FP4, 32 rows, 25.9 -> 23.7).  Smaller ones gain as much where they come from memory (14336 x 4096 FP8, 8 rows,
-// 16.1 -> 14.7) and lose more where two or three of them take turns (11.5 -> 14.3).  (Of a view or of overlapping rows: the bytes
-// that are read, once each.)
+// 16.1 -> 14.7) and lose more where two or three of them take turns (11.5 -> 14.3).  (Two alone that take turns with
+// nothing between still gain from the cache at 117 MB, 14336 x 8192 FP8 at 32 rows 21.8 against 24.6, three no longer, 27.7 against
+// 24.9; at 235 MB two do not, 48.7 against 45.2.)  Of a view or of overlapping rows the bytes that are read count, once each.
 // ... rows of whole 128-byte lines only.  A line that two rows share is asked for by two waves, the second time after it has gone
 // (25600 x 11392 MXFP4, rows of 44.5 lines: 33 rows 51.0 -> 52.6 us, 8 rows 38.9 -> 39.3).
 // The decode kernel keeps to this where it runs slab by slab of 32 rows, and where W starts inside a line, too: 28672 x 8192 at 33,
