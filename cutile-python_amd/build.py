@@ -21,7 +21,7 @@ INCLUDE = ROOT.parent / "include"
 OUT = ROOT / "cutile_amd" / "libmxgemm.so"
 HOST_OUT = ROOT / "cutile_amd" / "_mxhost.so"   # csrc/mx_host.cpp: the operators' native host path
 OBJ = ROOT / "build"
-SOURCES = ["mx_api.hip", "mx_gemm_mfma.hip", "mx_gemm_pp32.hip", "mx_gemm_w4.hip", "mx_gemm_generic.hip", "mx_gemm_decode.hip", "mx_gemm_stream.hip", "mx_moe.hip", "mx_aux.hip", "mx_probe.hip"]
+SOURCES = ["mx_api.hip", "mx_gemm_mfma.hip", "mx_gemm_pp32.hip", "mx_gemm_w4.hip", "mx_gemm_generic.hip", "mx_gemm_decode.hip", "mx_gemm_stream.hip", "mx_moe.hip", "mx_moe_tile.hip", "mx_aux.hip", "mx_probe.hip"]
 # sources compiled once per value of a macro, so that their instances build in parallel: (file, macro, count)
 SPLIT = [("mx_gemm_pp.hip", "MX_PP_PAIR", 4), ("mx_gemm_t128.hip", "T128_PAIR", 4)]
 UNITS = [(s, None) for s in SOURCES] + [(f, f"-D{m}={i}") for f, m, n in SPLIT for i in range(n)]

@@ -11,6 +11,7 @@
 #include "mx_common.h"
 #include "mx_gemm_pp.h"
 #include "mx_gemm_t128.h"
+#include "mx_moe_tile.h"
 #include "mx_stream.h"
 
 // Scratch of mx_gemm_static: lives in the library's device image, one copy per GPU the library runs on, held
@@ -1280,11 +1281,14 @@ namespace {
 // Sizes of a mixture-of-experts layer and where its pieces lie in the workspace.
 struct MoePlan {
   int64_t T, n, E, H, F, H_out;
-  bool stream;          // experts' weights streamed for a few rows each; otherwise grouped GEMMs on aligned slots
+  bool stream;          // experts' weights streamed for a few rows each
+  bool tiles;           // row tiles of their own (mx_moe_tile.hip); neither: grouped GEMMs on aligned slots
+  int32_t splits;       // tiles: K ranges of the down projection
+  int64_t max_tiles, info;
   int32_t tile_m;
   int64_t q, qs, c3, c1, slots, in_use, max_slots, blocks, align, grouped, grouped_bytes, total;   // offsets (bytes)
 };
-// Rows per expert up to which the weights are streamed.  us per layer, streamed | grouped with 256-slot tiles:
+// Rows per expert up to which the weights are streamed where the row tiles below do not take the layer.  us per layer, streamed | grouped with 256-slot tiles:
 //   16 experts of 4096 x 4096, FP8: 32 rows 218 | 266, 64 rows 336 | 283; FP4: 32 rows 139 | 183, 48 rows 173 | 187, 64 rows
 //   238 | 193
 //   8 experts of 4096 x 14336, FP8: 16 rows 231 | 358, 32 rows 372 | 366; FP4: 32 rows 239 | 282, 48 rows 274 | 286
@@ -1299,7 +1303,17 @@ struct MoePlan {
 //     455 | 369; FP4, 16 experts 421 | 430, 505 | 437, 516 | 442
 // so that the tiles are ahead from 1 GB of weights on, at 33 rows not yet everywhere.
 // (64 rows: with a longer list of ids, mx_stream.h.)
-constexpr int64_t kMoeStreamRows = 48, kMoeStreamTwiceBytes = 1000000000;
+constexpr int64_t kMoeStreamRows = 48, kMoeStreamTwiceBytes = 1000000000, kMoeTileFromRows = 24;
+
+// what keeps a layer from the row tiles of mx_moe_tile.hip (nullptr: nothing): both weights' scales packed, whole K-steps and
+// column tiles, a routing that one workgroup sorts out, and no tile height asked for that they don't have
+const char* moe_tiles_issue(const MoePlan& p, const mx_gemm_opts& o) {
+  if (o.a_scale_layout != MX_SCALE_NATIVE || o.b_scale_layout != MX_SCALE_NATIVE) return "scales are not packed";
+  if (p.H % 128 != 0 || p.F % 128 != 0) return "H or F is not a multiple of 128";
+  if (p.n > kMoeTileMaxIds || p.E > kMoeTileMaxExperts) return "too many ids or experts";
+  if (o.tile_m != 0 && o.tile_m != 256) return "tile_m";
+  return nullptr;
+}
 
 MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& W2, const mx_gemm_opts& o) {
   MoePlan p = {};
@@ -1307,12 +1321,29 @@ MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& 
   const int64_t weights = p.E * (2 * p.F * p.H + p.H_out * p.F) / (W1.dtype == MX_E2M1 ? 2 : 1);   // bytes
   const int64_t rows = weights > kMoeStreamTwiceBytes ? 32 : kMoeStreamRows;
   p.stream = p.n <= kMoeMaxIds && p.n <= p.E * rows && p.H % 128 == 0 && p.F % 128 == 0;
+  // Row tiles where the weights would be streamed more than once and as long as the 256-row tiles, which need more launches around
+  // them, are not ahead.  us per layer, streamed | row tiles, 20, 24, 28 and 32 rows per expert: 8 experts of 4096 x 14336 FP8 232 | 258, 238 |
+  // 260, 305 | 263, 336 | 267, FP4 148 | 160, 154 | 162, 193 | 166, 212 | 170; 64 of 1024 x 1024 FP8 61 | 62, 71 | 63, 78 | 64, 88 | 65.
+  // Row tiles | 256-row tiles, 96, 112, 128 and 160 rows each: 8 of 4096 x 14336 FP8 384 | 392, 418 | 402, 456 | 409, FP4 237 | 298, 258 | 314,
+  // 318 | 325, 377 | 352; 8 of 4096 x 7168 FP8 207 | 243, 228 | 248, 246 | 252, 271 | 264; 64 of 4096 x 1024 FP8 285 | 322, 307 | 332, 334 |
+  // 340, 387 | 364; 64 of 1024 x 1024 FP8 104 | 122, 114 | 125, 121 | 128, 140 | 143 (192: 160 | 149); 32 of 1024 x 2048 FP8 95 | 120, 105 | 122,
+  // 112 | 126, 127 | 134, FP4 78 | 108, 86 | 112, 92 | 117, 106 | 124.
+  const int64_t tile_limit = p.H <= 2048 ? 160 : weights > kMoeStreamTwiceBytes && W1.dtype != MX_E2M1 ? 96 : 128;
+  const bool can_tile = moe_tiles_issue(p, o) == nullptr && p.n <= p.E * tile_limit;
+  if (can_tile && p.n > p.E * kMoeTileFromRows) p.stream = false;
+  p.tiles = can_tile && !p.stream;
   int64_t off = 0;
   auto take = [&](int64_t bytes) { const int64_t at = off; off += round256(bytes); return at; };
   p.q = take(p.n * p.F);
   p.qs = take(p.n * (p.F / 32));
-  p.c3 = take(p.n * p.H_out * 4);
-  if (!p.stream) {
+  if (p.tiles) p.tile_m = moe_tile_rows(p.n, p.E, p.H, W1.dtype);
+  p.splits = p.tiles ? moe_tile_splits(p.n, p.E, p.tile_m, p.H_out, p.F) : 1;
+  p.c3 = take(p.n * p.H_out * 4 * p.splits);
+  if (p.tiles) {
+    p.max_tiles = moe_tiles_max(p.n, p.E, p.tile_m);
+    p.info = take(p.max_tiles * (int64_t)sizeof(MoeTile));
+    p.slots = take(p.max_tiles * p.tile_m * 4);
+  } else if (!p.stream) {
     p.tile_m = o.tile_m > 0 ? o.tile_m : 256;
     p.max_slots = mx_moe_align_max_slots(p.n, (int32_t)p.E, p.tile_m);
     p.c1 = take(p.n * p.F * 4);
@@ -1394,7 +1425,7 @@ int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1,
   if (!why && H_out <= 128) why = "H_out is too small";
   if (why) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: %s", why);
   const MoePlan p = moe_plan(T, topk, *W1, *W2, o);
-  if (!p.stream && p.tile_m % 128 != 0) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: tile_m is not a multiple of 128");
+  if (!p.stream && !p.tiles && p.tile_m % 128 != 0) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: tile_m is not a multiple of 128");
   if (p.n * p.F >= ((int64_t)1 << 31)) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: the activation spans 2 GiB or more");
   if (!workspace || workspace_bytes < p.total)
     return set_error(MX_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)p.total, (long long)workspace_bytes);
@@ -1422,6 +1453,29 @@ int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1,
     a.N = (int32_t)H_out; a.K = (int32_t)F;
     a.weights = topk_weights; a.C = (float*)(ws + p.c3);
     if (int rc = launch_moe_stream(a, false, st)) return rc;
+  } else if (p.tiles) {
+    MoeTileArgs a = {};
+    MoeTile* const tiles = (MoeTile*)(ws + p.info);
+    int32_t* const slots = (int32_t*)(ws + p.slots);
+    if (int rc = launch_moe_tiles(topk_ids, ids64, p.n, (int)E, p.tile_m, tiles, slots, p.max_tiles, st)) return rc;
+    a.tiles = tiles; a.slots = slots; a.max_tiles = (int32_t)p.max_tiles; a.tile_rows = p.tile_m;
+    a.n_ids = (int32_t)p.n; a.E = (int32_t)E;
+    a.w_fmt = W1->dtype; a.scale_mode = scale_mode;
+    a.X = (const uint8_t*)X->ptr; a.Xs = (const uint8_t*)Xs->ptr; a.ldx = X->stride[0]; a.ldxs = Xs->stride[0];
+    a.x_rows = (int32_t)T; a.replicas = topk;
+    a.W = (const uint8_t*)W1->ptr; a.ldw = W1->stride[1]; a.w_es = W1->stride[0];
+    a.Ws = (const uint8_t*)W1s->ptr; a.ws_es = mx_packed_scale_bytes(2 * F, H);
+    a.N = (int32_t)(2 * F); a.K = (int32_t)H; a.F = (int32_t)F; a.splits = 1;
+    a.q = ws + p.q; a.qs = ws + p.qs;
+    if (int rc = launch_moe_tile(a, true, st)) return rc;
+    a.X = ws + p.q; a.Xs = ws + p.qs; a.ldx = F; a.ldxs = F / 32;
+    a.x_rows = (int32_t)p.n; a.replicas = 1;
+    a.W = (const uint8_t*)W2->ptr; a.ldw = W2->stride[1]; a.w_es = W2->stride[0];
+    a.Ws = (const uint8_t*)W2s->ptr; a.ws_es = mx_packed_scale_bytes(H_out, F);
+    a.N = (int32_t)H_out; a.K = (int32_t)F; a.splits = p.splits;
+    a.C = (float*)(ws + p.c3); a.c_split = p.n * H_out;
+    if (int rc = launch_moe_tile(a, false, st)) return rc;
+    return launch_moe_combine(a.C, p.splits, a.c_split, topk_weights, topk_ids, ids64, (int)E, T, topk, H_out, out->ptr, out->dtype, st);
   } else {
     int32_t* const slots = (int32_t*)(ws + p.slots);
     int32_t* const blocks = (int32_t*)(ws + p.blocks);
@@ -1445,7 +1499,7 @@ int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1,
                                  ws + p.grouped, p.grouped_bytes, stream))
       return rc;
   }
-  return launch_moe_combine((const float*)(ws + p.c3), topk_ids, ids64, (int)E, T, topk, H_out, out->ptr, out->dtype, st);
+  return launch_moe_combine((const float*)(ws + p.c3), 1, 0, nullptr, topk_ids, ids64, (int)E, T, topk, H_out, out->ptr, out->dtype, st);
 }
 
 namespace {

@@ -159,8 +159,10 @@ __global__ __launch_bounds__(C::WAVES * 64, 2) void moe_stream_kernel(const MoeS
 }
 
 // out[t, :] = sum over the top-k copies of a token, in their order; a copy whose expert id is outside [0, E) was never
-// computed and counts as zero.  Four columns per thread.
-__global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ c, const void* __restrict__ ids, int ids64,
+// computed and counts as zero.  A copy is the sum of `splits` partial products, c_split elements apart, times its routed weight
+// (null: c holds the weighted ones).  Four columns per thread.
+__global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ c, int splits, int64_t c_split,
+                                                          const float* __restrict__ weights, const void* __restrict__ ids, int ids64,
                                                           int E, int64_t T, int topk, int64_t H, void* out, int out_dtype) {
   const int64_t h4 = (H + 3) / 4, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= T * h4) return;
@@ -171,10 +173,14 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restric
     const int64_t id = t * topk + k;
     const int e = ids64 ? (int)((const int64_t*)ids)[id] : ((const int32_t*)ids)[id];
     if (e < 0 || e >= E) continue;
-    const float* p = c + id * H + h;
-    if (n == 4 && (H & 3) == 0) s += *(const v4f*)p;
-    else
-      for (int x = 0; x < n; ++x) s[x] += p[x];
+    v4f v = {0.f, 0.f, 0.f, 0.f};
+    for (int sp = 0; sp < splits; ++sp) {
+      const float* p = c + sp * c_split + id * H + h;
+      if (n == 4 && (H & 3) == 0) v += *(const v4f*)p;
+      else
+        for (int x = 0; x < n; ++x) v[x] += p[x];
+    }
+    s += weights ? v * weights[id] : v;
   }
   if (out_dtype == MX_F32) store8_edge<float>((float*)out + t * H + h, s, s, n);
   else store8_edge<uint16_t>((uint16_t*)out + t * H + h, s, s, n);
@@ -240,11 +246,11 @@ int launch_moe_stream(const MoeStreamArgs& a0, bool up, hipStream_t stream) {
   return MX_ERR_DTYPE;
 }
 
-int launch_moe_combine(const float* c, const void* ids, int ids64, int E, int64_t T, int topk, int64_t H, void* out,
+int launch_moe_combine(const float* c, int splits, int64_t c_split, const float* weights, const void* ids, int ids64, int E, int64_t T, int topk, int64_t H, void* out,
                        int out_dtype, hipStream_t stream) {
   const int64_t threads = T * ((H + 3) / 4);
   if (threads <= 0) return MX_OK;
-  hipError_t e = launch_kernel(moe_combine_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, c, ids, ids64, E, T,
+  hipError_t e = launch_kernel(moe_combine_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, c, splits, c_split, weights, ids, ids64, E, T,
                                topk, H, out, out_dtype);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_combine_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;

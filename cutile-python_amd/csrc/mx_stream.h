@@ -39,7 +39,7 @@ struct MoeStreamArgs {
   int32_t kw, units;                   // chosen by the launcher
 };
 int launch_moe_stream(const MoeStreamArgs& a, bool up, hipStream_t stream);
-int launch_moe_combine(const float* c, const void* ids, int ids64, int E, int64_t T, int topk, int64_t H, void* out,
+int launch_moe_combine(const float* c, int splits, int64_t c_split, const float* weights, const void* ids, int ids64, int E, int64_t T, int topk, int64_t H, void* out,
                        int out_dtype, hipStream_t stream);
 
 }  // namespace mx

@@ -893,7 +893,8 @@ def cutile_moe_scaled(hidden_states: torch.Tensor, hidden_scale: torch.Tensor,
     call synchronises with the host.  Returns (tokens, H) in ``out_dtype``.
 
     ``tile_m`` is the number of slots that an expert's rows are padded to (128: less padding where experts get few
-    rows).  Where they get so few that the weights are streamed there are no slots, and it has no effect."""
+    rows).  Where they get so few that the weights are streamed there are no slots, and it has no effect; the default also
+    leaves the height of the row tiles to the library (medium sizes with packed scales)."""
     if kernel == "auto" and scale_mode in ("floor", "ceil"):
         # one library call for the whole layer
         r = L.host().moe(hidden_states, hidden_scale, w1, w1_scale, w2, w2_scale, topk_weights, topk_ids, out_dtype,
