@@ -7,7 +7,7 @@
 // Here the fragments of stage s + 1 are read into a second register set while the MFMAs of stage s run, behind one
 // barrier per stage, and the LDS-DMA runs NS stages ahead:
 //   iteration s:  wait until stage s + 1 has landed; barrier (everybody's part has landed, everybody has read stage s)
-//                 issue the DMA of stage s + NS into the buffer of stage s
+//                 issue the DMA of stage s + NS into the buffer of stage s (more than two stages: between the MFMAs, SPREAD)
 //                 16 (32) MFMAs of stage s, the fragment reads of stage s + 1 between them
 // (order of the requests and what the waits count: mx_t128_schedule.h).
 // 64 x 64 tiles (four waves of 32 x 32, eight stages in flight or four) take products that leave CUs idle: a stage is 0.25 us
@@ -43,6 +43,11 @@ template <class C, int NS, int AS, int BS, bool GROUPED>
 __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem, const int pid, const int split, const int bz) {
   constexpr int KS = C::KSUB, SPQ = 4 / KS, MT = C::MT, NT = C::NTL;
   constexpr bool AP = AS != kScaleNative, BP = BS != kScaleNative, ANY = AS == kScaleAny;
+  // A stage's requests go out between its MFMAs: all four waves' at once behind the barrier they keep the address unit busy for some
+  // 500 cycles, the length of a stage's MFMAs, in which none of these is issued.  2048 x 2048 x 2048 FP8 15.2 -> 13.5 us, x 8192 43.0 ->
+  // 40.9, FP4 26.9 -> 25.3, 200 x 14336 x 4096 24.3 -> 23.0.  Not with two stages, where a later request is a later stage (512 x 14336 x 4096
+  // 35.8 -> 39.6), nor beside the larger tile's scales through registers (1111 x 2100 x 4032 21.6 -> 22.2).
+  constexpr bool SPREAD = NS > 2 && !(ANY && C::BM == 128);
   static_assert(ANY == (BS == kScaleAny) && !(ANY && GROUPED) && MT == NT && (C::BM == 128 || !GROUPED), "");
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, gq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -110,15 +115,16 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
     bvo[q] = row < g.N ? (uint32_t)(row * g.ldb + b_col) : kOobOffset;
   }
   const int Ka = g.K * C::A_EB / 8, Kb = g.K * C::B_EB / 8;   // bytes of a row
-  auto issue = [&](int s, int buf) {   // stage s; one at or beyond s1 and the chunks beyond the end of K arrive as zeros
+  // part `part` of `parts` of stage s; a stage at or beyond s1 and the chunks beyond the end of K arrive as zeros
+  auto issue = [&](int s, int buf, int part, int parts) {
     lds_u8* const base = smem + buf * C::STAGE + wave * 1024;
     const int ka = s * C::A_RB, kb = s * C::B_RB;
     const bool la = s < s1 && a_col < Ka - ka, lb = s < s1 && b_col < Kb - kb;
 #pragma unroll
-    for (int q = 0; q < AL; ++q)
+    for (int q = part * AL / parts; q < (part + 1) * AL / parts; ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, (lds_void*)(base + q * 4096), 16, la ? avo[q] : kOobOffset, ka, 0, 0);
 #pragma unroll
-    for (int q = 0; q < BL; ++q)
+    for (int q = part * BL / parts; q < (part + 1) * BL / parts; ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, (lds_void*)(base + C::A_STAGE + q * 4096), 16, lb ? bvo[q] : kOobOffset, kb,
                                                0, 0);
   };
@@ -279,7 +285,7 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
     if (!ANY && Sched::prologue_scales(k)) load_scales(q0 + k / SPQ);
-    issue(s0 + k, k);
+    issue(s0 + k, k, 0, 1);
     __builtin_amdgcn_sched_barrier(0);   // the waits count on this order
   }
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(ANY ? Sched::any_prologue_wait() : Sched::prologue_wait()));
@@ -321,8 +327,10 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    issue(s + NS, buf);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!SPREAD) {
+      issue(s + NS, buf, 0, 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     const int nbuf = buf + 1 == NS ? 0 : buf + 1;
     // the next quad's scales landed before this iteration's barrier (they were requested ahead of stage s + 1)
     if constexpr (t == SPQ - 1) read_scales(Q + 1);
@@ -340,6 +348,10 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
                                                 AP ? u : i, AP ? sa[i] : sa[u]);
       }
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (SPREAD) {
+        issue(s + NS, buf, i, MT);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     buf = nbuf;
   };
