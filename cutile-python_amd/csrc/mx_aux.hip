@@ -433,7 +433,8 @@ __global__ __launch_bounds__(256) void pack_scales_list_kernel(const PackList pl
 // ================================================================================================
 // MoE slot alignment (replaces moe_align_tile_size_torch, test/kernels/fused_moe.py:113-173)
 // ================================================================================================
-// A stable counting sort of the flattened expert ids over several workgroups, without atomics on global
+// A stable counting sort of the flattened expert ids; up to 16384 ids and 256 experts in one workgroup (moe_align_one_kernel, below),
+// beyond over several, without atomics on global
 // memory and without any slot written twice.  The ids are cut into B contiguous chunks, one per workgroup.
 // (The ids may be int64: id_shift = 1 reads their low halves.)
 //   moe_hist_kernel (only when B > 1): workgroup b counts the ids of every expert in chunk b -> counts[b][e].
@@ -605,6 +606,98 @@ __global__ __launch_bounds__(kAlignThreads) void moe_place_kernel(const int32_t*
     expert_ids[blk] = 0;
 }
 
+// The same for up to 16384 ids and 256 experts, in one launch of one workgroup.  A wave owns a contiguous part of the ids, up to 16 per
+// lane, which stay in registers.  64 of them at a time: a ballot per bit of the expert's number leaves each lane the lanes of its own
+// expert, hence its place among them, and an LDS counter per wave and expert adds the steps before.  Thread e then sums the
+// waves' counters of expert e, and a scan over the experts gives the first slots.
+// Bound: latency, of one dependent round trip to memory and of the ballots (the two kernels above take three round trips, with a launch
+// between, and walk 256 counters one by one).  us, two kernels | this one, without the launch that is saved: 1000 ids, 8 experts 10.4 | 4.7
+// (one kernel already), 256 experts 59 | 13; 3000 ids, 8 experts 16.8 | 6.6; 8192 ids, 8 experts 15.8 | 10.2, 64 experts 18.1 |
+// 11.7, 256 experts 25.7 | 19.9; 16384 ids, 8 experts 15.5 | 12.7, 256 experts 24.6 | 27.2, the same with a launch of some 2 us: the
+// line.  (The sorted ids through LDS, so that whole lines are stored: no faster, 11.9 and 27.8.)
+constexpr int kAlignOneIds = 16384, kAlignOneExperts = 256, kAlignOneThreads = 1024;
+__global__ __launch_bounds__(kAlignOneThreads) void moe_align_one_kernel(const int32_t* __restrict__ topk_ids, int id_shift, int n, int E,
+                                                                         int tile_m, int32_t* __restrict__ sorted_ids,
+                                                                         int32_t* __restrict__ expert_ids,
+                                                                         int32_t* __restrict__ num_slots_out, int64_t max_slots,
+                                                                         int64_t max_blocks) {
+  constexpr int T = kAlignOneThreads, W = T / 64, PER = kAlignOneIds / T;
+  __shared__ int32_t count[W][kAlignOneExperts], start[kAlignOneExperts + 1], total[kAlignOneExperts], wave_sum[W];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int steps = (n + T - 1) / T, first = wave * steps * 64 + lane;
+  int e[PER], place[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = first + 64 * k;
+    e[k] = k < steps && i < n ? topk_ids[(int64_t)i << id_shift] : -1;
+    if (e[k] >= E) e[k] = -1;
+  }
+  for (int x = lane; x < E; x += 64) count[wave][x] = 0;
+  __syncthreads();
+  const int bits = E > 1 ? 32 - __builtin_clz(E - 1) : 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    if (k >= steps) break;                           // uniform
+    const bool valid = e[k] >= 0;
+    uint64_t same = __builtin_amdgcn_ballot_w64(valid);
+    for (int b = 0; b < bits; ++b) {
+      const bool set = e[k] >> b & 1;
+      const uint64_t m = __builtin_amdgcn_ballot_w64(set);
+      same &= set ? m : ~m;
+    }
+    const int rank = __builtin_popcountll(same & ((1ull << lane) - 1));
+    int before = 0;
+    if (valid) before = count[wave][e[k]];
+    place[k] = before + rank;
+    // wave-synchronous: every lane has read its counter when the first of each expert writes it, and reads the next step's after that
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (valid && rank == 0) count[wave][e[k]] = before + __builtin_popcountll(same);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  }
+  __syncthreads();
+  int mine = 0;
+  if (tid < E) {
+    int c[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w) c[w] = count[w][tid];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      count[w][tid] = mine;
+      mine += c[w];
+    }
+    total[tid] = mine;
+  }
+  const int padded = (mine + tile_m - 1) / tile_m * tile_m;
+  int sum = padded;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(sum, d);
+    if (lane >= d) sum += o;
+  }
+  if (lane == 63) wave_sum[wave] = sum;
+  __syncthreads();
+  if (tid < E) {
+    for (int w = 0; w < wave; ++w) sum += wave_sum[w];
+    start[tid] = sum - padded;
+    if (tid == E - 1) {
+      start[E] = sum;
+      if (num_slots_out) *num_slots_out = sum;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+    if (k < steps && e[k] >= 0) sorted_ids[start[e[k]] + count[wave][e[k]] + place[k]] = first + 64 * k;
+  // padding, block -> expert map, unused tail (as above)
+  for (int x = wave; x < E; x += W) {
+    for (int s = start[x] + total[x] + lane; s < start[x + 1]; s += 64) sorted_ids[s] = n;
+    for (int b = start[x] / tile_m + lane; b < start[x + 1] / tile_m; b += 64) expert_ids[b] = x;   // (whole tiles)
+  }
+  const int used = start[E];
+  for (int64_t i = used + tid; i < max_slots; i += T) sorted_ids[i] = n;
+  for (int64_t blk = used / tile_m + tid; blk < max_blocks; blk += T) expert_ids[blk] = 0;
+}
+
 // ================================================================================================
 // Split-K reduction: C = sum of the fp32 partial products (analogue of the second pass of
 // matmul_split_k_kernel, test/kernels/matmul.py:103-140)
@@ -760,6 +853,12 @@ int launch_moe_align(const void* ids, int ids64, int64_t num_ids, int32_t num_ex
   moe_align_plan(num_ids, chunk, blocks);
   const int32_t* topk_ids = (const int32_t*)ids;
   const int id_shift = ids64 ? 1 : 0;
+  if (num_ids > 0 && num_ids <= kAlignOneIds && num_experts > 0 && num_experts <= kAlignOneExperts) {
+    hipError_t e = launch_kernel(moe_align_one_kernel, dim3(1), dim3(kAlignOneThreads), 0, stream, topk_ids, id_shift, (int)num_ids, (int)num_experts,
+                                 (int)tile_m, sorted_token_ids, sorted_expert_ids, num_slots_out, max_slots, max_slots / tile_m);
+    if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_align_one_kernel launch: %s", hipGetErrorString(e));
+    return MX_OK;
+  }
   const bool seg = num_experts <= kAlignSegExperts;
   const size_t lds = (size_t)(3 * num_experts + 1 + kAlignThreads) * sizeof(int32_t) +
                      (seg ? (size_t)num_experts * (kAlignThreads + 2) * sizeof(uint16_t) : 0);

@@ -118,6 +118,23 @@ def test_moe_align_many_ids_per_expert(ct, dev, n, E, tile, skew):
     assert bool((all_ids[len(want_ids):] == n).all()) and bool((all_e[len(want_e):] == 0).all())
 
 
+@pytest.mark.parametrize("E", [1, 2, 65, 255, 256, 257])
+@pytest.mark.parametrize("n", [1, 63, 65, 1024, 1025, 9000, 16384, 16385])
+def test_moe_align_at_the_limits_of_one_workgroup(ct, dev, n, E):
+    """Either side of the ids and experts that one workgroup sorts, of a step of 64 and of 1024 ids; ids outside the experts
+    are dropped, half of the others go to one expert, and the order of an expert's ids is kept."""
+    rng = np.random.default_rng(n + E)
+    ids = rng.integers(-1, E + 1, size=n, dtype=np.int32)
+    ids[rng.random(n) < 0.5] = E // 2
+    tile = 32
+    got_ids, got_e = (t.cpu().numpy() for t in ct.moe_align_tile_size(torch.from_numpy(ids).to(dev).reshape(-1, 1), tile, E, exact=False))
+    runs = [np.flatnonzero(ids == e) for e in range(E)]
+    want_ids = np.concatenate([np.pad(r, (0, -len(r) % tile), constant_values=n) for r in runs])
+    want_e = np.repeat(np.arange(E), [(len(r) + tile - 1) // tile for r in runs])
+    assert np.array_equal(got_ids[:len(want_ids)], want_ids) and np.array_equal(got_e[:len(want_e)], want_e)
+    assert (got_ids[len(want_ids):] == n).all() and (got_e[len(want_e):] == 0).all()
+
+
 def _moe_case(T, K, N, E, topk, seed, dev, w_std=0.1):
     a = randn_operand(T, K, O.E4M3, seed, dev, std=0.5)
     w = randn_operand(E * N, K, O.E4M3, seed + 1, dev, std=w_std)
