@@ -89,3 +89,28 @@ def test_moe_forward_tile_m(ct, dev, T, E, topk, skew, tile_m):
                                torch.from_numpy(ids).to(dev), tile_m, out_dtype=torch.float32)
     # (tolerance as above)
     assert O.rel_fro(got.cpu(), want) < 2e-2
+
+
+@pytest.mark.parametrize("T,topk,H_out", [(9, 3, 1027), (5, 5, 2052), (7, 1, 1100), (40, 3, 1284)])
+def test_sum_of_copies(ct, dev, T, topk, H_out):
+    """The sum over a token's copies where it is taken apart: an odd number of copies, columns in several parts (more than 1024),
+    parts that leave lanes idle, rows that are not whole 16-byte pieces; one copy of every token is dropped, or the only copy of
+    every second one."""
+    H, F, E = 128, 256, 6
+    rng = np.random.default_rng(T + H_out)
+    hq, hs = O.block_quantize(rng.standard_normal((T, H)).astype(np.float32), 32, O.E4M3, "floor")
+    w1q, w1s = O.block_quantize((rng.standard_normal((E, 2 * F, H)) * 0.2).astype(np.float32), 32, O.E4M3, "floor")
+    w2q, w2s = O.block_quantize((rng.standard_normal((E, H_out, F)) * 0.2).astype(np.float32), 32, O.E4M3, "floor")
+    ids = np.stack([rng.permutation(E)[:topk] for _ in range(T)])
+    wts = rng.random((T, topk)).astype(np.float32)
+    lost = np.zeros((T, topk), bool)
+    lost[np.arange(T)[:: 2 if topk == 1 else 1], rng.integers(0, topk, T)[:: 2 if topk == 1 else 1]] = True
+    want = O.moe_forward(hq, hs, w1q, w1s, w2q, w2s, np.where(lost, 0, wts), ids, w_fmt=O.E4M3)
+    for out_dtype in (torch.float32, torch.bfloat16):
+        got = ct.cutile_moe_scaled(_elems(hq, O.E4M3, dev), _scale(hs, dev), _elems(w1q, O.E4M3, dev), _scale(w1s, dev),
+                                   _elems(w2q, O.E4M3, dev), _scale(w2s, dev), torch.from_numpy(wts).to(dev),
+                                   torch.from_numpy(np.where(lost, -1, ids)).to(dev), out_dtype=out_dtype)
+        # (the bound of test_moe_forward: the activation is rounded to bf16 and re-quantised on both sides)
+        assert O.rel_fro(got.float().cpu(), want) < 2e-2
+        if topk == 1:
+            assert not got[::2].any()
