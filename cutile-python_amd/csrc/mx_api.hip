@@ -1315,6 +1315,17 @@ const char* moe_tiles_issue(const MoePlan& p, const mx_gemm_opts& o) {
   return nullptr;
 }
 
+// Layers of short rows that row tiles take up to 160 rows per expert, i.e. with three tiles of 64, instead of 128.  The 256-row tiles still have one,
+// and are ahead where these fill their rounds of 256 CUs.  us, row tiles | 256-row tiles, random routing, 136 and 160 rows each: taken here 8 experts
+// of 1024 x 7168 FP8 112 | 129, 115 | 125, FP4 87 | 112, 91 | 114; 32 of 1024 x 2048 FP8 (144) 120 | 126, 123 | 129; 16 of 1024 x 8192 FP8 (level) 202 | 198,
+// 216 | 209; 8 of 2048 x 8192 FP8 172 | 182, 178 | 186; 16 of 2048 x 4096 FP8 166 | 174, 176 | 181, FP4 134 | 144, 145 | 149; 64 of 2048 x 1024 FP8
+// 197 | 205, 212 | 217, FP4 171 | 173, 186 | 192.  Left to the 256-row tiles 8 of 2048 x 14336 FP8 283 | 261, 295 | 269, FP4 223 | 215, 232 | 224; 16
+// of 1280 x 8192 FP8 249 | 239, 267 | 248; 32 of 1536 x 2048 FP4 132 | 125, 141 | 131; 32 of 2048 x 2048 FP4 146 | 138, 156 | 145; 64 of
+// 1536 x 1024 FP4 154 | 148, 168 | 156 (12 columns for eight XCDs).
+bool third_tile(const MoePlan& p) {
+  return p.H <= 1024 || (p.E * p.F <= 65536 && (p.E <= 16 || (p.F <= 1024 && p.H_out % 1024 == 0)));
+}
+
 MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& W2, const mx_gemm_opts& o) {
   MoePlan p = {};
   p.T = T; p.n = T * topk; p.E = W1.shape[0]; p.H = W1.shape[2]; p.F = W1.shape[1] / 2; p.H_out = W2.shape[1];
@@ -1322,13 +1333,16 @@ MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& 
   const int64_t rows = weights > kMoeStreamTwiceBytes ? 32 : kMoeStreamRows;
   p.stream = p.n <= kMoeMaxIds && p.n <= p.E * rows && p.H % 128 == 0 && p.F % 128 == 0;
   // Row tiles where the weights would be streamed more than once and as long as the 256-row tiles, which need more launches around
-  // them, are not ahead.  us per layer, streamed | row tiles, 20, 24, 28 and 32 rows per expert: 8 experts of 4096 x 14336 FP8 232 | 258, 238 |
-  // 260, 305 | 263, 336 | 267, FP4 148 | 160, 154 | 162, 193 | 166, 212 | 170; 64 of 1024 x 1024 FP8 61 | 62, 71 | 63, 78 | 64, 88 | 65.
-  // Row tiles | 256-row tiles, 96, 112, 128 and 160 rows each: 8 of 4096 x 14336 FP8 384 | 392, 418 | 402, 456 | 409, FP4 237 | 298, 258 | 314,
-  // 318 | 325, 377 | 352; 8 of 4096 x 7168 FP8 207 | 243, 228 | 248, 246 | 252, 271 | 264; 64 of 4096 x 1024 FP8 285 | 322, 307 | 332, 334 |
-  // 340, 387 | 364; 64 of 1024 x 1024 FP8 104 | 122, 114 | 125, 121 | 128, 140 | 143 (192: 160 | 149); 32 of 1024 x 2048 FP8 95 | 120, 105 | 122,
-  // 112 | 126, 127 | 134, FP4 78 | 108, 86 | 112, 92 | 117, 106 | 124.
-  const int64_t tile_limit = p.H <= 2048 ? 160 : weights > kMoeStreamTwiceBytes && W1.dtype != MX_E2M1 ? 96 : 128;
+  // them, are not ahead.  us per layer, streamed | row tiles, random routing, 25, 26 and 28 rows per expert on average: 8 experts of 4096 x
+  // 14336 FP8 278 | 260, 281 | 261, 288 | 261, FP4 174 | 162, 177 | 161, 181 | 165; 8 of 4096 x 7168 FP8 156 | 152, 158 | 153, 159 | 153; 16 of
+  // 4096 x 4096 FP8 169 | 178, 177 | 178, 186 | 179; 64 of 1024 x 1024 FP4 59 | 48, 60 | 48, 65 | 48.  (With exactly as many rows for
+  // each expert, up to 32, streaming is up to 10 % ahead: 16 of 4096 x 4096 FP8 162 | 180.)
+  // Row tiles | 256-row tiles, random routing, 112 and 128 rows each: 8 of 4096 x 14336 FP4 276 | 322, 316 | 327; 16 of 4096 x 4096 FP8 256 | 278,
+  // 272 | 283; 32 of 4096 x 2048 FP8 265 | 290, 287 | 297; 16 of 3584 x 4096 FP8 233 | 232, 249 | 237 (28 columns for eight XCDs), FP4 159 | 175,
+  // 187 | 179; 64 of 4096 x 1024 FP4 220 | 248, 267 | 258; 32 of 1536 x 2048 FP8 136 | 141, 146 | 144.  96 rows: 8 of 4096 x 14336 FP8 381 | 384, at
+  // 112 and 128 no longer.  Where one expert has half of the copies or the popularity falls with the rank the row tiles are further
+  // ahead: 8 of 4096 x 14336 FP4, 96 rows on average 278 | 328, 290 | 335.
+  const int64_t tile_limit = p.H <= 2048 ? (third_tile(p) ? 160 : 128) : weights > kMoeStreamTwiceBytes && W1.dtype != MX_E2M1 ? 96 : 128;
   const bool can_tile = moe_tiles_issue(p, o) == nullptr && p.n <= p.E * tile_limit;
   if (can_tile && p.n > p.E * kMoeTileFromRows) p.stream = false;
   p.tiles = can_tile && !p.stream;

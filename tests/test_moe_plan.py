@@ -1,0 +1,53 @@
+"""Which form a mixture-of-experts layer takes (csrc/mx_api.hip, moe_plan), on the host: each form's workspace has a size of its own."""
+import ctypes
+
+import pytest
+
+import cutile_amd
+from cutile_amd import _lib as L
+
+E4M3, E2M1 = L.MX_E4M3, L.MX_E2M1
+
+
+def form(rows, E, H, F, w, H_out=None, tile_m=0, packed=True, topk=2):
+    """"streamed", "grouped" or (row tiles of the library's own) their height and the ranges of K of the second product, for `rows` rows
+    per expert on average."""
+    lib, H_out, T = cutile_amd.lib(), H_out or H, int(rows * E) // topk
+    weight = lambda n, k: L.MxTensor(ptr=4096, dtype=w, ndim=3, shape=(E, n, k, 0), stride=(n * k, k, 1, 0), packed_dim=2 if w == E2M1 else -1)
+    layout = L.MX_SCALE_NATIVE if packed else L.MX_SCALE_2D
+    o = L.MxGemmOpts(struct_size=32, block_size=32, tile_m=tile_m, a_scale_layout=layout, b_scale_layout=layout)
+    W1, W2 = weight(2 * F, H), weight(H_out, F)
+    need = lib.mx_moe_forward_workspace_bytes(T, topk, ctypes.byref(W1), ctypes.byref(W2), ctypes.byref(o))
+    up, n = lambda b: (b + 255) // 256 * 256, T * topk
+    activation, out = up(n * F) + up(n * (F // 32)), n * H_out * 4
+    if need == activation + up(out):
+        return "streamed"
+    for height in (64, 128):
+        tiles = (n + min(E, n) * (height - 1)) // height
+        for splits in range(1, 9):
+            if need == activation + up(out * splits) + up(tiles * 16) + up(tiles * height * 4):
+                return height, splits
+    assert need > activation + up(out) + n * F * 4   # the bf16 activation of both halves
+    return "grouped"
+
+
+def tiled(*a, **kw):
+    return form(*a, **kw) not in ("streamed", "grouped")
+
+
+@pytest.mark.parametrize("w", [E4M3, E2M1])
+def test_forms_by_rows_per_expert(w):
+    for E, H, F in ((8, 2048, 7168), (8, 4096, 14336), (64, 1024, 1024)):
+        assert form(24, E, H, F, w) == "streamed"
+        assert all(tiled(r, E, H, F, w) for r in (24.5, 32, 64, 96))
+        assert form(161, E, H, F, w) == "grouped"
+    assert form(64, 8, 2048, 7168, w, packed=False) == "grouped" and form(32, 8, 2048, 7168, w, packed=False) == "streamed"
+
+
+def test_row_tiles_of_three_per_expert():
+    """Beyond 128 rows only where the 256-row tiles are not ahead."""
+    ahead = [(8, 2048, 7168), (8, 2048, 8192), (8, 1536, 7168), (4, 2048, 14336), (16, 2048, 4096), (64, 2048, 1024), (8, 1024, 14336), (32, 1024, 2048)]
+    behind = [(8, 2048, 14336), (8, 1536, 14336), (16, 1280, 8192), (32, 1536, 2048), (32, 2048, 2048), (64, 1536, 1024)]
+    for w in (E4M3, E2M1):
+        assert all(tiled(128, *s, w) for s in ahead + behind)
+        assert [tiled(r, *s, w) for r in (129, 160) for s in ahead + behind] == ([True] * len(ahead) + [False] * len(behind)) * 2
