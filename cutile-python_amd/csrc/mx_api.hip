@@ -1306,12 +1306,12 @@ struct MoePlan {
 constexpr int64_t kMoeStreamRows = 48, kMoeStreamTwiceBytes = 1000000000, kMoeTileFromRows = 24;
 
 // what keeps a layer from the row tiles of mx_moe_tile.hip (nullptr: nothing): both weights' scales packed, whole K-steps and
-// column tiles, a routing that one workgroup sorts out, and no tile height asked for that they don't have
+// column tiles, a routing that one workgroup sorts out, and no padding asked for, which they don't have
 const char* moe_tiles_issue(const MoePlan& p, const mx_gemm_opts& o) {
   if (o.a_scale_layout != MX_SCALE_NATIVE || o.b_scale_layout != MX_SCALE_NATIVE) return "scales are not packed";
   if (p.H % 128 != 0 || p.F % 128 != 0) return "H or F is not a multiple of 128";
   if (p.n > kMoeTileMaxIds || p.E > kMoeTileMaxExperts) return "too many ids or experts";
-  if (o.tile_m != 0 && o.tile_m != 256) return "tile_m";
+  if (o.tile_m != 0) return "tile_m";
   return nullptr;
 }
 

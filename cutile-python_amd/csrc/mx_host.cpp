@@ -390,7 +390,8 @@ PyObject* py_moe(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const long tile_m = PyLong_AsLong(a[11]);
   if (tile_m == -1 && PyErr_Occurred()) PyErr_Clear();
   if (tile_m <= 0 || tile_m > 0x7FFFFFFF) Py_RETURN_NONE;
-  mx_gemm_opts o = {sizeof(mx_gemm_opts), 0, 0, 0, MX_KERNEL_AUTO, 32, 0, (int32_t)tile_m};
+  // (the operator's default, 256, leaves the form of the layer to the library)
+  mx_gemm_opts o = {sizeof(mx_gemm_opts), 0, 0, 0, MX_KERNEL_AUTO, 32, 0, tile_m == 256 ? 0 : (int32_t)tile_m};
   if (!expert_scale_desc(a[3], E, dW1.shape[1], dW1.shape[2], dev, &dW1s, &o.a_scale_layout) ||
       !expert_scale_desc(a[5], E, dW2.shape[1], dW2.shape[2], dev, &dW2s, &o.b_scale_layout))
     Py_RETURN_NONE;

@@ -44,6 +44,13 @@ def test_forms_by_rows_per_expert(w):
     assert form(64, 8, 2048, 7168, w, packed=False) == "grouped" and form(32, 8, 2048, 7168, w, packed=False) == "streamed"
 
 
+def test_padding_that_the_caller_asks_for():
+    """An explicit tile_m is kept to where there are slots; 0 leaves the form to the library."""
+    for w in (E4M3, E2M1):
+        assert tiled(64, 8, 2048, 7168, w, tile_m=0)
+        assert [form(64, 8, 2048, 7168, w, tile_m=t) for t in (128, 256, 512)] == ["grouped"] * 3
+
+
 def test_row_tiles_of_three_per_expert():
     """Beyond 128 rows only where the 256-row tiles are not ahead."""
     ahead = [(8, 2048, 7168), (8, 2048, 8192), (8, 1536, 7168), (4, 2048, 14336), (16, 2048, 4096), (64, 2048, 1024), (8, 1024, 14336), (32, 1024, 2048)]
