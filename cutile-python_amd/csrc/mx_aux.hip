@@ -2,6 +2,7 @@
 // MoE slot alignment.  All integer / byte work; results must be bit-exact.
 #include "mx_common.h"
 #include "mx_load_once.h"
+#include "mx_moe_rules.h"
 #include "mx_quant.h"
 
 namespace mx {
@@ -434,8 +435,7 @@ __global__ __launch_bounds__(256) void pack_scales_list_kernel(const PackList pl
 // MoE slot alignment (replaces moe_align_tile_size_torch, test/kernels/fused_moe.py:113-173)
 // ================================================================================================
 // A stable counting sort of the flattened expert ids; up to 16384 ids and 256 experts in one workgroup (moe_align_one_kernel, below),
-// beyond over several, without atomics on global
-// memory and without any slot written twice.  The ids are cut into B contiguous chunks, one per workgroup.
+// beyond over several, without atomics on global memory and without any slot written twice.  The ids are cut into B contiguous chunks, one per workgroup.
 // (The ids may be int64: id_shift = 1 reads their low halves.)
 //   moe_hist_kernel (only when B > 1): workgroup b counts the ids of every expert in chunk b -> counts[b][e].
 //   moe_place_kernel: workgroup b
@@ -613,9 +613,9 @@ __global__ __launch_bounds__(kAlignThreads) void moe_place_kernel(const int32_t*
 // Bound: latency, of one dependent round trip to memory and of the ballots (the two kernels above take three round trips, with a launch
 // between, and walk 256 counters one by one).  us, two kernels | this one, without the launch that is saved: 1000 ids, 8 experts 10.4 | 4.7
 // (one kernel already), 256 experts 59 | 13; 3000 ids, 8 experts 16.8 | 6.6; 8192 ids, 8 experts 15.8 | 10.2, 64 experts 18.1 |
-// 11.7, 256 experts 25.7 | 19.9; 16384 ids, 8 experts 15.5 | 12.7, 256 experts 24.6 | 27.2, the same with a launch of some 2 us: the
-// line.  (The sorted ids through LDS, so that whole lines are stored: no faster, 11.9 and 27.8.)
-constexpr int kAlignOneIds = 16384, kAlignOneExperts = 256, kAlignOneThreads = 1024;
+// 11.7, 256 experts 25.7 | 19.9.  The line: moe_align_in_one_workgroup.  (The sorted ids through LDS, so that whole lines are stored: no
+// faster, 16384 ids of 8 experts 11.9, of 256 experts 27.8 against 12.7 and 27.2.)
+constexpr int kAlignOneThreads = 1024;
 __global__ __launch_bounds__(kAlignOneThreads) void moe_align_one_kernel(const int32_t* __restrict__ topk_ids, int id_shift, int n, int E,
                                                                          int tile_m, int32_t* __restrict__ sorted_ids,
                                                                          int32_t* __restrict__ expert_ids,
@@ -853,7 +853,7 @@ int launch_moe_align(const void* ids, int ids64, int64_t num_ids, int32_t num_ex
   moe_align_plan(num_ids, chunk, blocks);
   const int32_t* topk_ids = (const int32_t*)ids;
   const int id_shift = ids64 ? 1 : 0;
-  if (num_ids > 0 && num_ids <= kAlignOneIds && num_experts > 0 && num_experts <= kAlignOneExperts) {
+  if (moe_align_in_one_workgroup(num_ids, num_experts)) {
     hipError_t e = launch_kernel(moe_align_one_kernel, dim3(1), dim3(kAlignOneThreads), 0, stream, topk_ids, id_shift, (int)num_ids, (int)num_experts,
                                  (int)tile_m, sorted_token_ids, sorted_expert_ids, num_slots_out, max_slots, max_slots / tile_m);
     if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_align_one_kernel launch: %s", hipGetErrorString(e));

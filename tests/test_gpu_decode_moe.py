@@ -118,8 +118,8 @@ def test_moe_align_many_ids_per_expert(ct, dev, n, E, tile, skew):
     assert bool((all_ids[len(want_ids):] == n).all()) and bool((all_e[len(want_e):] == 0).all())
 
 
-@pytest.mark.parametrize("E", [1, 2, 65, 255, 256, 257])
-@pytest.mark.parametrize("n", [1, 63, 65, 1024, 1025, 9000, 16384, 16385])
+@pytest.mark.parametrize("E", [1, 2, 16, 17, 64, 65, 255, 256, 257])
+@pytest.mark.parametrize("n", [1, 63, 65, 1024, 1025, 9000, 12288, 12289, 14336, 14337, 16384, 16385])
 def test_moe_align_at_the_limits_of_one_workgroup(ct, dev, n, E):
     """Either side of the ids and experts that one workgroup sorts, of a step of 64 and of 1024 ids; ids outside the experts
     are dropped, half of the others go to one expert, and the order of an expert's ids is kept."""

@@ -1,5 +1,7 @@
 """Which form a mixture-of-experts layer takes (csrc/mx_api.hip, moe_plan), on the host: each form's workspace has a size of its own."""
 import ctypes
+import pathlib
+import subprocess
 
 import pytest
 
@@ -58,3 +60,13 @@ def test_row_tiles_of_three_per_expert():
     for w in (E4M3, E2M1):
         assert all(tiled(128, *s, w) for s in ahead + behind)
         assert [tiled(r, *s, w) for r in (129, 160) for s in ahead + behind] == ([True] * len(ahead) + [False] * len(behind)) * 2
+
+
+def test_routing_by_one_workgroup_where_it_is_the_faster_one(tmp_path):
+    cases = [(1, 1), (12288, 256), (12288, 257), (14336, 64), (12289, 65), (16384, 16), (16384, 17), (14337, 64), (16385, 1), (0, 8)]
+    src = pathlib.Path(__file__).resolve().parent.parent / "cutile-python_amd" / "csrc"
+    body = "".join(f'std::printf("%d\\n", (int)mx::moe_align_in_one_workgroup({n}, {e}));' for n, e in cases)
+    (tmp_path / "p.cpp").write_text('#include <cstdio>\n#include "mx_moe_rules.h"\nint main() { %s }\n' % body)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", f"-I{src}", "-o", str(tmp_path / "p"), str(tmp_path / "p.cpp")], check=True)
+    got = subprocess.run([str(tmp_path / "p")], check=True, capture_output=True, text=True).stdout.split()
+    assert got == ["1", "1", "0", "1", "0", "1", "0", "0", "0", "0"]
