@@ -39,15 +39,19 @@ namespace {
 // where an operand's scales are: native layout; plain rows that the DMA can fetch; plain rows at any byte (both operands)
 constexpr int kScaleNative = 0, kScalePlain = 1, kScaleAny = 2;
 
-template <class C, int NS, int AS, int BS, bool GROUPED>
+// A stage's requests go out between its MFMAs: all four waves' at once behind the barrier they keep the address unit busy for some
+// 500 cycles, the length of a stage's MFMAs, in which none of these is issued.  2048 x 2048 x 2048 FP8 15.2 -> 13.5 us, x 8192 43.0 ->
+// 40.9, FP4 26.9 -> 25.3, 200 x 14336 x 4096 24.3 -> 23.0; on tiles of 64 0 - 6 % (packed scales, 300 x 2000 x 7168 FP8
+// 18.4 -> 17.8, FP4 weights 16.8 -> 15.8, with two workgroups on a CU 1400 x 1400 x 8192 29.8 -> 28.8; plain ones 900 x 900 x 8192 21.1 -> 20.9).  Not with two stages, where a later request is a later stage (512 x 14336 x 4096 35.8 -> 39.6), nor beside the larger
+// tile's scales through registers (1111 x 2100 x 4032 21.6 -> 22.2), nor beside those of the smaller one where eight stages are in flight
+// for long (t128_any_spread).
+template <class C, int NS, int AS>
+constexpr bool kSpread = NS > 2 && !(AS == kScaleAny && C::BM == 128);
+
+template <class C, int NS, int AS, int BS, bool GROUPED, bool SPREAD = kSpread<C, NS, AS>>
 __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem, const int pid, const int split, const int bz) {
   constexpr int KS = C::KSUB, SPQ = 4 / KS, MT = C::MT, NT = C::NTL;
   constexpr bool AP = AS != kScaleNative, BP = BS != kScaleNative, ANY = AS == kScaleAny;
-  // A stage's requests go out between its MFMAs: all four waves' at once behind the barrier they keep the address unit busy for some
-  // 500 cycles, the length of a stage's MFMAs, in which none of these is issued.  2048 x 2048 x 2048 FP8 15.2 -> 13.5 us, x 8192 43.0 ->
-  // 40.9, FP4 26.9 -> 25.3, 200 x 14336 x 4096 24.3 -> 23.0.  Not with two stages, where a later request is a later stage (512 x 14336 x 4096
-  // 35.8 -> 39.6), nor beside the larger tile's scales through registers (1111 x 2100 x 4032 21.6 -> 22.2).
-  constexpr bool SPREAD = NS > 2 && !(ANY && C::BM == 128);
   static_assert(ANY == (BS == kScaleAny) && !(ANY && GROUPED) && MT == NT && (C::BM == 128 || !GROUPED), "");
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, gq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -403,10 +407,10 @@ __device__ __forceinline__ void t128_tile(const T128Args& g, lds_u8* const smem,
   else store(std::integral_constant<int, 1>{});
 }
 
-template <class C, int NS, int AS, int BS, bool GROUPED>
+template <class C, int NS, int AS, int BS, bool GROUPED, bool SPREAD>
 __global__ __launch_bounds__(256, NS == 2 || (C::BM == 64 && NS == 4) ? 2 : 1) void t128_kernel(const T128Args g) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem_generic[];
-  t128_tile<C, NS, AS, BS, GROUPED>(g, (lds_u8*)smem_generic, blockIdx.x, blockIdx.y, blockIdx.z);
+  t128_tile<C, NS, AS, BS, GROUPED, SPREAD>(g, (lds_u8*)smem_generic, blockIdx.x, blockIdx.y, blockIdx.z);
   __builtin_amdgcn_s_waitcnt(0x0F70);   // the trailing zero-fill DMA has left the queue before the LDS is given back
 }
 
@@ -452,9 +456,9 @@ __global__ __launch_bounds__(256, 2) void t128_list_kernel(const T128List gl) {
   }
 }
 
-template <class C, int NS, int AS, int BS, bool GROUPED>
+template <class C, int NS, int AS, int BS, bool GROUPED, bool SPREAD = kSpread<C, NS, AS>>
 int launch_one(const T128Args& g, hipStream_t stream) {
-  auto kern = t128_kernel<C, NS, AS, BS, GROUPED>;
+  auto kern = t128_kernel<C, NS, AS, BS, GROUPED, SPREAD>;
   constexpr int lds = NS * C::STAGE + ((NS + 4 / C::KSUB - 1) / (4 / C::KSUB) + 1) * 4096;
   static int attr_done = 0;   // benign race: the attribute call is idempotent
   if (!attr_done) {
@@ -500,7 +504,11 @@ int t128_pair(const T128Args& g, hipStream_t stream) {
   auto depth = [&](auto cfg, auto ns) {
     using D = decltype(cfg);
     constexpr int NS = decltype(ns)::value;
-    if (g.a_plain == kT128ScalesAny) return launch_one<D, NS, kScaleAny, kScaleAny, false>(g, stream);
+    if (g.a_plain == kT128ScalesAny) {
+      if constexpr (D::BM == 64 && NS == 8)
+        if (!t128_any_spread(g.K, g.k_splits, D::KSUB)) return launch_one<D, NS, kScaleAny, kScaleAny, false, false>(g, stream);
+      return launch_one<D, NS, kScaleAny, kScaleAny, false>(g, stream);
+    }
     return !g.a_plain   ? launch_one<D, NS, kScaleNative, kScaleNative, false>(g, stream)
            : !g.b_plain ? launch_one<D, NS, kScalePlain, kScaleNative, false>(g, stream)
                         : launch_one<D, NS, kScalePlain, kScalePlain, false>(g, stream);

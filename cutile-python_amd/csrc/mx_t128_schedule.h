@@ -37,6 +37,15 @@ struct T128Schedule {
   static constexpr int any_stage_wait() { return (NS - 2) * TL; }
 };
 
+// Whether 64 x 64 tiles with eight stages in flight and scales at any byte send a stage's requests between its MFMAs: for short K only.
+// (Why that costs them beyond, and neither packed nor aligned scales, is not measured.)
+// us, behind the barrier | between the MFMAs, K in one range: FP8 500 x 1500 and 900 x 900, K = 2048 8.5 | 8.4, 8.7 | 8.4, 3072 (E5M2) 10.8 | 10.5,
+// 11.1 | 10.7, 4096 12.8 | 12.5, 13.4 | 13.7, 5120 15.5 | 15.4, 16.5 | 17.0, 7168 21.1 | 21.8, 21.3 | 22.0, 14336 36.4 | 38.8, 37.0 | 39.2; FP4
+// weights 4096 12.0 | 11.9, 12.0 | 11.8, 5120 13.7 | 13.6, 14.3 | 15.4, 8192 19.9 | 21.9, 20.8 | 22.6; FP4 x FP4 4096 9.8 | 9.6, 9.8 | 9.6, 5120 11.1 |
+// 10.8, 10.9 | 11.0, 7168 13.5 | 13.4, 14.0 | 15.3, 14336 25.2 | 27.9, 25.7 | 28.3.  With four stages in flight, two workgroups per CU, level: 1000 x
+// 1900 FP8 4096 20.4 | 19.5, 8192 33.3 | 33.6.
+inline bool t128_any_spread(int K, int splits, int ksteps_per_stage) { return K <= (ksteps_per_stage == 2 ? 5120 : 4096) * (splits > 1 ? splits : 1); }
+
 // First stage of a product of `stages` stages at which something is read that the waits do not cover, -1 if none.  -2: the
 // first reads, behind the prologue.  `scales_first`: a prologue that requests all its scales ahead of the stages.
 template <class S>

@@ -46,6 +46,18 @@ def test_either_side_of_the_line(ct, dev, fa, fb, K):
     assert torch.equal(out, run(ct.pack_scales(a.scale_t, operand="a"), ct.pack_scales(b.scale_t, operand="b")))
 
 
+@pytest.mark.parametrize("fa,fb", PAIRS, ids=str)
+@pytest.mark.parametrize("K", [4096, 4128, 5120, 5152])   # the last whose requests are spread over a stage, the first whose are not
+def test_either_side_of_long_k_on_64_x_64_tiles(ct, dev, fa, fb, K):
+    M, N = 130, 70
+    a, b = raw_operand(M, K, fa, 1500 + K, dev), raw_operand(N, K, fb, 1600 + K, dev)
+    run = lambda sa, sb: ct.block_scaled_matmul(a.storage, sa, b.storage.T, sb, a_format=a.fmt_kw, b_format=b.fmt_kw,
+                                                kernel="mfma128", out_dtype=torch.float32, split_k=1)
+    out = run(_placed(a.scale_t, 1, 0), _placed(b.scale_t, 3, 5).T)
+    assert torch.equal(out, run(ct.pack_scales(a.scale_t, operand="a"), ct.pack_scales(b.scale_t, operand="b")))
+    assert O.rel_fro(out.cpu(), oracle_matmul(a, b)) <= TOL
+
+
 @pytest.mark.parametrize("fmt", [O.E4M3, O.E2M1])
 def test_in_lists_and_batches(ct, dev, fmt):
     shapes = [(96, 200, 96), (128, 128, 512), (300, 64, 1056), (33, 130, 32), (257, 129, 992)]

@@ -84,3 +84,12 @@ def test_kernel_takes_order_and_waits_from_the_schedule():
     first, last = body.split("if constexpr (t == 0)")[1], body.split("if constexpr (t == SPQ - 1)")
     assert "store_any(Q + 1);" in first.split("issue(s + NS, buf)")[0] and "read_scales(Q + 1);" in last[1].splitlines()[0]
     assert "s_barrier" in body.split("store_any(q0);")[1].split("read_scales(q0);")[0]
+
+
+def test_scales_at_any_byte_keep_the_requests_together_for_long_k(tmp_path):
+    cases = [(992, 1, 1), (4096, 1, 1), (4097, 1, 1), (8192, 2, 1), (8193, 2, 1), (5120, 0, 2), (5121, 1, 2), (14336, 3, 2)]
+    body = "".join('std::printf("%%d\\n", (int)mx::t128_any_spread(%d, %d, %d));' % c for c in cases)
+    (tmp_path / "p.cpp").write_text('#include <cstdio>\n#include "mx_t128_schedule.h"\nint main() { %s }\n' % body)
+    subprocess.run(["g++", "-std=c++17", f"-I{CSRC}", "-o", str(tmp_path / "p"), str(tmp_path / "p.cpp")], check=True)
+    got = subprocess.run([str(tmp_path / "p")], check=True, capture_output=True, text=True).stdout.split()
+    assert got == ["1", "1", "0", "1", "0", "1", "0", "1"]
