@@ -15,12 +15,15 @@ CASES = [(25, 128, 128, 2, 2, 0.0), (64, 256, 128, 1, 1, 0.0), (65, 384, 256, 1,
          (129, 640, 128, 1, 1, 0.0), (100, 256, 384, 4, 2, 0.9), (210, 1152, 128, 16, 4, 0.2),
          # K of the second product in several ranges, the last of them not a whole K-quad
          (60, 128, 5248, 2, 2, 0.4),
-         # FP4: tiles of 128 rows (long rows of W, more than 64 rows per expert)
-         (70, 2176, 128, 1, 1, 0.0), (129, 2304, 128, 2, 2, 0.6), (128, 2176, 256, 1, 1, 0.0)]
+         # FP4: tiles of 128 rows (long rows of W, more than 64 rows per expert): one of them, full; two of an expert
+         (70, 2176, 128, 1, 1, 0.0), (128, 2176, 256, 1, 1, 0.0), (120, 2304, 128, 2, 2, 0.6),
+         # ... three of one expert, none of another, K of the second product in two ranges
+         (160, 2176, 2176, 4, 2, 0.95)]
+GROUPED = [(129, 2304, 128, 2, 2, 0.6)]   # the first that 256-row tiles take
 
 
 @pytest.mark.parametrize("w_fmt", [O.E4M3, O.E2M1], ids=str)
-@pytest.mark.parametrize("T,H,F,E,topk,skew", CASES)
+@pytest.mark.parametrize("T,H,F,E,topk,skew", CASES + GROUPED)
 def test_moe_row_tiles(ct, dev, T, H, F, E, topk, skew, w_fmt):
     rng = np.random.default_rng(T * 7 + F)
     H_out = H + 72                       # not a multiple of a tile
@@ -29,6 +32,8 @@ def test_moe_row_tiles(ct, dev, T, H, F, E, topk, skew, w_fmt):
     w2q, w2s = O.block_quantize((rng.standard_normal((E, H_out, F)) * 0.2).astype(np.float32), 32, w_fmt, "floor")
     ids = rng.integers(0, E, (T, topk))
     ids[rng.random((T, topk)) < skew] = 0
+    if E == 4 and F == 2176:
+        ids[ids == 2] = 3
     lost = rng.random((T, topk)) < (0.1 if E > 1 else 0.0)   # copies that no expert claims
     wts = rng.random((T, topk)).astype(np.float32)
     want = O.moe_forward(hq, hs, w1q, w1s, w2q, w2s, np.where(lost, 0, wts), ids, w_fmt=w_fmt)
@@ -57,16 +62,32 @@ def _random_layer(ct, dev, T, H, F, E, H_out, w_format, seed):
             torch.rand((T, 2), generator=g, device=dev), torch.randint(0, E, (T, 2), generator=g, device=dev))
 
 
-@pytest.mark.parametrize("w_format", [None, "e2m1"])
-def test_moe_row_tiles_non_temporal(ct, dev, w_format):
-    """Weights of more than 96 MB, an odd number of K-steps (FP4 stages hold two), and a token whose scales are NaN: it stays alone."""
-    T, H, E, H_out = 30, 3968, 2, 256
-    F = 12928 if w_format else 6528
+# 96 MB of W and more, rows of whole lines, at most 48 rows per expert: T, H, F, E, H_out.  Both products of each layer; K of the second in
+# ranges; even numbers of K-steps, and odd ones (FP4 stages hold two), where FP4 rows have whole lines by their pitch only
+ONCE = {None: [(30, 3968, 6528, 2, 7808), (90, 2048, 6656, 4, 4096)],
+        "e2m1": [(30, 4096, 12288, 2, 8192), (30, 3968, 12928, 2, 7808), (90, 2048, 12544, 4, 4104)]}
+once_pitch = lambda K, w_format: (K // 2 if w_format else K) + 127 & -128   # bytes
+
+
+def _pitched(w, w_format):
+    """The same rows, of whole lines each, with NaN bytes between them."""
+    v = w.view(torch.uint8)
+    E, rows, row = v.shape
+    pitch = once_pitch(2 * row if w_format else row, w_format)
+    buf = torch.full((E, rows, pitch), 0xFF, dtype=torch.uint8, device=v.device)
+    buf[..., :row] = v
+    return buf.view(w.dtype)[..., :row]
+
+
+@pytest.mark.parametrize("w_format,T,H,F,E,H_out", [(f, *s) for f, layers in ONCE.items() for s in layers])
+def test_moe_row_tiles_non_temporal(ct, dev, w_format, T, H, F, E, H_out):
+    """Non-temporal weights of both products, and a token whose scales are NaN: it stays alone."""
     x, xs, w1, s1, w2, s2, wt, ids = _random_layer(ct, dev, T, H, F, E, H_out, w_format, 3)
+    w1, w2 = _pitched(w1, w_format), _pitched(w2, w_format)
     p1, p2 = ct.pack_scales(s1, operand="b"), ct.pack_scales(s2, operand="b")
     run = lambda scales, a, b: ct.cutile_moe_scaled(x, scales, w1, a, w2, b, wt, ids, out_dtype=torch.float32, w_format=w_format)
     got, plain = run(xs, p1, p2), run(xs, s1, s2)
-    # plain scales run the streamed form: the same products in another order (tolerance as above)
+    # plain scales run another form: the same products in another order (tolerance as above)
     assert ((got - plain).norm() / plain.norm()).item() < 2e-2
     bad = xs.view(torch.uint8).clone()
     bad[7] = 0xFF

@@ -7,6 +7,7 @@ import pytest
 
 import cutile_amd
 from cutile_amd import _lib as L
+from test_load_once import evaluate as load_once  # noqa: F401
 
 E4M3, E2M1 = L.MX_E4M3, L.MX_E2M1
 
@@ -31,6 +32,23 @@ def form(rows, E, H, F, w, H_out=None, tile_m=0, packed=True, topk=2):
                 return height, splits
     assert need > activation + up(out) + n * F * 4   # the bf16 activation of both halves
     return "grouped"
+
+
+def test_gpu_tests_reach_the_row_tiles_that_they_are_about(load_once):
+    import test_gpu_moe_tiles as g
+    at = lambda w, T, H, F, E, topk, _=0.0: form(T * topk / E, E, H, F, w, H + 72, topk=topk)
+    assert [at(E4M3, *c)[0] for c in g.CASES] == [64] * len(g.CASES)
+    # (the two cases of one expert before the last two need as much room with either height)
+    assert all(tiled(T * topk / E, E, H, F, E2M1, H + 72, topk=topk) for T, H, F, E, topk, _ in g.CASES)
+    assert [at(E2M1, *c)[0] for c in g.CASES[-2:]] == [128] * 2 and at(E2M1, *g.CASES[-1])[1] == 2
+    assert all(at(w, *c) == "grouped" for w in (E4M3, E2M1) for c in g.GROUPED)
+    # both products of the layers with non-temporal weights; some of the second ones in ranges of K
+    ranges = [form(2 * T / E, E, H, F, E2M1 if f else E4M3, H_out) for f, layers in g.ONCE.items() for T, H, F, E, H_out in layers]
+    assert all(height == 64 for height, _ in ranges) and any(n > 1 for _, n in ranges[:2]) and any(n > 1 for _, n in ranges[2:])
+    row = lambda K, f: K // 2 if f else K
+    assert load_once(*[f"stream_loads_once({min(2 * T, E) * n}LL, {row(K, f)}, {g.once_pitch(K, f)}, 0, 1)" for f, layers in g.ONCE.items()
+                       for T, H, F, E, H_out in layers for n, K in ((2 * F, H), (H_out, F))]) == [1] * 10
+    assert all(2 * T <= 48 * E for layers in g.ONCE.values() for T, _, _, E, _ in layers)
 
 
 def tiled(*a, **kw):
