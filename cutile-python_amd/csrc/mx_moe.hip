@@ -160,15 +160,19 @@ __global__ __launch_bounds__(C::WAVES * 64, 2) void moe_stream_kernel(const MoeS
 
 // out[t, :] = sum over the top-k copies of a token, in their order; a copy whose expert id is outside [0, E) was never
 // computed and counts as zero.  A copy is the sum of `splits` partial products, c_split elements apart, times its routed weight
-// (null: c holds the weighted ones).  Four columns per thread, one token per workgroup, KU copies requested at a time.
-// Bound: reading the copies.  4096 tokens x 2 copies of 4096 33.6 -> 31.2 us (6.4 TB/s), 3500 x 4 of 2048 22.3 -> 20.4, 1500 x 2 of 4096
-// 12.7 -> 12.0: a thread for every four columns of all tokens took a 64-bit division each and waited for one copy after the
-// other.  (Four copies at a time: 23.5 for the second.)
+// (null: c holds the weighted ones).  Four columns per thread, whole waves per token, KU copies requested at a time.
+// Bound: reading the copies.  Against a thread for every four columns of all tokens, which takes a 64-bit division each and waits for one
+// copy after the other: 4096 tokens x 2 copies of 4096 behind the MoE layer's product 33.6 -> 31.2 us (6.4 TB/s), 3500 x 4 of 2048 22.3 ->
+// 20.4, 8192 x 4 of 2048 53.4 -> 44.2, 300 x 8 of 2048 7.0 -> 5.6; columns that leave part of a wave idle cost what is idle: 6000 x 2 of 1028 11.7 ->
+// 13.2, of 2560 columns 31.0 -> 32.6.  (Four copies at a time: 23.5 for the second.  Workgroups of five waves 34.6 for the last, whole threads
+// counted over all columns with a 32-bit division 35.3; rows that are not whole 16-byte pieces, two copies at a time: 3000 x 3 of 1030 14.2 | 16.7.)
 template <int KU>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const float* __restrict__ c, int splits, int64_t c_split,
                                                           const float* __restrict__ weights, const void* __restrict__ ids, int ids64,
                                                           int E, int64_t T, int topk, int64_t H, void* out, int out_dtype) {
-  const int64_t t = (int64_t)blockIdx.z * gridDim.x + blockIdx.x, h = ((int64_t)blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  // (the parts of a token next to each other: they share lines where its rows don't start at one)
+  const int64_t t = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * blockDim.y + __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int64_t h = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (t >= T || h >= H) return;
   const int n = H - h < 4 ? (int)(H - h) : 4;
   const bool whole = n == 4 && (H & 3) == 0;
@@ -267,13 +271,18 @@ int launch_moe_stream(const MoeStreamArgs& a0, bool up, hipStream_t stream) {
 int launch_moe_combine(const float* c, int splits, int64_t c_split, const float* weights, const void* ids, int ids64, int E, int64_t T, int topk, int64_t H, void* out,
                        int out_dtype, hipStream_t stream) {
   if (T <= 0 || H <= 0) return MX_OK;
-  // a token's columns in equal parts of at most 256 threads, whole waves
-  const int64_t h4 = (H + 3) / 4, parts = (h4 + 255) / 256, threads = ((h4 + parts - 1) / parts + 63) / 64 * 64;
-  const int64_t x = T < 1 << 23 ? T : 1 << 23;       // (below 2^32 threads along a dimension)
-  const dim3 grid((unsigned)x, (unsigned)parts, (unsigned)((T + x - 1) / x)), block((unsigned)threads);
+  // A token's columns in parts of one, two or four waves, as few idle lanes as can be and then as long as can be; workgroups of four waves, several
+  // tokens together, where that leaves two for each CU.
+  const int64_t h4 = (H + 3) / 4;
+  int64_t threads = 256;
+  for (int64_t n = 128; n >= 64; n /= 2)
+    if ((h4 + n - 1) / n * n < (h4 + threads - 1) / threads * threads) threads = n;
+  const int64_t parts = (h4 + threads - 1) / threads, tokens = T * parts >= 512 * (256 / threads) ? 256 / threads : 1;
+  const int64_t groups = (T + tokens - 1) / tokens, z = (groups + 65534) / 65535;   // (a grid has less than 65536 of y and z)
+  const dim3 grid((unsigned)parts, (unsigned)((groups + z - 1) / z), (unsigned)z), block((unsigned)threads, (unsigned)tokens);
   auto run = [&](auto kern) { return launch_kernel(kern, grid, block, 0, stream, c, splits, c_split, weights, ids, ids64, E, T, topk, H, out,
                                                              out_dtype); };
-  hipError_t e = topk == 1 ? run(moe_combine_kernel<1>) : run(moe_combine_kernel<2>);
+  hipError_t e = topk == 1 || H % 4 != 0 ? run(moe_combine_kernel<1>) : run(moe_combine_kernel<2>);
   if (e != hipSuccess) return set_error(MX_ERR_LAUNCH, "moe_combine_kernel launch: %s", hipGetErrorString(e));
   return MX_OK;
 }

@@ -91,7 +91,9 @@ def test_moe_forward_tile_m(ct, dev, T, E, topk, skew, tile_m):
     assert O.rel_fro(got.cpu(), want) < 2e-2
 
 
-@pytest.mark.parametrize("T,topk,H_out", [(9, 3, 1027), (5, 5, 2052), (7, 1, 1100), (40, 3, 1284)])
+@pytest.mark.parametrize("T,topk,H_out", [(9, 3, 1027), (5, 5, 2052), (7, 1, 1100), (40, 3, 1284),
+                                          # several tokens per workgroup (the last one not full), of one wave, two, and 17 parts
+                                          (2049, 1, 260), (2050, 3, 136), (1025, 2, 516), (127, 1, 4100), (122, 2, 4100)])
 def test_sum_of_copies(ct, dev, T, topk, H_out):
     """The sum over a token's copies where it is taken apart: an odd number of copies, columns in several parts (more than 1024),
     parts that leave lanes idle, rows that are not whole 16-byte pieces; one copy of every token is dropped, or the only copy of
