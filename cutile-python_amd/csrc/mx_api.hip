@@ -11,6 +11,7 @@
 #include "mx_common.h"
 #include "mx_gemm_pp.h"
 #include "mx_gemm_t128.h"
+#include "mx_moe_rules.h"
 #include "mx_moe_tile.h"
 #include "mx_stream.h"
 
@@ -1303,7 +1304,7 @@ struct MoePlan {
 //     455 | 369; FP4, 16 experts 421 | 430, 505 | 437, 516 | 442
 // so that the tiles are ahead from 1 GB of weights on, at 33 rows not yet everywhere.
 // (64 rows: with a longer list of ids, mx_stream.h.)
-constexpr int64_t kMoeStreamRows = 48, kMoeStreamTwiceBytes = 1000000000, kMoeTileFromRows = 24;
+constexpr int64_t kMoeStreamRows = 48, kMoeStreamTwiceBytes = 1000000000;
 
 // what keeps a layer from the row tiles of mx_moe_tile.hip (nullptr: nothing): both weights' scales packed, whole K-steps and
 // column tiles, a routing that one workgroup sorts out, and no padding asked for, which they don't have
@@ -1332,11 +1333,8 @@ MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& 
   const int64_t weights = p.E * (2 * p.F * p.H + p.H_out * p.F) / (W1.dtype == MX_E2M1 ? 2 : 1);   // bytes
   const int64_t rows = weights > kMoeStreamTwiceBytes ? 32 : kMoeStreamRows;
   p.stream = p.n <= kMoeMaxIds && p.n <= p.E * rows && p.H % 128 == 0 && p.F % 128 == 0;
-  // Row tiles where the weights would be streamed more than once and as long as the 256-row tiles, which need more launches around
-  // them, are not ahead.  us per layer, streamed | row tiles, random routing, 25, 26 and 28 rows per expert on average: 8 experts of 4096 x
-  // 14336 FP8 278 | 260, 281 | 261, 288 | 261, FP4 174 | 162, 177 | 161, 181 | 165; 8 of 4096 x 7168 FP8 156 | 152, 158 | 153, 159 | 153; 16 of
-  // 4096 x 4096 FP8 169 | 178, 177 | 178, 186 | 179; 64 of 1024 x 1024 FP4 59 | 48, 60 | 48, 65 | 48.  (With exactly as many rows for
-  // each expert, up to 32, streaming is up to 10 % ahead: 16 of 4096 x 4096 FP8 162 | 180.)
+  // Row tiles where the weights would be streamed more than once (moe_leaves_streaming) and as long as the 256-row tiles, which need more
+  // launches around them, are not ahead.
   // Row tiles | 256-row tiles, random routing, 112 and 128 rows each: 8 of 4096 x 14336 FP4 276 | 322, 316 | 327; 16 of 4096 x 4096 FP8 256 | 278,
   // 272 | 283; 32 of 4096 x 2048 FP8 265 | 290, 287 | 297; 16 of 3584 x 4096 FP8 233 | 232, 249 | 237 (28 columns for eight XCDs), FP4 159 | 175,
   // 187 | 179; 64 of 4096 x 1024 FP4 220 | 248, 267 | 258; 32 of 1536 x 2048 FP8 136 | 141, 146 | 144.  96 rows: 8 of 4096 x 14336 FP8 381 | 384, at
@@ -1344,7 +1342,7 @@ MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& 
   // ahead: 8 of 4096 x 14336 FP4, 96 rows on average 278 | 328, 290 | 335.
   const int64_t tile_limit = p.H <= 2048 ? (third_tile(p) ? 160 : 128) : weights > kMoeStreamTwiceBytes && W1.dtype != MX_E2M1 ? 96 : 128;
   const bool can_tile = moe_tiles_issue(p, o) == nullptr && p.n <= p.E * tile_limit;
-  if (can_tile && p.n > p.E * kMoeTileFromRows) p.stream = false;
+  if (can_tile && moe_leaves_streaming(p.n, p.E, topk)) p.stream = false;
   p.tiles = can_tile && !p.stream;
   int64_t off = 0;
   auto take = [&](int64_t bytes) { const int64_t at = off; off += round256(bytes); return at; };

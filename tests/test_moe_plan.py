@@ -42,6 +42,7 @@ def test_gpu_tests_reach_the_row_tiles_that_they_are_about(load_once):
     assert all(tiled(T * topk / E, E, H, F, E2M1, H + 72, topk=topk) for T, H, F, E, topk, _ in g.CASES)
     assert [at(E2M1, *c)[0] for c in g.CASES[-2:]] == [128] * 2 and at(E2M1, *g.CASES[-1])[1] == 2
     assert all(at(w, *c) == "grouped" for w in (E4M3, E2M1) for c in g.GROUPED)
+    assert all(at(w, *c) == "streamed" for w in (E4M3, E2M1) for c in g.STREAMED)
     # both products of the layers with non-temporal weights; some of the second ones in ranges of K
     ranges = [form(2 * T / E, E, H, F, E2M1 if f else E4M3, H_out) for f, layers in g.ONCE.items() for T, H, F, E, H_out in layers]
     assert all(height == 64 for height, _ in ranges) and any(n > 1 for _, n in ranges[:2]) and any(n > 1 for _, n in ranges[2:])
@@ -59,9 +60,17 @@ def tiled(*a, **kw):
 def test_forms_by_rows_per_expert(w):
     for E, H, F in ((8, 2048, 7168), (8, 4096, 14336), (64, 1024, 1024)):
         assert form(24, E, H, F, w) == "streamed"
-        assert all(tiled(r, E, H, F, w) for r in (24.5, 32, 64, 96))
+        assert all(tiled(r, E, H, F, w) for r in (25.5, 32, 64, 96))
         assert form(161, E, H, F, w) == "grouped"
     assert form(64, 8, 2048, 7168, w, packed=False) == "grouped" and form(32, 8, 2048, 7168, w, packed=False) == "streamed"
+
+
+def test_streaming_ends_where_random_routing_gives_an_expert_more_than_32_rows():
+    for w in (E4M3, E2M1):
+        at = lambda E, topk: next(T * topk / E for T in range(1, 1000) if form(T * topk / E, E, 2048, 4096, w, topk=topk) != "streamed")
+        assert [at(E, E) for E in (1, 2, 4, 8)] == [33] * 4            # every expert has the same
+        assert [at(2, 1), at(4, 2), at(4, 1), at(8, 4), at(8, 2), at(8, 1)] == [27, 27, 25.5, 27, 25.5, 25]
+        assert at(16, 2) == 24.125 and at(64, 2) == 24.03125
 
 
 def test_padding_that_the_caller_asks_for():
