@@ -1335,12 +1335,18 @@ MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& 
   p.stream = p.n <= kMoeMaxIds && p.n <= p.E * rows && p.H % 128 == 0 && p.F % 128 == 0;
   // Row tiles where the weights would be streamed more than once (moe_leaves_streaming) and as long as the 256-row tiles, which need more
   // launches around them, are not ahead.
-  // Row tiles | 256-row tiles, random routing, 112 and 128 rows each: 8 of 4096 x 14336 FP4 276 | 322, 316 | 327; 16 of 4096 x 4096 FP8 256 | 278,
-  // 272 | 283; 32 of 4096 x 2048 FP8 265 | 290, 287 | 297; 16 of 3584 x 4096 FP8 233 | 232, 249 | 237 (28 columns for eight XCDs), FP4 159 | 175,
-  // 187 | 179; 64 of 4096 x 1024 FP4 220 | 248, 267 | 258; 32 of 1536 x 2048 FP8 136 | 141, 146 | 144.  96 rows: 8 of 4096 x 14336 FP8 381 | 384, at
-  // 112 and 128 no longer.  Where one expert has half of the copies or the popularity falls with the rank the row tiles are further
-  // ahead: 8 of 4096 x 14336 FP4, 96 rows on average 278 | 328, 290 | 335.
-  const int64_t tile_limit = p.H <= 2048 ? (third_tile(p) ? 160 : 128) : weights > kMoeStreamTwiceBytes && W1.dtype != MX_E2M1 ? 96 : 128;
+  // Row tiles | 256-row tiles, random routing, 120 and 128 rows each: 8 of 4096 x 7168 FP8 241 | 255, 244 | 259, FP4 160 | 191, 187 | 194; 8 of 4096 x
+  // 14336 FP4 294 | 317, 322 | 320; 32 of 4096 x 2048 FP8 278 | 303, 292 | 307, FP4 201 | 214, 222 | 218; 64 of 4096 x 1024 FP4 241 | 263, 270 | 268.  From
+  // 16 experts of 4096 or more on, the experts that get a second (third) tile are more than one round of 256 CUs: 16 of 2560 x 4096 FP8 202 | 194,
+  // 210 | 197; 16 of 3584 x 4096 FP8 247 | 244, 254 | 247; 16 of 4096 x 4096 FP8 268 | 289, 287 | 292, FP4 183 | 190, 212 | 198; 16 of 3584 x 8192 FP4
+  // 293 | 302, 370 | 306; 32 of 4096 x 4096 FP4 353 | 346, 391 | 353.  8 of 4096 x 14336 FP8, 96 rows: 381 | 384, at 112 and 128 no longer.
+  // Where one expert has half of the copies or the popularity falls with the rank the row tiles are further ahead: 8 of 4096 x 14336 FP4, 96 rows
+  // on average 278 | 328, 290 | 335.
+  const bool many = p.E >= 16 && (p.F >= 4096 || p.E * p.F > 65536);
+  const int64_t tile_limit = p.H <= 2048                                             ? (third_tile(p) ? 160 : 128)
+                             : weights > kMoeStreamTwiceBytes && W1.dtype != MX_E2M1 ? 96
+                             : many                                                  ? 120
+                                                                                     : 128;
   const bool can_tile = moe_tiles_issue(p, o) == nullptr && p.n <= p.E * tile_limit;
   if (can_tile && moe_leaves_streaming(p.n, p.E, topk)) p.stream = false;
   p.tiles = can_tile && !p.stream;

@@ -89,6 +89,13 @@ def test_row_tiles_of_three_per_expert():
         assert [tiled(r, *s, w) for r in (129, 160) for s in ahead + behind] == ([True] * len(ahead) + [False] * len(behind)) * 2
 
 
+def test_many_wide_experts_leave_row_tiles_before_most_have_a_second_one():
+    for E, H, F, w in ((16, 4096, 4096, E4M3), (16, 4096, 4096, E2M1), (16, 3584, 8192, E2M1), (32, 4096, 4096, E2M1)):
+        assert tiled(120, E, H, F, w) and form(121, E, H, F, w) == "grouped"
+    for E, H, F in ((8, 4096, 7168), (32, 4096, 2048), (64, 4096, 1024), (8, 2560, 14336)):
+        assert all(tiled(128, E, H, F, w) and form(129, E, H, F, w) == "grouped" for w in (E4M3, E2M1))
+
+
 def test_routing_by_one_workgroup_where_it_is_the_faster_one(tmp_path):
     cases = [(1, 1), (12288, 256), (12288, 257), (14336, 64), (12289, 65), (16384, 16), (16384, 17), (14337, 64), (16385, 1), (0, 8)]
     src = pathlib.Path(__file__).resolve().parent.parent / "cutile-python_amd" / "csrc"
