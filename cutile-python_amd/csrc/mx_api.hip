@@ -1316,15 +1316,36 @@ const char* moe_tiles_issue(const MoePlan& p, const mx_gemm_opts& o) {
   return nullptr;
 }
 
-// Layers of short rows that row tiles take up to 160 rows per expert, i.e. with three tiles of 64, instead of 128.  The 256-row tiles still have one,
-// and are ahead where these fill their rounds of 256 CUs.  us, row tiles | 256-row tiles, random routing, 136 and 160 rows each: taken here 8 experts
-// of 1024 x 7168 FP8 112 | 129, 115 | 125, FP4 87 | 112, 91 | 114; 32 of 1024 x 2048 FP8 (144) 120 | 126, 123 | 129; 16 of 1024 x 8192 FP8 (level) 202 | 198,
-// 216 | 209; 8 of 2048 x 8192 FP8 172 | 182, 178 | 186; 16 of 2048 x 4096 FP8 166 | 174, 176 | 181, FP4 134 | 144, 145 | 149; 64 of 2048 x 1024 FP8
-// 197 | 205, 212 | 217, FP4 171 | 173, 186 | 192.  Left to the 256-row tiles 8 of 2048 x 14336 FP8 283 | 261, 295 | 269, FP4 223 | 215, 232 | 224; 16
-// of 1280 x 8192 FP8 249 | 239, 267 | 248; 32 of 1536 x 2048 FP4 132 | 125, 141 | 131; 32 of 2048 x 2048 FP4 146 | 138, 156 | 145; 64 of
-// 1536 x 1024 FP4 154 | 148, 168 | 156 (12 columns for eight XCDs).
-bool third_tile(const MoePlan& p) {
-  return p.H <= 1024 || (p.E * p.F <= 65536 && (p.E <= 16 || (p.F <= 1024 && p.H_out % 1024 == 0)));
+// Rows per expert on average up to which the row tiles are mostly not behind the 256-row tiles, which need more launches around them.  Random routing
+// gives some experts one tile of 64 (FP4 and long rows 128) more than the average; where the layer is large that is at once another round of
+// workgroups, while 256-row tiles still have one each.  us, row tiles | 256-row tiles, random routing, at the rows in front:
+//   long rows, FP8 beyond 1 GB of weights.  96: 8 experts of 4096 x 14336 381 | 384 (at 112 and 128 no longer), 16 of 3072 x 8192 349 | 350, 64 of 3072 x
+//     2048 377 | 384, 16 of 4096 x 7168 392 | 373.  Larger ones, 64, 72 and 88: 16 of 4096 x 8192 392 | 400, 422 | 405, 438 | 414; 12 of 3584 x 14336 440 |
+//     473, 515 | 478, 512 | 488; 32 of 3584 x 8192 658 | 642, 714 | 653, 769 | 671; 32 of 4096 x 4096 (1.6 GB) 404 | 426, 432 | 432, 447 | 448
+//   long rows, many experts.  120 and 128: 16 of 2560 x 4096 FP8 202 | 194, 210 | 197; 16 of 4096 x 4096 FP8 268 | 289, 287 | 292, FP4 183 | 190, 212 | 198; 16 of
+//     3584 x 8192 FP4 293 | 302, 370 | 306; 32 of 4096 x 4096 FP4 353 | 346, 391 | 353.  Others: 8 of 4096 x 7168 FP8 241 | 255, 244 | 259, FP4 160 |
+//     191, 187 | 194; 8 of 4096 x 14336 FP4 294 | 317, 322 | 320; 32 of 4096 x 2048 FP8 278 | 303, 292 | 307, FP4 201 | 214, 222 | 218
+//   short rows, large layers.  72 and 88: 32 of 1536 x 8192 FP8 398 | 367, 397 | 378, FP4 297 | 289, 312 | 299; 32 of 2048 x 8192 FP8 452 | 441, 478 | 455; 64 of
+//     2048 x 4096 FP8 456 | 469, 470 | 484, FP4 345 | 353, 363 | 367; 64 of 1024 x 4096, 88 and 112: FP8 309 | 305, 320 | 321, FP4 249 | 242, 268 | 256.
+//     Medium ones of many experts, 120 and 128: 32 of 1536 x 4096 FP8 246 | 235, 265 | 239, FP4 198 | 191, 214 | 194; 128 of 1536 x 1024 FP8 295 | 288, 311 |
+//     292; 64 of 2048 x 2048 FP8 290 | 298, 306 | 303
+//   short rows, small layers, a third tile of 64.  136 and 160: 8 of 1024 x 7168 FP8 112 | 129, 115 | 125, FP4 87 | 112, 91 | 114; 32 of 1024 x 2048 FP8 (144) 120 |
+//     126, 123 | 129; 16 of 1024 x 8192 FP8 203 | 200, 215 | 209, FP4 165 | 173, 174 | 184; 8 of 2048 x 8192 FP8 172 | 182, 178 | 186; 16 of 2048 x 4096 FP8
+//     166 | 174, 176 | 181; 64 of 2048 x 1024 FP8 197 | 205, 212 | 217.  Not: 32 of 1024 x 4096 FP8 203 | 197, 213 | 205; 64 of 1024 x 2048 FP8 208 |
+//     200, 227 | 212; 8 of 2048 x 14336 FP8 283 | 261, 295 | 269, FP4 223 | 215, 232 | 224; 16 of 1280 x 8192 FP8 249 | 239, 267 | 248; 32 of 1536 x 2048
+//     FP4 132 | 125, 141 | 131; 32 of 2048 x 2048 FP4 146 | 138, 156 | 145; 64 of 1536 x 1024 FP4 154 | 148, 168 | 156 (12 columns for eight XCDs)
+// Where one expert has half of the copies or the popularity falls with the rank the row tiles are further ahead: 8 of 4096 x 14336 FP4, 96 rows
+// on average 278 | 328, 290 | 335.
+int64_t moe_tile_limit(const MoePlan& p, int64_t weight_bytes, bool fp4) {
+  const int64_t cols = p.E * p.F;
+  if (p.H > 2048) {
+    if (!fp4 && weight_bytes > kMoeStreamTwiceBytes) return weight_bytes > 1500000000 ? 64 : 96;
+    return p.E >= 16 && (p.F >= 4096 || cols > 65536) ? 120 : 128;
+  }
+  if (cols > 196608) return p.H <= 1024 ? 96 : 72;
+  if (p.H <= 1024 && cols <= 131072 && (p.E <= 16 || cols < 131072)) return 160;
+  if (cols <= 65536 && (p.E <= 16 || (p.F <= 1024 && p.H_out % 1024 == 0))) return 160;
+  return p.H > 1024 && p.E >= 32 && cols >= 131072 ? 120 : 128;
 }
 
 MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& W2, const mx_gemm_opts& o) {
@@ -1333,21 +1354,8 @@ MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& 
   const int64_t weights = p.E * (2 * p.F * p.H + p.H_out * p.F) / (W1.dtype == MX_E2M1 ? 2 : 1);   // bytes
   const int64_t rows = weights > kMoeStreamTwiceBytes ? 32 : kMoeStreamRows;
   p.stream = p.n <= kMoeMaxIds && p.n <= p.E * rows && p.H % 128 == 0 && p.F % 128 == 0;
-  // Row tiles where the weights would be streamed more than once (moe_leaves_streaming) and as long as the 256-row tiles, which need more
-  // launches around them, are not ahead.
-  // Row tiles | 256-row tiles, random routing, 120 and 128 rows each: 8 of 4096 x 7168 FP8 241 | 255, 244 | 259, FP4 160 | 191, 187 | 194; 8 of 4096 x
-  // 14336 FP4 294 | 317, 322 | 320; 32 of 4096 x 2048 FP8 278 | 303, 292 | 307, FP4 201 | 214, 222 | 218; 64 of 4096 x 1024 FP4 241 | 263, 270 | 268.  From
-  // 16 experts of 4096 or more on, the experts that get a second (third) tile are more than one round of 256 CUs: 16 of 2560 x 4096 FP8 202 | 194,
-  // 210 | 197; 16 of 3584 x 4096 FP8 247 | 244, 254 | 247; 16 of 4096 x 4096 FP8 268 | 289, 287 | 292, FP4 183 | 190, 212 | 198; 16 of 3584 x 8192 FP4
-  // 293 | 302, 370 | 306; 32 of 4096 x 4096 FP4 353 | 346, 391 | 353.  8 of 4096 x 14336 FP8, 96 rows: 381 | 384, at 112 and 128 no longer.
-  // Where one expert has half of the copies or the popularity falls with the rank the row tiles are further ahead: 8 of 4096 x 14336 FP4, 96 rows
-  // on average 278 | 328, 290 | 335.
-  const bool many = p.E >= 16 && (p.F >= 4096 || p.E * p.F > 65536);
-  const int64_t tile_limit = p.H <= 2048                                             ? (third_tile(p) ? 160 : 128)
-                             : weights > kMoeStreamTwiceBytes && W1.dtype != MX_E2M1 ? 96
-                             : many                                                  ? 120
-                                                                                     : 128;
-  const bool can_tile = moe_tiles_issue(p, o) == nullptr && p.n <= p.E * tile_limit;
+  // Row tiles where the weights would be streamed more than once and the 256-row tiles are not ahead.
+  const bool can_tile = moe_tiles_issue(p, o) == nullptr && p.n <= p.E * moe_tile_limit(p, weights, W1.dtype == MX_E2M1);
   if (can_tile && moe_leaves_streaming(p.n, p.E, topk)) p.stream = false;
   p.tiles = can_tile && !p.stream;
   int64_t off = 0;

@@ -89,11 +89,15 @@ def test_row_tiles_of_three_per_expert():
         assert [tiled(r, *s, w) for r in (129, 160) for s in ahead + behind] == ([True] * len(ahead) + [False] * len(behind)) * 2
 
 
-def test_many_wide_experts_leave_row_tiles_before_most_have_a_second_one():
-    for E, H, F, w in ((16, 4096, 4096, E4M3), (16, 4096, 4096, E2M1), (16, 3584, 8192, E2M1), (32, 4096, 4096, E2M1)):
-        assert tiled(120, E, H, F, w) and form(121, E, H, F, w) == "grouped"
-    for E, H, F in ((8, 4096, 7168), (32, 4096, 2048), (64, 4096, 1024), (8, 2560, 14336)):
-        assert all(tiled(128, E, H, F, w) and form(129, E, H, F, w) == "grouped" for w in (E4M3, E2M1))
+@pytest.mark.parametrize("E,H,F,limits", [
+    (8, 4096, 7168, (128, 128)), (8, 4096, 14336, (96, 128)), (16, 3072, 8192, (96, 120)), (16, 4096, 8192, (64, 120)), (12, 3584, 14336, (64, 128)),
+    (16, 4096, 4096, (120, 120)), (32, 4096, 2048, (128, 128)), (64, 4096, 1024, (128, 128)),      # long rows
+    (32, 1536, 8192, (72, 72)), (64, 2048, 4096, (72, 72)), (64, 1024, 4096, (96, 96)),            # short ones, large layers
+    (32, 1536, 4096, (120, 120)), (128, 1536, 1024, (120, 120)), (16, 2048, 8192, (128, 128)), (12, 1536, 14336, (128, 128)),
+    (16, 1024, 8192, (160, 160)), (32, 1024, 4096, (128, 128)), (64, 1024, 2048, (128, 128)), (32, 1024, 2048, (160, 160))])
+def test_rows_up_to_which_a_layer_has_row_tiles(E, H, F, limits):
+    for w, limit in zip((E4M3, E2M1), limits):
+        assert tiled(limit, E, H, F, w) and form(limit + 1, E, H, F, w) == "grouped"
 
 
 def test_routing_by_one_workgroup_where_it_is_the_faster_one(tmp_path):
