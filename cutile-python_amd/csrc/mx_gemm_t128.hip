@@ -42,9 +42,10 @@ constexpr int kScaleNative = 0, kScalePlain = 1, kScaleAny = 2;
 // A stage's requests go out between its MFMAs: all four waves' at once behind the barrier they keep the address unit busy for some
 // 500 cycles, the length of a stage's MFMAs, in which none of these is issued.  2048 x 2048 x 2048 FP8 15.2 -> 13.5 us, x 8192 43.0 ->
 // 40.9, FP4 26.9 -> 25.3, 200 x 14336 x 4096 24.3 -> 23.0; on tiles of 64 0 - 6 % (packed scales, 300 x 2000 x 7168 FP8
-// 18.4 -> 17.8, FP4 weights 16.8 -> 15.8, with two workgroups on a CU 1400 x 1400 x 8192 29.8 -> 28.8; plain ones 900 x 900 x 8192 21.1 -> 20.9).  Not with two stages, where a later request is a later stage (512 x 14336 x 4096 35.8 -> 39.6), nor beside the larger
-// tile's scales through registers (1111 x 2100 x 4032 21.6 -> 22.2), nor beside those of the smaller one where eight stages are in flight
-// for long (t128_any_spread).
+// 18.4 -> 17.8, FP4 weights 16.8 -> 15.8, with two workgroups on a CU 1400 x 1400 x 8192 29.8 -> 28.8; plain ones 900 x 900 x 8192 21.1 ->
+// 20.9).  Not with two stages, where a later request is a later stage (512 x 14336 x 4096 35.8 -> 39.6), nor beside the larger tile's
+// scales through registers (1111 x 2100 x 4032 21.6 -> 22.2), nor beside those of the smaller one where eight stages are in flight for long
+// (t128_any_spread).
 template <class C, int NS, int AS>
 constexpr bool kSpread = NS > 2 && !(AS == kScaleAny && C::BM == 128);
 

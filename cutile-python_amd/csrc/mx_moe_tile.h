@@ -1,4 +1,4 @@
-// Interface of the mixture-of-experts layer at medium sizes (mx_moe_tile.hip): experts of some 24 to 160 rows each.
+// Interface of the mixture-of-experts layer at medium sizes (mx_moe_tile.hip): experts of some 24 to 128 rows each.
 #pragma once
 #include "mx_common.h"
 

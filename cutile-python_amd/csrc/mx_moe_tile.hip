@@ -1,13 +1,13 @@
-// Mixture-of-experts layer at medium sizes: experts of some 16 to 256 rows.
+// Mixture-of-experts layer at medium sizes: experts of some 24 to 128 rows (which layers: moe_plan in mx_api.hip).
 //
 // Bound: reading the experts' weights once.  Streaming them past every few rows (mx_moe.hip) reads them again for each 32 rows;
 // the grouped 256 x 256 kernel has one workgroup per CU, whose two stages in flight ask for 4 TB/s of them, and needs slot
 // arrays, re-laid scales, a bf16 activation written and read and a launch that adds up the split last round around it.  Here:
-//   moe_tiles_kernel:       the routed copies of every expert, in tiles of 64;
-//   moe_tile_kernel<UP>:    64 rows x (64 gate + 64 up columns), SiLU(gate) * up and its MX quantisation in the epilogue;
-//   moe_tile_kernel<DOWN>:  64 rows x 128 columns, fp32, K in several ranges where there would be too few workgroups;
+//   moe_tiles_kernel:       the routed copies of every expert, in tiles of 64 (FP4 and long rows of W: 128, moe_tile_rows);
+//   moe_tile_kernel<UP>:    a tile x (64 gate + 64 up columns), SiLU(gate) * up and its MX quantisation in the epilogue;
+//   moe_tile_kernel<DOWN>:  a tile x 128 columns, fp32, K in several ranges where there would be too few workgroups;
 //   moe_combine_kernel:     adds up the ranges and a token's copies (mx_moe.hip).
-// A workgroup is four waves of 32 x 64 on the schedule of the 128 x 128 kernel (order of the requests and counted waits:
+// A workgroup is four waves of 32 x 64 (64 x 64) on the schedule of the 128 x 128 kernel (order of the requests and counted waits:
 // mx_t128_schedule.h): 80 KiB of LDS, two workgroups on a CU, so that one's start and output lie behind the other's stream and
 // together they have up to six stages of 16 KiB of weights in flight.  (Eight waves on 128 or 256 rows, one workgroup per CU and
 // four or three stages deep, leave start and output open: 8 experts of 2048 x 7168, 32 and 64 rows each, FP8 93 | 112 | 147 and

@@ -318,7 +318,7 @@ MX_API int mx_silu_mul_quantize(const mx_tensor* gate_up, mx_tensor* xq, mx_tens
  *   their copy.  The activation between the projections is E4M3, quantised by scale_mode as in mx_quantize.
  *   out [T,H_out] MX_F32 or MX_BF16, contiguous.
  * A few rows per expert stream the experts' weights (three launches in all, no slots and hence no tile_m).  Medium numbers
- * of rows (some 24 to 160 per expert, both scales MX_SCALE_NATIVE, H and F multiples of 128, tile_m 0) run on row tiles
+ * of rows (some 24 to 128 per expert, both scales MX_SCALE_NATIVE, H and F multiples of 128, tile_m 0) run on row tiles
  * of the library's own choice, with the activation in the first product's epilogue; the rest as alignment to opts->tile_m (0: 256), grouped
  * GEMM, activation, grouped GEMM and sum.  No host synchronisation.  Returns MX_ERR_LAYOUT, with nothing enqueued, for
  * operands that only the single entry points take (generic-kernel layouts).
