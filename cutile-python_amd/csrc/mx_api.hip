@@ -1348,7 +1348,7 @@ int64_t moe_tile_limit(const MoePlan& p, int64_t weight_bytes, bool fp4) {
   return p.H > 1024 && p.E >= 32 && cols >= 131072 ? 120 : 128;
 }
 
-MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& W2, const mx_gemm_opts& o) {
+MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& W2, const mx_gemm_opts& o, int32_t max_splits = 8) {
   MoePlan p = {};
   p.T = T; p.n = T * topk; p.E = W1.shape[0]; p.H = W1.shape[2]; p.F = W1.shape[1] / 2; p.H_out = W2.shape[1];
   const int64_t weights = p.E * (2 * p.F * p.H + p.H_out * p.F) / (W1.dtype == MX_E2M1 ? 2 : 1);   // bytes
@@ -1364,6 +1364,7 @@ MoePlan moe_plan(int64_t T, int32_t topk, const mx_tensor& W1, const mx_tensor& 
   p.qs = take(p.n * (p.F / 32));
   if (p.tiles) p.tile_m = moe_tile_rows(p.n, p.E, p.H, W1.dtype);
   p.splits = p.tiles ? moe_tile_splits(p.n, p.E, p.tile_m, p.H_out, p.F) : 1;
+  if (p.splits > max_splits) p.splits = max_splits;
   p.c3 = take(p.n * p.H_out * 4 * p.splits);
   if (p.tiles) {
     p.max_tiles = moe_tiles_max(p.n, p.E, p.tile_m);
@@ -1450,7 +1451,9 @@ int mx_moe_forward(const mx_tensor* X, const mx_tensor* Xs, const mx_tensor* W1,
   if (!why && 2 * F <= 128) why = "F is too small";
   if (!why && H_out <= 128) why = "H_out is too small";
   if (why) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: %s", why);
-  const MoePlan p = moe_plan(T, topk, *W1, *W2, o);
+  MoePlan p = moe_plan(T, topk, *W1, *W2, o);
+  // ranges of K are optional: fewer copies can ask for more of them than more copies do, and the room may have been laid out for the latter
+  while (p.splits > 1 && workspace_bytes < p.total) p = moe_plan(T, topk, *W1, *W2, o, p.splits - 1);
   if (!p.stream && !p.tiles && p.tile_m % 128 != 0) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: tile_m is not a multiple of 128");
   if (p.n * p.F >= ((int64_t)1 << 31)) return set_error(MX_ERR_LAYOUT, "mx_moe_forward: the activation spans 2 GiB or more");
   if (!workspace || workspace_bytes < p.total)

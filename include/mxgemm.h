@@ -322,6 +322,8 @@ MX_API int mx_silu_mul_quantize(const mx_tensor* gate_up, mx_tensor* xq, mx_tens
  * of the library's own choice, with the activation in the first product's epilogue; the rest as alignment to opts->tile_m (0: 256), grouped
  * GEMM, activation, grouped GEMM and sum.  No host synchronisation.  Returns MX_ERR_LAYOUT, with nothing enqueued, for
  * operands that only the single entry points take (generic-kernel layouts).
+ * Workspace: mx_moe_forward_workspace_bytes(), which includes the fp32 partial sums of the row tiles' second product split along K.
+ * They are optional: what is enough for T tokens is also enough for fewer, with fewer ranges of K where less is left for them.
  */
 MX_API int64_t mx_moe_forward_workspace_bytes(int64_t T, int32_t topk, const mx_tensor* W1, const mx_tensor* W2,
                                        const mx_gemm_opts* opts);

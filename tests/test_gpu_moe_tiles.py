@@ -1,10 +1,13 @@
 """GPU parity of the mixture-of-experts layer at medium sizes (row tiles, mx_moe_tile.hip): rows around the tiles of 64 and 128,
 experts with no row and with several tiles, ids outside the experts, odd K-steps and column counts, K in several ranges,
 non-temporal weights, and replays of a captured call."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
+from cutile_amd import _lib as L
 from oracle import mx_oracle as O
 from test_gpu_moe_forward import _elems, _scale
 
@@ -96,6 +99,36 @@ def test_moe_row_tiles_non_temporal(ct, dev, w_format, T, H, F, E, H_out):
     lone = run(bad.view(xs.dtype), p1, p2)
     others = [t for t in range(T) if t != 7]
     assert torch.equal(lone[others], got[others]) and not torch.isfinite(lone[7]).any()
+
+
+@pytest.mark.parametrize("w_format", [None, "e2m1"])
+def test_moe_row_tiles_in_less_room(ct, dev, w_format):
+    """A workspace that leaves room for fewer ranges of K than the layer would take, down to one: the same sums in another order."""
+    T, H, F, E, H_out, topk = 60, 128, 5248, 2, 200, 2
+    x, xs, w1, s1, w2, s2, wt, ids = _random_layer(ct, dev, T, H, F, E, H_out, w_format, 7)
+    p1, p2 = ct.pack_scales(s1, operand="b"), ct.pack_scales(s2, operand="b")
+    want = ct.cutile_moe_scaled(x, xs, w1, p1, w2, p2, wt, ids, out_dtype=torch.float32, w_format=w_format)
+    lib, out = ct.lib(), torch.empty((T, H_out), device=dev)
+    o = L.MxGemmOpts(struct_size=32, block_size=32, a_scale_layout=L.MX_SCALE_NATIVE, b_scale_layout=L.MX_SCALE_NATIVE)
+    wd = lambda w: L.desc(w.view(torch.uint8), L.MX_E2M1 if w_format else L.MX_E4M3, 2 if w_format else -1)
+    packed = [L.MxTensor(ptr=p.data.data_ptr(), dtype=L.MX_E8M0, ndim=3, shape=(E, 1, 1, 0), stride=(1, 1, 1, 0), packed_dim=-1) for p in (p1, p2)]
+    args = [L.desc(x.view(torch.uint8), L.MX_E4M3), L.desc(xs.view(torch.uint8), L.MX_E8M0), wd(w1), packed[0], wd(w2), packed[1]]
+    ref = [ctypes.byref(a) for a in args]
+    need = lib.mx_moe_forward_workspace_bytes(T, topk, ref[2], ref[4], ctypes.byref(o))
+    one = T * topk * H_out * 4
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    done = 0
+    for ranges_less in range(8):
+        out.fill_(float("nan"))
+        rc = lib.mx_moe_forward(*ref, wt.data_ptr(), ids.data_ptr(), 1, topk, ctypes.byref(L.desc(out, L.MX_F32)), 1, ctypes.byref(o),
+                                ws.data_ptr(), need - ranges_less * one, L.stream_ptr(dev))
+        if rc == L.MX_ERR_WORKSPACE:
+            break
+        assert rc == L.MX_OK, L.last_error()
+        # (fp32 sums of 5248 products in another order, 2^-24 for each of their some 16 roundings)
+        assert ((out - want).norm() / want.norm()).item() < 1e-6
+        done += 1
+    assert done > 2
 
 
 def test_moe_row_tiles_replayed(ct, dev):

@@ -4,6 +4,7 @@ import pathlib
 import subprocess
 
 import pytest
+import torch
 
 import cutile_amd
 from cutile_amd import _lib as L
@@ -87,6 +88,33 @@ def test_row_tiles_of_three_per_expert():
     for w in (E4M3, E2M1):
         assert all(tiled(128, *s, w) for s in ahead + behind)
         assert [tiled(r, *s, w) for r in (129, 160) for s in ahead + behind] == ([True] * len(ahead) + [False] * len(behind)) * 2
+
+
+@pytest.mark.parametrize("E,H,F,w", [(8, 1024, 14336, E4M3), (8, 2048, 7168, E2M1), (16, 2048, 4096, E4M3), (2, 4096, 14336, E2M1), (1, 1024, 14336, E4M3),
+                                     (64, 1024, 1024, E2M1)])
+def test_room_for_many_tokens_is_enough_for_fewer(E, H, F, w):
+    """A row-tiled layer asks for more ranges of K, and more room for their sums, with fewer rows; it makes do with fewer of them."""
+    if torch.cuda.is_available():
+        pytest.skip("these pointers are the host's")
+    lib, packed, topk = cutile_amd.lib(), 2 if w == E2M1 else -1, 1 if E == 1 else 2
+    p = (torch.zeros(1 << 16, dtype=torch.uint8).data_ptr() + 255) // 256 * 256
+    desc = lambda dtype, shape, strides, packed_dim=-1: L.MxTensor(ptr=p, dtype=dtype, ndim=len(shape), shape=shape + (0,) * (4 - len(shape)),
+                                                                   stride=strides + (0,) * (4 - len(strides)), packed_dim=packed_dim)
+    W = [desc(w, (E, n, k), (n * k, k, 1), packed) for n, k in ((2 * F, H), (H, F))]
+    o = L.MxGemmOpts(struct_size=32, block_size=32, a_scale_layout=L.MX_SCALE_NATIVE, b_scale_layout=L.MX_SCALE_NATIVE)
+    Ws = desc(L.MX_E8M0, (E, 1, 1), (1, 1, 1))
+    need = lambda T: lib.mx_moe_forward_workspace_bytes(T, topk, *(ctypes.byref(t) for t in W), ctypes.byref(o))
+
+    def forward(T, room):
+        X, Xs = desc(E4M3, (T, H), (H, 1)), desc(L.MX_E8M0, (T, H // 32), (H // 32, 1))
+        return lib.mx_moe_forward(*(ctypes.byref(t) for t in (X, Xs, W[0], Ws, W[1], Ws)), p, p, 0, topk,
+                                  ctypes.byref(desc(L.MX_F32, (T, H), (H, 1))), 1, ctypes.byref(o), p, room, None)
+    tokens = [t for t in range(1, 180 * E // topk, max(1, E // 2))]
+    for i, T in enumerate(tokens):
+        assert forward(T, min(need(t) for t in tokens[i:])) == L.MX_ERR_LAUNCH   # (no GPU here: everything before was in order)
+        f = form(T * topk / E, E, H, F, w, topk=topk)
+        ranges = 1 if isinstance(f, str) else f[1]
+        assert forward(T, need(T) - (ranges - 1) * T * topk * H * 4 - 1) == L.MX_ERR_WORKSPACE
 
 
 @pytest.mark.parametrize("E,H,F,limits", [
